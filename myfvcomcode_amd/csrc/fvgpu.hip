@@ -1589,10 +1589,14 @@ struct fvmlp {
   int bmax = 0;
   int step = 0;
   hipStream_t stream = nullptr;
-  float *X = nullptr, *Y = nullptr, *P = nullptr, *G = nullptr, *Mo = nullptr, *Ve = nullptr;
-  float *H1 = nullptr, *H2 = nullptr, *D1 = nullptr, *D2 = nullptr, *DO = nullptr, *loss = nullptr, *lsum = nullptr;
+  float *X = nullptr, *Y = nullptr, *P = nullptr, *Mo = nullptr, *Ve = nullptr;
+  float* G = nullptr;          // the batch's gradient, then its summed loss
+  float* part = nullptr;       // the workgroups' partials of it
   float* Yp = nullptr;
   int* idx = nullptr;
+  // pinned host staging of the small copies: the batch's indices, and G
+  int* hidx = nullptr;
+  float* hG = nullptr;
   MlpPacked* packed = nullptr;
   std::vector<void*> allocs;
 };
@@ -1608,20 +1612,22 @@ int malloc_mlp(fvmlp* t, T** p, size_t n) {
   return 0;
 }
 
-// Minibatch of one training step: fwd/bwd, weight gradients, loss sum.
-int mlp_batch(fvmlp* t, const int* didx, int B, float* loss_out) {
-  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3((B + 255) / 256), dim3(256), 0, t->stream, t->P, t->X, t->Y, didx, B, t->H1,
-                     t->H2, t->D1, t->D2, t->DO, t->loss);
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, t->stream, t->X, didx, B, t->H1, t->H2,
-                     t->D1, t->D2, t->DO, t->G);
-  hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, t->stream, t->loss, (long)B, t->lsum);
+// One minibatch of B samples, given by index (didx), drawn (draw.n > 0) or
+// the first B: its gradient and loss into G, and with step >= 1 the AdamW
+// step.
+int mlp_batch(fvmlp* t, const int* didx, MlpDraw draw, int B, int step, float lr, float wd) {
+  const int blocks = std::min((B + MLP_GRP - 1) / MLP_GRP, MLP_BLOCKS);
+  hipLaunchKernelGGL(k_mlp_batch, dim3(blocks), dim3(256), 0, t->stream, t->P, t->X, t->Y, didx, draw, B, t->part);
+  hipLaunchKernelGGL(k_mlp_update, dim3((MLP_PART + 31) / 32), dim3(256), 0, t->stream, t->part, blocks, t->G, t->P,
+                     t->Mo, t->Ve, step, lr, wd, 0.9f, 0.999f, 1e-8f);
   HIPCHK(hipGetLastError());
-  if (loss_out) {
-    float l = 0.0f;
-    HIPCHK(hipMemcpyAsync(&l, t->lsum, sizeof(float), hipMemcpyDeviceToHost, t->stream));
-    HIPCHK(hipStreamSynchronize(t->stream));
-    *loss_out = l / (float)B;
-  }
+  return 0;
+}
+
+// The last batch's gradient and summed loss, in the pinned copy.
+int mlp_fetch(fvmlp* t) {
+  HIPCHK(hipMemcpyAsync(t->hG, t->G, MLP_PART * sizeof(float), hipMemcpyDeviceToHost, t->stream));
+  HIPCHK(hipStreamSynchronize(t->stream));
   return 0;
 }
 }  // namespace
@@ -1636,13 +1642,16 @@ int fvmlp_create(int64_t n, const float* x, const float* y, int32_t bmax, fvmlp*
   fvmlp* t = new fvmlp();
   t->n = n;
   t->bmax = bmax;
-  const size_t bb = (size_t)bmax;
+  const size_t bb = (size_t)bmax, nb_ = std::min<size_t>((bb + MLP_GRP - 1) / MLP_GRP, MLP_BLOCKS);
   if (hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking) != hipSuccess ||
-      malloc_mlp(t, &t->X, (size_t)n * MLP_IN) || malloc_mlp(t, &t->Y, (size_t)n * MLP_OUT) ||
-      malloc_mlp(t, &t->P, MLP_NPARAM) || malloc_mlp(t, &t->G, MLP_NPARAM) || malloc_mlp(t, &t->Mo, MLP_NPARAM) ||
-      malloc_mlp(t, &t->Ve, MLP_NPARAM) || malloc_mlp(t, &t->H1, bb * MLP_H) || malloc_mlp(t, &t->H2, bb * MLP_H) ||
-      malloc_mlp(t, &t->D1, bb * MLP_H) || malloc_mlp(t, &t->D2, bb * MLP_H) || malloc_mlp(t, &t->DO, bb * MLP_OUT) ||
-      malloc_mlp(t, &t->loss, bb) || malloc_mlp(t, &t->lsum, 1) || malloc_mlp(t, &t->idx, bb) ||
+      hipHostMalloc((void**)&t->hidx, bb * sizeof(int), hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&t->hG, MLP_PART * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+    fvmlp_destroy(t);
+    return fail("fvmlp_create: stream or pinned staging");
+  }
+  if (malloc_mlp(t, &t->X, (size_t)n * MLP_IN) || malloc_mlp(t, &t->Y, (size_t)n * MLP_OUT) ||
+      malloc_mlp(t, &t->P, MLP_NPARAM) || malloc_mlp(t, &t->G, MLP_PART) || malloc_mlp(t, &t->Mo, MLP_NPARAM) ||
+      malloc_mlp(t, &t->Ve, MLP_NPARAM) || malloc_mlp(t, &t->part, nb_ * MLP_PART) || malloc_mlp(t, &t->idx, bb) ||
       malloc_mlp(t, &t->Yp, (size_t)n * MLP_OUT) || malloc_mlp(t, &t->packed, 1)) {
     fvmlp_destroy(t);
     return 1;
@@ -1654,9 +1663,10 @@ int fvmlp_create(int64_t n, const float* x, const float* y, int32_t bmax, fvmlp*
 }
 
 int fvmlp_set_params(fvmlp* t, const float* p) {
-  HIPCHK(hipMemcpy(t->P, p, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice));
-  HIPCHK(hipMemset(t->Mo, 0, MLP_NPARAM * sizeof(float)));
-  HIPCHK(hipMemset(t->Ve, 0, MLP_NPARAM * sizeof(float)));
+  HIPCHK(hipMemcpyAsync(t->P, p, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice, t->stream));
+  HIPCHK(hipMemsetAsync(t->Mo, 0, MLP_NPARAM * sizeof(float), t->stream));
+  HIPCHK(hipMemsetAsync(t->Ve, 0, MLP_NPARAM * sizeof(float), t->stream));
+  HIPCHK(hipStreamSynchronize(t->stream));
   t->step = 0;
   return 0;
 }
@@ -1675,13 +1685,15 @@ int fvmlp_grad(fvmlp* t, const int32_t* idx, int32_t B, float* grad, float* loss
   if (idx) {
     for (int b = 0; b < B; ++b)
       if (idx[b] < 0 || idx[b] >= t->n) return fail("fvmlp_grad: sample index out of range");
-    HIPCHK(hipMemcpy(t->idx, idx, (size_t)B * sizeof(int), hipMemcpyHostToDevice));
+    std::memcpy(t->hidx, idx, (size_t)B * sizeof(int));
+    HIPCHK(hipMemcpyAsync(t->idx, t->hidx, (size_t)B * sizeof(int), hipMemcpyHostToDevice, t->stream));
     didx = t->idx;
   } else if (B > t->n) {
     return fail("fvmlp_grad: batch larger than the sample set");
   }
-  if (mlp_batch(t, didx, B, loss)) return 1;
-  HIPCHK(hipMemcpy(grad, t->G, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost));
+  if (mlp_batch(t, didx, MlpDraw{0, 0}, B, 0, 0.0f, 0.0f) || mlp_fetch(t)) return 1;
+  std::memcpy(grad, t->hG, MLP_NPARAM * sizeof(float));
+  if (loss) *loss = t->hG[MLP_NPARAM] / (float)B;
   return 0;
 }
 
@@ -1689,21 +1701,19 @@ int fvmlp_train(fvmlp* t, int32_t steps, int32_t batch, int64_t ntrain, float lr
                 float* last_loss) {
   if (batch < 1 || batch > t->bmax) return fail("fvmlp_train: batch size outside [1, bmax]");
   if (ntrain < 1 || ntrain > t->n) return fail("fvmlp_train: ntrain outside [1, n]");
-  std::vector<int> hidx((size_t)batch);
-  uint64_t st = seed * 6364136223846793005ull + 1442695040888963407ull;
-  float l = 0.0f;
+  // seeded minibatches (PCG-style LCG, high bits), drawn on the device: the
+  // host only carries the generator's state from batch to batch, so the
+  // steps are enqueued without waiting for one another
+  unsigned long long st = seed * MLP_LCG_A + MLP_LCG_C;
   for (int it = 0; it < steps; ++it) {
-    for (int b = 0; b < batch; ++b) {   // seeded minibatch (PCG-style LCG, high bits)
-      st = st * 6364136223846793005ull + 1442695040888963407ull;
-      hidx[b] = (int)((st >> 33) % (uint64_t)ntrain);
-    }
-    HIPCHK(hipMemcpyAsync(t->idx, hidx.data(), (size_t)batch * sizeof(int), hipMemcpyHostToDevice, t->stream));
-    if (mlp_batch(t, t->idx, batch, it + 1 == steps ? &l : nullptr)) return 1;
     t->step += 1;
-    hipLaunchKernelGGL(k_adamw, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, t->stream, t->P, t->G, t->Mo, t->Ve,
-                       t->step, lr, wd, 0.9f, 0.999f, 1e-8f);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(t->stream));   // the host index buffer is reused
+    if (mlp_batch(t, nullptr, MlpDraw{st, (long)ntrain}, batch, t->step, lr, wd)) return 1;
+    st = mlp_lcg_skip(st, (unsigned long long)batch);
+  }
+  float l = 0.0f;
+  if (steps > 0) {
+    if (mlp_fetch(t)) return 1;
+    l = t->hG[MLP_NPARAM] / (float)batch;
   }
   if (last_loss) *last_loss = l;
   return 0;
@@ -1730,6 +1740,8 @@ void fvmlp_destroy(fvmlp* t) {
   if (!t) return;
   if (t->stream) (void)hipStreamSynchronize(t->stream);
   for (void* p : t->allocs) (void)hipFree(p);
+  if (t->hidx) (void)hipHostFree(t->hidx);
+  if (t->hG) (void)hipHostFree(t->hG);
   if (t->stream) (void)hipStreamDestroy(t->stream);
   delete t;
 }

@@ -45,10 +45,6 @@
 
 __device__ __forceinline__ float mlp_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float mlp_silu(float z) { return z * mlp_sigmoid(z); }
-__device__ __forceinline__ float mlp_dsilu(float z) {
-  const float s = mlp_sigmoid(z);
-  return s * (1.0f + z * (1.0f - s));
-}
 __device__ __forceinline__ float mlp_softplus(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 
 // ------------------------------------------------------------ features
@@ -116,132 +112,246 @@ __global__ __launch_bounds__(256) void k_closure_features(DevGrid g, IntArgs a, 
 }
 
 // ------------------------------------------------------------ training (FP32)
-// Forward pass and the per-sample deltas of one minibatch; thread per sample.
-// Stores H1, H2 (activations), D1, D2 (deltas) and DO (output deltas) for
-// the weight-gradient kernel, and the sample's loss.  D1 holds the
-// first-layer pre-activations until the deltas overwrite them.
-__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float* __restrict__ P, const float* __restrict__ X,
-                                                      const float* __restrict__ Y, const int* __restrict__ idx,
-                                                      int B, float* H1, float* H2, float* D1, float* D2, float* DO,
-                                                      float* loss) {
-  __shared__ float sP[MLP_NPARAM];
-  for (int t = threadIdx.x; t < MLP_NPARAM; t += blockDim.x) sP[t] = P[t];
-  __syncthreads();
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const long s = idx ? idx[b] : b;
-  float* h1g = H1 + (long)b * MLP_H;
-  float* d1g = D1 + (long)b * MLP_H;
-  float xin[5];
-#pragma unroll
-  for (int c = 0; c < 5; ++c) xin[c] = X[s * MLP_IN + c];
-  float h1[MLP_H];
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) {
-    float acc = sP[MLP_OFF_B1 + j];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) acc += sP[MLP_OFF_W1 + j * 5 + c] * xin[c];
-    d1g[j] = acc;
-    h1[j] = mlp_silu(acc);
-    h1g[j] = h1[j];
+// One training step is two kernels.  k_mlp_batch takes groups of
+// MLP_GRP = 32 samples through the forward pass, the loss, the backward pass
+// and the group's share of the gradient without leaving LDS: the three
+// 64x64 products (H1*W2', D2*W2 and D2'*H1) and the narrow ones (D1, D2 and
+// H2 against the inputs, ones and output deltas, packed as one 16-column
+// operand) run on the FP32 matrix cores (v_mfma_f32_16x16x4_f32: FP32
+// operands and accumulation).  Each workgroup adds its groups' gradients in
+// registers and writes one partial vector; k_mlp_update sums the partials in
+// a fixed order and, when training, takes the AdamW step.  Bound: latency of
+// a step's two launches (the arithmetic is 0.2 GFLOP at 8,192 samples).  A
+// group of 32 gives one workgroup per CU at the 8,192-sample batch.
+// Measured at 8,192 samples: 2450 us a step with one thread per parameter
+// summing over the batch and the deltas in HBM, 27 us now.
+#define MLP_GRP 32
+#define MLP_LD 68                 // LDS row of 64 hidden units: rows 4 banks apart
+#define MLP_LX 20                 // LDS row of the packed narrow operand (16 columns)
+#define MLP_PART (MLP_NPARAM + 1) // a workgroup's partial: gradient, then loss
+#define MLP_BLOCKS 256            // most partials of a batch
+
+typedef float mlp_f32x4 __attribute__((ext_vector_type(4)));
+
+// A minibatch drawn from samples [0, n): sample b is the high 31 bits of the
+// (b+1)-th state after `state` of the 64-bit LCG, modulo n.  n = 0: none.
+#define MLP_LCG_A 6364136223846793005ull
+#define MLP_LCG_C 1442695040888963407ull
+struct MlpDraw { unsigned long long state; long n; };
+
+// The LCG's state `steps` steps on (composition by doubling).
+__host__ __device__ inline unsigned long long mlp_lcg_skip(unsigned long long st, unsigned long long steps) {
+  unsigned long long a = MLP_LCG_A, c = MLP_LCG_C;
+  for (; steps; steps >>= 1) {
+    if (steps & 1) st = a * st + c;
+    c = (a + 1) * c;
+    a = a * a;
   }
-  float z2[MLP_H];
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) {
-    float acc = sP[MLP_OFF_B2 + j];
-#pragma unroll
-    for (int c = 0; c < MLP_H; ++c) acc += sP[MLP_OFF_W2 + j * MLP_H + c] * h1[c];
-    z2[j] = acc;
-  }
-  float o0 = sP[MLP_OFF_B3], o1 = sP[MLP_OFF_B3 + 1];
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) {
-    const float h2 = mlp_silu(z2[j]);
-    H2[(long)b * MLP_H + j] = h2;
-    o0 += sP[MLP_OFF_W3 + j] * h2;
-    o1 += sP[MLP_OFF_W3 + MLP_H + j] * h2;
-  }
-  float dout[MLP_OUT], l = 0.0f;
-  const float oo[MLP_OUT] = {o0, o1};
-#pragma unroll
-  for (int c = 0; c < MLP_OUT; ++c) {
-    const float k = mlp_softplus(oo[c]) + MLP_KEPS;
-    const float r = logf(k) - logf(fmaxf(Y[s * 2 + c], MLP_KEPS));
-    l += r * r;
-    dout[c] = 2.0f * r / k * mlp_sigmoid(oo[c]) / (float)B;   // d(mean loss)/do
-    DO[(long)b * MLP_OUT + c] = dout[c];
-  }
-  loss[b] = l;
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) {
-    const float acc = sP[MLP_OFF_W3 + j] * dout[0] + sP[MLP_OFF_W3 + MLP_H + j] * dout[1];
-    z2[j] = acc * mlp_dsilu(z2[j]);          // z2 now holds delta2
-    D2[(long)b * MLP_H + j] = z2[j];
-  }
-#pragma unroll
-  for (int j = 0; j < MLP_H; ++j) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int c = 0; c < MLP_H; ++c) acc += sP[MLP_OFF_W2 + c * MLP_H + j] * z2[c];
-    d1g[j] = acc * mlp_dsilu(d1g[j]);
-  }
+  return st;
 }
 
-// Gradient of every parameter over the minibatch, one thread per parameter
-// (a fixed-order sum over the samples, so the result is deterministic).
-__global__ void k_mlp_wgrad(const float* __restrict__ X, const int* __restrict__ idx, int B,
-                            const float* __restrict__ H1, const float* __restrict__ H2,
-                            const float* __restrict__ D1, const float* __restrict__ D2,
-                            const float* __restrict__ DO, float* G) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
-  float acc = 0.0f;
-  if (p < MLP_OFF_B1) {
-    const int j = (p - MLP_OFF_W1) / 5, c = (p - MLP_OFF_W1) % 5;
-    for (int b = 0; b < B; ++b) acc += D1[(long)b * MLP_H + j] * X[(long)(idx ? idx[b] : b) * MLP_IN + c];
-  } else if (p < MLP_OFF_W2) {
-    const int j = p - MLP_OFF_B1;
-    for (int b = 0; b < B; ++b) acc += D1[(long)b * MLP_H + j];
-  } else if (p < MLP_OFF_B2) {
-    const int j = (p - MLP_OFF_W2) / MLP_H, c = (p - MLP_OFF_W2) % MLP_H;
-    for (int b = 0; b < B; ++b) acc += D2[(long)b * MLP_H + j] * H1[(long)b * MLP_H + c];
-  } else if (p < MLP_OFF_W3) {
-    const int j = p - MLP_OFF_B2;
-    for (int b = 0; b < B; ++b) acc += D2[(long)b * MLP_H + j];
-  } else if (p < MLP_OFF_B3) {
-    const int c = (p - MLP_OFF_W3) / MLP_H, j = (p - MLP_OFF_W3) % MLP_H;
-    for (int b = 0; b < B; ++b) acc += DO[(long)b * MLP_OUT + c] * H2[(long)b * MLP_H + j];
-  } else {
-    const int c = p - MLP_OFF_B3;
-    for (int b = 0; b < B; ++b) acc += DO[(long)b * MLP_OUT + c];
-  }
-  G[p] = acc;
-}
-
-// Sum of n values in a fixed order by one workgroup of 256 threads.
-__global__ void k_sum_fixed(const float* v, long n, float* out) {
-  __shared__ float sh[256];
-  float acc = 0.0f;
-  for (long t = threadIdx.x; t < n; t += 256) acc += v[t];
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+__global__ __launch_bounds__(256) void k_mlp_batch(const float* __restrict__ P, const float* __restrict__ X,
+                                                   const float* __restrict__ Y, const int* __restrict__ idx,
+                                                   MlpDraw draw, int B, float* __restrict__ part) {
+  __shared__ float sW2[MLP_H * MLP_LD], sH1[MLP_GRP * MLP_LD], sG1[MLP_GRP * MLP_LD], sH2[MLP_GRP * MLP_LD],
+      sD1[MLP_GRP * MLP_LD], sD2[MLP_GRP * MLP_LD];
+  __shared__ float sW1[MLP_H * 5], sB1[MLP_H], sW3[MLP_OUT * MLP_H], sX[MLP_GRP * MLP_LX], sY[MLP_GRP * MLP_OUT];
+  __shared__ float sRed[2][MLP_GRP * MLP_OUT];
+  const int t = threadIdx.x, w = t >> 6, l = t & 63, col = l & 15, kq = l >> 4;
+  for (int q = t; q < MLP_H * MLP_H; q += 256) sW2[(q >> 6) * MLP_LD + (q & 63)] = P[MLP_OFF_W2 + q];
+  for (int q = t; q < MLP_H * 5; q += 256) sW1[q] = P[MLP_OFF_W1 + q];
+  if (t < MLP_H) sB1[t] = P[MLP_OFF_B1 + t];
+  if (t < MLP_OUT * MLP_H) sW3[t] = P[MLP_OFF_W3 + t];
+  const int j2 = 16 * w + col;                      // this lane's column of the 64-wide products
+  const float b2 = P[MLP_OFF_B2 + j2];
+  const float w30 = P[MLP_OFF_W3 + j2], w31 = P[MLP_OFF_W3 + MLP_H + j2];
+  const float b3 = P[MLP_OFF_B3 + (t & 1)];
+  mlp_f32x4 gW2[4] = {}, gW1 = {}, gB2 = {}, gW3 = {};
+  float lacc = 0.0f, dacc = 0.0f;
+  for (int g0 = blockIdx.x * MLP_GRP; g0 < B; g0 += gridDim.x * MLP_GRP) {
+    if (t < MLP_GRP) {
+      const int b = g0 + t;
+      float4 xa = make_float4(0.f, 0.f, 0.f, 0.f);
+      float x4 = 0.0f;
+      float2 y = make_float2(1.f, 1.f);
+      if (b < B) {
+        long s = b;
+        if (draw.n > 0) {
+          const unsigned r = (unsigned)(mlp_lcg_skip(draw.state, (unsigned long long)b + 1) >> 33);
+          s = draw.n < 0x80000000l ? (long)(r % (unsigned)draw.n) : (long)r;
+        } else if (idx) {
+          s = idx[b];
+        }
+        xa = *(const float4*)(X + s * MLP_IN);
+        x4 = X[s * MLP_IN + 4];
+        y = *(const float2*)(Y + s * MLP_OUT);
+      }
+      float* xr = sX + t * MLP_LX;
+      xr[0] = xa.x; xr[1] = xa.y; xr[2] = xa.z; xr[3] = xa.w; xr[4] = x4; xr[5] = 1.0f;
+#pragma unroll
+      for (int c = 6; c < 16; ++c) xr[c] = 0.0f;
+      sY[2 * t] = y.x;
+      sY[2 * t + 1] = y.y;
+    }
     __syncthreads();
+    {   // layer 1: sample t%32, hidden units 8*(t/32) .. +7
+      const int b = t & 31, j0 = 8 * (t >> 5);
+      const float* xr = sX + b * MLP_LX;
+      float h[8], gr[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        float z = sB1[j0 + q];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) z += sW1[(j0 + q) * 5 + c] * xr[c];
+        const float sg = mlp_sigmoid(z);
+        h[q] = z * sg;
+        gr[q] = sg * (1.0f + z * (1.0f - sg));
+      }
+      float4* ph = (float4*)(sH1 + b * MLP_LD + j0);
+      float4* pg = (float4*)(sG1 + b * MLP_LD + j0);
+      ph[0] = make_float4(h[0], h[1], h[2], h[3]); ph[1] = make_float4(h[4], h[5], h[6], h[7]);
+      pg[0] = make_float4(gr[0], gr[1], gr[2], gr[3]); pg[1] = make_float4(gr[4], gr[5], gr[6], gr[7]);
+    }
+    __syncthreads();
+    // layer 2: rows = samples (two tiles), columns = hidden units 16w..16w+15
+    float g2[2][4];
+    {
+      mlp_f32x4 z[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) z[m] = mlp_f32x4{b2, b2, b2, b2};
+#pragma unroll
+      for (int s = 0; s < MLP_H / 4; ++s) {
+        const float wb = sW2[j2 * MLP_LD + 4 * s + kq];
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          z[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sH1[(16 * m + col) * MLP_LD + 4 * s + kq], wb, z[m], 0, 0, 0);
+      }
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float sg = mlp_sigmoid(z[m][r]);
+          sH2[(16 * m + 4 * kq + r) * MLP_LD + j2] = z[m][r] * sg;
+          g2[m][r] = sg * (1.0f + z[m][r] * (1.0f - sg));
+        }
+    }
+    __syncthreads();
+    {   // layer 3, loss and output deltas: sample t/8, eighth t%8 of the hidden units
+      const int b = t >> 3, p = t & 7;
+      float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float h = sH2[b * MLP_LD + 8 * p + q];
+        o0 += sW3[8 * p + q] * h;
+        o1 += sW3[MLP_H + 8 * p + q] * h;
+      }
+#pragma unroll
+      for (int m = 1; m < 8; m <<= 1) {
+        o0 += __shfl_xor(o0, m);
+        o1 += __shfl_xor(o1, m);
+      }
+      if (p < MLP_OUT && g0 + b < B) {
+        const float o = (p ? o1 : o0) + b3;
+        const float k = mlp_softplus(o) + MLP_KEPS;
+        const float r = logf(k) - logf(fmaxf(sY[2 * b + p], MLP_KEPS));
+        const float d = 2.0f * r / k * mlp_sigmoid(o) / (float)B;   // d(mean loss)/do
+        sX[b * MLP_LX + 6 + p] = d;
+        lacc += r * r;
+        dacc += d;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int b = 16 * m + 4 * kq + r;
+        sD2[b * MLP_LD + j2] = (w30 * sX[b * MLP_LX + 6] + w31 * sX[b * MLP_LX + 7]) * g2[m][r];
+      }
+    __syncthreads();
+    {   // deltas of layer 1: rows = samples, columns = first-layer units 16w..16w+15
+      mlp_f32x4 d[2] = {};
+#pragma unroll
+      for (int s = 0; s < MLP_H / 4; ++s) {
+        const float wb = sW2[(4 * s + kq) * MLP_LD + j2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          d[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sD2[(16 * m + col) * MLP_LD + 4 * s + kq], wb, d[m], 0, 0, 0);
+      }
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int q = (16 * m + 4 * kq + r) * MLP_LD + j2;
+          sD1[q] = d[m][r] * sG1[q];
+        }
+    }
+    __syncthreads();
+    // gradient: rows = hidden units 16w..16w+15, summed over the group's samples
+#pragma unroll
+    for (int s = 0; s < MLP_GRP / 4; ++s) {
+      const int b = 4 * s + kq, q = b * MLP_LD + 16 * w + col;
+      const float bx = sX[b * MLP_LX + col], d2 = sD2[q];
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        gW2[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(d2, sH1[b * MLP_LD + 16 * n + col], gW2[n], 0, 0, 0);
+      gB2 = __builtin_amdgcn_mfma_f32_16x16x4f32(d2, bx, gB2, 0, 0, 0);
+      gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(sD1[q], bx, gW1, 0, 0, 0);
+      gW3 = __builtin_amdgcn_mfma_f32_16x16x4f32(sH2[q], bx, gW3, 0, 0, 0);
+    }
+    __syncthreads();   // the next group overwrites the LDS operands
   }
-  if (threadIdx.x == 0) out[0] = sh[0];
+  float* out = part + (long)blockIdx.x * MLP_PART;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int j = 16 * w + 4 * kq + r;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) out[MLP_OFF_W2 + j * MLP_H + 16 * n + col] = gW2[n][r];
+    if (col < 5) out[MLP_OFF_W1 + j * 5 + col] = gW1[r];
+    if (col == 5) {
+      out[MLP_OFF_B1 + j] = gW1[r];
+      out[MLP_OFF_B2 + j] = gB2[r];
+    }
+    if (col == 6 || col == 7) out[MLP_OFF_W3 + (col - 6) * MLP_H + j] = gW3[r];
+  }
+  if ((t & 7) < MLP_OUT) {
+    sRed[0][(t >> 3) * MLP_OUT + (t & 7)] = dacc;
+    sRed[1][(t >> 3) * MLP_OUT + (t & 7)] = lacc;
+  }
+  __syncthreads();
+  if (t < 3) {   // the output biases' gradients and the loss
+    float acc = 0.0f;
+    for (int q = 0; q < MLP_GRP; ++q)
+      acc += t < 2 ? sRed[0][q * MLP_OUT + t] : sRed[1][q * MLP_OUT] + sRed[1][q * MLP_OUT + 1];
+    out[t < 2 ? MLP_OFF_B3 + t : MLP_NPARAM] = acc;
+  }
 }
 
-// AdamW step on the FP32 master weights (decoupled weight decay on the
-// weight matrices, not the biases).
-__global__ void k_adamw(float* P, const float* G, float* Mo, float* Ve, int step, float lr, float wd,
-                        float b1, float b2, float eps) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
+// Sums the batch's partials (the gradient into G[0, NPARAM), the loss into
+// G[NPARAM]) in a fixed order: 32 parameters x 8 slices of the partials per
+// workgroup, the slices combined in order.  With step >= 1 also the AdamW
+// step on the FP32 master weights (decoupled weight decay on the weight
+// matrices, not the biases).
+__global__ __launch_bounds__(256) void k_mlp_update(const float* __restrict__ part, int nblk, float* G, float* P,
+                                                    float* Mo, float* Ve, int step, float lr, float wd, float b1,
+                                                    float b2, float eps) {
+  __shared__ float sh[8][32];
+  const int q = threadIdx.x & 31, sl = threadIdx.x >> 5;
+  const int p = blockIdx.x * 32 + q;
+  float acc = 0.0f;
+  if (p < MLP_PART)
+#pragma unroll 8
+    for (int b = sl; b < nblk; b += 8) acc += part[(long)b * MLP_PART + p];
+  sh[sl][q] = acc;
+  __syncthreads();
+  if (sl != 0 || p >= MLP_PART) return;
+#pragma unroll
+  for (int s = 1; s < 8; ++s) acc += sh[s][q];
+  G[p] = acc;
+  if (step < 1 || p >= MLP_NPARAM) return;
   const bool is_bias = (p >= MLP_OFF_B1 && p < MLP_OFF_W2) || (p >= MLP_OFF_B2 && p < MLP_OFF_W3) || p >= MLP_OFF_B3;
-  const float g = G[p];
-  const float m = b1 * Mo[p] + (1.0f - b1) * g;
-  const float v = b2 * Ve[p] + (1.0f - b2) * g * g;
+  const float m = b1 * Mo[p] + (1.0f - b1) * acc;
+  const float v = b2 * Ve[p] + (1.0f - b2) * acc * acc;
   Mo[p] = m;
   Ve[p] = v;
   const float mh = m / (1.0f - powf(b1, (float)step)), vh = v / (1.0f - powf(b2, (float)step));
