@@ -448,8 +448,8 @@ class DeviceModel:
 
     def set_concurrency(self, mode):
         """Independent chains of the step on a second stream, a bit mask:
-        1 the T/S and Q2/Q2L pairs, 2 the 2-D stage pair (default 3, both),
-        0 every chain on the main stream (per-kernel timing)."""
+        1 the T/S and Q2/Q2L pairs (2 has no effect; default 3), 0 every
+        chain on the main stream (per-kernel timing)."""
         _check(gpu_lib(), gpu_lib().fvgpu_set_concurrency(self._h, int(mode)), "fvgpu_set_concurrency")
 
     def closure_fallbacks(self):

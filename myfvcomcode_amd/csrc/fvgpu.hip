@@ -10,7 +10,8 @@
 //  * every scatter loop of the reference becomes a gather through sorted
 //    CSR lists (node -> control-volume sub-edges, element -> edges), so no
 //    atomics are used and sums are formed in the reference's order;
-//  * the RK stages of the 2-D mode ping-pong between three buffer sets with
+//  * an RK stage of the 2-D mode is one launch over compact element tiles;
+//    the stages ping-pong between three buffer sets with
 //    the fourth stage written in place over the RK base (pointwise reads
 //    only), so the state returns to fixed buffers after every external step
 //    and one internal step can be captured as a replayable hipGraph;
@@ -86,13 +87,12 @@ struct fvgpu_handle {
   int device = 0;
   int cu_count = 0;       // compute units of the device
   hipStream_t stream = nullptr;
-  // Independent chains of the step (the 2-D elevation and edge terms, the
-  // T and S passes, the Q2 and Q2L advection) fork onto stream2 and join
-  // back; both streams have the default priority.  `cur` is the stream the
+  // Independent chains of the step (the T and S passes, the Q2 and Q2L
+  // advection) fork onto stream2 and join back; both streams have the default priority.  `cur` is the stream the
   // launch macros enqueue on.
   hipStream_t stream2 = nullptr, cur = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  int concurrent = 3;     // bit 0: 3-D chain pairs, bit 1: the 2-D stage pair on stream2
+  int concurrent = 3;     // bit 0: the 3-D chain pairs on stream2
   // CV records then face fluxes in two launches (1) or one fused launch
   // (0), for ADV_T/ADV_S and for ADV_Q
   int two_phase_ts = 0, two_phase_q = 0;
@@ -102,14 +102,17 @@ struct fvgpu_handle {
   double *wu0 = nullptr, *wv0 = nullptr, *wu1 = nullptr, *wv1 = nullptr, *ws2x = nullptr, *ws2y = nullptr;
   int wind_varies = 0;
   DevGrid g{};
+  const DevGrid* dg = nullptr;   // its device copy
   std::vector<void*> allocs;
   // device state
   DevClock* clk = nullptr;
   Ext2DState ext[3];      // ext[0] = state / RK base, ext[1], ext[2] stage buffers
   IntArgs ia{};
   IntArgs ib{};           // ia with its own scratch, for the chain on stream2
-  double *xflux_obcn = nullptr, *fobn = nullptr;
-  double* phi = nullptr;  // per sub-edge EXTEL term of the 2-D stage input, element-major
+  double* phi[2] = {};    // per sub-edge EXTEL terms of a 2-D stage's input and output, element-major
+  double* elrk = nullptr; // the RK base elevation of stages 2-4
+  double* own2d = nullptr;   // block-order constants of the external steps (ExtArgs::own2d)
+  ExtClock* ec = nullptr; // clocks of the external steps (ISPLIT of them, at least one)
   double* ens_buf = nullptr;  // X5 and member offsets of fvgpu_ensemble_update
   // graph
   hipGraph_t graph = nullptr;
@@ -137,12 +140,14 @@ struct fvgpu_handle {
 
 namespace {
 
+// Device memory of n values, zero, or a copy of src where given.
 template <typename T>
-int dalloc(fvgpu_handle* h, T** p, size_t n) {
+int dalloc(fvgpu_handle* h, T** p, size_t n, const T* src = nullptr) {
   void* q = nullptr;
   HIPCHK(hipMalloc(&q, (n ? n : 1) * sizeof(T)));
-  HIPCHK(hipMemset(q, 0, (n ? n : 1) * sizeof(T)));
   h->allocs.push_back(q);
+  if (n && src) HIPCHK(hipMemcpy(q, src, n * sizeof(T), hipMemcpyHostToDevice));
+  else HIPCHK(hipMemset(q, 0, (n ? n : 1) * sizeof(T)));
   *p = (T*)q;
   return 0;
 }
@@ -150,16 +155,14 @@ int dalloc(fvgpu_handle* h, T** p, size_t n) {
 template <typename T>
 int dupload(fvgpu_handle* h, const T** p, const T* src, size_t n) {
   T* q = nullptr;
-  if (dalloc(h, &q, n)) return 1;
-  if (n) HIPCHK(hipMemcpy(q, src, n * sizeof(T), hipMemcpyHostToDevice));
+  if (dalloc(h, &q, n, src)) return 1;
   *p = q;
   return 0;
 }
 
 int dupload_rw(fvgpu_handle* h, double** p, const double* src, size_t n) {
-  if (dalloc(h, p, n)) return 1;
+  if (dalloc(h, p, n, src)) return 1;
   h->rw.push_back({(void*)*p, (n ? n : 1) * sizeof(double)});
-  if (n && src) HIPCHK(hipMemcpy(*p, src, n * sizeof(double), hipMemcpyHostToDevice));
   return 0;
 }
 
@@ -247,9 +250,9 @@ int block_of(const fvgpu_handle* h, const char* name) {
 // Fork: work enqueued on stream2 after this waits for everything enqueued
 // on the main stream so far.  Join: the main stream waits for stream2.
 // Under graph capture the events become dependency edges of the graph.
-// `what` is the concurrency bit of the pair (FV_CONC_3D or FV_CONC_2D);
-// with that bit clear both chains go to the main stream in turn.
-enum { FV_CONC_3D = 1, FV_CONC_2D = 2 };
+// `what` is the concurrency bit of the pair; with that bit clear both chains
+// go to the main stream in turn.
+enum { FV_CONC_3D = 1 };
 void fork_streams(fvgpu_handle* h, int what) {
   if (!(h->concurrent & what)) return;
   (void)hipEventRecord(h->ev_fork, h->stream);
@@ -267,15 +270,17 @@ void on_stream1(fvgpu_handle* h) { h->cur = h->stream; }
 const double ALPHA_RK[5] = {0.0, 0.2500, 1.0 / 3.0, 0.5000, 1.0};
 
 // ------------------------------------------------------------- the steps
-ExtArgs make_ext_args(fvgpu_handle* h, int K, const Ext2DState& cur, const Ext2DState& nxt) {
+// Arguments of the RK stage K (0: the INT form) of the external step whose
+// clock is ec.
+ExtArgs make_ext_args(fvgpu_handle* h, int K, const Ext2DState& cur, const Ext2DState& nxt, const ExtClock* ec) {
   ExtArgs a{};
   a.cur = cur;
   a.base = h->ext[0];
   a.nxt = nxt;
   a.K = K;
   a.alpha = ALPHA_RK[K];
-  a.xflux_obcn = h->xflux_obcn;
-  a.fobn = h->fobn;
+  a.elrk = K <= 1 ? h->ext[0].el : h->elrk;
+  a.elrk_copy = K == 1 ? h->elrk : nullptr;
   a.uard_obcn = h->ia.uard_obcn;
   a.egf = h->ia.egf;
   a.fluxobn = h->ia.fluxobn;
@@ -283,45 +288,37 @@ ExtArgs make_ext_args(fvgpu_handle* h, int K, const Ext2DState& cur, const Ext2D
   a.vard = h->ia.vard;
   a.adx2d = h->ia.adx2d; a.ady2d = h->ia.ady2d; a.drx2d = h->ia.drx2d; a.dry2d = h->ia.dry2d;
   a.wubot = h->ia.wubot; a.wvbot = h->ia.wvbot;
+  a.own2d = h->own2d;
   a.qdis = h->ia.qdis;
-  a.ef = h->ia.ef2;
-  a.elij = h->ia.elij2;
-  a.phi = h->phi;
+  // stage K reads the terms that the INT form or k_ext_begin (phi[0]) or the
+  // previous stage left and writes the other buffer; four stages later they
+  // are in phi[0] again
+  a.phi = h->phi[(K + 1) & 1];
+  a.phi_next = K == 0 ? h->phi[0] : h->phi[K & 1];
   a.ws2x = h->wind_varies ? h->ws2x : h->g.wsx;
   a.ws2y = h->wind_varies ? h->ws2y : h->g.wsy;
+  a.ec = ec;
   a.clk = h->clk;
   a.elm1 = h->ia.elm1;
   a.elm2 = h->ia.elm2;
   return a;
 }
 
-// `fresh`: the 2-D state may have changed since the last stage (first
-// external step of an internal step, or a direct EXTERNAL_STEP call), so
-// the EXTEL terms are formed from it first; otherwise the last stage's
-// k_ext_momentum left them.
+// One EXTERNAL_STEP; phi[0] holds the EXTEL terms of the 2-D state, ec its
+// clock.
 template <typename FT>
-void enqueue_external_step_t(fvgpu_handle* h, int iext, bool fresh) {
+void enqueue_external_step_t(fvgpu_handle* h, int iext, const ExtClock* ec) {
   const DevGrid& g = h->g;
-  LAUNCH("ext_clock", k_ext_clock, 1, 64, h->clk, iext);
-  if (fresh) TLAUNCH("ext_phi", k_ext_phi, g.N, g, h->ext[0].ua, h->ext[0].va, h->ext[0].d1, h->phi);
   if (h->wind_varies)
     TLAUNCH("ext_wind", k_ext_wind, g.N, g, h->wu0, h->wv0, h->wu1, h->wv1, iext, h->ws2x, h->ws2y);
   // stage buffers: 1: A->B, 2: B->C, 3: C->B, 4: B->A (in place on the RK base)
   const Ext2DState* cur[5] = {nullptr, &h->ext[0], &h->ext[1], &h->ext[2], &h->ext[1]};
   const Ext2DState* nxt[5] = {nullptr, &h->ext[1], &h->ext[2], &h->ext[1], &h->ext[0]};
   for (int K = 1; K <= 4; ++K) {
-    ExtArgs a = make_ext_args(h, K, *cur[K], *nxt[K]);
-    // the edge terms and the elevation both read only the stage input
-    fork_streams(h, FV_CONC_2D);
-    on_stream2(h, FV_CONC_2D);
-    TLAUNCH("advave_edge", k_advave_edge<FT>, g.NE + 1, g, a.cur.ua, a.cur.va, a.cur.d, a.cur.el, a.ef, a.elij);
-    on_stream1(h);
-#define EXTEL_CALL(SM) TLAUNCH("ext_elevation", k_ext_elevation<SM>, g.M + 1, g, a)
-    FV_SMAX_DISPATCH(g.cv_max, EXTEL_CALL);
-    if (g.obc_radiate) LAUNCH("ext_obc_radiate", k_ext_obc_radiate, nb(g.IOBCN), 256, g, a);
+    ExtArgs a = make_ext_args(h, K, *cur[K], *nxt[K], ec);
+#define EXT_STAGE_CALL(SM) LAUNCH("ext_momentum", (k_ext_stage<SM, FT, false>), g.ub_tile.nblk, 256, h->dg, a)
+    FV_SMAX_DISPATCH(g.cv_max, EXT_STAGE_CALL);
     if (g.obc_ore) LAUNCH("elm_shift", k_elm_shift, nb(g.M + 1), 256, g, a);
-    join_streams(h, FV_CONC_2D);
-    TLAUNCH("ext_momentum", k_ext_momentum<FT>, g.N + 1, g, a);
   }
 }
 
@@ -385,17 +382,17 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
   const DevGrid& g = h->g;
   IntArgs& a = h->ia;
   const long mk = g.m1 * g.KB, nk = g.n1 * g.KB;
-  LAUNCH("int_clock", k_int_clock, 1, 64, g, h->clk, a.qdis);
+  LAUNCH("int_clock", k_int_clock, 1, 64, g, h->clk, a.qdis, h->ec, 1, g.isplit);
 #define ADJ1_CALL(KM) TLAUNCH("adjust1_brough", k_adjust1_brough<KM>, g.N + 1, g, a)
   FV_KMAX_DISPATCH(g.KBM1, ADJ1_CALL);
   LAUNCH("adv3d_blk", (k_uv_blk<0, FT>), g.ub_tile.nblk, 256, g, a);
   TLAUNCH("baropg", k_baropg, g.N + 1, g, a, (int)h->md->p.barotropic);
   if (!h->md->p.barotropic) TLAUNCH("rho1_roundtrip", k_rho1_roundtrip, (long)g.KBM1 * g.m1, g, a);
-  TLAUNCH("advave_edge", k_advave_edge<FT>, g.NE + 1, g, a.ua, a.va, a.d, a.el, a.ef2, a.elij2);
-  TLAUNCH("advave_int", k_advave_int<FT>, g.N + 1, g, a);
-  TLAUNCH("zero", k_zero, g.m1, a.egf, g.m1);
-  if (g.IOBCN > 0) TLAUNCH("zero", k_zero, g.IOBCN, a.uard_obcn, (long)g.IOBCN);
-  for (int iext = 1; iext <= g.isplit; ++iext) enqueue_external_step_t<FT>(h, iext, iext == 1);
+  {
+    ExtArgs e = make_ext_args(h, 0, h->ext[0], h->ext[0], nullptr);
+    LAUNCH("advave_int", (k_ext_stage<16, FT, true>), g.ub_tile.nblk, 256, h->dg, e);
+  }
+  for (int iext = 1; iext <= g.isplit; ++iext) enqueue_external_step_t<FT>(h, iext, h->ec + (iext - 1));
 #define ADJ2_CALL(KM) TLAUNCH("adjust2", k_adjust2<KM>, g.N + 1, g, a)
   FV_KMAX_DISPATCH(g.KBM1, ADJ2_CALL);
 #define VERTVL_CALL(SM) LAUNCH("vertvl", k_vertvl_tile<SM>, g.nt_nblk, 256, g, a)
@@ -471,9 +468,14 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
   TLAUNCH("end_2d", k_end_2d, std::max(g.M, g.N) + 1, g, a);
 }
 
+// One EXTERNAL_STEP by itself: its EXTEL terms and constants are formed
+// from the state.
 void enqueue_external_step(fvgpu_handle* h, int iext) {
-  if (h->precision == FV_MIXED) enqueue_external_step_t<float>(h, iext, true);
-  else enqueue_external_step_t<double>(h, iext, true);
+  const DevGrid& g = h->g;
+  LAUNCH("int_clock", k_int_clock, 1, 64, g, h->clk, h->ia.qdis, h->ec, iext, 1);
+  LAUNCH("ext_begin", k_ext_begin, g.cvb_nblk, FV_CVB, g, make_ext_args(h, 0, h->ext[0], h->ext[0], nullptr));
+  if (h->precision == FV_MIXED) enqueue_external_step_t<float>(h, iext, h->ec);
+  else enqueue_external_step_t<double>(h, iext, h->ec);
 }
 
 void enqueue_internal_step(fvgpu_handle* h) {
@@ -505,6 +507,7 @@ int build_lists(fvgpu_handle* h) {
   }
   // element -> 3 sub-edges, and each sub-edge's element-major flux position
   std::vector<int> pos(NCV + 1, 0);
+  std::vector<double> edx, edy;   // DLTXE, DLTYE of the element's sub-edges (ecv_dx, ecv_dy)
   {
     const size_t n1 = (size_t)N + 1;
     std::vector<int> ec(3 * n1, 0), esw(3 * n1, 0), ecnt(n1, 0);
@@ -531,7 +534,8 @@ int build_lists(fvgpu_handle* h) {
     }
     for (int e = 1; e <= N; ++e)
       if (ecnt[e] != 3) return fail("an element has fewer than 3 control-volume sub-edges");
-    std::vector<double> edx(3 * n1, 0.0), edy(3 * n1, 0.0);
+    edx.assign(3 * n1, 0.0);
+    edy.assign(3 * n1, 0.0);
     for (size_t q = 0; q < 3 * n1; ++q)
       if (ec[q] > 0) { edx[q] = md->dltxe[ec[q]]; edy[q] = md->dltye[ec[q]]; }
     if (dupload(h, &g.ecv_dx, edx.data(), edx.size())) return 1;
@@ -580,6 +584,12 @@ int build_lists(fvgpu_handle* h) {
     if (md->nadjc_obc[i] > 0) fo[md->adjc_obc[i]].push_back((i << 1) | 0);
     if (md->nadjc_obc[i] > 1) fo[md->adjc_obc[(size_t)IOBCN + i]].push_back((i << 1) | 1);
   }
+  for (int i = 1; i <= N; ++i)
+    for (int x : fo[i]) {
+      const int j = md->i_obc_n[x >> 1];
+      if (md->nv[i] != j && md->nv[(size_t)N + 1 + i] != j && md->nv[2 * ((size_t)N + 1) + i] != j)
+        return fail("an OBC node's adjacent cell does not have the node");
+    }
   std::vector<int> fo_off(N + 2, 0), fo_ent;
   for (int i = 0; i <= N; ++i) { fo_off[i + 1] = fo_off[i] + (int)fo[i].size(); for (int x : fo[i]) fo_ent.push_back(x); }
   if (dupload(h, &g.fo_off, fo_off.data(), fo_off.size())) return 1;
@@ -598,7 +608,23 @@ int build_lists(fvgpu_handle* h) {
   if (dupload(h, &g.node_obc, nobc.data(), nobc.size())) return 1;
   if (dupload(h, &g.node_riv, nriv.data(), nriv.size())) return 1;
   if (dupload(h, &g.fct_skip, skip.data(), skip.size())) return 1;
+  // element -> rivers in river order: NBVE(J,1) then NBVE(J,NTVE(J)) of a
+  // node river's node, an edge river's own cell
+  std::vector<std::vector<int>> re(N + 1);
+  for (int k = 0; k < md->numqbc; ++k) {
+    if (md->icellq[k] > 0) { re[md->icellq[k]].push_back(k); continue; }
+    const int j = md->inodeq[k];
+    const int i1 = md->nbve[md->nbve_off[j]], i2 = md->nbve[md->nbve_off[j] + md->ntve[j] - 1];
+    re[i1].push_back(k);
+    re[i2].push_back(k);
+  }
+  std::vector<int> re_off(N + 2, 0), re_ent;
+  for (int i = 0; i <= N; ++i) { re_off[i + 1] = re_off[i] + (int)re[i].size(); for (int x : re[i]) re_ent.push_back(x); }
+  if (dupload(h, &g.re_off, re_off.data(), re_off.size())) return 1;
+  if (dupload(h, &g.re_riv, re_ent.data(), re_ent.size())) return 1;
   std::vector<std::vector<int>> tile_own;   // the element tiles below, for the momentum blocks too
+  std::vector<int> tile_nn, tile_nodes, tile_stn;   // their nodes: cvb_nn, cvb_nodes, 2*node + 1 where first
+  std::vector<int> tile_loc;                         // cvb_loc
   // element blocks of the fused record + face-flux kernels: recursive
   // coordinate bisection of the element centroids (each range halved at the
   // median of its longer extent) down to blocks of at most FV_CVB elements
@@ -655,12 +681,34 @@ int build_lists(fvgpu_handle* h) {
         }
       return n;
     };
+    // the elements' edges, and they with the other elements of those edges,
+    // number at most 256 each (the blocked momentum kernels)
+    std::vector<int> emark(N + 1, -1), cmark(NE + 1, -1);
+    auto tile_fits = [&](int lo, int hi) {
+      ++stamp;
+      int nr = 0, nc = 0;
+      for (int q = lo; q < hi; ++q) {
+        const int e = ids[q];
+        if (emark[e] != stamp) { emark[e] = stamp; ++nr; }
+        for (int j = 0; j < 3; ++j) {
+          const int c = ed[3 * (size_t)e + j] >> 1;
+          if (cmark[c] == stamp) continue;
+          cmark[c] = stamp;
+          ++nc;
+          for (int side = 0; side < 2; ++side) {
+            const int x = md->iec[(size_t)side * (NE + 1) + c];
+            if (emark[x] != stamp) { emark[x] = stamp; ++nr; }
+          }
+        }
+      }
+      return nr <= 256 && nc <= 256;
+    };
     std::vector<std::pair<int, int>> stack = component_ranges(ids, ecomp), leaves;
     while (!stack.empty()) {
       const std::pair<int, int> r = stack.back();
       stack.pop_back();
       const int lo = r.first, hi = r.second, n = hi - lo;
-      if (n <= FV_CVB && distinct_nodes(lo, hi) <= FV_CVB) { leaves.push_back(r); continue; }
+      if (n <= FV_CVB && distinct_nodes(lo, hi) <= FV_CVB && tile_fits(lo, hi)) { leaves.push_back(r); continue; }
       double x0 = md->xc[ids[lo]], x1 = x0, y0 = md->yc[ids[lo]], y1 = y0;
       for (int q = lo + 1; q < hi; ++q) {
         const double x = md->xc[ids[q]], y = md->yc[ids[q]];
@@ -675,7 +723,8 @@ int build_lists(fvgpu_handle* h) {
     }
     const int nblk = (int)leaves.size();
     std::vector<int> bnn(nblk, 0), bne(nblk, 0), bnodes((size_t)nblk * FV_CVB, 1), belems((size_t)nblk * FV_CVB, 1);
-    std::vector<int> loc((size_t)N + 1, 0), nloc(M + 1, 0);
+    std::vector<int> loc((size_t)N + 1, 0), nloc(M + 1, 0), stn((size_t)nblk * FV_CVB, 2);
+    std::vector<char> seen(M + 1, 0);
     for (int b = 0; b < nblk; ++b) {
       const int lo = leaves[b].first, hi = leaves[b].second;
       std::sort(ids.begin() + lo, ids.begin() + hi);
@@ -690,6 +739,8 @@ int build_lists(fvgpu_handle* h) {
           if (mark[nd] != stamp) {
             mark[nd] = stamp;
             nloc[nd] = nn;
+            stn[(size_t)b * FV_CVB + nn] = (nd << 1) | (seen[nd] ? 0 : 1);
+            seen[nd] = 1;
             bnodes[(size_t)b * FV_CVB + nn++] = nd;
           }
           packed |= nloc[nd] << (8 * j);
@@ -791,19 +842,25 @@ int build_lists(fvgpu_handle* h) {
     }
     if (dupload(h, &g.cvb_nn, bnn.data(), bnn.size())) return 1;
     if (dupload(h, &g.cvb_nodes, bnodes.data(), bnodes.size())) return 1;
+    for (int i = 1; i <= M; ++i)
+      if (!seen[i]) return fail("a node belongs to no element");
+    tile_stn.swap(stn);
     if (dupload(h, &g.cvb_ne, bne.data(), bne.size())) return 1;
     if (dupload(h, &g.cvb_elems, belems.data(), belems.size())) return 1;
     if (dupload(h, &g.cvb_loc, loc.data(), loc.size())) return 1;
     if (dupload(h, &g.rec_keep, keep.data(), keep.size())) return 1;
+    tile_nn.swap(bnn);
+    tile_nodes.swap(bnodes);
+    tile_loc.swap(loc);
   }
-  // element blocks of the blocked ADVECTION / ADV_UV kernels.  ADVECTION
-  // takes the element tiles above (compact, so few neighbours form their
-  // records twice) if every tile needs at most 256 records (its own
-  // elements and the other elements of their edges) and at most 256 edges;
+  // element blocks of the blocked momentum kernels.  The 2-D stage and
+  // ADVECTION take the element tiles above (compact, so few neighbours form
+  // their records twice; each needs at most 256 records -- its own elements
+  // and the other elements of their edges -- and at most 256 edges);
   // ADV_UV, whose element part reads and writes many element-layer
   // arrays, takes runs of consecutive elements (contiguous addresses), the
   // largest run length (a multiple of 8, at most 128) that keeps every
-  // block within both, and so does ADVECTION where a tile would not fit
+  // block within both
   {
     std::vector<int> bns, bnown, belems, bne, bedges, beloc, epos;
     std::vector<int> rslot(N + 1, -1), rblk(N + 1, -1), eslot(NE + 1, -1), eblk(NE + 1, -1);
@@ -840,7 +897,7 @@ int build_lists(fvgpu_handle* h) {
               eblk[c] = b;
               eslot[c] = ne++;
             }
-            packed |= (eslot[c] & 255) << (8 * q);
+            packed |= (eslot[c] & 255) << (8 * q) | (ed[3 * (size_t)e + q] & 1) << (24 + q);
           }
           epos[e] = packed;
         }
@@ -869,28 +926,64 @@ int build_lists(fvgpu_handle* h) {
       eb = std::min(eb - 8, (int)((long)eb * 256 / worst) / 8 * 8);
     }
     if (upload_blocks(g.ub_run)) return 1;
-    bool tiles_fit = true;
-    for (const auto& t : tile_own) tiles_fit = tiles_fit && t.size() <= 128;
-    if (tiles_fit && build_blocks(tile_own) <= 256) {
-      if (upload_blocks(g.ub_tile)) return 1;
-    } else {
-      g.ub_tile = g.ub_run;
+    if (build_blocks(tile_own) > 256) return fail("an element tile exceeds the blocked momentum kernels' records");
+    // the 2-D stage's tables, in block order
+    const size_t nt = tile_own.size(), n1 = (size_t)N + 1, ne1 = (size_t)NE + 1;
+    std::vector<int4> nb4(nt * 256, int4{0, 0, 0, 0});
+    std::vector<double> egeo(nt * 6 * 256, 0.0);
+    std::vector<int> nslot(M + 1, 0);
+    for (size_t b = 0; b < nt; ++b) {
+      for (int t = 0; t < tile_nn[b]; ++t) nslot[tile_nodes[b * FV_CVB + t]] = t;
+      for (int t = 0; t < bns[b]; ++t) {
+        const int x = belems[b * 256 + t];
+        nb4[b * 256 + t] = int4{x, md->nbe[x], md->nbe[n1 + x], md->nbe[2 * n1 + x]};
+      }
+      for (int t = 0; t < bne[b]; ++t) {
+        const int c = bedges[b * 256 + t], ia = md->iec[c], ib = md->iec[ne1 + c];
+        if (md->isbc[c] < 0 || md->isbc[c] > 3) return fail("ISBC outside 0..3");
+        const unsigned lo = (unsigned)beloc[b * 256 + t], j1 = (unsigned)nslot[md->ienode[c]],
+                       j2 = (unsigned)nslot[md->ienode[ne1 + c]];
+        beloc[b * 256 + t] = (int)(lo | j1 << 16 | j2 << 23 | (unsigned)md->isbc[c] << 30);
+        const double v[6] = {md->xijc[c] - md->xc[ia], md->yijc[c] - md->yc[ia], md->xijc[c] - md->xc[ib],
+                             md->yijc[c] - md->yc[ib], md->dltxc[c], md->dltyc[c]};
+        for (int q = 0; q < 6; ++q) egeo[(b * 6 + q) * 256 + t] = v[q];
+      }
     }
+    if (upload_blocks(g.ub_tile) || dupload(h, &g.ub_tile.nb4, nb4.data(), nb4.size()) ||
+        dupload(h, &g.ub_tile.egeo, egeo.data(), egeo.size()))
+      return 1;
+    const size_t SM = (size_t)std::max(g.cv_max, 1);
+    std::vector<int4> snode(nt * FV_CVB, int4{2, 0, -1, -1}), selem(nt * FV_CVB, int4{0, 0, 0, 0});
+    std::vector<int> slist(nt * SM * FV_CVB, 0);
+    std::vector<double> snd(nt * 2 * FV_CVB, 1.0), sed(nt * 12 * FV_CVB, 0.0);
+    for (size_t b = 0; b < nt; ++b) {
+      for (int t = 0; t < tile_nn[b]; ++t) {
+        const int i = tile_nodes[b * FV_CVB + t];
+        snode[b * FV_CVB + t] = int4{tile_stn[b * FV_CVB + t], cnt[i], nobc[i], nriv[i]};
+        for (int j = 0; j < cnt[i]; ++j) {
+          const int en = ent[off[i] + j];
+          slist[(b * SM + j) * FV_CVB + t] = (pos[en >> 1] << 1) | (en & 1);
+        }
+        snd[(2 * b) * FV_CVB + t] = md->art1[i];
+        snd[(2 * b + 1) * FV_CVB + t] = md->h[i];
+      }
+      for (int t = 0; t < bnown[b]; ++t) {
+        const int e = belems[b * 256 + t];
+        selem[b * FV_CVB + t] = int4{epos[e], tile_loc[e], (md->isbce[e] & 3) | (re_off[e] < re_off[e + 1] ? 4 : 0),
+                                     md->iucp[e]};
+        double v[12] = {md->epor[e], md->grav_e[e], md->art[e], md->cor[e], md->h1[e], md->cc_sponge[e]};
+        for (int j = 0; j < 3; ++j) {
+          v[6 + j] = edx[(size_t)j * n1 + e];
+          v[9 + j] = edy[(size_t)j * n1 + e];
+        }
+        for (int q = 0; q < 12; ++q) sed[(b * 12 + q) * FV_CVB + t] = v[q];
+      }
+    }
+    if (dupload(h, &g.st_node, snode.data(), snode.size()) || dupload(h, &g.st_elem, selem.data(), selem.size()) ||
+        dupload(h, &g.st_list, slist.data(), slist.size()) || dupload(h, &g.st_nd, snd.data(), snd.size()) ||
+        dupload(h, &g.st_ed, sed.data(), sed.size()))
+      return 1;
   }
-  // element -> rivers in river order: NBVE(J,1) then NBVE(J,NTVE(J)) of a
-  // node river's node, an edge river's own cell
-  std::vector<std::vector<int>> re(N + 1);
-  for (int k = 0; k < md->numqbc; ++k) {
-    if (md->icellq[k] > 0) { re[md->icellq[k]].push_back(k); continue; }
-    const int j = md->inodeq[k];
-    const int i1 = md->nbve[md->nbve_off[j]], i2 = md->nbve[md->nbve_off[j] + md->ntve[j] - 1];
-    re[i1].push_back(k);
-    re[i2].push_back(k);
-  }
-  std::vector<int> re_off(N + 2, 0), re_ent;
-  for (int i = 0; i <= N; ++i) { re_off[i + 1] = re_off[i] + (int)re[i].size(); for (int x : re[i]) re_ent.push_back(x); }
-  if (dupload(h, &g.re_off, re_off.data(), re_off.size())) return 1;
-  if (dupload(h, &g.re_riv, re_ent.data(), re_ent.size())) return 1;
   return 0;
 }
 
@@ -1058,14 +1151,12 @@ int upload_state(fvgpu_handle* h) {
   RW(gx, nullptr, mk);
   // flux buffers sized for FP64 (the mixed form uses the first half)
   {
-    EdgeFlux4T<double>* p2 = nullptr; CvRecT<double>* pr = nullptr;
+    CvRecT<double>* pr = nullptr;
     double* pc = nullptr;
-    if (dalloc(h, &p2, (size_t)g.NE + 1)) return 1;
     if (dalloc(h, &pr, mk)) return 1;
     if (dalloc(h, &pc, ((size_t)g.NCV + 1) * g.KB)) return 1;
-    a.ef2 = p2; a.rec = pr; a.cvflux = pc;
+    a.rec = pr; a.cvflux = pc;
   }
-  RW(elij2, nullptr, (size_t)g.NE + 1);
   if (dalloc(h, &a.vhpair, mk)) return 1;
   if (dalloc(h, &a.obcsum, 5 * (size_t)g.IOBCN)) return 1;
   RW(adx2d, nullptr, n1); RW(ady2d, nullptr, n1); RW(drx2d, nullptr, n1); RW(dry2d, nullptr, n1);
@@ -1075,9 +1166,9 @@ int upload_state(fvgpu_handle* h) {
   RW(qdis, nullptr, (size_t)g.NUMQBC); RW(xflux_obc, nullptr, (size_t)g.IOBCN * g.KB);
   RW(uard_obcn, nullptr, (size_t)g.IOBCN);
 #undef RW
-  if (dalloc(h, &h->xflux_obcn, (size_t)g.IOBCN)) return 1;
-  if (dalloc(h, &h->phi, (size_t)g.NCV + 1)) return 1;
-  if (dalloc(h, &h->fobn, (size_t)g.IOBCN)) return 1;
+  if (dalloc(h, &h->phi[0], (size_t)g.NCV + 1) || dalloc(h, &h->phi[1], (size_t)g.NCV + 1)) return 1;
+  if (dalloc(h, &h->own2d, (size_t)g.cvb_nblk * 6 * FV_CVB)) return 1;
+  if (dalloc(h, &h->elrk, m1) || dalloc(h, &h->ec, (size_t)std::max(g.isplit, 1))) return 1;
   if (dalloc(h, &h->clk, 1)) return 1;
   {
     double* dp = nullptr;
@@ -1085,8 +1176,8 @@ int upload_state(fvgpu_handle* h) {
     h->diag_part = dp;
   }
   DevClock c{};
-  c.iint = md->p.iint0; c.iext = 0; c.ramp_int = 0; c.ramp_ext = 0;
-  c.ext_time = md->p.time0; c.time0 = md->p.time0; c.dti = g.dti; c.dte = g.dte;
+  c.iint = md->p.iint0; c.ramp_int = 0;
+  c.time0 = md->p.time0; c.dti = g.dti; c.dte = g.dte;
   c.isplit = g.isplit; c.iramp = g.iramp; c.depth_fail = 0;
   HIPCHK(hipMemcpy(h->clk, &c, sizeof(c), hipMemcpyHostToDevice));
   a.clk = h->clk;
@@ -1174,7 +1265,7 @@ int fvgpu_create(const fv_model* md, int32_t precision, fvgpu_handle** out) {
     fvgpu_destroy(h);
     return fail("stream2 / events");
   }
-  if (upload_grid(h) || upload_state(h)) { fvgpu_destroy(h); return 1; }
+  if (upload_grid(h) || upload_state(h) || dupload(h, &h->dg, &h->g, 1)) { fvgpu_destroy(h); return 1; }
   HIPCHK(hipStreamSynchronize(h->stream));
   *out = h;
   return 0;
@@ -1189,7 +1280,6 @@ int fvgpu_internal_step(fvgpu_handle* h) {
 
 int fvgpu_external_step(fvgpu_handle* h, int32_t iext) {
   // the clock as INTERNAL_STEP would set it for IINT+1, then one EXTERNAL_STEP
-  LAUNCH("int_clock", k_int_clock, 1, 64, h->g, h->clk, h->ia.qdis);
   enqueue_external_step(h, iext);
   // restore IINT (this call does not complete an internal step)
   DevClock c;
@@ -1766,7 +1856,7 @@ int fvgpu_set_concurrency(fvgpu_handle* h, int32_t mode) {
 }
 
 int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_len) {
-  static const char* fams[] = {"ext_elevation", "advave_edge", "ext_momentum", "cvrec_ts", "cvrec_q", "cvflux_ts",
+  static const char* fams[] = {"cvrec_ts", "cvrec_q", "cvflux_ts",
                                "cvflux_q", "adv_ts", "adv_q",
                                "viscofh", "vdif_q", "vdif_ts", "adjust1_brough", "adjust2", "baropg",
                                "uv_finish", "copy", "closure_features", "closure_apply"};

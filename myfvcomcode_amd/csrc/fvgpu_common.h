@@ -28,10 +28,18 @@
 // elems[256*b + t]; its ne[b] (<= 256) edges edges[256*b + t], with the
 // record slots of IA and IB in bits 0-7 and 8-15 of eloc[256*b + t];
 // epos[e] packs the edge slots of element e's three edges (in ed_ent
-// order) in bits 0-7, 8-15, 16-23.
+// order) in bits 0-7, 8-15, 16-23, and in bits 24-26 whether e is their IB.
+// For the element tiles also, in block order so that the 2-D stage reads
+// them directly: nb4[256*b + t] the record's element and its three
+// neighbours NBE; egeo[(6*b + q)*256 + t] the edge's XIJC-XC and YIJC-YC of
+// IA, the same of IB, DLTXC, DLTYC; and in eloc the local indices (of
+// cvb_nodes) of the edge's nodes IENODE in bits 16-22 and 23-29 and ISBC in
+// bits 30-31.
 struct UvBlocks {
   int nblk;
   const int *nown, *ns, *elems, *ne, *edges, *eloc, *epos;
+  const int4* nb4;
+  const double* egeo;
 };
 
 struct DevGrid {
@@ -87,6 +95,17 @@ struct DevGrid {
   // at every layer (the OBC nodes and the other ends of their sub-edges).
   int cvb_nblk;
   const int *cvb_nn, *cvb_nodes, *cvb_ne, *cvb_elems, *cvb_loc, *rec_keep;
+  // The 2-D stage's constants of the same blocks in block order (read
+  // directly and contiguously, without waiting for an index): node t:
+  // st_node[FV_CVB*b + t] = {2*node + 1 in the first block that has it,
+  // sub-edge count, OBC index or -1, river index or -1}, its cvl_ent list
+  // st_list[(cv_max*b + j)*FV_CVB + t] and {ART1, H} in
+  // st_nd[(2*b + q)*FV_CVB + t]; element t: st_elem = {epos, cvb_loc, ISBCE
+  // + 4 if it has rivers, IUCP} and EPOR, GRAV_E, ART, COR, H1, CC_SPONGE,
+  // DLTXE and DLTYE of its three sub-edges in st_ed[(12*b + q)*FV_CVB + t].
+  const int4 *st_node, *st_elem;
+  const int* st_list;
+  const double *st_nd, *st_ed;
   // Node tiles (VERTVL): tile b owns the nt_nown[b] (<= FV_NTN) nodes
   // nt_nodes[FV_NTN*b + t]; nt_elems[FV_NTE*b + t] are the nt_nel[b]
   // (<= FV_NTE) elements that have one of them as a vertex.  Slot j of
@@ -94,8 +113,9 @@ struct DevGrid {
   // | side, in the order of cvl_ent.
   int nt_nblk;
   const int *nt_nown, *nt_nodes, *nt_nel, *nt_elems, *nt_lpos;
-  // Element blocks of the blocked ADVECTION / ADV_UV kernels (UvBlocks):
-  // compact tiles for ADVECTION, runs of consecutive elements for ADV_UV.
+  // Element blocks of the blocked momentum kernels (UvBlocks): the blocks of
+  // cvb_* (compact tiles) for the 2-D stage and ADVECTION, runs of
+  // consecutive elements for ADV_UV.
   UvBlocks ub_tile, ub_run;
   // OBC / tide / rivers
   const int *i_obc_n, *next_obc, *nadjc_obc, *adjc_obc, *type_obc;
@@ -182,10 +202,7 @@ __device__ __forceinline__ bool river_share(const DevGrid& g, int j, int i, doub
 // tiny kernels so that a captured graph replays correctly.
 struct DevClock {
   long long iint;
-  int iext;
   double ramp_int;      // RAMP of INTERNAL_STEP
-  double ramp_ext;      // RAMP of the current EXTERNAL_STEP
-  double ext_time;      // ExtTime (s since SpecTime)
   double time0, dti, dte;
   int isplit, iramp;
   int depth_fail;

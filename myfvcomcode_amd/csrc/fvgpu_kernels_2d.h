@@ -1,23 +1,16 @@
 // fvgpu_kernels_2d.h -- the barotropic (external) mode on the device.
 //
 // One Runge-Kutta stage of EXTERNAL_STEP (FVCOM_source/external_step.F:159-438)
-// is three kernels:
-//   k_ext_elevation  node-parallel: EXTEL_EDGE (extel_edge.F:32-229) as a
-//                    gather of each node's control-volume sub-edge terms
-//                    (formed per sub-edge by the previous stage's
-//                    k_ext_momentum, or by k_ext_phi), the
-//                    OBC tide and RK blend (BCOND_GCN(1,K), bcond_gcn.F:116;
-//                    BCOND_ASL, mod_obcs.F:509-592), the OBC flux of FLUX_OBN
-//                    (mod_obcs.F:1181-1215), D = H + EL, DEPTH_CHECK, and the
-//                    stage-3 EGF / stage-4 UARD_OBCN accumulations.
-//   k_advave_edge    edge-parallel: the ADVAVE_EDGE_GCN edge terms
-//                    (advave_edge_gcn.F:546-884) of the stage input, once per edge;
-//   k_ext_momentum   element-parallel: N2E2D of the new elevation, the
-//                    element's three edge terms gathered in edge order,
-//                    EXTUV_EDGE (extuv_edge.F:33-196),
-//                    the wall projection BCOND_GCN(2,K) (bcond_gcn.F:325-420),
-//                    D1 = H1 + EL1, the stage-3 UARD/VARD accumulation and
-//                    the EXTEL terms of its sub-edges for the next stage.
+// is one kernel over compact element tiles, k_ext_stage: EXTEL_EDGE
+// (extel_edge.F:32-229) as a gather of each node's control-volume sub-edge
+// terms (formed per sub-edge by the previous stage, or by k_ext_begin), the
+// open-boundary conditions and RK blend (BCOND_GCN(1,K), bcond_gcn.F:116;
+// mod_obcs.F:509-737), FLUX_OBN (mod_obcs.F:1181-1215), D = H + EL,
+// DEPTH_CHECK, N2E2D, the ADVAVE_EDGE_GCN edge terms
+// (advave_edge_gcn.F:546-884), EXTUV_EDGE (extuv_edge.F:33-196), the wall
+// projection BCOND_GCN(2,K) (bcond_gcn.F:325-420), D1 = H1 + EL1, the
+// stage-3 EGF / UARD / VARD and stage-4 UARD_OBCN accumulations, and the
+// EXTEL terms of the next stage.
 // The per-node and per-element gather lists are sorted by sub-edge / edge
 // index, so every sum is formed in the order of the reference's scatter loop.
 #pragma once
@@ -29,29 +22,30 @@ struct Ext2DState {      // one buffer set of the 2-D state
   double *ua, *va, *el1, *d1;  // elements
 };
 
-// Per edge (and layer) momentum-flux terms of the edge loops of
-// ADVAVE_EDGE_GCN / ADVECTION_EDGE_GCN / ADV_UV_EDGE_GCN, written once per
-// edge by an edge kernel and gathered by the two adjacent elements.
-template <typename T>
-struct __align__(16) EdgeFlux4T {
-  T xadv, yadv, fx, fy;
-};
+// RAMP and ExtTime of one external step (k_int_clock).
+struct ExtClock { double ramp, time; };
 
 struct ExtArgs {
   Ext2DState cur;        // stage input
-  Ext2DState base;       // RK base (ELRK, UARK, VARK, ELRK1)
+  Ext2DState base;       // RK base (UARK, VARK, ELRK1)
   Ext2DState nxt;        // stage output (may alias base: pointwise use only)
   int K;                 // RK stage 1..4
   double alpha;          // ALPHA_RK(K)
-  double *xflux_obcn, *fobn, *uard_obcn, *egf, *fluxobn, *uard, *vard;
-  const double *adx2d, *ady2d, *drx2d, *dry2d, *wubot, *wvbot;
+  const double* elrk;    // RK base elevation: the base's own array in stage 1, its copy afterwards
+  double* elrk_copy;     // stage 1 fills the copy, else null
+  double *uard_obcn, *egf, *fluxobn, *uard, *vard;
+  double *adx2d, *ady2d; // written by the INT form only
+  const double *drx2d, *dry2d, *wubot, *wvbot;
+  // the six constants of the external steps in block order: ADX2D, ADY2D,
+  // DRX2D, DRY2D, WUBOT, WVBOT of element t at (6*b + q)*FV_CVB + t
+  // (written by the INT form)
+  double* own2d;
   const double *qdis;    // QDIS (internal-mode river discharge)
-  void* ef;              // per-edge ADVAVE terms of the stage input, EdgeFlux4T<FT>
-  double* elij;          // per-edge mean elevation of the stage input
-  double* phi;           // per sub-edge EXTEL terms (read for the stage input,
-                         // written by k_ext_momentum for the next stage)
+  const double* phi;     // per sub-edge EXTEL terms of the stage input
+  double* phi_next;      // those of the stage output
   const double *ws2x, *ws2y;   // wind stress of the external step (before RAMP*0.001)
   double *elm1, *elm2;         // the elevation one and two RK stages back (Orlanski OBC)
+  const ExtClock* ec;    // of this external step
   DevClock* clk;
 };
 
@@ -140,42 +134,24 @@ __device__ __forceinline__ double tide_force(const DevGrid& g, int obc, double r
   return force * ramp;
 }
 
-// FLUX_OBN's flux defect of OBC node i (mod_obcs.F:1196) and, in the last
-// stage, its UARD_OBCN share (external_step.F:423-430).
-__device__ __forceinline__ void ext_obc_flux(const DevGrid& g, const ExtArgs& a, int i, int obc, double elf,
-                                             double elrk, double xobc) {
-  a.fobn[obc] = -(elf - elrk) * g.art1[i] / (a.alpha * g.dte) - xobc;
-  if (a.K == 4) {
-    const double tmp = -(elf - elrk) * g.art1[i] / g.dte - xobc;
-    a.uard_obcn[obc] = a.uard_obcn[obc] + tmp / (double)g.isplit;
-  }
-}
-
-// The new elevation of node i: EL, D = H + EL, the stage-3 EGF sum and
-// DEPTH_CHECK.
-__device__ __forceinline__ void ext_node_store(const DevGrid& g, const ExtArgs& a, int i, double elf) {
-  const double dnew = g.h[i] + elf;
-  a.nxt.el[i] = elf;
-  a.nxt.d[i] = dnew;
-  if (a.K == 3) a.egf[i] = a.egf[i] + elf / (double)g.isplit;
-  if (i >= 1 && dnew < g.min_depth) a.clk->depth_fail = 1;
-}
-
+// The new elevation of node i before its open-boundary condition:
+// EXTEL_EDGE's sum over the node's sub-edges in sub-edge order, its rivers
+// (rv: the first, or -1) and the RK update; at an OBC node `xobc` is the sum
+// itself (extel_edge.F:155-160).  The term of sub-edge c, D1*(-UA*DLTYE +
+// VA*DLTXE) of its element for side IB, is exactly the negative for side IA
+// (DLTXE/DLTYE negated; round to nearest is symmetric), so the stored term
+// is added or subtracted.  The node's n list entries are at lst[j*stride];
+// SMAX >= the slots of the list (nslot), the slots past n hold the unused
+// entry 0, so all list and term loads are unconditional and issue together.
 template <int SMAX>
-__global__ void k_ext_elevation(DevGrid g, ExtArgs a) {
-  const int i = (int)xcd_thread();
-  if (i > g.M) return;
-  // EXTEL_EDGE sum over the node's sub-edges in sub-edge order.  The term of
-  // sub-edge c, D1*(-UA*DLTYE + VA*DLTXE) of its element for side IB, is
-  // exactly the negative for side IA (DLTXE/DLTYE negated; round to
-  // nearest is symmetric), so the stored term is added or subtracted.
-  // SMAX >= the node's sub-edge count: the slots past it re-read slot 0,
-  // so all list and term loads are unconditional and issue together.
-  const int n = g.cv_cnt[i];
+__device__ __forceinline__ double ext_node_update(const DevGrid& g, const ExtArgs& a, int i, const int* lst,
+                                                  long stride, int n, int rv, bool obc, double art1, double elrk,
+                                                  double& xobc) {
+  const int nslot = g.cv_max;
   int ce[SMAX];
   static_for<SMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    ce[j] = g.cvl_ent[(long)(j < n ? j : 0) * g.m1 + i];
+    ce[j] = lst[(j < nslot ? j : 0) * stride];
   });
   double t[SMAX];
   static_for<SMAX>([&](auto jc) {
@@ -187,10 +163,8 @@ __global__ void k_ext_elevation(DevGrid g, ExtArgs a) {
     constexpr int j = decltype(jc)::value;
     if (j < n) xflux = (ce[j] & 1) ? xflux + t[j] : xflux - t[j];
   });
-  const int obc = g.node_obc[i];
-  double xobc = 0.0;
-  if (obc >= 0) { xobc = xflux; xflux = 0.0; a.xflux_obcn[obc] = xobc; }
-  const int rv = g.node_riv[i];
+  xobc = 0.0;
+  if (obc) { xobc = xflux; xflux = 0.0; }
   if (rv >= 0) {
     for (int j = rv; j < g.NUMQBC; ++j) {
       double w;
@@ -198,59 +172,43 @@ __global__ void k_ext_elevation(DevGrid g, ExtArgs a) {
     }
   }
   const double dtk = a.alpha * g.dte;
-  const double elrk = a.base.el[i];
-  double elf = elrk - dtk * xflux / g.art1[i];
-  if (obc >= 0) {
-    const int ty = g.type_obc[obc];
-    if (ty >= 5) return;   // radiation conditions: k_ext_obc_radiate, once every interior ELF is formed
-    if (ty <= 2) {         // BCOND_ASL, then the RK blend (external_step.F:262-266)
-      if (g.obc_elev) {
-        const double rk_time = a.clk->ext_time + g.dte * (a.alpha - 1.0);
-        elf = tide_force(g, obc, rk_time, a.clk->ramp_ext);
-      }
-      elf = elrk + a.alpha * (elf - elrk);
-    } else {               // BCOND_ASL_CLP (mod_obcs.F:599-617)
-      elf = 0.0;
-    }
-    ext_obc_flux(g, a, i, obc, elf, elrk, xobc);
-  }
-  ext_node_store(g, a, i, elf);
+  return elrk - dtk * xflux / art1;
 }
 
-// BCOND_GWI (TYPE_OBC 5/6, mod_obcs.F:624-658) and BCOND_BKI (7/8,
-// mod_obcs.F:665-699): the OBC node's ELF from its interior neighbour
-// NEXT_OBC's new ELF (formed by k_ext_elevation, which leaves these nodes
-// alone); BCOND_ORE (9/10, mod_obcs.F:706-737): from the stage input EL
-// and the elevations ELM1/ELM2 one and two stages back.  One thread per
-// OBC node.
-__global__ void k_ext_obc_radiate(DevGrid g, ExtArgs a) {
-  const int obc = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (obc >= g.IOBCN) return;
-  const int ty = g.type_obc[obc];
-  if (ty < 5) return;
-  const int i1 = g.i_obc_n[obc], i2 = g.next_obc[obc];
-  const double elrk = a.base.el[i1];
-  double elf;
+// The open-boundary condition of OBC node i (index obc): its elevation from
+// the unconstrained one.  1/2: BCOND_ASL (mod_obcs.F:552-582), then the RK
+// blend (external_step.F:262-266); 3/4: BCOND_ASL_CLP (mod_obcs.F:599-617);
+// 5/6: BCOND_GWI (mod_obcs.F:624-658) and 7/8: BCOND_BKI (mod_obcs.F:665-699)
+// from the new elevation el2 of the interior neighbour NEXT_OBC; 9/10:
+// BCOND_ORE (mod_obcs.F:706-737) from the stage input EL and the elevations
+// ELM1/ELM2 one and two stages back.
+__device__ __forceinline__ double ext_obc_value(const DevGrid& g, const ExtArgs& a, int i, int obc, int ty,
+                                                double elrk, double elf, double el2) {
+  if (ty <= 2) {
+    if (g.obc_elev) {
+      const double rk_time = a.ec->time + g.dte * (a.alpha - 1.0);
+      elf = tide_force(g, obc, rk_time, a.ec->ramp);
+    }
+    return elrk + a.alpha * (elf - elrk);
+  }
+  if (ty <= 4) return 0.0;
   if (ty >= 9) {
-    const int i3 = g.next_obc2[obc];
+    const int i2 = g.next_obc[obc], i3 = g.next_obc2[obc];
     const double cl = (a.elm2[i2] - a.cur.el[i2]) / (a.cur.el[i2] + a.elm2[i2] - 2.0 * a.elm1[i3]);
     double mu;                            // a NaN CL (0/0 at rest) gives MU = 0, as in the reference
     if (cl >= 1.0) mu = 1.0;
     else if (cl > 0.0 && cl < 1.0) mu = cl;
     else mu = 0.0;
-    elf = (a.elm1[i1] * (1.0 - mu) + 2.0 * mu * a.cur.el[i2]) / (1.0 + mu);
-  } else {
-    const double cc = sqrt(g.grav_n[i1] * g.h[i1]) * g.dte / g.dltn_obc[obc] * a.alpha;
-    const double cp = cc + 1.0;
-    elf = ty <= 6 ? (cc * a.nxt.el[i2] + elrk) / cp : (cc * a.nxt.el[i2] + elrk * (1.0 - g.dte / 10800.0)) / cp;
+    return (a.elm1[i] * (1.0 - mu) + 2.0 * mu * a.cur.el[i2]) / (1.0 + mu);
   }
-  ext_obc_flux(g, a, i1, obc, elf, elrk, a.xflux_obcn[obc]);
-  ext_node_store(g, a, i1, elf);
+  const double cc = sqrt(g.grav_n[i] * g.h[i]) * g.dte / g.dltn_obc[obc] * a.alpha;
+  const double cp = cc + 1.0;
+  return ty <= 6 ? (cc * el2 + elrk) / cp : (cc * el2 + elrk * (1.0 - g.dte / 10800.0)) / cp;
 }
 
 // ASSIGN_ELM1_TO_ELM2 (mod_obcs.F:178-199) at the end of a stage
 // (external_step.F:333): ELM2 = ELM1, ELM1 = the stage input EL.  Run
-// after k_ext_obc_radiate, the only reader.
+// after k_ext_stage, the only reader; launched only when Orlanski nodes exist.
 __global__ void k_elm_shift(DevGrid g, ExtArgs a) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i > g.M) return;
@@ -258,189 +216,317 @@ __global__ void k_elm_shift(DevGrid g, ExtArgs a) {
   a.elm1[i] = a.cur.el[i];
 }
 
-// ADVAVE_EDGE_GCN edge loop body (advave_edge_gcn.F:546-884) for edge e of
-// the state (ua, va, d, el), one thread per edge: least-squares velocity
-// gradients on both sides, face velocities, upwind advective flux, the
-// Smagorinsky stresses; the side-dependent factors (EPOR, IUCP, ISBC, the
-// pressure term) are applied by the gathering element.  Arithmetic in the
-// flux type FT (FP64: the reference's expressions bit for bit).
-template <typename FT>
-__global__ __launch_bounds__(256) void k_advave_edge(DevGrid g, const double* ua_, const double* va_,
-                                                     const double* d, const double* el,
-                                                     void* ef_, double* elij_out) {
-  const int e = (int)xcd_thread();
-  if (e < 1 || e > g.NE) return;
-  EdgeFlux4T<FT>* ef = (EdgeFlux4T<FT>*)ef_;
-  const FT half = (FT)0.5, one = (FT)1.0;
-  const int ia = IEC_(e, 1), ib = IEC_(e, 2), j1 = IENODE_(e, 1), j2 = IENODE_(e, 2);
-  const FT dij = half * ((FT)d[j1] + (FT)d[j2]);
-  const double elij = 0.5 * (el[j1] + el[j2]);
-  auto U = [&](int i) { return (FT)ua_[i]; };
-  auto V = [&](int i) { return (FT)va_[i]; };
-  auto A1 = [&](int i, int j) { return (FT)A1U_(i, j); };
-  auto A2 = [&](int i, int j) { return (FT)A2U_(i, j); };
-  int k1 = NBE_(ia, 1), k2 = NBE_(ia, 2), k3 = NBE_(ia, 3);
-  const FT cofa1 = A1(ia, 1) * U(ia) + A1(ia, 2) * U(k1) + A1(ia, 3) * U(k2) + A1(ia, 4) * U(k3);
-  const FT cofa2 = A2(ia, 1) * U(ia) + A2(ia, 2) * U(k1) + A2(ia, 3) * U(k2) + A2(ia, 4) * U(k3);
-  const FT cofa5 = A1(ia, 1) * V(ia) + A1(ia, 2) * V(k1) + A1(ia, 3) * V(k2) + A1(ia, 4) * V(k3);
-  const FT cofa6 = A2(ia, 1) * V(ia) + A2(ia, 2) * V(k1) + A2(ia, 3) * V(k2) + A2(ia, 4) * V(k3);
-  FT xij = (FT)(g.xijc[e] - g.xc[ia]), yij = (FT)(g.yijc[e] - g.yc[ia]);
-  const FT uij1 = U(ia) + cofa1 * xij + cofa2 * yij;
-  const FT vij1 = V(ia) + cofa5 * xij + cofa6 * yij;
-  k1 = NBE_(ib, 1); k2 = NBE_(ib, 2); k3 = NBE_(ib, 3);
-  const FT cofa3 = A1(ib, 1) * U(ib) + A1(ib, 2) * U(k1) + A1(ib, 3) * U(k2) + A1(ib, 4) * U(k3);
-  const FT cofa4 = A2(ib, 1) * U(ib) + A2(ib, 2) * U(k1) + A2(ib, 3) * U(k2) + A2(ib, 4) * U(k3);
-  const FT cofa7 = A1(ib, 1) * V(ib) + A1(ib, 2) * V(k1) + A1(ib, 3) * V(k2) + A1(ib, 4) * V(k3);
-  const FT cofa8 = A2(ib, 1) * V(ib) + A2(ib, 2) * V(k1) + A2(ib, 3) * V(k2) + A2(ib, 4) * V(k3);
-  xij = (FT)(g.xijc[e] - g.xc[ib]); yij = (FT)(g.yijc[e] - g.yc[ib]);
-  const FT uij2 = U(ib) + cofa3 * xij + cofa4 * yij;
-  const FT vij2 = V(ib) + cofa7 * xij + cofa8 * yij;
-  const FT uij = half * (uij1 + uij2), vij = half * (vij1 + vij2);
-  const FT dlx = (FT)g.dltxc[e], dly = (FT)g.dltyc[e];
-  const FT un_tmp = -uij * dly + vij * dlx;
-  const FT viscof1 = (FT)g.art[ia] * sqrt(sq(cofa1) + sq(cofa6) + half * sq(cofa2 + cofa5));
-  const FT viscof2 = (FT)g.art[ib] * sqrt(sq(cofa3) + sq(cofa8) + half * sq(cofa4 + cofa7));
-  const FT cca = (FT)g.cc_hvc[ia], ccb = (FT)g.cc_hvc[ib];
-  const FT viscof = ((FT)g.fact * half * (viscof1 * cca + viscof2 * ccb) +
-                     (FT)g.fm1 * half * (cca + ccb)) / (FT)g.hprnu;
-  const FT txxij = (cofa1 + cofa3) * viscof;
-  const FT tyyij = (cofa6 + cofa8) * viscof;
-  const FT txyij = half * (cofa2 + cofa4 + cofa5 + cofa7) * viscof;
-  EdgeFlux4T<FT> r;
-  r.fx = dij * (txxij * dly - txyij * dlx);
-  r.fy = dij * (txyij * dly - tyyij * dlx);
-  const FT sgn = fsign1(un_tmp);
-  r.xadv = dij * un_tmp * ((one - sgn) * uij2 + (one + sgn) * uij1) * half;
-  r.yadv = dij * un_tmp * ((one - sgn) * vij2 + (one + sgn) * vij1) * half;
-  ef[e] = r;
-  elij_out[e] = elij;
+// What the INT form of k_ext_stage leaves for the external steps, from the
+// current state: the EXTEL terms and the block-order constants.  For a
+// direct EXTERNAL_STEP call; one workgroup per element tile.
+__global__ __launch_bounds__(FV_CVB) void k_ext_begin(DevGrid g, ExtArgs a) {
+  const int b = (int)blockIdx.x, t = threadIdx.x;
+  if (t >= g.cvb_ne[b]) return;
+  const int i = g.cvb_elems[(long)FV_CVB * b + t];
+  const double v[6] = {a.adx2d[i], a.ady2d[i], a.drx2d[i], a.dry2d[i], a.wubot[i], a.wvbot[i]};
+#pragma unroll
+  for (int q = 0; q < 6; ++q) a.own2d[(6L * b + q) * FV_CVB + t] = v[q];
+  const double ua = a.cur.ua[i], va = a.cur.va[i], d1 = a.cur.d1[i];
+  const long p0 = 3L * (i - 1) + 1;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const long q = (long)j * g.n1 + i;
+    a.phi_next[p0 + j] = d1 * (-ua * g.ecv_dy[q] + va * g.ecv_dx[q]);
+  }
 }
 
-// ADVAVE_EDGE_GCN for element i: its three edges' terms gathered in edge
-// order (the reference's scatter order), OBC flux and rivers
-// (advave_edge_gcn.F:746-992).  The element sums are FP64.
+// One 2-D stage by element tile.  A workgroup of 256 lanes takes a compact
+// tile of at most 128 elements (DevGrid::ub_tile; its nodes in st_nodes) and
+// does the whole stage for it, so that neither the edge terms nor the new
+// elevation cross HBM between launches:
+//   1. lanes 0, 1, ..: the least-squares velocity gradients of the tile's
+//      elements and of the other elements of their edges (at most 256), one
+//      element a lane, into LDS; lanes 255, 254, ..: the new elevation of
+//      the tile's nodes, one node a lane;
+//   2. one edge a lane: the ADVAVE_EDGE_GCN edge terms from the two
+//      elements' gradients (at most 256 edges), into LDS;
+//   3. one own element a lane: its three edges' terms summed in edge order,
+//      EXTUV_EDGE, the wall projection and the sub-edge terms of the next
+//      stage.
+// A node on a tile's border is formed by every tile that has it, with the
+// same operations on the same operands, and stored by the first of them.
+// So that no lane can read what another workgroup has already replaced, the
+// sub-edge terms go from one buffer to another, and stages 2-4 read the RK
+// base elevation from a copy (stage 4 writes over the base).
+//
+// Bound: on a large mesh HBM (1,000,000 elements in FP64: 622 MB a stage,
+// 151 us, 4.1 TB/s; as separate elevation, edge and momentum kernels 196 us,
+// 180 with the first two side by side), on a small one the launches and the
+// dependent loads of one tile (3,200 elements: 21 -> 8 us a stage).  The
+// constants come in block order because gathering them by index had every
+// tile wait for one more load and fetch rows of partly used lines (206 ->
+// 164 us); the own elements' data is loaded after the node part, so that
+// their registers do not add up (159 -> 112 VGPRs, 153 us).
+//
+// INT: the same edge terms for ADVAVE_EDGE_GCN of INTERNAL_STEP
+// (internal_step.F:387-392) instead of a stage: ADX2D/ADY2D -= the sums, the
+// accumulators of the coming external steps set to zero
+// (internal_step.F:395-397) and the first stage's sub-edge terms formed.
 template <typename FT>
-__device__ __forceinline__ void advave_gather(const DevGrid& g, int i, const void* ef_, const double* elij,
-                                              const double* ua, const double* va, const double* d1,
-                                              const double* fluxobn, const double* qdis,
-                                              double& xf, double& yf, double& px, double& py) {
-  const EdgeFlux4T<FT>* ef = (const EdgeFlux4T<FT>*)ef_;
-  xf = 0.0; yf = 0.0; px = 0.0; py = 0.0;
-  const double ep = g.epor[i], iu = (double)g.iucp[i], gdi = g.grav_e[i] * d1[i];
-  // the three edges' loads first, then the sums with the side chosen by a
-  // select: no branch separates the loads, so they issue together
-  int ent[3];
-  EdgeFlux4T<FT> r[3];
-  double isbc_tmp[3], el[3], dlx[3], dly[3];
+struct ExtRecsLds {   // one array per quantity: a wave's reads of one spread over the banks
+  FT u[256], v[256], c1[256], c2[256], c5[256], c6[256], p[256], cc[256];
+};
+template <typename FT>
+struct ExtFluxLds {
+  FT xadv[256], yadv[256], fx[256], fy[256];
+  double elij[256], dlx[256], dly[256];
+  int isbc[256];
+};
+
+template <int SMAX, typename FT, bool INT>
+__global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ gp, ExtArgs a) {
+  const DevGrid& g = *gp;   // in device memory: by value its pointers overflow the scalar registers
+  __shared__ ExtRecsLds<FT> sr;
+  __shared__ ExtFluxLds<FT> sf;
+  __shared__ double s_elf[FV_CVB], s_el[FV_CVB], s_d[FV_CVB], s_fobn[FV_CVB];
+  const FT half = (FT)0.5, one = (FT)1.0;
+  const int b = xcd_block(), t = threadIdx.x;
+  const UvBlocks& B = g.ub_tile;
+  // the block-order constants of the first two parts, so that their
+  // latencies overlap
+  const bool ract = t < B.ns[b], eact = t < B.ne[b], oact = t < B.nown[b];
+  const int tn = 255 - t, nn = g.cvb_nn[b];   // lane 255 - tn: the tile's node tn
+  const bool nact = tn < nn, n0 = b == 0 && tn == nn;   // node 0 by block 0
+  const int4 xs = ract ? B.nb4[256L * b + t] : make_int4(0, 0, 0, 0);
+  int4 nd = make_int4(1, 0, -1, -1);
+  if (nact) nd = g.st_node[(long)FV_CVB * b + tn];
+  unsigned pl = 0;
+  double eg[6];   // XIJC-XC, YIJC-YC of IA, the same of IB, DLTXC, DLTYC
+  if (eact) {
+    pl = (unsigned)B.eloc[256L * b + t];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) ent[q] = g.ed_ent[3 * i + q];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int e = ent[q] >> 1;
-    r[q] = ef[e];
-    isbc_tmp[q] = (double)g.isbc[e];
-    el[q] = elij[e];
-    dlx[q] = g.dltxc[e];
-    dly[q] = g.dltyc[e];
+    for (int q = 0; q < 6; ++q) eg[q] = B.egeo[(6L * b + q) * 256 + t];
   }
+  const int i = xs.x;
+  double ua = 0.0, va = 0.0;
+  // 1. gradients
+  if (ract) {
+    FT ra1[4], ra2[4];
+    lsq_coef<FT>(g, i, ra1, ra2);
+    const FT rart = (FT)g.art[i], rcc = (FT)g.cc_hvc[i];
+    ua = a.cur.ua[i];
+    va = a.cur.va[i];
+    const FT us = (FT)ua, u1 = (FT)a.cur.ua[xs.y], u2 = (FT)a.cur.ua[xs.z], u3 = (FT)a.cur.ua[xs.w];
+    const FT vs = (FT)va, v1 = (FT)a.cur.va[xs.y], v2 = (FT)a.cur.va[xs.z], v3 = (FT)a.cur.va[xs.w];
+    const FT c1 = ra1[0] * us + ra1[1] * u1 + ra1[2] * u2 + ra1[3] * u3;
+    const FT c2 = ra2[0] * us + ra2[1] * u1 + ra2[2] * u2 + ra2[3] * u3;
+    const FT c5 = ra1[0] * vs + ra1[1] * v1 + ra1[2] * v2 + ra1[3] * v3;
+    const FT c6 = ra2[0] * vs + ra2[1] * v1 + ra2[2] * v2 + ra2[3] * v3;
+    const FT vis = rart * sqrt(sq(c1) + sq(c6) + half * sq(c2 + c5));
+    sr.u[t] = us; sr.v[t] = vs;
+    sr.c1[t] = c1; sr.c2[t] = c2; sr.c5[t] = c5; sr.c6[t] = c6;
+    sr.p[t] = vis * rcc;
+    sr.cc[t] = rcc;
+  }
+  // 1. nodes
+  if (nact || n0) {
+    const int j = nd.x >> 1, obc = nd.z;
+    const bool keep = (nd.x & 1) != 0;   // this tile stores the node
+    if (nact) {
+      s_el[tn] = a.cur.el[j];
+      s_d[tn] = a.cur.d[j];
+    }
+    if constexpr (INT) {
+      if (keep) {
+        a.egf[j] = 0.0;
+        if (obc >= 0) a.uard_obcn[obc] = 0.0;
+      }
+      if (n0) { a.uard[0] = 0.0; a.vard[0] = 0.0; }
+    } else {
+      double art1, hn;
+      if (nact) {
+        art1 = g.st_nd[2L * b * FV_CVB + tn];
+        hn = g.st_nd[(2L * b + 1) * FV_CVB + tn];
+      } else {
+        art1 = g.art1[0];
+        hn = g.h[0];
+      }
+      const double elrk = a.elrk[j];
+      if (keep && a.elrk_copy) a.elrk_copy[j] = elrk;
+      const int ty = obc >= 0 ? g.type_obc[obc] : 0;
+      // GWI / BKI need their interior neighbour's new elevation: a second
+      // pass forms it, as the tile that has that node does
+      double elf = 0.0, el2 = 0.0, xobc = 0.0;
+      const int* lst = nact ? g.st_list + (long)g.cv_max * b * FV_CVB + tn : g.cvl_ent;
+      long stride = nact ? FV_CVB : g.m1;
+      int id = j, cnt = nd.y, rv = nd.w;
+      double ar = art1, er = elrk;
+      for (bool next = false;;) {
+        double xo;
+        const double e = ext_node_update<SMAX>(g, a, id, lst, stride, cnt, rv, !next && obc >= 0, ar, er, xo);
+        if (next) { el2 = e; break; }
+        elf = e;
+        xobc = xo;
+        if (ty < 5 || ty > 8) break;
+        id = g.next_obc[obc];
+        lst = g.cvl_ent + id;
+        stride = g.m1;
+        cnt = g.cv_cnt[id]; rv = g.node_riv[id];
+        ar = g.art1[id]; er = a.elrk[id];
+        next = true;
+      }
+      if (obc >= 0) {
+        elf = ext_obc_value(g, a, j, obc, ty, elrk, elf, el2);
+        // FLUX_OBN's flux defect (mod_obcs.F:1196) and, in the last stage,
+        // the node's UARD_OBCN share (external_step.F:423-430)
+        if (nact) s_fobn[tn] = -(elf - elrk) * art1 / (a.alpha * g.dte) - xobc;
+        if (a.K == 4 && keep) {
+          const double tmp = -(elf - elrk) * art1 / g.dte - xobc;
+          a.uard_obcn[obc] = a.uard_obcn[obc] + tmp / (double)g.isplit;
+        }
+      }
+      if (nact) s_elf[tn] = elf;
+      if (keep) {
+        const double dnew = hn + elf;
+        a.nxt.el[j] = elf;
+        a.nxt.d[j] = dnew;
+        if (a.K == 3) a.egf[j] = a.egf[j] + elf / (double)g.isplit;
+        if (j >= 1 && dnew < g.min_depth) a.clk->depth_fail = 1;
+      }
+    }
+  }
+  // the element part's constants and state (the block's own elements are its
+  // first records): issued before the barrier, after the node part, whose
+  // registers are free again
+  int4 oe = make_int4(0, 0, 0, 0);
+  double ed[12], own[6], d1 = 0.0, el1b = 0.0, uab = 0.0, vab = 0.0, wsx = 0.0, wsy = 0.0;
+  if (oact) {
+    oe = g.st_elem[(long)FV_CVB * b + t];
+#pragma unroll
+    for (int q = 0; q < 12; ++q) ed[q] = g.st_ed[(12L * b + q) * FV_CVB + t];
+    d1 = a.cur.d1[i];
+    if constexpr (INT) {
+      own[0] = a.adx2d[i]; own[1] = a.ady2d[i]; own[2] = a.drx2d[i]; own[3] = a.dry2d[i];
+      own[4] = a.wubot[i]; own[5] = a.wvbot[i];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) own[q] = a.own2d[(6L * b + q) * FV_CVB + t];
+      el1b = a.base.el1[i]; uab = a.base.ua[i]; vab = a.base.va[i];
+      if (g.wind_on) { wsx = a.ws2x[i]; wsy = a.ws2y[i]; }
+    }
+  }
+  __syncthreads();
+  // 2. edge terms
+  if (eact) {
+    const int sa = pl & 255, sb = (pl >> 8) & 255, n1 = (pl >> 16) & 127, n2 = (pl >> 23) & 127;
+    const FT dij = half * ((FT)s_d[n1] + (FT)s_d[n2]);
+    const FT xija = (FT)eg[0], yija = (FT)eg[1], xijb = (FT)eg[2], yijb = (FT)eg[3], dlx = (FT)eg[4],
+             dly = (FT)eg[5];
+    const FT cofa1 = sr.c1[sa], cofa2 = sr.c2[sa], cofa5 = sr.c5[sa], cofa6 = sr.c6[sa];
+    const FT cofa3 = sr.c1[sb], cofa4 = sr.c2[sb], cofa7 = sr.c5[sb], cofa8 = sr.c6[sb];
+    const FT uij1 = sr.u[sa] + cofa1 * xija + cofa2 * yija;
+    const FT vij1 = sr.v[sa] + cofa5 * xija + cofa6 * yija;
+    const FT uij2 = sr.u[sb] + cofa3 * xijb + cofa4 * yijb;
+    const FT vij2 = sr.v[sb] + cofa7 * xijb + cofa8 * yijb;
+    const FT uij = half * (uij1 + uij2), vij = half * (vij1 + vij2);
+    const FT un_tmp = -uij * dly + vij * dlx;
+    FT viscof = (FT)g.fact * half * (sr.p[sa] + sr.p[sb]) + (FT)g.fm1 * half * (sr.cc[sa] + sr.cc[sb]);
+    if ((FT)g.hprnu != one) viscof = viscof / (FT)g.hprnu;   // x / 1 is x
+    const FT txxij = (cofa1 + cofa3) * viscof;
+    const FT tyyij = (cofa6 + cofa8) * viscof;
+    const FT txyij = half * (cofa2 + cofa4 + cofa5 + cofa7) * viscof;
+    sf.fx[t] = dij * (txxij * dly - txyij * dlx);
+    sf.fy[t] = dij * (txyij * dly - tyyij * dlx);
+    const FT sgn = fsign1(un_tmp);
+    sf.xadv[t] = dij * un_tmp * ((one - sgn) * uij2 + (one + sgn) * uij1) * half;
+    sf.yadv[t] = dij * un_tmp * ((one - sgn) * vij2 + (one + sgn) * vij1) * half;
+    sf.elij[t] = 0.5 * (s_el[n1] + s_el[n2]);
+    sf.dlx[t] = eg[4];
+    sf.dly[t] = eg[5];
+    sf.isbc[t] = (int)(pl >> 30);
+  }
+  __syncthreads();
+  if (!oact) return;
+  // 3. FLUX_OBN: contributions to this open-boundary element, in OBC order
+  const int ep3 = oe.x, nl = oe.y, isb = oe.z & 3;
+  const double ep = ed[0], ge = ed[1], art = ed[2], cor = ed[3], h1 = ed[4], spg = ed[5], iu = (double)oe.w;
+  double fl = 0.0;
+  if (isb == 2) {
+    if constexpr (INT) {
+      fl = a.fluxobn[i];
+    } else {
+      for (int p = g.fo_off[i]; p < g.fo_off[i + 1]; ++p) {
+        const int ent = g.fo_obc[p], ob = ent >> 1, slot = ent & 1;
+        const int j = g.i_obc_n[ob];   // one of the element's nodes
+        const int ln = j == NV_(i, 1) ? nl & 255 : j == NV_(i, 2) ? (nl >> 8) & 255 : (nl >> 16) & 255;
+        fl = fl + g.fluxf_obc[(long)slot * g.IOBCN + ob] * s_fobn[ln];
+      }
+      a.fluxobn[i] = fl;
+    }
+  }
+  // ADVAVE_EDGE_GCN's sums (advave_edge_gcn.F:746-992) in edge order
+  double xf = 0.0, yf = 0.0, px = 0.0, py = 0.0;
+  const double gdi = ge * d1;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    const double xadv = (double)r[q].xadv, yadv = (double)r[q].yadv, fx = (double)r[q].fx, fy = (double)r[q].fy;
-    const double gd = gdi * el[q];
-    const double tx = (xadv + fx * ep) * (1.0 - isbc_tmp[q]) * iu;
-    const double ty = (yadv + fy * ep) * (1.0 - isbc_tmp[q]) * iu;
-    const double gy = gd * dly[q], gx = gd * dlx[q];
-    const bool ib = (ent[q] & 1) != 0;
+    const int s = (ep3 >> (8 * q)) & 255;
+    const bool ib = (ep3 >> (24 + q)) & 1;   // the element is IB of the edge
+    const double xadv = (double)sf.xadv[s], yadv = (double)sf.yadv[s], fx = (double)sf.fx[s], fy = (double)sf.fy[s];
+    const double isbc_tmp = (double)sf.isbc[s];
+    const double gd = gdi * sf.elij[s];
+    const double tx = (xadv + fx * ep) * (1.0 - isbc_tmp) * iu;
+    const double ty = (yadv + fy * ep) * (1.0 - isbc_tmp) * iu;
+    const double gy = gd * sf.dly[s], gx = gd * sf.dlx[s];
     xf = ib ? xf - tx : xf + tx;
     yf = ib ? yf - ty : yf + ty;
     px = ib ? px + gy : px - gy;
     py = ib ? py - gx : py + gx;
   }
-  if (g.isbce[i] == 2) {
-    xf = (xf + fluxobn[i] * ua[i]) * (double)g.iucp[i];
-    yf = (yf + fluxobn[i] * va[i]) * (double)g.iucp[i];
+  if (isb == 2) {
+    xf = (xf + fl * ua) * iu;
+    yf = (yf + fl * va) * iu;
   }
-  for (int p = g.re_off[i]; p < g.re_off[i + 1]; ++p) {
-    // a node river's momentum is split between two cells, an edge river's
-    // enters its cell whole (advave_edge_gcn.F:971-992)
-    const int k = g.re_riv[p];
-    const double fq = g.icellq[k] > 0 ? 1.0 : 0.5;
-    const double vlctyq = qdis[k] / g.qarea[k];
-    xf = xf - fq * qdis[k] * vlctyq * g.cos_angleq[k];
-    yf = yf - fq * qdis[k] * vlctyq * g.sin_angleq[k];
+  if (oe.z & 4) {
+    for (int p = g.re_off[i]; p < g.re_off[i + 1]; ++p) {
+      // a node river's momentum is split between two cells, an edge river's
+      // enters its cell whole (advave_edge_gcn.F:971-992)
+      const int k = g.re_riv[p];
+      const double fq = g.icellq[k] > 0 ? 1.0 : 0.5;
+      const double vlctyq = a.qdis[k] / g.qarea[k];
+      xf = xf - fq * a.qdis[k] * vlctyq * g.cos_angleq[k];
+      yf = yf - fq * a.qdis[k] * vlctyq * g.sin_angleq[k];
+    }
   }
-}
-
-// EXTEL terms of element i's three sub-edges (side IB), element-major.
-__device__ __forceinline__ void ext_phi_store(const DevGrid& g, int i, double ua, double va, double d1,
-                                              double* phi) {
+  double un = ua, vn = va, dn = d1;
+  if constexpr (INT) {
+    own[0] = own[0] - xf;
+    own[1] = own[1] - yf;
+    a.adx2d[i] = own[0];
+    a.ady2d[i] = own[1];
+    a.uard[i] = 0.0;
+    a.vard[i] = 0.0;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) a.own2d[(6L * b + q) * FV_CVB + t] = own[q];
+  } else {
+    // EXTUV_EDGE
+    const double one_third = 1.0 / 3.0, ramp = a.ec->ramp;
+    const double elf1 = one_third * (s_elf[nl & 255] + s_elf[(nl >> 8) & 255] + s_elf[(nl >> 16) & 255]);
+    const double wus2 = g.wind_on ? wsx * ramp * 0.001 : 0.0;
+    const double wvs2 = g.wind_on ? wsy * ramp * 0.001 : 0.0;
+    const double resx = own[0] + xf + own[2] + px - cor * va * d1 * art - (wus2 + own[4]) * art;
+    const double resy = own[1] + yf + own[3] + py + cor * ua * d1 * art - (wvs2 + own[5]) * art;
+    un = (uab * (h1 + el1b) - a.alpha * g.dte * resx / art) / (h1 + elf1);
+    vn = (vab * (h1 + el1b) - a.alpha * g.dte * resy / art) / (h1 + elf1);
+    un = un / (1.0 + spg * un * un);
+    vn = vn / (1.0 + spg * vn * vn);
+    if (isb != 0) wall_project(g, i, un, vn);
+    dn = h1 + elf1;
+    a.nxt.ua[i] = un;
+    a.nxt.va[i] = vn;
+    a.nxt.el1[i] = elf1;
+    a.nxt.d1[i] = dn;
+    if (a.K == 3) {
+      a.uard[i] = a.uard[i] + un * dn;
+      a.vard[i] = a.vard[i] + vn * dn;
+    }
+  }
+  // the next stage's EXTEL terms of the element's sub-edges (side IB)
   const long p0 = 3L * (i - 1) + 1;
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const long q = (long)j * g.n1 + i;
-    phi[p0 + j] = d1 * (-ua * g.ecv_dy[q] + va * g.ecv_dx[q]);
-  }
-}
-
-// The EXTEL terms of a 2-D state (before its first stage).
-__global__ __launch_bounds__(256) void k_ext_phi(DevGrid g, const double* ua, const double* va, const double* d1,
-                                                 double* phi) {
-  const int i = (int)xcd_thread() + 1;
-  if (i > g.N) return;
-  ext_phi_store(g, i, ua[i], va[i], d1[i], phi);
-}
-
-template <typename FT>
-__global__ void k_ext_momentum(DevGrid g, ExtArgs a) {
-  const int i = (int)xcd_thread();
-  if (i < 1 || i > g.N) return;
-  const double one_third = 1.0 / 3.0;
-  const double elf1 = one_third * (a.nxt.el[NV_(i, 1)] + a.nxt.el[NV_(i, 2)] + a.nxt.el[NV_(i, 3)]);
-  // FLUX_OBN: contributions to this open-boundary element, in OBC order
-  if (g.isbce[i] == 2) {
-    double f = 0.0;
-    for (int p = g.fo_off[i]; p < g.fo_off[i + 1]; ++p) {
-      const int ent = g.fo_obc[p], ob = ent >> 1, slot = ent & 1;
-      f = f + g.fluxf_obc[(long)slot * g.IOBCN + ob] * a.fobn[ob];
-    }
-    a.fluxobn[i] = f;
-  }
-  double xf, yf, px, py;
-  advave_gather<FT>(g, i, a.ef, a.elij, a.cur.ua, a.cur.va, a.cur.d1, a.fluxobn, a.qdis, xf, yf, px, py);
-  // EXTUV_EDGE
-  const double ua = a.cur.ua[i], va = a.cur.va[i], d1 = a.cur.d1[i], art = g.art[i], cor = g.cor[i];
-  const double ramp = a.clk->ramp_ext;
-  const double wus2 = g.wind_on ? a.ws2x[i] * ramp * 0.001 : 0.0;
-  const double wvs2 = g.wind_on ? a.ws2y[i] * ramp * 0.001 : 0.0;
-  const double resx = a.adx2d[i] + xf + a.drx2d[i] + px - cor * va * d1 * art - (wus2 + a.wubot[i]) * art;
-  const double resy = a.ady2d[i] + yf + a.dry2d[i] + py + cor * ua * d1 * art - (wvs2 + a.wvbot[i]) * art;
-  const double h1 = g.h1[i], elrk1 = a.base.el1[i];
-  double uaf = (a.base.ua[i] * (h1 + elrk1) - a.alpha * g.dte * resx / art) / (h1 + elf1);
-  double vaf = (a.base.va[i] * (h1 + elrk1) - a.alpha * g.dte * resy / art) / (h1 + elf1);
-  uaf = uaf / (1.0 + g.cc_sponge[i] * uaf * uaf);
-  vaf = vaf / (1.0 + g.cc_sponge[i] * vaf * vaf);
-  wall_project(g, i, uaf, vaf);
-  const double d1n = h1 + elf1;
-  a.nxt.ua[i] = uaf;
-  a.nxt.va[i] = vaf;
-  a.nxt.el1[i] = elf1;
-  a.nxt.d1[i] = d1n;
-  ext_phi_store(g, i, uaf, vaf, d1n, a.phi);
-  if (a.K == 3) {
-    a.uard[i] = a.uard[i] + uaf * d1n;
-    a.vard[i] = a.vard[i] + vaf * d1n;
-  }
-}
-
-// Start of EXTERNAL_STEP: clock and RAMP (external_step.F:83-88).
-__global__ void k_ext_clock(DevClock* c, int iext) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  c->iext = iext;
-  c->ext_time = c->time0 + (double)(c->iint - 1) * c->dti + (double)iext * c->dte;
-  if (c->iramp != 0) {
-    const double tmp = (double)(c->iint - 1) + (double)iext / (double)c->isplit;
-    c->ramp_ext = fv_tanh(tmp / (double)c->iramp);
-  } else {
-    c->ramp_ext = 1.0;
-  }
+  for (int j = 0; j < 3; ++j) a.phi_next[p0 + j] = dn * (-un * ed[9 + j] + vn * ed[6 + j]);
 }

@@ -27,8 +27,6 @@ struct IntArgs {
   double* gx;            // node-layer scratch (PROD of VDIF_Q)
   double *elm1, *elm2;   // the elevation one and two RK stages back (Orlanski OBC)
   // flux buffers, of the flux type FT (double, or float in the mixed form)
-  void* ef2;             // per-edge ADVAVE terms (2-D), EdgeFlux4T<FT>
-  double* elij2;         // per-edge mean elevation (2-D)
   void* rec;             // node-layer records of the field being advected, CvRecT<FT>
   double2* vhpair;       // node-layer pair scratch: VDIF_Q's elimination coefficients
   double* obcsum;        // BCOND_TS column sums, 5 per OBC node
@@ -44,13 +42,24 @@ struct IntArgs {
 
 #define GRID1(n) (((n) + 255) / 256), 256
 
-// Start of INTERNAL_STEP (internal_step.F:115-120) and BCOND_GCN(8,0) rivers.
-__global__ void k_int_clock(DevGrid g, DevClock* c, double* qdis) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  c->iint += 1;
-  if (c->iramp != 0) c->ramp_int = fv_tanh((double)c->iint / (double)c->iramp);
-  else c->ramp_int = 1.0;
-  for (int j = 0; j < g.NUMQBC; ++j) qdis[j] = g.qdis0[j] * c->ramp_int;
+// Start of INTERNAL_STEP (internal_step.F:115-120), BCOND_GCN(8,0) rivers,
+// and the clocks and RAMPs of its external steps iext0 .. iext0+n-1
+// (external_step.F:83-88) into ec[0 .. n-1].  One workgroup.
+__global__ void k_int_clock(DevGrid g, DevClock* c, double* qdis, ExtClock* ec, int iext0, int n) {
+  const long long iint = c->iint + 1;
+  const double ramp = c->iramp != 0 ? fv_tanh((double)iint / (double)c->iramp) : 1.0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    c->iint = iint;
+    c->ramp_int = ramp;
+  }
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    const int iext = iext0 + q;
+    ec[q].time = c->time0 + (double)(iint - 1) * c->dti + (double)iext * c->dte;
+    const double tmp = (double)(iint - 1) + (double)iext / (double)c->isplit;
+    ec[q].ramp = c->iramp != 0 ? fv_tanh(tmp / (double)c->iramp) : 1.0;
+  }
+  for (int j = threadIdx.x; j < g.NUMQBC; j += blockDim.x) qdis[j] = g.qdis0[j] * ramp;
 }
 
 __global__ void k_zero(double* p, long n) {
@@ -208,21 +217,6 @@ __global__ void k_rho1_roundtrip(DevGrid g, IntArgs a) {
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= (long)g.KBM1 * g.m1) return;
   a.rho1[q] = (a.rho1[q] - a.rmean1[q]) + a.rmean1[q];
-}
-
-// Ext-mode ADVAVE of INTERNAL_STEP and GX/GY (internal_step.F:387-392),
-// plus the zeroing of UARD/VARD (internal_step.F:395-397).
-template <typename FT>
-__global__ void k_advave_int(DevGrid g, IntArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > g.N) return;
-  a.uard[i] = 0.0;
-  a.vard[i] = 0.0;
-  if (i < 1) return;
-  double xf, yf, px, py;
-  advave_gather<FT>(g, i, a.ef2, a.elij2, a.ua, a.va, a.d1, a.fluxobn, a.qdis, xf, yf, px, py);
-  a.adx2d[i] = a.adx2d[i] - xf;
-  a.ady2d[i] = a.ady2d[i] - yf;
 }
 
 // ADJUST2D3D(2) (adjust2d3d.F:65-110).

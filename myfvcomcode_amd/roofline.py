@@ -24,36 +24,19 @@ def sizes(model):
 
 
 # ----------------------------------------------------------------- 2-D mode
-def ext_elevation(s, real=R8):
-    """EXTEL_EDGE gather + elevation update (one RK stage)."""
-    M, N, NCV = s["M"], s["N"], s["NCV"]
-    reads = (M * (3 * I4 + 3 * real)          # cv_cnt, node_obc, node_riv; ELRK, ART1, H
-             + 2 * NCV * I4                   # slot-major sub-edge lists (term position, side)
-             + NCV * real)                    # the stage input's EXTEL term of every sub-edge
-    writes = M * 2 * real                     # EL, D of the stage output
-    return reads + writes
-
-
-def advave_edge(s, real=R8):
-    """ADVAVE_EDGE_GCN edge terms, one thread per edge."""
-    M, N, NE = s["M"], s["N"], s["NE"]
-    reads = (NE * (4 * I4 + 4 * real)         # IEC, IENODE; XIJC, YIJC, DLTXC, DLTYC
-             + N * (3 * I4 + 8 * real + 4 * real + 2 * real)  # NBE; A1U, A2U; XC, YC, ART, CC_HVC; UA, VA
-             + M * 2 * real)                  # D, EL
-    writes = NE * (4 * real + real)           # EdgeFlux4 + ELIJ
-    return reads + writes
-
-
 def ext_momentum(s, real=R8):
-    """Edge-term gather + EXTUV_EDGE + wall projection (one RK stage)."""
-    M, N, NE = s["M"], s["N"], s["NE"]
-    elem_reals = 20   # EPOR GRAV_E D1 UA VA ART COR WSX WSY ADX2D ADY2D DRX2D DRY2D WUBOT WVBOT H1 EL1 UARK VARK CC_SPONGE
-    elem_ints = 9     # NV(3), edge list(3), IUCP, ISBCE, river offset
-    reads = (N * (elem_reals * real + elem_ints * I4)
-             + NE * (4 * real + real + I4 + 2 * real)  # EdgeFlux4, ELIJ, ISBC, DLTXC, DLTYC
-             + N * 6 * real                            # DLTXE/DLTYE of the element's 3 sub-edges
-             + M * real)                               # new EL
-    writes = N * 4 * real + N * 3 * real               # UA, VA, EL1, D1; EXTEL terms of the next stage
+    """One RK stage by element tile (k_ext_stage): elevation, edge terms and
+    momentum in one launch.  Each element's, edge's and node's constants and
+    state once; a tile's halo (about 0.35 records, 0.26 edges and 0.15 nodes
+    per element again) is traffic, not counted here."""
+    M, N, NE, NCV = s["M"], s["N"], s["NE"], s["NCV"]
+    reads = (N * (4 * I4 + 10 * real)                  # neighbours; A1U, A2U, ART, CC_HVC
+             + N * (4 * I4 + 12 * real + 6 * real)     # flags; EPOR .. DLTYE; ADX2D .. WVBOT
+             + N * (2 + 3 + 1 + 2) * real              # UA, VA; UARK, VARK, ELRK1; D1; wind stress
+             + NE * (I4 + 6 * real)                    # edge slots; edge geometry
+             + M * (4 * I4 + 5 * real) + 2 * NCV * I4  # node flags; ART1, H, ELRK, EL, D; sub-edge lists
+             + NCV * real)                             # EXTEL terms
+    writes = N * 4 * real + NCV * real + M * 2 * real  # UA, VA, EL1, D1; next EXTEL terms; EL, D
     return reads + writes
 
 
@@ -220,7 +203,7 @@ def n2e3d(s, real=R8):
 
 
 FAMILIES = {f.__name__: f for f in (
-    ext_elevation, advave_edge, ext_momentum, cvrec_ts, cvrec_q, cvflux_ts, cvflux_q, cvrecflux_ts, cvrecflux_q,
+    ext_momentum, cvrec_ts, cvrec_q, cvflux_ts, cvflux_q, cvrecflux_ts, cvrecflux_q,
     adv_ts, adv_q,
     adv3d_blk, advuv_blk, vertvl, viscofh, vdif_q, vdif_uv, vdif_ts,
     n2e3d)}
