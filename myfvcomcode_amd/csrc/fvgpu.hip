@@ -247,6 +247,32 @@ int block_of(const fvgpu_handle* h, const char* name) {
                        h->cur, __VA_ARGS__);                                                      \
   } while (0)
 
+// How many shares the n layers of a kernel are split into (its grid's y
+// extent) whose layers are independent of one another, given its workgroups
+// per layer: so many that about `per_cu` workgroups a CU are in the grid -- a
+// mesh with fewer leaves CUs idle while each of its lanes walks the column
+// alone -- but at least 2 layers a share, over which a lane's constants and
+// lists are read once.  3 is what the registers of these kernels let a CU
+// hold: more measured slower (62,500 elements x 40 layers, one graph a step:
+// 2.14 ms unsplit, 1.94 at 3, 1.96 at 6, 2.02 at 12; 250,000 x 20: 3.28,
+// 3.27, 3.28, 3.35; from 768 workgroups a layer on, nothing is split and
+// nothing changes), but for ADV_UV, whose grid is the most uneven, 6 (62,500
+// elements: 161 us unsplit, 137 at 3, 130 at 6).  adv_ts at 17,000 elements x
+// 20: 52 -> 17 us, at 62,500 x 40: 101 -> 48 us.
+unsigned layer_chunks(const fvgpu_handle* h, long workgroups, int n, int per_cu) {
+  const long want = ((long)per_cu * h->cu_count + workgroups - 1) / std::max(workgroups, 1l);
+  return (unsigned)std::max(1l, std::min(want, (long)n / 2));
+}
+// TLAUNCH of such a kernel over n layers.
+#define TLAUNCH_LAYERS(NAME, KERNEL, NITEMS, NLAYERS, PER_CU, ...)                                  \
+  do {                                                                                            \
+    const int bs_ = block_of(h, NAME);                                                            \
+    const unsigned nb_ = (unsigned)(((long)(NITEMS) + bs_ - 1) / bs_);                            \
+    Launch l_(h, NAME);                                                                           \
+    hipLaunchKernelGGL(KERNEL, dim3(nb_, layer_chunks(h, nb_, NLAYERS, PER_CU)), dim3(bs_), 0,     \
+                       h->cur, __VA_ARGS__);                                                      \
+  } while (0)
+
 // Fork: work enqueued on stream2 after this waits for everything enqueued
 // on the main stream so far.  Join: the main stream waits for stream2.
 // Under graph capture the events become dependency edges of the graph.
@@ -337,11 +363,11 @@ void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
     FV_RMAX_DISPATCH(g.ring_max, CVREC_TS_CALL);
     TLAUNCH("cvflux_ts", k_cvflux_ts<FT>, g.N + 1, g, a);
   } else {
-#define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT>), g.cvb_nblk, 256, g, a, f1, fm, 0.0)
+#define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1, 3)), 256, g, a, f1, fm, 0.0)
     FV_RMAX_DISPATCH(g.ring_max, CVRF_TS_CALL);
   }
-#define ADV_TS_CALL10(SM) TLAUNCH("adv_ts", (k_adv_ts_gather<SM, 10, FT>), g.M + 1, g, a, f1, ff, fdis, which, fct)
-#define ADV_TS_CALL16(SM) TLAUNCH("adv_ts", (k_adv_ts_gather<SM, 16, FT>), g.M + 1, g, a, f1, ff, fdis, which, fct)
+#define ADV_TS_CALL10(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 10, FT>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
+#define ADV_TS_CALL16(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 16, FT>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL10);
   else FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL16);
   if (g.IOBCN > 0) {
@@ -368,11 +394,11 @@ void enqueue_adv_q(fvgpu_handle* h, IntArgs& a, double* q, double* qf, int fct) 
     FV_RMAX_DISPATCH(g.ring_max, CVREC_Q_CALL);
     TLAUNCH("cvflux_q", k_cvflux_q<FT>, g.N + 1, g, a);
   } else {
-#define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT>), g.cvb_nblk, 256, g, a, q, nullptr, qmean1)
+#define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1 - 1, 3)), 256, g, a, q, nullptr, qmean1)
     FV_RMAX_DISPATCH(g.ring_max, CVRF_Q_CALL);
   }
-#define ADV_Q_CALL10(SM) TLAUNCH("adv_q", (k_adv_q_gather<SM, 10, FT>), g.M + 1, g, a, q, qf, fct)
-#define ADV_Q_CALL16(SM) TLAUNCH("adv_q", (k_adv_q_gather<SM, 16, FT>), g.M + 1, g, a, q, qf, fct)
+#define ADV_Q_CALL10(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 10, FT>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
+#define ADV_Q_CALL16(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 16, FT>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL10);
   else FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL16);
 }
@@ -398,9 +424,9 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
 #define VERTVL_CALL(SM) LAUNCH("vertvl", k_vertvl_tile<SM>, g.nt_nblk, 256, g, a)
   FV_SMAX_DISPATCH(g.cv_max, VERTVL_CALL);
   N2E3D(a.wts, a.w);
-#define VISCOFH_CALL(RM) TLAUNCH("viscofh", k_viscofh_r<RM>, g.M + 1, g, a)
+#define VISCOFH_CALL(RM) TLAUNCH_LAYERS("viscofh", k_viscofh_r<RM>, g.M + 1, g.KBM1, 3, g, a)
   FV_RMAX_DISPATCH(g.ve_max, VISCOFH_CALL);
-  LAUNCH("advuv_blk", (k_uv_blk<1, FT>), g.ub_run.nblk, 256, g, a);
+  LAUNCH("advuv_blk", (k_uv_blk<1, FT>), dim3(g.ub_run.nblk, layer_chunks(h, g.ub_run.nblk, g.KBM1, 6)), 256, g, a);
 #define VDIF_UV_CALL(KM) LAUNCH("vdif_uv", k_vdif_uv_r<KM>, dim3(nb(g.N + 1), 2), 256, g, a)
   FV_KMAX_DISPATCH(g.KBM1, VDIF_UV_CALL);
   TLAUNCH("uv_finish", k_uv_finish, (long)g.N * g.KBM1, g, a);
@@ -411,7 +437,7 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     // MY2.5 column solve (without horizontal advection of Q2/Q2L) for the
     // rejected columns only
     const long ns = (long)g.M * (g.KBM1 - 1);
-#define CLF_CALL(RM) TLAUNCH("closure_features", k_closure_features<RM>, g.M, g, a, h->cl_x, (float*)nullptr)
+#define CLF_CALL(RM) TLAUNCH_LAYERS("closure_features", k_closure_features<RM>, g.M, g.KBM1 - 1, 3, g, a, h->cl_x, (float*)nullptr)
     FV_RMAX_DISPATCH(g.ve_max, CLF_CALL);
     LAUNCH("closure_infer", k_mlp_infer_mfma, (unsigned)std::min<long>((ns + 31) / 32, 8192), 64, h->cl_w, h->cl_x, ns,
            h->cl_yp);

@@ -85,9 +85,12 @@ __global__ __launch_bounds__(256) void k_closure_features(DevGrid g, IntArgs a, 
     });
     return s / ntd;
   };
-  double um = ring_avg(a.u, 0), vm = ring_avg(a.v, 0);
+  int k0, k1;
+  layer_share(2, g.KBM1, k0, k1);
+  if (k0 > k1) return;
+  double um = ring_avg(a.u, (long)(k0 - 2) * g.n1), vm = ring_avg(a.v, (long)(k0 - 2) * g.n1);
   const float ld = (float)log10(d > 1e-3 ? d : 1e-3) - 1.0f;
-  for (int k = 2; k <= g.KBM1; ++k) {
+  for (int k = k0; k <= k1; ++k) {
     const long q = NI(g, i, k), eo = (long)(k - 1) * g.n1;
     const double dzd = DZZ(i, k - 1) * d;
     const double n2 = -g.grav_n[i] * (a.rho1[q - g.m1] - a.rho1[q]) / dzd;

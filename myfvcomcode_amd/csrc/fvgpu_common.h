@@ -141,6 +141,15 @@ __device__ __forceinline__ int xcd_block() {
 }
 __device__ __forceinline__ long xcd_thread() { return (long)xcd_block() * blockDim.x + threadIdx.x; }
 
+// The layers of this workgroup's share of [first, last] where a kernel's
+// layers are split over gridDim.y (layer_chunks of the host side); k0 > k1:
+// none.
+__device__ __forceinline__ void layer_share(int first, int last, int& k0, int& k1) {
+  const int c = (last - first + (int)gridDim.y) / (int)gridDim.y;
+  k0 = first + (int)blockIdx.y * c;
+  k1 = min(k0 + c - 1, last);
+}
+
 // 1-based layer accessors
 __device__ __forceinline__ long NI(const DevGrid& g, int i, int k) { return (long)(k - 1) * g.m1 + i; }
 __device__ __forceinline__ long EI(const DevGrid& g, int i, int k) { return (long)(k - 1) * g.n1 + i; }

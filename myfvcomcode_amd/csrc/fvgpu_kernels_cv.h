@@ -369,7 +369,9 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
   const long cs = (long)g.NCV + 1;
   int rn[RMAX];
   const int nt = clip ? load_ring<RMAX>(g, i, rn) : 0;
-  for (int k = 1; k <= g.KBM1; ++k) {
+  int k0, k1;
+  layer_share(1, g.KBM1, k0, k1);
+  for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.m1;
     const FT* fl = (const FT*)a.cvflux + (long)(k - 1) * cs;
     // all SMAX loads issue together (slots past the node's count read the
@@ -513,8 +515,10 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
                                                    double cmean) {
   __shared__ CvRecLds<FT> srec[2];
   const int b = xcd_block(), t = threadIdx.x;
-  const int k0 = KIND == 0 ? 1 : 2;
-  const int nk = g.KBM1 - k0 + 1;   // layers (interfaces) of the pass
+  int k0, k1;
+  layer_share(KIND == 0 ? 1 : 2, g.KBM1, k0, k1);
+  const int nk = k1 - k0 + 1;       // layers (interfaces) of this workgroup
+  if (nk < 1) return;
   // The role is taken from the wave's first lane, so that the branch is
   // uniform over each wave and both roles pass nk + 1 barriers.
   if (__builtin_amdgcn_readfirstlane(t) < FV_CVB) {
@@ -556,7 +560,9 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
     const FT fact = (FT)g.fact, rhprnu = (FT)g.hprnu, one = (FT)1.0;
     const double dt1 = a.dt1[e];
     const long cs = (long)g.NCV + 1, p0 = 3L * (e - 1) + 1;
-    double um = a.u[e], vm = a.v[e];   // layer 1 (ADV_Q's interface interpolation)
+    // the layer above (ADV_Q's interface interpolation)
+    const long em = (long)(KIND == 1 ? k0 - 2 : 0) * g.n1 + e;
+    double um = a.u[em], vm = a.v[em];
     for (int s = 0; s <= nk; ++s) {
       if (s > 0) {
         const int k = k0 + s - 1;
@@ -591,7 +597,8 @@ __global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, cons
   const int i = (int)xcd_thread();
   if (i > g.M) return;
   if (i == 0) {
-    for (int k = 1; k <= g.KB; ++k) qf[NI(g, 0, k)] = 0.0;
+    if (blockIdx.y == 0)
+      for (int k = 1; k <= g.KB; ++k) qf[NI(g, 0, k)] = 0.0;
     return;
   }
   const int n = g.cv_cnt[i];
@@ -605,9 +612,13 @@ __global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, cons
   const bool clip = fct && !g.fct_skip[i];
   int rn[RMAX];
   const int nt = clip ? load_ring<RMAX>(g, i, rn) : 0;
-  qf[NI(g, i, 1)] = 0.0;
-  qf[NI(g, i, g.KB)] = 0.0;
-  for (int k = 2; k <= g.KBM1; ++k) {
+  if (blockIdx.y == 0) {
+    qf[NI(g, i, 1)] = 0.0;
+    qf[NI(g, i, g.KB)] = 0.0;
+  }
+  int k0, k1;
+  layer_share(2, g.KBM1, k0, k1);
+  for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.m1;
     const FT* fl = (const FT*)a.cvflux + (long)(k - 1) * cs;
     // all SMAX loads issue together (slots past the node's count read the
@@ -801,7 +812,9 @@ __global__ __launch_bounds__(256) void k_viscofh_r(DevGrid g, IntArgs a) {
   const double nx0 = bnd ? g.dltxnec[o] : 0.0, ny0 = bnd ? g.dltynec[o] : 0.0;
   const double nxl = bnd ? g.dltxnec[o + jl] : 0.0, nyl = bnd ? g.dltynec[o + jl] : 0.0;
   const double art1 = g.art1[i];
-  for (int k = 1; k <= g.KBM1; ++k) {
+  int k0, k1;
+  layer_share(1, g.KBM1, k0, k1);
+  for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.n1;
     // the ring's velocities are loaded unconditionally (slots past the ring
     // read element 0) so that the loads issue together

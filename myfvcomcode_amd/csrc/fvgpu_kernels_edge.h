@@ -50,7 +50,11 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
   const FT half = (FT)0.5, one = (FT)1.0;
   const double* U = a.u;
   const double* V = a.v;
-  if (MODE == 1 && b == 0 && t == 0)
+  // ADVECTION sums over the column: its layers are not split
+  int k0 = 1, k1 = g.KBM1;
+  if (MODE == 1) layer_share(1, g.KBM1, k0, k1);
+  if (k0 > k1) return;
+  if (MODE == 1 && b == 0 && t == 0 && k0 == 1)
     for (int k = 1; k <= g.KB; ++k) a.viscofm[EI(g, 0, k)] = 0.0;
   // 1. record part: element x
   const UvBlocks& B = MODE == 0 ? g.ub_tile : g.ub_run;
@@ -104,8 +108,12 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
   double pu[4], pv[4];
   const int xs[4] = {x, x1, x2, x3};
 #pragma unroll
-  for (int q = 0; q < 4; ++q) { pu[q] = U[xs[q]]; pv[q] = V[xs[q]]; }
-  for (int k = 1; k <= g.KBM1; ++k) {
+  for (int q = 0; q < 4; ++q) {
+    const long f = (long)(k0 - 1) * g.n1 + xs[q];
+    pu[q] = U[f];
+    pv[q] = V[f];
+  }
+  for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.n1;
     // this layer's inputs of the edge and element parts, issued before the
     // record arithmetic and the barriers (every index is valid for idle lanes)
@@ -130,7 +138,7 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
       sr.c1[t] = c1; sr.c2[t] = c2; sr.c5[t] = c5; sr.c6[t] = c6;
       sr.p[t] = vis * rcc;
     }
-    if (k < g.KBM1) {
+    if (k < k1) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) { pu[q] = U[kp + xs[q]]; pv[q] = V[kp + xs[q]]; }
     }
@@ -233,7 +241,7 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
   if (oact) {
     if (MODE == 0) {
       (cy ? a.ady2d : a.adx2d)[i] = sc;
-    } else if (!cy) {
+    } else if (!cy && k1 == g.KBM1) {
       a.viscofm[EI(g, i, g.KB)] = 0.0 / art;
     }
   }
