@@ -444,11 +444,9 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     LAUNCH("zero", k_zero_int, 1, 64, h->cl_nfall, 1);
     TLAUNCH("closure_apply", k_closure_apply, g.M, g, a, h->cl_yp, a.gx, h->cl_flag, h->cl_nfall);
     TLAUNCH("fallback_q2f", k_fallback_q2f, g.M + 1, g, a, (const int*)h->cl_flag);
-#define VDIF_QM_CALL(KM) TLAUNCH("vdif_q", (k_vdif_q_r<KM, 10, FV_VDIFQ_VHREG>), g.M + 1, g, a, a.vhpair, h->cl_flag)
-#define VDIF_QM_CALL16(KM) TLAUNCH("vdif_q", (k_vdif_q_r<KM, 16, FV_VDIFQ_VHREG>), g.M + 1, g, a, a.vhpair, h->cl_flag)
+#define VDIF_QM_CALL(RM) TLAUNCH("vdif_q", k_vdif_q<RM>, g.M + 1, g, a, a.vhpair, h->cl_flag)
     // (vdif_q also stores Q2 = Q2F, Q2L = Q2LF for its columns)
-    if (g.ve_max <= 10) FV_KMAX_DISPATCH(g.KBM1, VDIF_QM_CALL);
-    else FV_KMAX_DISPATCH(g.KBM1, VDIF_QM_CALL16);
+    FV_RMAX_DISPATCH(g.ve_max, VDIF_QM_CALL);
   } else if (h->md->p.vertical_closure) {
     // ADV_Q of Q2 on the main stream, of Q2L on stream2 (own scratch)
     fork_streams(h, FV_CONC_3D);
@@ -457,12 +455,10 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     on_stream1(h);
     enqueue_adv_q<FT>(h, a, a.q2, a.q2f, fct);
     join_streams(h, FV_CONC_3D);
-#define VDIF_Q_CALL(KM) TLAUNCH("vdif_q", (k_vdif_q_r<KM, 10, FV_VDIFQ_VHREG>), g.M + 1, g, a, a.vhpair, (const int*)nullptr)
-#define VDIF_Q_CALL16(KM) TLAUNCH("vdif_q", (k_vdif_q_r<KM, 16, FV_VDIFQ_VHREG>), g.M + 1, g, a, a.vhpair, (const int*)nullptr)
+#define VDIF_Q_CALL(RM) TLAUNCH("vdif_q", k_vdif_q<RM>, g.M + 1, g, a, a.vhpair, (const int*)nullptr)
     // VDIF_Q, then Q2 = Q2F and Q2L = Q2LF (internal_step.F:1029-1035) in
     // the same kernel, the elimination coefficients in `vhpair`.
-    if (g.ve_max <= 10) FV_KMAX_DISPATCH(g.KBM1, VDIF_Q_CALL);
-    else FV_KMAX_DISPATCH(g.KBM1, VDIF_Q_CALL16);
+    FV_RMAX_DISPATCH(g.ve_max, VDIF_Q_CALL);
   } else {
     // VERTICAL_MIXING_TYPE 'constant'
     const double umol = h->md->p.umol;
@@ -1117,13 +1113,15 @@ int upload_grid(fvgpu_handle* h) {
                   columns_uniform(md->dzz, m1, KB, 0) && columns_uniform(md->zz, m1, KB, 0);
   const bool ue = columns_uniform(md->z1, n1, KB, 1) && columns_uniform(md->dz1, n1, KB, 1) &&
                   columns_uniform(md->dzz1, n1, KB, 1) && columns_uniform(md->zz1, n1, KB, 1);
-  g.sig_uniform = (un && ue) ? 1 : 0;
+  const bool sig_uniform = un && ue;
+  g.nsk = sig_uniform ? 1 : (long)m1; g.nsi = sig_uniform ? 0 : 1;
+  g.esk = sig_uniform ? 1 : (long)n1; g.esi = sig_uniform ? 0 : 1;
   auto col = [&](const double* a, size_t l1, size_t first) {
     std::vector<double> c(KB);
     for (int k = 0; k < KB; ++k) c[k] = a[(size_t)k * l1 + first];
     return c;
   };
-  if (g.sig_uniform) {
+  if (sig_uniform) {
     std::vector<double> c;
     c = col(md->z, m1, 0); if (dupload(h, &g.z, c.data(), KB)) return 1;
     c = col(md->zz, m1, 0); if (dupload(h, &g.zz, c.data(), KB)) return 1;

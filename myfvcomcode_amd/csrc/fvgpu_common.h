@@ -10,12 +10,6 @@
 #include <utility>
 
 #define FV_MAXKB 64
-// VDIF_Q keeps the elimination coefficients of its two solves in registers
-// (1) or in a node-layer scratch pair (0: unrolled level loops, 2: rolled),
-// trading VGPRs for occupancy.
-#ifndef FV_VDIFQ_VHREG
-#define FV_VDIFQ_VHREG 0
-#endif
 #define FV_MAX_CV 32   // control-volume sub-edges per node (twice the node degree)
 #define FV_MAX_RING 16 // NTSN / NTVE bound of the node rings held in registers
 #define FV_CVB 128     // elements and nodes per block of the fused CV kernels
@@ -45,7 +39,9 @@ struct UvBlocks {
 struct DevGrid {
   int M, N, NE, NCV, KB, KBM1, KBM2, IOBCN, NUMQBC, NTIDE;
   long m1, n1;
-  int sig_uniform;          // all node (and all element) sigma columns identical
+  // sigma value of layer k at entity i: a[(k-1)*sk + i*si], one column for
+  // all (sk = 1, si = 0) when all node and all element columns are identical
+  long nsk, nsi, esk, esi;
   double dte, dti, umol, vprnu, hprnu, cbcmin, min_depth;
   double fact, fm1;         // horizontal mixing closure / constant switches
   double const1, cvhp1;     // 16.6**.6666667*SEF and (15.8*CBCNST)**0.6666667
@@ -63,7 +59,7 @@ struct DevGrid {
   // edges and CV sub-edges
   const int *iec, *ienode, *isbc, *niec, *ntrg;
   const double *xijc, *yijc, *dltxc, *dltyc, *dltxe, *dltye, *dltxncve, *dltyncve;
-  // sigma (per column, or one column when sig_uniform)
+  // sigma (per column, or one column for all: nsk ..)
   const double *z, *zz, *dz, *dzz, *z1, *zz1, *dz1, *dzz1;
   // gather lists
   const int *cv_off, *cv_ent;      // node -> (cv<<1 | side), sorted by cv
@@ -153,11 +149,12 @@ __device__ __forceinline__ void layer_share(int first, int last, int& k0, int& k
 // 1-based layer accessors
 __device__ __forceinline__ long NI(const DevGrid& g, int i, int k) { return (long)(k - 1) * g.m1 + i; }
 __device__ __forceinline__ long EI(const DevGrid& g, int i, int k) { return (long)(k - 1) * g.n1 + i; }
+// (by strides, not by a branch, which no other load could cross)
 __device__ __forceinline__ double SIGN_(const DevGrid& g, const double* a, int i, int k) {
-  return g.sig_uniform ? a[k - 1] : a[NI(g, i, k)];
+  return a[(long)(k - 1) * g.nsk + (long)i * g.nsi];
 }
 __device__ __forceinline__ double SIGE_(const DevGrid& g, const double* a, int i, int k) {
-  return g.sig_uniform ? a[k - 1] : a[EI(g, i, k)];
+  return a[(long)(k - 1) * g.esk + (long)i * g.esi];
 }
 #define DZ(i, k) SIGN_(g, g.dz, i, k)
 #define DZZ(i, k) SIGN_(g, g.dzz, i, k)

@@ -134,22 +134,22 @@ __global__ __launch_bounds__(256) void k_vdif_ts_r(DevGrid g, IntArgs a, double*
 }
 
 // Per-level quantities of VDIF_Q (vdif_q.F:255-368): from Q2, Q2L and RHO1
-// at levels k-1 and k of node i (the values passed in).
+// at levels k-1 and k of node i, DZZ(k-1) and Z(k) (the values passed in).
 struct Q25Level { double q2, boy, ll, gh, stf, dtef; };
 
 __device__ __forceinline__ Q25Level q25_eval(const DevGrid& g, int i, int k, double d, double l0, double q2raw,
-                                             double q2l, double rho_km1, double rho_k) {
+                                             double q2l, double rho_km1, double rho_k, double dzz, double z) {
   const double SMALL = 1.E-8, KAPPA = 0.40, GH_MAX = .0233, GHC = -6.0, GH_MIN = -.281, B1 = 16.6;
   const double p9 = (double)0.9f, p1 = (double)0.1f;
   Q25Level r;
   r.q2 = fabs(q2raw + SMALL);
   r.boy = 0.0;
-  if (k >= 2 && k <= g.KBM1) r.boy = g.grav_n[i] * (rho_km1 - rho_k) / (DZZ(i, k - 1) * d);
+  if (k >= 2 && k <= g.KBM1) r.boy = g.grav_n[i] * (rho_km1 - rho_k) / (dzz * d);
   if (k == 1) r.ll = KAPPA * l0;
   else if (k == g.KB) r.ll = 0.0;
   else {
     double ll = fabs(q2l) / r.q2;
-    if (ZN(i, k) > -0.5) ll = fmax(ll, KAPPA * l0);
+    if (z > -0.5) ll = fmax(ll, KAPPA * l0);
     if (r.boy < 0.0) {
       const double lmax = sqrt(fabs(GH_MIN) * r.q2 / (-r.boy + SMALL));
       ll = fmin(ll, lmax);
@@ -165,6 +165,15 @@ __device__ __forceinline__ Q25Level q25_eval(const DevGrid& g, int i, int k, dou
   return r;
 }
 
+// What VDIF_Q's downward sweep reads at one level: RHO1, KQ of the level
+// below, Q2, Q2L, KM, KH, Q2F, Q2LF of the node, DZZ(k-1), DZ(k), Z(k) and
+// U, V of its element ring.  (The sigma values too: a load issued inside the
+// level's arithmetic is waited for after every load before it.)
+template <int RMAX>
+struct Q25Loads {
+  double rho, kq, q2, q2l, km, kh, q2f, q2lf, dzz, dz, z, ur[RMAX], vr[RMAX];
+};
+
 // VDIF_Q, MY2.5 (vdif_q.F:34-551), one thread per node column in two
 // sweeps.  The downward sweep k = 1..KB reads every node-layer value once
 // (sliding windows over RHO1 and KQ, the ring averages of U/V): it forms the
@@ -172,17 +181,25 @@ __device__ __forceinline__ Q25Level q25_eval(const DevGrid& g, int i, int k, dou
 // forward elimination of both the Q2 solve (vdif_q.F:372-378) and the Q2L
 // solve (vdif_q.F:398-417), and updates KQ/KM/KH and L, which depend on the
 // old Q2/Q2L only (vdif_q.F:466-487; L(1)=KAPPA*L0, L(KB)=0).  The
-// elimination coefficients VH of both solves go to registers (VHMODE 1,
-// loops unrolled) or to the node-layer pair scratch `vhs` (VHMODE 0 with
-// unrolled loops, 2 with rolled ones); VHP(k) is parked in Q2F(k)/Q2LF(k),
-// which the elimination has just consumed.  The upward
+// elimination coefficients VH of both solves go to the node-layer pair
+// scratch `vhs`; VHP(k) is parked in Q2F(k)/Q2LF(k), which the elimination
+// has just consumed.  The upward
 // sweep does both back-substitutions (vdif_q.F:380-391, 420-431) and the
 // threshold (vdif_q.F:440-448), and stores each final value both to
 // Q2F/Q2LF and to Q2/Q2L, the copy that follows VDIF_Q in INTERNAL_STEP
 // (internal_step.F:1034-1035); column 0 is copied by its thread.  Every value is formed by the reference's
 // operations in its order; only the loops are fused.
-template <int KMAX, int RMAX, int VHMODE>
-__global__ __launch_bounds__(256) void k_vdif_q_r(DevGrid g, IntArgs a, double2* vhs, const int* only) {
+//
+// Bound: the latency of a level's loads where the mesh has few columns, HBM
+// where it has many.  So the downward sweep issues the loads of level k+1
+// before it works on level k, and the upward sweep takes UP levels' loads at
+// once; both loops stay rolled (unrolled to 40 levels the code outgrew the
+// instruction cache, and no load could cross a level's branch).  62,500
+// elements x 40 layers: 257 -> 173 us; 1,000,000 x 40: 1277 -> 1082 us (4.9 GB,
+// 4.5 TB/s; 2 waves a SIMD instead of 3).
+template <int RMAX>
+__global__ __launch_bounds__(256) void k_vdif_q(DevGrid g, IntArgs a, double2* vhs, const int* only) {
+  constexpr int UP = 4;
   const int i = (int)xcd_thread();
   if (i > g.M) return;
   if (only && !only[i]) return;   // column subset (the learned closure's fallback)
@@ -234,12 +251,15 @@ __global__ __launch_bounds__(256) void k_vdif_q_r(DevGrid g, IntArgs a, double2*
   });
   // ring values loaded unconditionally (slots past the ring read element
   // 0) so that the loads issue together; the sum takes the ring in order
-  auto ring_avg = [&](const double* f, long eo) {
-    double fv[RMAX];
+  auto load_ring_uv = [&](int k, double (&ur)[RMAX], double (&vr)[RMAX]) {
+    const long eo = (long)(k - 1) * g.n1;
     static_for<RMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      fv[j] = f[eo + re[j]];
+      ur[j] = a.u[eo + re[j]];
+      vr[j] = a.v[eo + re[j]];
     });
+  };
+  auto ring_avg = [&](const double (&fv)[RMAX]) {
     double x = 0.0;
     static_for<RMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
@@ -247,9 +267,26 @@ __global__ __launch_bounds__(256) void k_vdif_q_r(DevGrid g, IntArgs a, double2*
     });
     return x / ntd;
   };
+  auto load_level = [&](int k) {
+    Q25Loads<RMAX> r;
+    const long q = (long)(k - 1) * m1 + i;
+    r.rho = a.rho1[q];
+    r.kq = KQ[q + m1];
+    r.q2 = a.q2[q];
+    r.q2l = a.q2l[q];
+    r.km = KM[q];
+    r.kh = KH[q];
+    r.q2f = Q2F[q];
+    r.q2lf = Q2LF[q];
+    r.dzz = DZZ(i, k - 1);
+    r.dz = DZ(i, k);
+    r.z = ZN(i, k);
+    load_ring_uv(k, r.ur, r.vr);
+    return r;
+  };
   const double coef4 = 18.0 * A1 * A1 + 9.0 * A1 * A2, coef5 = 9.0 * A1 * A2;
   // stability functions and the under-relaxed mixing coefficients at level k
-  auto mix = [&](long q, const Q25Level& lv, double kq_old) {
+  auto mix = [&](long q, const Q25Level& lv, double kq_old, double km_old, double kh_old) {
     const double coef1 = A2 * (1.0 - 6.0 * A1 / B1 * lv.stf);
     const double coef2 = 3.0 * A2 * B2 / lv.stf + 18.0 * A1 * A2;
     const double coef3 = A1 * (1.0 - 3.0 * C1 - 6.0 * A1 / B1 * lv.stf);
@@ -257,109 +294,115 @@ __global__ __launch_bounds__(256) void k_vdif_q_r(DevGrid g, IntArgs a, double2*
     const double sm = (coef3 + sh * coef4 * lv.gh) / (1. - coef5 * lv.gh);
     const double kn = lv.ll * sqrt(lv.q2);
     KQ[q] = 0.5 * (kn * KAPPA * sm + kq_old);
-    KM[q] = 0.5 * (kn * sm + KM[q]);
-    KH[q] = 0.5 * (kn * sh * g.vprnu + KH[q]);
+    KM[q] = 0.5 * (kn * sm + km_old);
+    KH[q] = 0.5 * (kn * sh * g.vprnu + kh_old);
     L[q] = lv.ll;
   };
   const double z1 = ZN(i, 1), zkb = ZN(i, KB);
-  constexpr int NVH = VHMODE == 1 ? KMAX + 1 : 1;
-  double VH1[NVH], VH2[NVH];
   double vh1p = 0.0, vh2p = 0.0;             // VH(k-1) of the two solves
   const double vhp1_1 = g.cvhp1 * utau2;
   double vhp1 = vhp1_1, vhp2 = 0.0;          // VHP(k-1) of the two solves
-  // level 1
+  // level 1, and the loads of level 2
   double rho_km1 = a.rho1[NI(g, i, 1)];
   double kq_km1 = KQ[NI(g, i, 1)];           // old KQ(k-1)
   double kq_k = KQ[NI(g, i, 2)];             // old KQ(k)
+  double dz_km1 = DZ(i, 1);
+  double ukm1 = 0.0, vkm1 = 0.0;
+  Q25Loads<RMAX> nx;
   {
     const long q = NI(g, i, 1);
-    const Q25Level lv = q25_eval(g, i, 1, d, l0, a.q2[q], a.q2l[q], 0.0, 0.0);
-    mix(q, lv, kq_km1);
+    const double q21 = a.q2[q], q2l1 = a.q2l[q], km1 = KM[q], kh1 = KH[q];
+    double ur[RMAX], vr[RMAX];
+    load_ring_uv(1, ur, vr);
+    nx = load_level(min(2, KBM1));
+    __builtin_amdgcn_sched_barrier(0);
+    const Q25Level lv = q25_eval(g, i, 1, d, l0, q21, q2l1, 0.0, 0.0, 0.0, 0.0);
+    mix(q, lv, kq_km1, km1, kh1);
+    if (d > 0.0) { ukm1 = ring_avg(ur); vkm1 = ring_avg(vr); }
   }
-  double ukm1 = 0.0, vkm1 = 0.0;
-  if (d > 0.0) { ukm1 = ring_avg(a.u, 0); vkm1 = ring_avg(a.v, 0); }
-  auto fwd = [&](const int k) __attribute__((always_inline)) {
-    {
-      const long q = (long)(k - 1) * m1 + i;
-      const double rho_k = a.rho1[q];
-      const double kq_kp1 = KQ[q + m1];
-      const Q25Level lv = q25_eval(g, i, k, d, l0, a.q2[q], a.q2l[q], rho_km1, rho_k);
-      // PROD (vdif_q.F:259-302)
-      const double boy = lv.boy;
-      const double kmq = KM[q];
-      double pr = kmq * 0.0 * fv_pow15(.5 * (-boy + fabs(boy)));
-      if (d > 0.0) {
-        const long eo = (long)(k - 1) * g.n1;
-        const double uk = ring_avg(a.u, eo), vk = ring_avg(a.v, eo);
-        pr = pr + kmq * SEF * (sq(uk - ukm1) + sq(vk - vkm1)) / sq(DZZ(i, k - 1) * d);
-        pr = pr + KH[q] * boy;
-        ukm1 = uk;
-        vkm1 = vk;
-      }
-      // the threshold before the solves (vdif_q.F:136-145): both to SMALL
-      // if either is at or below it
-      double q2f = Q2F[q], q2lf = Q2LF[q];
-      if (q2f <= SMALL || q2lf <= SMALL) { q2f = SMALL; q2lf = SMALL; }
-      const double ak = -0.5 * dti * (kq_kp1 + kq_k + 2.0 * umol) / (DZZ(i, k - 1) * DZ(i, k) * d * d);
-      const double ck = -0.5 * dti * (kq_km1 + kq_k + 2.0 * umol) / (DZZ(i, k - 1) * DZ(i, k - 1) * d * d);
-      const double t1 = 1. / (ak + ck * (1. - vh1p) - (2. * dti * lv.dtef + 1.));
-      const double vh1 = ak * t1;
-      const double p1 = (-2. * dti * pr + ck * vhp1 - q2f) * t1;
-      double vh2, p2;
-      if (d > 0.0) {
-        const double zk = ZN(i, k);
-        const double dtef = lv.dtef * (1. + E2 * sq((1. / fabs(zk - z1) + 1. / fabs(zk - zkb)) * lv.ll / (d * KAPPA)));
-        const double t2 = 1. / (ak + ck * (1. - vh2p) - (dti * dtef + 1.));
-        vh2 = ak * t2;
-        p2 = (dti * (-pr * lv.ll * E1) + ck * vhp2 - q2lf) * t2;
-      } else {              // D <= 0: VH/VHP keep the first solve's values
-        vh2 = vh1;
-        p2 = p1;
-      }
-      if constexpr (VHMODE == 1) { VH1[k] = vh1; VH2[k] = vh2; }
-      else vhs[q] = make_double2(vh1, vh2);
-      Q2F[q] = p1;
-      Q2LF[q] = p2;
-      vh1p = vh1;
-      vh2p = vh2;
-      vhp1 = p1;
-      vhp2 = p2;
-      mix(q, lv, kq_k);
-      rho_km1 = rho_k;
-      kq_km1 = kq_k;
-      kq_k = kq_kp1;
+#pragma unroll 2
+  for (int k = 2; k <= KBM1; ++k) {
+    const Q25Loads<RMAX> c = nx;
+    nx = load_level(min(k + 1, KBM1));   // past the last level: reloads it, unused
+    __builtin_amdgcn_sched_barrier(0);
+    const long q = (long)(k - 1) * m1 + i;
+    const Q25Level lv = q25_eval(g, i, k, d, l0, c.q2, c.q2l, rho_km1, c.rho, c.dzz, c.z);
+    // PROD (vdif_q.F:259-302)
+    const double boy = lv.boy;
+    // the reference's KM*0*x**1.5, x >= 0: zero (or NaN) whatever the power
+    double pr = c.km * 0.0 * (.5 * (-boy + fabs(boy)));
+    if (d > 0.0) {
+      const double uk = ring_avg(c.ur), vk = ring_avg(c.vr);
+      pr = pr + c.km * SEF * (sq(uk - ukm1) + sq(vk - vkm1)) / sq(c.dzz * d);
+      pr = pr + c.kh * boy;
+      ukm1 = uk;
+      vkm1 = vk;
     }
-  };
-  if constexpr (VHMODE != 2) {
-    static_for<KMAX - 1>([&](auto kc) {
-      constexpr int k = decltype(kc)::value + 2;
-      if (k <= KBM1) fwd(k);
-    });
-  } else {
-    for (int k = 2; k <= KBM1; ++k) fwd(k);
+    // the threshold before the solves (vdif_q.F:136-145): both to SMALL
+    // if either is at or below it
+    double q2f = c.q2f, q2lf = c.q2lf;
+    if (q2f <= SMALL || q2lf <= SMALL) { q2f = SMALL; q2lf = SMALL; }
+    const double ak = -0.5 * dti * (c.kq + kq_k + 2.0 * umol) / (c.dzz * c.dz * d * d);
+    const double ck = -0.5 * dti * (kq_km1 + kq_k + 2.0 * umol) / (c.dzz * dz_km1 * d * d);
+    const double t1 = 1. / (ak + ck * (1. - vh1p) - (2. * dti * lv.dtef + 1.));
+    const double vh1 = ak * t1;
+    const double p1 = (-2. * dti * pr + ck * vhp1 - q2f) * t1;
+    double vh2, p2;
+    if (d > 0.0) {
+      const double zk = c.z;
+      const double dtef = lv.dtef * (1. + E2 * sq((1. / fabs(zk - z1) + 1. / fabs(zk - zkb)) * lv.ll / (d * KAPPA)));
+      const double t2 = 1. / (ak + ck * (1. - vh2p) - (dti * dtef + 1.));
+      vh2 = ak * t2;
+      p2 = (dti * (-pr * lv.ll * E1) + ck * vhp2 - q2lf) * t2;
+    } else {              // D <= 0: VH/VHP keep the first solve's values
+      vh2 = vh1;
+      p2 = p1;
+    }
+    vhs[q] = make_double2(vh1, vh2);
+    Q2F[q] = p1;
+    Q2LF[q] = p2;
+    vh1p = vh1;
+    vh2p = vh2;
+    vhp1 = p1;
+    vhp2 = p2;
+    mix(q, lv, kq_k, c.km, c.kh);
+    rho_km1 = c.rho;
+    kq_km1 = kq_k;
+    kq_k = c.kq;
+    dz_km1 = c.dz;
   }
   {
     // level KB (kq_k is the old KQ(KB) here)
     const long q = NI(g, i, KB);
-    const Q25Level lv = q25_eval(g, i, KB, d, l0, a.q2[q], a.q2l[q], 0.0, 0.0);
-    mix(q, lv, kq_k);
+    const Q25Level lv = q25_eval(g, i, KB, d, l0, a.q2[q], a.q2l[q], 0.0, 0.0, 0.0, 0.0);
+    mix(q, lv, kq_k, KM[q], KH[q]);
   }
   // upward sweep: both back-substitutions, then the threshold on each level
   double x1 = q2f_kb, x2 = Q2LF[NI(g, i, KB)];
   a.q2[NI(g, i, KB)] = x1;
   a.q2l[NI(g, i, KB)] = x2;
-  auto bwd = [&](const int k) __attribute__((always_inline)) {
-    {
+  for (int kt = KBM1; kt >= 1; kt -= UP) {
+    double2 w[UP];
+    double p1[UP], p2[UP];
+#pragma unroll
+    for (int j = 0; j < UP; ++j) {
+      const long q = (long)(max(kt - j, 1) - 1) * m1 + i;
+      w[j] = vhs[q];
+      p1[j] = Q2F[q];
+      p2[j] = Q2LF[q];
+    }
+#pragma unroll
+    for (int j = 0; j < UP; ++j) {
+      const int k = kt - j;
+      if (k < 1) break;
       const long q = (long)(k - 1) * m1 + i;
-      double v1 = 0.0, v2 = 0.0, p1 = vhp1_1, p2 = 0.0;   // VH(1) = 0, VHP(1) of the two solves
-      if (k >= 2) {
-        if constexpr (VHMODE == 1) { v1 = VH1[k]; v2 = VH2[k]; }
-        else { const double2 w = vhs[q]; v1 = w.x; v2 = w.y; }
-        p1 = Q2F[q];
-        p2 = Q2LF[q];
+      if (k == 1) {   // VH(1) = 0, VHP(1) of the two solves
+        x1 = 0.0 * x1 + vhp1_1;
+        x2 = 0.0 * x2 + 0.0;
+      } else {
+        x1 = w[j].x * x1 + p1[j];
+        x2 = w[j].y * x2 + p2[j];
       }
-      x1 = v1 * x1 + p1;
-      x2 = v2 * x2 + p2;
       double y1 = x1, y2 = x2;
       if (k >= 2 && (x1 <= SMALL || x2 <= SMALL)) { y1 = SMALL; y2 = SMALL; }
       Q2F[q] = y1;
@@ -367,13 +410,5 @@ __global__ __launch_bounds__(256) void k_vdif_q_r(DevGrid g, IntArgs a, double2*
       a.q2[q] = y1;
       a.q2l[q] = y2;
     }
-  };
-  if constexpr (VHMODE != 2) {
-    static_for<KMAX>([&](auto kc) {
-      constexpr int k = KMAX - decltype(kc)::value;
-      if (k <= KBM1) bwd(k);
-    });
-  } else {
-    for (int k = KBM1; k >= 1; --k) bwd(k);
   }
 }
