@@ -20,6 +20,7 @@
 #include "fvgpu_closure.h"
 #include "../../include/fvgpu.h"
 
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -327,6 +328,7 @@ ExtArgs make_ext_args(fvgpu_handle* h, int K, const Ext2DState& cur, const Ext2D
   a.clk = h->clk;
   a.elm1 = h->ia.elm1;
   a.elm2 = h->ia.elm2;
+  a.st = h->g.st;
   return a;
 }
 
@@ -516,6 +518,9 @@ int build_lists(fvgpu_handle* h) {
   const fv_model* md = h->md;
   const int M = md->m, N = md->n, NE = md->ne, NCV = md->ncv;
   DevGrid& g = h->g;
+  // per-layer byte offsets of entities and flux positions are 32-bit (at())
+  if (8ll * std::max<long long>({(long long)M + 1, (long long)N + 1, (long long)NCV + 1}) >= (1ll << 32))
+    return fail("the mesh exceeds 32-bit byte offsets per layer");
   // node -> CV sub-edges sorted by sub-edge index
   std::vector<int> cnt(M + 2, 0);
   for (int c = 1; c <= NCV; ++c) { cnt[md->niec[c]]++; cnt[md->niec[(size_t)(NCV + 1) + c]]++; }
@@ -951,37 +956,42 @@ int build_lists(fvgpu_handle* h) {
     if (build_blocks(tile_own) > 256) return fail("an element tile exceeds the blocked momentum kernels' records");
     // the 2-D stage's tables, in block order
     const size_t nt = tile_own.size(), n1 = (size_t)N + 1, ne1 = (size_t)NE + 1;
-    std::vector<int4> nb4(nt * 256, int4{0, 0, 0, 0});
+    StageTab& st = g.st;
+    st = StageTab{0, 0, 0, std::max(g.cv_max, 1)};
+    std::vector<int4> nb4(nt * 256, int4{INT_MIN, 0, 0, 0});
+    std::vector<unsigned> sedge(nt * 256, ~0u);
     std::vector<double> egeo(nt * 6 * 256, 0.0);
     std::vector<int> nslot(M + 1, 0);
     for (size_t b = 0; b < nt; ++b) {
       for (int t = 0; t < tile_nn[b]; ++t) nslot[tile_nodes[b * FV_CVB + t]] = t;
       for (int t = 0; t < bns[b]; ++t) {
         const int x = belems[b * 256 + t];
-        nb4[b * 256 + t] = int4{x, md->nbe[x], md->nbe[n1 + x], md->nbe[2 * n1 + x]};
+        nb4[b * 256 + t] = int4{t < bnown[b] ? x : ~x, md->nbe[x], md->nbe[n1 + x], md->nbe[2 * n1 + x]};
       }
       for (int t = 0; t < bne[b]; ++t) {
         const int c = bedges[b * 256 + t], ia = md->iec[c], ib = md->iec[ne1 + c];
-        if (md->isbc[c] < 0 || md->isbc[c] > 3) return fail("ISBC outside 0..3");
-        const unsigned lo = (unsigned)beloc[b * 256 + t], j1 = (unsigned)nslot[md->ienode[c]],
-                       j2 = (unsigned)nslot[md->ienode[ne1 + c]];
-        beloc[b * 256 + t] = (int)(lo | j1 << 16 | j2 << 23 | (unsigned)md->isbc[c] << 30);
+        if (md->isbc[c] < 0 || md->isbc[c] > 2) return fail("ISBC outside 0..2");
+        sedge[b * 256 + t] = (unsigned)beloc[b * 256 + t] | (unsigned)nslot[md->ienode[c]] << 16 |
+                             (unsigned)nslot[md->ienode[ne1 + c]] << 23 | (unsigned)md->isbc[c] << 30;
         const double v[6] = {md->xijc[c] - md->xc[ia], md->yijc[c] - md->yc[ia], md->xijc[c] - md->xc[ib],
                              md->yijc[c] - md->yc[ib], md->dltxc[c], md->dltyc[c]};
         for (int q = 0; q < 6; ++q) egeo[(b * 6 + q) * 256 + t] = v[q];
       }
+      st.n_rec = std::max(st.n_rec, bns[b]);
+      st.n_edge = std::max(st.n_edge, bne[b]);
+      st.n_node = std::max(st.n_node, tile_nn[b]);
     }
-    if (upload_blocks(g.ub_tile) || dupload(h, &g.ub_tile.nb4, nb4.data(), nb4.size()) ||
-        dupload(h, &g.ub_tile.egeo, egeo.data(), egeo.size()))
+    if (upload_blocks(g.ub_tile) || dupload(h, &st.rec, nb4.data(), nb4.size()) ||
+        dupload(h, &st.edge, sedge.data(), sedge.size()) || dupload(h, &st.egeo, egeo.data(), egeo.size()))
       return 1;
     const size_t SM = (size_t)std::max(g.cv_max, 1);
-    std::vector<int4> snode(nt * FV_CVB, int4{2, 0, -1, -1}), selem(nt * FV_CVB, int4{0, 0, 0, 0});
+    std::vector<int4> snode(nt * FV_CVB, int4{-1, 0, -1, -1}), selem(nt * FV_CVB, int4{0, 0, 0, 0});
     std::vector<int> slist(nt * SM * FV_CVB, 0);
     std::vector<double> snd(nt * 2 * FV_CVB, 1.0), sed(nt * 12 * FV_CVB, 0.0);
     for (size_t b = 0; b < nt; ++b) {
       for (int t = 0; t < tile_nn[b]; ++t) {
         const int i = tile_nodes[b * FV_CVB + t];
-        snode[b * FV_CVB + t] = int4{tile_stn[b * FV_CVB + t], cnt[i], nobc[i], nriv[i]};
+        snode[b * FV_CVB + t] = int4{tile_stn[b * FV_CVB + t], 0, nobc[i], nriv[i]};
         for (int j = 0; j < cnt[i]; ++j) {
           const int en = ent[off[i] + j];
           slist[(b * SM + j) * FV_CVB + t] = (pos[en >> 1] << 1) | (en & 1);
@@ -1001,10 +1011,13 @@ int build_lists(fvgpu_handle* h) {
         for (int q = 0; q < 12; ++q) sed[(b * 12 + q) * FV_CVB + t] = v[q];
       }
     }
-    if (dupload(h, &g.st_node, snode.data(), snode.size()) || dupload(h, &g.st_elem, selem.data(), selem.size()) ||
-        dupload(h, &g.st_list, slist.data(), slist.size()) || dupload(h, &g.st_nd, snd.data(), snd.size()) ||
-        dupload(h, &g.st_ed, sed.data(), sed.size()))
+    if (dupload(h, &st.node, snode.data(), snode.size()) || dupload(h, &st.elem, selem.data(), selem.size()) ||
+        dupload(h, &st.list, slist.data(), slist.size()) || dupload(h, &st.nd, snd.data(), snd.size()) ||
+        dupload(h, &st.ed, sed.data(), sed.size()))
       return 1;
+    st.a12 = g.a12;
+    st.art = g.art;
+    st.cc_hvc = g.cc_hvc;
   }
   return 0;
 }

@@ -5,6 +5,7 @@
 // nodes/elements at one layer reads consecutive addresses.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 #include <utility>
@@ -23,17 +24,43 @@
 // record slots of IA and IB in bits 0-7 and 8-15 of eloc[256*b + t];
 // epos[e] packs the edge slots of element e's three edges (in ed_ent
 // order) in bits 0-7, 8-15, 16-23, and in bits 24-26 whether e is their IB.
-// For the element tiles also, in block order so that the 2-D stage reads
-// them directly: nb4[256*b + t] the record's element and its three
-// neighbours NBE; egeo[(6*b + q)*256 + t] the edge's XIJC-XC and YIJC-YC of
-// IA, the same of IB, DLTXC, DLTYC; and in eloc the local indices (of
-// cvb_nodes) of the edge's nodes IENODE in bits 16-22 and 23-29 and ISBC in
-// bits 30-31.
 struct UvBlocks {
   int nblk;
   const int *nown, *ns, *elems, *ne, *edges, *eloc, *epos;
-  const int4* nb4;
+};
+
+// The 2-D stage's tables of the element tiles (DevGrid::ub_tile, the same
+// blocks as cvb_*), in block order so that a stage reads them directly and
+// contiguously: no list length or index has to arrive before the first
+// loads go out.  Lanes past a block's entries read a marked pad; n_* are the
+// most entries of any block.
+//   rec[256*b + t]   the gradient record's element x and its neighbours
+//                    NBE; x = e for the block's own element t, ~e for
+//                    another element, INT_MIN for a pad
+//   edge[256*b + t]  the record slots of IA and IB in bits 0-7 and 8-15, the
+//                    node slots of IENODE in bits 16-22 and 23-29, ISBC in
+//                    bits 30-31; all ones for a pad
+//   egeo[(6*b + q)*256 + t]  XIJC-XC and YIJC-YC of IA, the same of IB,
+//                    DLTXC, DLTYC
+//   node[FV_CVB*b + t]  {2*node + 1 in the first block that has it, 0, OBC
+//                    index or -1, river index or -1}, x = -1 for a pad
+//   list[(nslot*b + j)*FV_CVB + t]  the node's cvl_ent list
+//   nd[(2*b + q)*FV_CVB + t]  ART1, H
+//   elem[FV_CVB*b + t]  {epos, cvb_loc, ISBCE + 4 if it has rivers, IUCP}
+//   ed[(12*b + q)*FV_CVB + t]  EPOR, GRAV_E, ART, COR, H1, CC_SPONGE, DLTXE
+//                    and DLTYE of the three sub-edges
+// a12, art and cc_hvc are DevGrid's.
+struct StageTab {
+  int n_rec, n_edge, n_node, nslot;
+  const int4* rec;
+  const unsigned* edge;
   const double* egeo;
+  const int4* node;
+  const int* list;
+  const double* nd;
+  const int4* elem;
+  const double* ed;
+  const double *a12, *art, *cc_hvc;
 };
 
 struct DevGrid {
@@ -91,17 +118,7 @@ struct DevGrid {
   // at every layer (the OBC nodes and the other ends of their sub-edges).
   int cvb_nblk;
   const int *cvb_nn, *cvb_nodes, *cvb_ne, *cvb_elems, *cvb_loc, *rec_keep;
-  // The 2-D stage's constants of the same blocks in block order (read
-  // directly and contiguously, without waiting for an index): node t:
-  // st_node[FV_CVB*b + t] = {2*node + 1 in the first block that has it,
-  // sub-edge count, OBC index or -1, river index or -1}, its cvl_ent list
-  // st_list[(cv_max*b + j)*FV_CVB + t] and {ART1, H} in
-  // st_nd[(2*b + q)*FV_CVB + t]; element t: st_elem = {epos, cvb_loc, ISBCE
-  // + 4 if it has rivers, IUCP} and EPOR, GRAV_E, ART, COR, H1, CC_SPONGE,
-  // DLTXE and DLTYE of its three sub-edges in st_ed[(12*b + q)*FV_CVB + t].
-  const int4 *st_node, *st_elem;
-  const int* st_list;
-  const double *st_nd, *st_ed;
+  StageTab st;
   // Node tiles (VERTVL): tile b owns the nt_nown[b] (<= FV_NTN) nodes
   // nt_nodes[FV_NTN*b + t]; nt_elems[FV_NTE*b + t] are the nt_nel[b]
   // (<= FV_NTE) elements that have one of them as a vertex.  Slot j of
@@ -146,6 +163,14 @@ __device__ __forceinline__ void layer_share(int first, int last, int& k0, int& k
   k1 = min(k0 + c - 1, last);
 }
 
+// p[i] where p is the same for every lane and i an entity or flux position:
+// the address is the scalar base plus a 32-bit byte offset (no 64-bit lane
+// arithmetic).  fvgpu_create refuses meshes whose offsets would not fit.
+template <typename T>
+__device__ __forceinline__ T at(const T* p, int i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (unsigned)i * (unsigned)sizeof(T));
+}
+
 // 1-based layer accessors
 __device__ __forceinline__ long NI(const DevGrid& g, int i, int k) { return (long)(k - 1) * g.m1 + i; }
 __device__ __forceinline__ long EI(const DevGrid& g, int i, int k) { return (long)(k - 1) * g.n1 + i; }
@@ -179,8 +204,8 @@ __device__ __forceinline__ double SIGE_(const DevGrid& g, const double* a, int i
 // The least-squares coefficients A1U(e,1..4) and A2U(e,1..4) of element
 // e, in the flux type, from the interleaved copy (two 32-byte loads each).
 template <typename FT>
-__device__ __forceinline__ void lsq_coef(const DevGrid& g, int e, FT (&a1)[4], FT (&a2)[4]) {
-  const double4* p = reinterpret_cast<const double4*>(g.a12) + 2L * e;
+__device__ __forceinline__ void lsq_coef(const double* a12, int e, FT (&a1)[4], FT (&a2)[4]) {
+  const double4* p = reinterpret_cast<const double4*>(a12) + 2L * e;
   const double4 u = p[0], w = p[1];
   a1[0] = (FT)u.x; a1[1] = (FT)u.y; a1[2] = (FT)u.z; a1[3] = (FT)u.w;
   a2[0] = (FT)w.x; a2[1] = (FT)w.y; a2[2] = (FT)w.z; a2[3] = (FT)w.w;
@@ -188,6 +213,10 @@ __device__ __forceinline__ void lsq_coef(const DevGrid& g, int e, FT (&a1)[4], F
 
 __device__ __forceinline__ double fsign1(double b) { return b >= 0.0 ? 1.0 : -1.0; }
 __device__ __forceinline__ float fsign1(float b) { return b >= 0.0f ? 1.0f : -1.0f; }
+// x, negated where bit 0 of m is set
+__device__ __forceinline__ double flip_sign(double x, int m) {
+  return __hiloint2double(__double2hiint(x) ^ (m << 31), __double2loint(x));
+}
 __device__ __forceinline__ double sq(double x) { return x * x; }
 __device__ __forceinline__ float sq(float x) { return x * x; }
 

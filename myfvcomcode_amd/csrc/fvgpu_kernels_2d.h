@@ -47,6 +47,7 @@ struct ExtArgs {
   double *elm1, *elm2;         // the elevation one and two RK stages back (Orlanski OBC)
   const ExtClock* ec;    // of this external step
   DevClock* clk;
+  StageTab st;
 };
 
 // PSIMPLE_DRAG (mod_bulk.F:58-90): wind stress of a wind speed (Large and
@@ -140,28 +141,21 @@ __device__ __forceinline__ double tide_force(const DevGrid& g, int obc, double r
 // itself (extel_edge.F:155-160).  The term of sub-edge c, D1*(-UA*DLTYE +
 // VA*DLTXE) of its element for side IB, is exactly the negative for side IA
 // (DLTXE/DLTYE negated; round to nearest is symmetric), so the stored term
-// is added or subtracted.  The node's n list entries are at lst[j*stride];
-// SMAX >= the slots of the list (nslot), the slots past n hold the unused
-// entry 0, so all list and term loads are unconditional and issue together.
+// is added or subtracted.  ce: the node's list entries; the slots past them
+// hold the unused entry 0, whose term is zero and leaves the sum as it is
+// (x - 0 is x), so all term loads are unconditional and issue together.
 template <int SMAX>
-__device__ __forceinline__ double ext_node_update(const DevGrid& g, const ExtArgs& a, int i, const int* lst,
-                                                  long stride, int n, int rv, bool obc, double art1, double elrk,
-                                                  double& xobc) {
-  const int nslot = g.cv_max;
-  int ce[SMAX];
-  static_for<SMAX>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    ce[j] = lst[(j < nslot ? j : 0) * stride];
-  });
+__device__ __forceinline__ double ext_node_update(const DevGrid& g, const ExtArgs& a, int i, const int (&ce)[SMAX],
+                                                  int rv, bool obc, double art1, double elrk, double& xobc) {
   double t[SMAX];
   static_for<SMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    t[j] = a.phi[ce[j] >> 1];
+    t[j] = at(a.phi, ce[j] >> 1);
   });
   double xflux = 0.0;
   static_for<SMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    if (j < n) xflux = (ce[j] & 1) ? xflux + t[j] : xflux - t[j];
+    xflux = xflux + flip_sign(t[j], ~ce[j]);
   });
   xobc = 0.0;
   if (obc) { xobc = xflux; xflux = 0.0; }
@@ -280,39 +274,50 @@ struct ExtFluxLds {
 
 template <int SMAX, typename FT, bool INT>
 __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ gp, ExtArgs a) {
-  const DevGrid& g = *gp;   // in device memory: by value its pointers overflow the scalar registers
+  const DevGrid& g = *gp;   // in device memory, for the boundary parts: by value its pointers
+                            // overflow the scalar registers
   __shared__ ExtRecsLds<FT> sr;
   __shared__ ExtFluxLds<FT> sf;
   __shared__ double s_elf[FV_CVB], s_el[FV_CVB], s_d[FV_CVB], s_fobn[FV_CVB];
   const FT half = (FT)0.5, one = (FT)1.0;
   const int b = xcd_block(), t = threadIdx.x;
-  const UvBlocks& B = g.ub_tile;
+  const StageTab& st = a.st;
   // the block-order constants of the first two parts, so that their
   // latencies overlap
-  const bool ract = t < B.ns[b], eact = t < B.ne[b], oact = t < B.nown[b];
-  const int tn = 255 - t, nn = g.cvb_nn[b];   // lane 255 - tn: the tile's node tn
-  const bool nact = tn < nn, n0 = b == 0 && tn == nn;   // node 0 by block 0
-  const int4 xs = ract ? B.nb4[256L * b + t] : make_int4(0, 0, 0, 0);
-  int4 nd = make_int4(1, 0, -1, -1);
-  if (nact) nd = g.st_node[(long)FV_CVB * b + tn];
-  unsigned pl = 0;
-  double eg[6];   // XIJC-XC, YIJC-YC of IA, the same of IB, DLTXC, DLTYC
-  if (eact) {
-    pl = (unsigned)B.eloc[256L * b + t];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) eg[q] = B.egeo[(6L * b + q) * 256 + t];
+  int4 xs = make_int4(INT_MIN, 0, 0, 0), nd = make_int4(-1, 0, -1, -1);
+  if (t < st.n_rec) xs = st.rec[256L * b + t];
+  const int tn = 255 - t;   // lane 255 - tn: the tile's node tn
+  if (tn < st.n_node) nd = st.node[(long)FV_CVB * b + tn];
+  int ce[SMAX];
+  if constexpr (!INT) {
+    const int* lst = st.list + (long)st.nslot * b * FV_CVB + min(tn, FV_CVB - 1);
+    if (tn < st.n_node)
+      static_for<SMAX>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        ce[j] = lst[(j < st.nslot ? j : 0) * FV_CVB];
+      });
   }
-  const int i = xs.x;
+  unsigned pl = ~0u;
+  double eg[6];   // XIJC-XC, YIJC-YC of IA, the same of IB, DLTXC, DLTYC
+  if (t < st.n_edge) {
+    pl = st.edge[256L * b + t];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) eg[q] = st.egeo[(6L * b + q) * 256 + t];
+  }
+  const bool ract = xs.x != INT_MIN, oact = xs.x > 0, eact = pl != ~0u, nact = nd.x >= 0;
+  const bool n0 = b == 0 && tn == FV_CVB;   // node 0 by block 0
+  if (n0) nd.x = 1;
+  const int i = xs.x >= 0 ? xs.x : ~xs.x;
   double ua = 0.0, va = 0.0;
   // 1. gradients
   if (ract) {
     FT ra1[4], ra2[4];
-    lsq_coef<FT>(g, i, ra1, ra2);
-    const FT rart = (FT)g.art[i], rcc = (FT)g.cc_hvc[i];
-    ua = a.cur.ua[i];
-    va = a.cur.va[i];
-    const FT us = (FT)ua, u1 = (FT)a.cur.ua[xs.y], u2 = (FT)a.cur.ua[xs.z], u3 = (FT)a.cur.ua[xs.w];
-    const FT vs = (FT)va, v1 = (FT)a.cur.va[xs.y], v2 = (FT)a.cur.va[xs.z], v3 = (FT)a.cur.va[xs.w];
+    lsq_coef<FT>(st.a12, i, ra1, ra2);
+    const FT rart = (FT)at(st.art, i), rcc = (FT)at(st.cc_hvc, i);
+    ua = at(a.cur.ua, i);
+    va = at(a.cur.va, i);
+    const FT us = (FT)ua, u1 = (FT)at(a.cur.ua, xs.y), u2 = (FT)at(a.cur.ua, xs.z), u3 = (FT)at(a.cur.ua, xs.w);
+    const FT vs = (FT)va, v1 = (FT)at(a.cur.va, xs.y), v2 = (FT)at(a.cur.va, xs.z), v3 = (FT)at(a.cur.va, xs.w);
     const FT c1 = ra1[0] * us + ra1[1] * u1 + ra1[2] * u2 + ra1[3] * u3;
     const FT c2 = ra2[0] * us + ra2[1] * u1 + ra2[2] * u2 + ra2[3] * u3;
     const FT c5 = ra1[0] * vs + ra1[1] * v1 + ra1[2] * v2 + ra1[3] * v3;
@@ -328,8 +333,8 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     const int j = nd.x >> 1, obc = nd.z;
     const bool keep = (nd.x & 1) != 0;   // this tile stores the node
     if (nact) {
-      s_el[tn] = a.cur.el[j];
-      s_d[tn] = a.cur.d[j];
+      s_el[tn] = at(a.cur.el, j);
+      s_d[tn] = at(a.cur.d, j);
     }
     if constexpr (INT) {
       if (keep) {
@@ -340,33 +345,35 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     } else {
       double art1, hn;
       if (nact) {
-        art1 = g.st_nd[2L * b * FV_CVB + tn];
-        hn = g.st_nd[(2L * b + 1) * FV_CVB + tn];
+        art1 = st.nd[2L * b * FV_CVB + tn];
+        hn = st.nd[(2L * b + 1) * FV_CVB + tn];
       } else {
         art1 = g.art1[0];
         hn = g.h[0];
       }
-      const double elrk = a.elrk[j];
+      const double elrk = at(a.elrk, j);
       if (keep && a.elrk_copy) a.elrk_copy[j] = elrk;
       const int ty = obc >= 0 ? g.type_obc[obc] : 0;
       // GWI / BKI need their interior neighbour's new elevation: a second
       // pass forms it, as the tile that has that node does
       double elf = 0.0, el2 = 0.0, xobc = 0.0;
-      const int* lst = nact ? g.st_list + (long)g.cv_max * b * FV_CVB + tn : g.cvl_ent;
-      long stride = nact ? FV_CVB : g.m1;
-      int id = j, cnt = nd.y, rv = nd.w;
+      int id = j, rv = nd.w;
       double ar = art1, er = elrk;
+      if (n0)
+        static_for<SMAX>([&](auto jc) { ce[decltype(jc)::value] = 0; });
       for (bool next = false;;) {
         double xo;
-        const double e = ext_node_update<SMAX>(g, a, id, lst, stride, cnt, rv, !next && obc >= 0, ar, er, xo);
+        const double e = ext_node_update<SMAX>(g, a, id, ce, rv, !next && obc >= 0, ar, er, xo);
         if (next) { el2 = e; break; }
         elf = e;
         xobc = xo;
         if (ty < 5 || ty > 8) break;
         id = g.next_obc[obc];
-        lst = g.cvl_ent + id;
-        stride = g.m1;
-        cnt = g.cv_cnt[id]; rv = g.node_riv[id];
+        static_for<SMAX>([&](auto jc) {
+          constexpr int q = decltype(jc)::value;
+          ce[q] = g.cvl_ent[(long)(q < st.nslot ? q : 0) * g.m1 + id];
+        });
+        rv = g.node_riv[id];
         ar = g.art1[id]; er = a.elrk[id];
         next = true;
       }
@@ -396,18 +403,18 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
   int4 oe = make_int4(0, 0, 0, 0);
   double ed[12], own[6], d1 = 0.0, el1b = 0.0, uab = 0.0, vab = 0.0, wsx = 0.0, wsy = 0.0;
   if (oact) {
-    oe = g.st_elem[(long)FV_CVB * b + t];
+    oe = st.elem[(long)FV_CVB * b + t];
 #pragma unroll
-    for (int q = 0; q < 12; ++q) ed[q] = g.st_ed[(12L * b + q) * FV_CVB + t];
-    d1 = a.cur.d1[i];
+    for (int q = 0; q < 12; ++q) ed[q] = st.ed[(12L * b + q) * FV_CVB + t];
+    d1 = at(a.cur.d1, i);
     if constexpr (INT) {
       own[0] = a.adx2d[i]; own[1] = a.ady2d[i]; own[2] = a.drx2d[i]; own[3] = a.dry2d[i];
       own[4] = a.wubot[i]; own[5] = a.wvbot[i];
     } else {
 #pragma unroll
       for (int q = 0; q < 6; ++q) own[q] = a.own2d[(6L * b + q) * FV_CVB + t];
-      el1b = a.base.el1[i]; uab = a.base.ua[i]; vab = a.base.va[i];
-      if (g.wind_on) { wsx = a.ws2x[i]; wsy = a.ws2y[i]; }
+      el1b = at(a.base.el1, i); uab = at(a.base.ua, i); vab = at(a.base.va, i);
+      if (g.wind_on) { wsx = at(a.ws2x, i); wsy = at(a.ws2y, i); }
     }
   }
   __syncthreads();

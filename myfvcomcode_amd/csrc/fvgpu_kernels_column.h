@@ -320,7 +320,6 @@ __global__ __launch_bounds__(256) void k_vdif_q(DevGrid g, IntArgs a, double2* v
     mix(q, lv, kq_km1, km1, kh1);
     if (d > 0.0) { ukm1 = ring_avg(ur); vkm1 = ring_avg(vr); }
   }
-#pragma unroll 2
   for (int k = 2; k <= KBM1; ++k) {
     const Q25Loads<RMAX> c = nx;
     nx = load_level(min(k + 1, KBM1));   // past the last level: reloads it, unused

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
   const int x = ract ? B.elems[256L * b + t] : 0;
   const int x1 = NBE_(x, 1), x2 = NBE_(x, 2), x3 = NBE_(x, 3);
   FT ra1[4], ra2[4];
-  lsq_coef<FT>(g, x, ra1, ra2);
+  lsq_coef<FT>(g.a12, x, ra1, ra2);
   const FT rart = (FT)g.art[x], rcc = (FT)g.cc_hvc[x];
   // 2. edge part: edge c
   const bool eact = t < B.ne[b];
