@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     if (tn < st.n_node)
       static_for<SMAX>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        ce[j] = lst[(j < st.nslot ? j : 0) * FV_CVB];
+        ce[j] = j < st.nslot ? lst[j * FV_CVB] : 0;   // 0: the zero term
       });
   }
   unsigned pl = ~0u;
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
         id = g.next_obc[obc];
         static_for<SMAX>([&](auto jc) {
           constexpr int q = decltype(jc)::value;
-          ce[q] = g.cvl_ent[(long)(q < st.nslot ? q : 0) * g.m1 + id];
+          ce[q] = q < st.nslot ? g.cvl_ent[(long)q * g.m1 + id] : 0;
         });
         rv = g.node_riv[id];
         ar = g.art1[id]; er = a.elrk[id];
