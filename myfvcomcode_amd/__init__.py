@@ -463,8 +463,8 @@ class DeviceModel:
         L = gpu_lib()
         n = C.c_int64()
         _check(L, L.fvgpu_closure_samples(self._h, None, None, 0, C.byref(n)), "fvgpu_closure_samples")
-        x = np.zeros((n.value, 8), np.float32)
-        y = np.zeros((n.value, 2), np.float32)
+        x = np.empty((n.value, 8), np.float32)
+        y = np.empty((n.value, 2), np.float32)
         fp = C.POINTER(C.c_float)
         _check(L, L.fvgpu_closure_samples(self._h, x.ctypes.data_as(fp), y.ctypes.data_as(fp), n.value,
                                           C.byref(n)), "fvgpu_closure_samples")
@@ -577,7 +577,7 @@ class Trainer:
     def infer(self, lo=0, n=None, mfma=True):
         L = gpu_lib()
         n = int(n if n is not None else self.n - lo)
-        y = np.zeros((n, 2), np.float32)
+        y = np.empty((n, 2), np.float32)
         _check(L, L.fvmlp_infer(self._h, int(lo), n, 1 if mfma else 0, y.ctypes.data_as(C.POINTER(C.c_float))),
                "fvmlp_infer")
         return y

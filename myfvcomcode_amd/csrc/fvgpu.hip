@@ -18,6 +18,7 @@
 //  * time-dependent scalars (RAMP, ExtTime) live in a device clock updated
 //    by single-thread kernels, never by host writes between launches.
 #include "fvgpu_closure.h"
+#include "fvgpu_stage.h"
 #include "../../include/fvgpu.h"
 
 #include <climits>
@@ -87,6 +88,7 @@ struct fvgpu_handle {
   int precision = 0;
   int device = 0;
   int cu_count = 0;       // compute units of the device
+  HostStage stage;        // pinned staging of the copies to and from the caller's memory
   hipStream_t stream = nullptr;
   // Independent chains of the step (the T and S passes, the Q2 and Q2L
   // advection) fork onto stream2 and join back; both streams have the default priority.  `cur` is the stream the
@@ -102,6 +104,7 @@ struct fvgpu_handle {
   // stress (ws2x, ws2y), otherwise it uses the end stress g.wsx/g.wsy
   double *wu0 = nullptr, *wv0 = nullptr, *wu1 = nullptr, *wv1 = nullptr, *ws2x = nullptr, *ws2y = nullptr;
   int wind_varies = 0;
+  std::vector<double> wind_end;   // wu1 then wv1, kept on the host until the wind first varies
   DevGrid g{};
   const DevGrid* dg = nullptr;   // its device copy
   std::vector<void*> allocs;
@@ -147,8 +150,8 @@ int dalloc(fvgpu_handle* h, T** p, size_t n, const T* src = nullptr) {
   void* q = nullptr;
   HIPCHK(hipMalloc(&q, (n ? n : 1) * sizeof(T)));
   h->allocs.push_back(q);
-  if (n && src) HIPCHK(hipMemcpy(q, src, n * sizeof(T), hipMemcpyHostToDevice));
-  else HIPCHK(hipMemset(q, 0, (n ? n : 1) * sizeof(T)));
+  if (n && src) HIPCHK(h->stage.to_device(q, src, n * sizeof(T), h->stream, h->device));
+  else HIPCHK(hipMemsetAsync(q, 0, (n ? n : 1) * sizeof(T), h->stream));
   *p = (T*)q;
   return 0;
 }
@@ -1120,6 +1123,10 @@ int upload_grid(fvgpu_handle* h) {
     if (dalloc(h, &h->ws2x, n1) || dalloc(h, &h->ws2y, n1)) return 1;
     h->wind_varies = std::memcmp(md->uuwind0, md->uuwind, n1 * sizeof(double)) != 0 ||
                      std::memcmp(md->vvwind0, md->vvwind, n1 * sizeof(double)) != 0;
+    if (!h->wind_varies) {
+      h->wind_end.assign(md->uuwind, md->uuwind + n1);
+      h->wind_end.insert(h->wind_end.end(), md->vvwind, md->vvwind + n1);
+    }
   }
   // sigma: one column when every column is identical
   const bool un = columns_uniform(md->z, m1, KB, 0) && columns_uniform(md->dz, m1, KB, 0) &&
@@ -1216,7 +1223,7 @@ int upload_state(fvgpu_handle* h) {
   c.iint = md->p.iint0; c.ramp_int = 0;
   c.time0 = md->p.time0; c.dti = g.dti; c.dte = g.dte;
   c.isplit = g.isplit; c.iramp = g.iramp; c.depth_fail = 0;
-  HIPCHK(hipMemcpy(h->clk, &c, sizeof(c), hipMemcpyHostToDevice));
+  HIPCHK(h->stage.to_device(h->clk, &c, sizeof(c), h->stream, h->device));
   a.clk = h->clk;
   // the stream2 chains: the same arrays, their own scratch (node-layer
   // records, face fluxes, bottom gradients, OBC fluxes)
@@ -1296,6 +1303,7 @@ int fvgpu_create(const fv_model* md, int32_t precision, fvgpu_handle** out) {
   h->two_phase_q = precision == FV_MIXED ? 1 : 0;
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) { delete h; return fail("stream"); }
   h->cur = h->stream;
+  h->stage.reserve();
   if (hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming) != hipSuccess) {
@@ -1320,11 +1328,9 @@ int fvgpu_external_step(fvgpu_handle* h, int32_t iext) {
   enqueue_external_step(h, iext);
   // restore IINT (this call does not complete an internal step)
   DevClock c;
-  HIPCHK(hipMemcpyAsync(&c, h->clk, sizeof(c), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  HIPCHK(h->stage.to_host(&c, h->clk, sizeof(c), h->stream, h->device));
   c.iint -= 1;
-  HIPCHK(hipMemcpyAsync(h->clk, &c, sizeof(c), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  HIPCHK(h->stage.to_device(h->clk, &c, sizeof(c), h->stream, h->device));
   return 0;
 }
 
@@ -1355,8 +1361,7 @@ int fvgpu_get_state(fvgpu_handle* h, const char* name, double* host, int64_t len
   double* p = lookup(h, name, &l);
   if (!p) return fail(std::string("unknown state array ") + name);
   if ((size_t)len != l) return fail(std::string("length mismatch for ") + name);
-  HIPCHK(hipMemcpyAsync(host, p, l * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  HIPCHK(h->stage.to_host(host, p, l * sizeof(double), h->stream, h->device));
   return 0;
 }
 
@@ -1365,8 +1370,7 @@ int fvgpu_put_state(fvgpu_handle* h, const char* name, const double* host, int64
   double* p = lookup(h, name, &l);
   if (!p) return fail(std::string("unknown state array ") + name);
   if ((size_t)len != l) return fail(std::string("length mismatch for ") + name);
-  HIPCHK(hipMemcpyAsync(p, host, l * sizeof(double), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  HIPCHK(h->stage.to_device(p, host, l * sizeof(double), h->stream, h->device));
   return 0;
 }
 
@@ -1406,9 +1410,15 @@ int ens_update(fvgpu_handle* h, const char* name, int32_t nrens, const int64_t* 
   }
   double* dx5 = stage;
   long* doff = (long*)(stage + FV_ENS_MAX * FV_ENS_MAX);
-  std::vector<long> offl(off, off + nrens);
-  HIPCHK(hipMemcpyAsync(dx5, x5, (size_t)nrens * nrens * sizeof(double), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(hipMemcpyAsync(doff, offl.data(), (size_t)nrens * sizeof(long), hipMemcpyHostToDevice, h->stream));
+  static_assert(sizeof(long) == sizeof(double), "offsets are staged beside X5");
+  double up[FV_ENS_MAX * FV_ENS_MAX + FV_ENS_MAX];
+  std::memcpy(up, x5, (size_t)nrens * nrens * sizeof(double));
+  for (int i = 0; i < nrens; ++i) {
+    const long o = (long)off[i];
+    std::memcpy(&up[FV_ENS_MAX * FV_ENS_MAX + i], &o, sizeof(o));
+  }
+  HIPCHK(h->stage.to_device(stage, up, (size_t)(FV_ENS_MAX * FV_ENS_MAX + nrens) * sizeof(double), h->stream,
+                            h->device));
   const long total = (long)len * nl;
   // persistent blocks: two per CU (the 65 KB of LDS each allows two)
   const long ntiles = (total + FV_ENS_TILE - 1) / FV_ENS_TILE;
@@ -1446,30 +1456,26 @@ int fvgpu_set_forcing(fvgpu_handle* h, const char* name, const double* host, int
   if (n == "wind") {
     if (!h->md->p.wind_on) return fail("the model was created without wind");
     if ((size_t)len != 2 * n1) return fail("wind: expected UUWIND then VVWIND, 2*(N+1) values");
-    std::vector<double> wx(n1, 0.0), wy(n1, 0.0);
-    wind_stress(host, host + n1, n1, wx.data(), wy.data());
-    HIPCHK(hipMemcpyAsync((void*)g.wsx, wx.data(), n1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipMemcpyAsync((void*)g.wsy, wy.data(), n1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    // the previous end speeds become the start of the coming step
-    std::vector<double> old_u(n1), old_v(n1);
-    HIPCHK(hipMemcpyAsync(old_u.data(), h->wu1, n1 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(old_v.data(), h->wv1, n1 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpyAsync(h->wu0, old_u.data(), n1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipMemcpyAsync(h->wv0, old_v.data(), n1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipMemcpyAsync(h->wu1, host, n1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipMemcpyAsync(h->wv1, host + n1, n1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    const bool varies = std::memcmp(old_u.data(), host, n1 * sizeof(double)) != 0 ||
-                        std::memcmp(old_v.data(), host + n1, n1 * sizeof(double)) != 0;
-    if (varies && !h->wind_varies) {
+    const bool varies =
+        !h->wind_varies && std::memcmp(h->wind_end.data(), host, 2 * n1 * sizeof(double)) != 0;
+    // the new speeds (by way of the external steps' stress buffers, which
+    // every external step fills again) become the end of the coming step,
+    // the previous end its start
+    HIPCHK(h->stage.to_device(h->ws2x, host, n1 * sizeof(double), h->stream, h->device));
+    HIPCHK(h->stage.to_device(h->ws2y, host + n1, n1 * sizeof(double), h->stream, h->device));
+    hipLaunchKernelGGL(k_wind_shift, dim3(nb((long)n1)), dim3(256), 0, h->stream, (long)n1, h->wu0, h->wv0, h->wu1,
+                       h->wv1, (const double*)h->ws2x, (const double*)h->ws2y, (double*)g.wsx, (double*)g.wsy);
+    HIPCHK(hipGetLastError());
+    if (varies) {
       // the captured step gains the per-external-step stress kernel
       h->wind_varies = 1;
+      std::vector<double>().swap(h->wind_end);
       drop_graphs(h);
     }
   } else if (n == "qdis" || n == "tdis" || n == "sdis") {
     if ((size_t)len != nr) return fail(n + ": expected one value per river (NUMQBC)");
     const double* dst = n == "qdis" ? g.qdis0 : n == "tdis" ? g.tdis : g.sdis;
-    if (nr) HIPCHK(hipMemcpyAsync((void*)dst, host, nr * sizeof(double), hipMemcpyHostToDevice, h->stream));
+    if (nr) HIPCHK(h->stage.to_device((void*)dst, host, nr * sizeof(double), h->stream, h->device));
   } else {
     return fail("unknown forcing " + n + " (wind, qdis, tdis, sdis)");
   }
@@ -1555,6 +1561,7 @@ void fvgpu_destroy(fvgpu_handle* h) {
   drop_graphs(h);
   for (hipEvent_t e : h->event_pool) (void)hipEventDestroy(e);
   for (void* p : h->allocs) (void)hipFree(p);
+  h->stage.release();
   if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
   if (h->ev_join) (void)hipEventDestroy(h->ev_join);
   if (h->stream2) (void)hipStreamDestroy(h->stream2);
@@ -1620,10 +1627,9 @@ extern "C" int fvgpu_diagnostics(fvgpu_handle* h, fv_diag* out) {
   DiagAcc* part = (DiagAcc*)h->diag_part;
   hipLaunchKernelGGL(k_diag_partial, dim3(nblk), dim3(256), 0, h->stream, h->g, h->ia, part);
   std::vector<DiagAcc> hp(nblk);
-  HIPCHK(hipMemcpyAsync(hp.data(), part, sizeof(DiagAcc) * nblk, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h->stage.to_host(hp.data(), part, sizeof(DiagAcc) * nblk, h->stream, h->device));
   DevClock c;
-  HIPCHK(hipMemcpyAsync(&c, h->clk, sizeof(c), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  HIPCHK(h->stage.to_host(&c, h->clk, sizeof(c), h->stream, h->device));
   double vol = 0, vc = 0, salt = 0, sc = 0, heat = 0, hc = 0, dmin = 1e300;
   int bad = 0;
   auto nm = [](double& s, double& cc, double x) {
@@ -1700,9 +1706,8 @@ int fvgpu_closure_samples(fvgpu_handle* h, float* x, float* y, int64_t max_sampl
 #define CLD_CALL(RM) hipLaunchKernelGGL(k_closure_features<RM>, dim3(nb(g.M)), dim3(256), 0, h->stream, g, a, dx, dy)
   FV_RMAX_DISPATCH(g.ve_max, CLD_CALL);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(x, dx, ns * MLP_IN * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipMemcpyAsync(y, dy, ns * MLP_OUT * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  HIPCHK(h->stage.to_host(x, dx, ns * MLP_IN * sizeof(float), h->stream, h->device));
+  HIPCHK(h->stage.to_host(y, dy, ns * MLP_OUT * sizeof(float), h->stream, h->device));
   HIPCHK(hipFree(dx));
   HIPCHK(hipFree(dy));
   return 0;
@@ -1715,7 +1720,9 @@ struct fvmlp {
   int64_t n = 0;
   int bmax = 0;
   int step = 0;
+  int device = 0;
   hipStream_t stream = nullptr;
+  HostStage stage;
   float *X = nullptr, *Y = nullptr, *P = nullptr, *Mo = nullptr, *Ve = nullptr;
   float* G = nullptr;          // the batch's gradient, then its summed loss
   float* part = nullptr;       // the workgroups' partials of it
@@ -1733,8 +1740,8 @@ template <typename T>
 int malloc_mlp(fvmlp* t, T** p, size_t n) {
   void* q = nullptr;
   HIPCHK(hipMalloc(&q, (n ? n : 1) * sizeof(T)));
-  HIPCHK(hipMemset(q, 0, (n ? n : 1) * sizeof(T)));
   t->allocs.push_back(q);
+  HIPCHK(hipMemsetAsync(q, 0, (n ? n : 1) * sizeof(T), t->stream));
   *p = (T*)q;
   return 0;
 }
@@ -1769,6 +1776,7 @@ int fvmlp_create(int64_t n, const float* x, const float* y, int32_t bmax, fvmlp*
   fvmlp* t = new fvmlp();
   t->n = n;
   t->bmax = bmax;
+  (void)hipGetDevice(&t->device);
   const size_t bb = (size_t)bmax, nb_ = std::min<size_t>((bb + MLP_GRP - 1) / MLP_GRP, MLP_BLOCKS);
   if (hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking) != hipSuccess ||
       hipHostMalloc((void**)&t->hidx, bb * sizeof(int), hipHostMallocDefault) != hipSuccess ||
@@ -1783,14 +1791,17 @@ int fvmlp_create(int64_t n, const float* x, const float* y, int32_t bmax, fvmlp*
     fvmlp_destroy(t);
     return 1;
   }
-  HIPCHK(hipMemcpy(t->X, x, (size_t)n * MLP_IN * sizeof(float), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(t->Y, y, (size_t)n * MLP_OUT * sizeof(float), hipMemcpyHostToDevice));
+  if (t->stage.to_device(t->X, x, (size_t)n * MLP_IN * sizeof(float), t->stream, t->device) != hipSuccess ||
+      t->stage.to_device(t->Y, y, (size_t)n * MLP_OUT * sizeof(float), t->stream, t->device) != hipSuccess) {
+    fvmlp_destroy(t);
+    return fail("fvmlp_create: copying the samples");
+  }
   *out = t;
   return 0;
 }
 
 int fvmlp_set_params(fvmlp* t, const float* p) {
-  HIPCHK(hipMemcpyAsync(t->P, p, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice, t->stream));
+  HIPCHK(t->stage.to_device(t->P, p, MLP_NPARAM * sizeof(float), t->stream, t->device));
   HIPCHK(hipMemsetAsync(t->Mo, 0, MLP_NPARAM * sizeof(float), t->stream));
   HIPCHK(hipMemsetAsync(t->Ve, 0, MLP_NPARAM * sizeof(float), t->stream));
   HIPCHK(hipStreamSynchronize(t->stream));
@@ -1799,8 +1810,7 @@ int fvmlp_set_params(fvmlp* t, const float* p) {
 }
 
 int fvmlp_get_params(fvmlp* t, float* p) {
-  HIPCHK(hipStreamSynchronize(t->stream));
-  HIPCHK(hipMemcpy(p, t->P, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost));
+  HIPCHK(t->stage.to_host(p, t->P, MLP_NPARAM * sizeof(float), t->stream, t->device));
   return 0;
 }
 
@@ -1858,8 +1868,7 @@ int fvmlp_infer(fvmlp* t, int64_t lo, int64_t n, int32_t use_mfma, float* y) {
                        t->X + lo * MLP_IN, (long)n, t->Yp);
   }
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(y, t->Yp, (size_t)n * MLP_OUT * sizeof(float), hipMemcpyDeviceToHost, t->stream));
-  HIPCHK(hipStreamSynchronize(t->stream));
+  HIPCHK(t->stage.to_host(y, t->Yp, (size_t)n * MLP_OUT * sizeof(float), t->stream, t->device));
   return 0;
 }
 
@@ -1867,6 +1876,7 @@ void fvmlp_destroy(fvmlp* t) {
   if (!t) return;
   if (t->stream) (void)hipStreamSynchronize(t->stream);
   for (void* p : t->allocs) (void)hipFree(p);
+  t->stage.release();
   if (t->hidx) (void)hipHostFree(t->hidx);
   if (t->hG) (void)hipHostFree(t->hG);
   if (t->stream) (void)hipStreamDestroy(t->stream);

@@ -74,6 +74,21 @@ __global__ void k_ext_wind(DevGrid g, const double* u0, const double* v0, const 
   psimple_drag(uu, vv, sx[i], sy[i]);
 }
 
+// New end-of-step wind speeds (nu, nv) at elements 0..n1-1: the previous ones
+// become the start of the step; the stress of the new ones at elements 1...
+__global__ void k_wind_shift(long n1, double* u0, double* v0, double* u1, double* v1, const double* nu,
+                             const double* nv, double* sx, double* sy) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n1) return;
+  u0[i] = u1[i];
+  v0[i] = v1[i];
+  u1[i] = nu[i];
+  v1[i] = nv[i];
+  sx[i] = 0.0;
+  sy[i] = 0.0;
+  if (i >= 1) psimple_drag(nu[i], nv[i], sx[i], sy[i]);
+}
+
 // Wall projection of a velocity pair (BCOND_GCN cases 2/3/5): the element's
 // case, found once (wall_prep), then applied to any number of pairs of its
 // column (wall_apply).  Case 3 zeroes the pair; on a solid wall (ISBCE 1)
