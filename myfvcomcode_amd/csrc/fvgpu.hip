@@ -144,15 +144,22 @@ struct fvgpu_handle {
 
 namespace {
 
-// Device memory of n values, zero, or a copy of src where given.
+// Device memory of n values, not initialised.
 template <typename T>
-int dalloc(fvgpu_handle* h, T** p, size_t n, const T* src = nullptr) {
+int dalloc_raw(fvgpu_handle* h, T** p, size_t n) {
   void* q = nullptr;
   HIPCHK(hipMalloc(&q, (n ? n : 1) * sizeof(T)));
   h->allocs.push_back(q);
-  if (n && src) HIPCHK(h->stage.to_device(q, src, n * sizeof(T), h->stream, h->device));
-  else HIPCHK(hipMemsetAsync(q, 0, (n ? n : 1) * sizeof(T), h->stream));
   *p = (T*)q;
+  return 0;
+}
+
+// Device memory of n values, zero, or a copy of src where given.
+template <typename T>
+int dalloc(fvgpu_handle* h, T** p, size_t n, const T* src = nullptr) {
+  if (dalloc_raw(h, p, n)) return 1;
+  if (n && src) HIPCHK(h->stage.to_device(*p, src, n * sizeof(T), h->stream, h->device));
+  else HIPCHK(hipMemsetAsync(*p, 0, (n ? n : 1) * sizeof(T), h->stream));
   return 0;
 }
 
@@ -537,7 +544,6 @@ int build_lists(fvgpu_handle* h) {
   }
   // element -> 3 sub-edges, and each sub-edge's element-major flux position
   std::vector<int> pos(NCV + 1, 0);
-  std::vector<double> edx, edy;   // DLTXE, DLTYE of the element's sub-edges (ecv_dx, ecv_dy)
   {
     const size_t n1 = (size_t)N + 1;
     std::vector<int> ec(3 * n1, 0), esw(3 * n1, 0), ecnt(n1, 0);
@@ -564,8 +570,7 @@ int build_lists(fvgpu_handle* h) {
     }
     for (int e = 1; e <= N; ++e)
       if (ecnt[e] != 3) return fail("an element has fewer than 3 control-volume sub-edges");
-    edx.assign(3 * n1, 0.0);
-    edy.assign(3 * n1, 0.0);
+    std::vector<double> edx(3 * n1, 0.0), edy(3 * n1, 0.0);
     for (size_t q = 0; q < 3 * n1; ++q)
       if (ec[q] > 0) { edx[q] = md->dltxe[ec[q]]; edy[q] = md->dltye[ec[q]]; }
     if (dupload(h, &g.ecv_dx, edx.data(), edx.size())) return 1;
@@ -609,19 +614,29 @@ int build_lists(fvgpu_handle* h) {
   if (dupload(h, &g.ed_ent, ed.data(), ed.size())) return 1;
   // FLUXOBN contributions per element in OBC order
   const int IOBCN = md->iobcn;
-  std::vector<std::vector<int>> fo(N + 1);
+  std::vector<std::pair<int, int>> fo;   // (element, entry) by element, OBC order kept
   for (int i = 0; i < IOBCN; ++i) {
-    if (md->nadjc_obc[i] > 0) fo[md->adjc_obc[i]].push_back((i << 1) | 0);
-    if (md->nadjc_obc[i] > 1) fo[md->adjc_obc[(size_t)IOBCN + i]].push_back((i << 1) | 1);
+    if (md->nadjc_obc[i] > 0) fo.push_back({md->adjc_obc[i], (i << 1) | 0});
+    if (md->nadjc_obc[i] > 1) fo.push_back({md->adjc_obc[(size_t)IOBCN + i], (i << 1) | 1});
   }
-  for (int i = 1; i <= N; ++i)
-    for (int x : fo[i]) {
-      const int j = md->i_obc_n[x >> 1];
-      if (md->nv[i] != j && md->nv[(size_t)N + 1 + i] != j && md->nv[2 * ((size_t)N + 1) + i] != j)
-        return fail("an OBC node's adjacent cell does not have the node");
+  for (const auto& [e, x] : fo) {
+    const int j = md->i_obc_n[x >> 1];
+    if (md->nv[e] != j && md->nv[(size_t)N + 1 + e] != j && md->nv[2 * ((size_t)N + 1) + e] != j)
+      return fail("an OBC node's adjacent cell does not have the node");
+  }
+  // CSR over elements 0..N of (element, entry) pairs, each element's entries in their order
+  auto element_csr = [&](std::vector<std::pair<int, int>>& v, std::vector<int>& off, std::vector<int>& ent_) {
+    std::stable_sort(v.begin(), v.end(), [](const auto& p, const auto& q) { return p.first < q.first; });
+    off.assign(N + 2, (int)v.size());
+    size_t q = 0;
+    for (int i = 0; i <= N + 1; ++i) {
+      while (q < v.size() && v[q].first < i) ++q;
+      off[i] = (int)q;
     }
-  std::vector<int> fo_off(N + 2, 0), fo_ent;
-  for (int i = 0; i <= N; ++i) { fo_off[i + 1] = fo_off[i] + (int)fo[i].size(); for (int x : fo[i]) fo_ent.push_back(x); }
+    for (const auto& p : v) ent_.push_back(p.second);
+  };
+  std::vector<int> fo_off, fo_ent;
+  element_csr(fo, fo_off, fo_ent);
   if (dupload(h, &g.fo_off, fo_off.data(), fo_off.size())) return 1;
   if (dupload(h, &g.fo_obc, fo_ent.data(), fo_ent.size())) return 1;
   std::vector<int> nobc(M + 1, -1), nriv(M + 1, -1), skip(M + 1, 0);
@@ -640,21 +655,19 @@ int build_lists(fvgpu_handle* h) {
   if (dupload(h, &g.fct_skip, skip.data(), skip.size())) return 1;
   // element -> rivers in river order: NBVE(J,1) then NBVE(J,NTVE(J)) of a
   // node river's node, an edge river's own cell
-  std::vector<std::vector<int>> re(N + 1);
+  std::vector<std::pair<int, int>> re;
   for (int k = 0; k < md->numqbc; ++k) {
-    if (md->icellq[k] > 0) { re[md->icellq[k]].push_back(k); continue; }
+    if (md->icellq[k] > 0) { re.push_back({md->icellq[k], k}); continue; }
     const int j = md->inodeq[k];
-    const int i1 = md->nbve[md->nbve_off[j]], i2 = md->nbve[md->nbve_off[j] + md->ntve[j] - 1];
-    re[i1].push_back(k);
-    re[i2].push_back(k);
+    re.push_back({md->nbve[md->nbve_off[j]], k});
+    re.push_back({md->nbve[md->nbve_off[j] + md->ntve[j] - 1], k});
   }
-  std::vector<int> re_off(N + 2, 0), re_ent;
-  for (int i = 0; i <= N; ++i) { re_off[i + 1] = re_off[i] + (int)re[i].size(); for (int x : re[i]) re_ent.push_back(x); }
+  std::vector<int> re_off, re_ent;
+  element_csr(re, re_off, re_ent);
   if (dupload(h, &g.re_off, re_off.data(), re_off.size())) return 1;
   if (dupload(h, &g.re_riv, re_ent.data(), re_ent.size())) return 1;
   std::vector<std::vector<int>> tile_own;   // the element tiles below, for the momentum blocks too
-  std::vector<int> tile_nn, tile_nodes, tile_stn;   // their nodes: cvb_nn, cvb_nodes, 2*node + 1 where first
-  std::vector<int> tile_loc;                         // cvb_loc
+  std::vector<int> tile_nn, tile_stn;       // their nodes: cvb_nn; 2*node, + 1 in the first tile that has it
   // element blocks of the fused record + face-flux kernels: recursive
   // coordinate bisection of the element centroids (each range halved at the
   // median of its longer extent) down to blocks of at most FV_CVB elements
@@ -880,8 +893,6 @@ int build_lists(fvgpu_handle* h) {
     if (dupload(h, &g.cvb_loc, loc.data(), loc.size())) return 1;
     if (dupload(h, &g.rec_keep, keep.data(), keep.size())) return 1;
     tile_nn.swap(bnn);
-    tile_nodes.swap(bnodes);
-    tile_loc.swap(loc);
   }
   // element blocks of the blocked momentum kernels.  The 2-D stage and
   // ADVECTION take the element tiles above (compact, so few neighbours form
@@ -957,70 +968,26 @@ int build_lists(fvgpu_handle* h) {
     }
     if (upload_blocks(g.ub_run)) return 1;
     if (build_blocks(tile_own) > 256) return fail("an element tile exceeds the blocked momentum kernels' records");
-    // the 2-D stage's tables, in block order
-    const size_t nt = tile_own.size(), n1 = (size_t)N + 1, ne1 = (size_t)NE + 1;
+    for (int c = 1; c <= NE; ++c)
+      if (md->isbc[c] < 0 || md->isbc[c] > 2) return fail("ISBC outside 0..2");
+    if (upload_blocks(g.ub_tile)) return 1;
+    // the 2-D stage's tables, filled on the device
+    const size_t nt = tile_own.size();
     StageTab& st = g.st;
-    st = StageTab{0, 0, 0, std::max(g.cv_max, 1)};
-    std::vector<int4> nb4(nt * 256, int4{INT_MIN, 0, 0, 0});
-    std::vector<unsigned> sedge(nt * 256, ~0u);
-    std::vector<double> egeo(nt * 6 * 256, 0.0);
-    std::vector<int> nslot(M + 1, 0);
-    for (size_t b = 0; b < nt; ++b) {
-      for (int t = 0; t < tile_nn[b]; ++t) nslot[tile_nodes[b * FV_CVB + t]] = t;
-      for (int t = 0; t < bns[b]; ++t) {
-        const int x = belems[b * 256 + t];
-        nb4[b * 256 + t] = int4{t < bnown[b] ? x : ~x, md->nbe[x], md->nbe[n1 + x], md->nbe[2 * n1 + x]};
-      }
-      for (int t = 0; t < bne[b]; ++t) {
-        const int c = bedges[b * 256 + t], ia = md->iec[c], ib = md->iec[ne1 + c];
-        if (md->isbc[c] < 0 || md->isbc[c] > 2) return fail("ISBC outside 0..2");
-        sedge[b * 256 + t] = (unsigned)beloc[b * 256 + t] | (unsigned)nslot[md->ienode[c]] << 16 |
-                             (unsigned)nslot[md->ienode[ne1 + c]] << 23 | (unsigned)md->isbc[c] << 30;
-        const double v[6] = {md->xijc[c] - md->xc[ia], md->yijc[c] - md->yc[ia], md->xijc[c] - md->xc[ib],
-                             md->yijc[c] - md->yc[ib], md->dltxc[c], md->dltyc[c]};
-        for (int q = 0; q < 6; ++q) egeo[(b * 6 + q) * 256 + t] = v[q];
-      }
-      st.n_rec = std::max(st.n_rec, bns[b]);
-      st.n_edge = std::max(st.n_edge, bne[b]);
-      st.n_node = std::max(st.n_node, tile_nn[b]);
-    }
-    if (upload_blocks(g.ub_tile) || dupload(h, &st.rec, nb4.data(), nb4.size()) ||
-        dupload(h, &st.edge, sedge.data(), sedge.size()) || dupload(h, &st.egeo, egeo.data(), egeo.size()))
-      return 1;
-    const size_t SM = (size_t)std::max(g.cv_max, 1);
-    std::vector<int4> snode(nt * FV_CVB, int4{-1, 0, -1, -1}), selem(nt * FV_CVB, int4{0, 0, 0, 0});
-    std::vector<int> slist(nt * SM * FV_CVB, 0);
-    std::vector<double> snd(nt * 2 * FV_CVB, 1.0), sed(nt * 12 * FV_CVB, 0.0);
-    for (size_t b = 0; b < nt; ++b) {
-      for (int t = 0; t < tile_nn[b]; ++t) {
-        const int i = tile_nodes[b * FV_CVB + t];
-        snode[b * FV_CVB + t] = int4{tile_stn[b * FV_CVB + t], 0, nobc[i], nriv[i]};
-        for (int j = 0; j < cnt[i]; ++j) {
-          const int en = ent[off[i] + j];
-          slist[(b * SM + j) * FV_CVB + t] = (pos[en >> 1] << 1) | (en & 1);
-        }
-        snd[(2 * b) * FV_CVB + t] = md->art1[i];
-        snd[(2 * b + 1) * FV_CVB + t] = md->h[i];
-      }
-      for (int t = 0; t < bnown[b]; ++t) {
-        const int e = belems[b * 256 + t];
-        selem[b * FV_CVB + t] = int4{epos[e], tile_loc[e], (md->isbce[e] & 3) | (re_off[e] < re_off[e + 1] ? 4 : 0),
-                                     md->iucp[e]};
-        double v[12] = {md->epor[e], md->grav_e[e], md->art[e], md->cor[e], md->h1[e], md->cc_sponge[e]};
-        for (int j = 0; j < 3; ++j) {
-          v[6 + j] = edx[(size_t)j * n1 + e];
-          v[9 + j] = edy[(size_t)j * n1 + e];
-        }
-        for (int q = 0; q < 12; ++q) sed[(b * 12 + q) * FV_CVB + t] = v[q];
-      }
-    }
-    if (dupload(h, &st.node, snode.data(), snode.size()) || dupload(h, &st.elem, selem.data(), selem.size()) ||
-        dupload(h, &st.list, slist.data(), slist.size()) || dupload(h, &st.nd, snd.data(), snd.size()) ||
-        dupload(h, &st.ed, sed.data(), sed.size()))
-      return 1;
+    st = StageTab{*std::max_element(bns.begin(), bns.end()), *std::max_element(bne.begin(), bne.end()),
+                  *std::max_element(tile_nn.begin(), tile_nn.end()), std::max(g.cv_max, 1)};
     st.a12 = g.a12;
     st.art = g.art;
     st.cc_hvc = g.cc_hvc;
+    const int* stn = nullptr;
+    if (dupload(h, &stn, tile_stn.data(), tile_stn.size())) return 1;
+    if (dalloc_raw(h, &st.rec, nt * 256) || dalloc_raw(h, &st.edge, nt * 256) || dalloc_raw(h, &st.egeo, nt * 6 * 256) ||
+        dalloc_raw(h, &st.node, nt * FV_CVB) || dalloc_raw(h, &st.elem, nt * FV_CVB) ||
+        dalloc_raw(h, &st.list, nt * st.nslot * FV_CVB) || dalloc_raw(h, &st.nd, nt * 2 * FV_CVB) ||
+        dalloc_raw(h, &st.ed, nt * 12 * FV_CVB))
+      return 1;
+    hipLaunchKernelGGL(k_stage_tables, dim3((unsigned)nt), dim3(256), 0, h->stream, g, st, stn);
+    HIPCHK(hipGetLastError());
   }
   return 0;
 }

@@ -52,14 +52,14 @@ struct UvBlocks {
 // a12, art and cc_hvc are DevGrid's.
 struct StageTab {
   int n_rec, n_edge, n_node, nslot;
-  const int4* rec;
-  const unsigned* edge;
-  const double* egeo;
-  const int4* node;
-  const int* list;
-  const double* nd;
-  const int4* elem;
-  const double* ed;
+  int4* rec;
+  unsigned* edge;
+  double* egeo;
+  int4* node;
+  int* list;
+  double* nd;
+  int4* elem;
+  double* ed;
   const double *a12, *art, *cc_hvc;
 };
 

@@ -244,6 +244,63 @@ __global__ __launch_bounds__(FV_CVB) void k_ext_begin(DevGrid g, ExtArgs a) {
   }
 }
 
+// Fills the 2-D stage's tables (StageTab) from the grid, one workgroup per
+// element tile; stn[FV_CVB*b + t]: 2*node + 1 in the first tile that has it.
+__global__ __launch_bounds__(256) void k_stage_tables(DevGrid g, StageTab st, const int* stn) {
+  const long b = blockIdx.x;
+  const int t = threadIdx.x;
+  const UvBlocks& B = g.ub_tile;
+  const int nown = B.nown[b];
+  int4 rec = make_int4(INT_MIN, 0, 0, 0);
+  if (t < B.ns[b]) {
+    const int x = B.elems[256 * b + t];
+    rec = make_int4(t < nown ? x : ~x, NBE_(x, 1), NBE_(x, 2), NBE_(x, 3));
+  }
+  st.rec[256 * b + t] = rec;
+  unsigned pl = ~0u;
+  double v[6] = {};
+  if (t < B.ne[b]) {
+    const int c = B.edges[256 * b + t], ia = IEC_(c, 1), ib = IEC_(c, 2);
+    pl = (unsigned)B.eloc[256 * b + t] | (unsigned)g.isbc[c] << 30;
+    // the edge's nodes are nodes of whichever of its elements the tile owns
+    const int sa = pl & 255, sb = (pl >> 8) & 255;
+    const int e = B.elems[256 * b + (sa < nown ? sa : sb)], loc = g.cvb_loc[e];
+    for (int q = 0; q < 2; ++q) {
+      const int j = IENODE_(c, q + 1);
+      const int l = j == NV_(e, 1) ? loc & 255 : j == NV_(e, 2) ? (loc >> 8) & 255 : (loc >> 16) & 255;
+      pl |= (unsigned)l << (16 + 7 * q);
+    }
+    v[0] = g.xijc[c] - g.xc[ia]; v[1] = g.yijc[c] - g.yc[ia];
+    v[2] = g.xijc[c] - g.xc[ib]; v[3] = g.yijc[c] - g.yc[ib];
+    v[4] = g.dltxc[c]; v[5] = g.dltyc[c];
+  }
+  st.edge[256 * b + t] = pl;
+  for (int q = 0; q < 6; ++q) st.egeo[(6 * b + q) * 256 + t] = v[q];
+  if (t >= FV_CVB) return;
+  const bool nact = t < g.cvb_nn[b];
+  const int i = nact ? g.cvb_nodes[FV_CVB * b + t] : 0;
+  st.node[FV_CVB * b + t] = nact ? make_int4(stn[FV_CVB * b + t], 0, g.node_obc[i], g.node_riv[i])
+                                 : make_int4(-1, 0, -1, -1);
+  for (int j = 0; j < st.nslot; ++j)
+    st.list[(st.nslot * b + j) * FV_CVB + t] = nact && j < g.cv_max ? g.cvl_ent[(long)j * g.m1 + i] : 0;
+  st.nd[2 * b * FV_CVB + t] = nact ? g.art1[i] : 1.0;
+  st.nd[(2 * b + 1) * FV_CVB + t] = nact ? g.h[i] : 0.0;
+  const bool oact = t < nown;
+  const int e = oact ? B.elems[256 * b + t] : 0;
+  st.elem[FV_CVB * b + t] = oact ? make_int4(B.epos[e], g.cvb_loc[e],
+                                             (g.isbce[e] & 3) | (g.re_off[e] < g.re_off[e + 1] ? 4 : 0), g.iucp[e])
+                                 : make_int4(0, 0, 0, 0);
+  double w[12] = {};
+  if (oact) {
+    w[0] = g.epor[e]; w[1] = g.grav_e[e]; w[2] = g.art[e]; w[3] = g.cor[e]; w[4] = g.h1[e]; w[5] = g.cc_sponge[e];
+    for (int j = 0; j < 3; ++j) {
+      w[6 + j] = g.ecv_dx[(long)j * g.n1 + e];
+      w[9 + j] = g.ecv_dy[(long)j * g.n1 + e];
+    }
+  }
+  for (int q = 0; q < 12; ++q) st.ed[(12 * b + q) * FV_CVB + t] = w[q];
+}
+
 // One 2-D stage by element tile.  A workgroup of 256 lanes takes a compact
 // tile of at most 128 elements (DevGrid::ub_tile; its nodes in st_nodes) and
 // does the whole stage for it, so that neither the edge terms nor the new
