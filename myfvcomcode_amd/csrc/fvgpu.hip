@@ -387,7 +387,11 @@ void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
     if (g.cv_max <= 16) LAUNCH("adv_ts_obc", (k_adv_ts_obc<16, FT>), (unsigned)((np + 15) / 16), 256, g, a);
     else LAUNCH("adv_ts_obc", (k_adv_ts_obc<32, FT>), (unsigned)((np + 7) / 8), 256, g, a);
   }
-#define VDIF_TS_CALL(KM) TLAUNCH("vdif_ts", k_vdif_ts_r<KM>, g.M + 1, g, a, ff, which)
+#define VDIF_TS_CALL(KM)                                                                          \
+  do {                                                                                             \
+    if (g.nsi == 0) TLAUNCH("vdif_ts", (k_vdif_ts_r<KM, true>), g.M + 1, g, a, ff, which);         \
+    else TLAUNCH("vdif_ts", (k_vdif_ts_r<KM, false>), g.M + 1, g, a, ff, which);                   \
+  } while (0)
   FV_KMAX_DISPATCH(g.KBM1, VDIF_TS_CALL);
   TLAUNCH("bcond_ts", k_bcond_ts_sums, g.IOBCN + 1, g, a, which, a.obcsum);
   if (g.IOBCN > 0) TLAUNCH("bcond_ts", k_bcond_ts_layers, (long)g.IOBCN * g.KBM1, g, a, which, (const double*)a.obcsum);
@@ -439,9 +443,11 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
 #define VISCOFH_CALL(RM) TLAUNCH_LAYERS("viscofh", k_viscofh_r<RM>, g.M + 1, g.KBM1, 3, g, a)
   FV_RMAX_DISPATCH(g.ve_max, VISCOFH_CALL);
   LAUNCH("advuv_blk", (k_uv_blk<1, FT>), dim3(g.ub_run.nblk, layer_chunks(h, g.ub_run.nblk, g.KBM1, 6)), 256, g, a);
-#define VDIF_UV_CALL(KM) LAUNCH("vdif_uv", k_vdif_uv_r<KM>, dim3(nb(g.N + 1), 2), 256, g, a)
+#define VDIF_UV_CALL(KM) do {                                                              \
+    if (g.esi == 0) LAUNCH("vdif_uv", (k_vdif_uv_r<KM, true>), (unsigned)((g.N + 127) / 128), 256, g, a);      \
+    else LAUNCH("vdif_uv", (k_vdif_uv_r<KM, false>), (unsigned)((g.N + 127) / 128), 256, g, a);                \
+  } while (0)
   FV_KMAX_DISPATCH(g.KBM1, VDIF_UV_CALL);
-  TLAUNCH("uv_finish", k_uv_finish, (long)g.N * g.KBM1, g, a);
   LAUNCH("wreal", k_wreal, nb(g.N), 256, g, a);
   const int fct = h->md->p.scalar_positivity ? 1 : 0;
   if (h->md->p.vertical_closure && h->closure_mode == 1) {
@@ -1873,7 +1879,7 @@ int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_
   static const char* fams[] = {"cvrec_ts", "cvrec_q", "cvflux_ts",
                                "cvflux_q", "adv_ts", "adv_q",
                                "viscofh", "vdif_q", "vdif_ts", "adjust1_brough", "adjust2", "baropg",
-                               "uv_finish", "copy", "closure_features", "closure_apply"};
+                               "copy", "closure_features", "closure_apply"};
   static const int cands[] = {64, 128, 256};
   if (steps < 1) return fail("autotune needs at least one step per candidate");
   // save the state; every candidate runs real steps

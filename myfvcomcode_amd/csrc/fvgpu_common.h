@@ -181,6 +181,18 @@ __device__ __forceinline__ double SIGN_(const DevGrid& g, const double* a, int i
 __device__ __forceinline__ double SIGE_(const DevGrid& g, const double* a, int i, int k) {
   return a[(long)(k - 1) * g.esk + (long)i * g.esi];
 }
+// The same for kernels instantiated for identical columns (UNI): a scalar
+// load, which waits for no other load.
+template <bool UNI>
+__device__ __forceinline__ double sign_u(const DevGrid& g, const double* a, int i, int k) {
+  if constexpr (UNI) return ((const __attribute__((address_space(4))) double*)a)[k - 1];
+  else return SIGN_(g, a, i, k);
+}
+template <bool UNI>
+__device__ __forceinline__ double sige_u(const DevGrid& g, const double* a, int i, int k) {
+  if constexpr (UNI) return ((const __attribute__((address_space(4))) double*)a)[k - 1];
+  else return SIGE_(g, a, i, k);
+}
 #define DZ(i, k) SIGN_(g, g.dz, i, k)
 #define DZZ(i, k) SIGN_(g, g.dzz, i, k)
 #define ZN(i, k) SIGN_(g, g.z, i, k)
