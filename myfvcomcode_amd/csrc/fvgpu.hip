@@ -362,7 +362,7 @@ void enqueue_external_step_t(fvgpu_handle* h, int iext, const ExtClock* ec) {
 
 // ADV_T or ADV_S with FCT, VDIF_TS, BCOND_TS, F1 = FF and N2E3D of one
 // tracer (internal_step.F), on h->cur with the scratch of `a`.
-template <typename FT>
+template <typename FT, bool UN>
 void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
   const DevGrid& g = h->g;
   const long mk = g.m1 * g.KB;
@@ -371,15 +371,15 @@ void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
   const double* fm = which == 1 ? a.tmean1 : a.smean1;
   const double* fdis = which == 1 ? g.tdis : g.sdis;
   if (h->two_phase_ts) {
-#define CVREC_TS_CALL(RM) TLAUNCH("cvrec_ts", (k_cvrec<0, RM, FT>), g.M + 1, g, a, f1, fm, 0.0, 1, g.KBM1)
+#define CVREC_TS_CALL(RM) TLAUNCH("cvrec_ts", (k_cvrec<0, RM, FT, UN>), g.M + 1, g, a, f1, fm, 0.0, 1, g.KBM1)
     FV_RMAX_DISPATCH(g.ring_max, CVREC_TS_CALL);
-    TLAUNCH("cvflux_ts", k_cvflux_ts<FT>, g.N + 1, g, a);
+    TLAUNCH("cvflux_ts", (k_cvflux_ts<FT, UN>), g.N + 1, g, a);
   } else {
-#define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1, 3)), 256, g, a, f1, fm, 0.0)
+#define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT, UN>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1, 3)), 256, g, a, f1, fm, 0.0)
     FV_RMAX_DISPATCH(g.ring_max, CVRF_TS_CALL);
   }
-#define ADV_TS_CALL10(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 10, FT>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
-#define ADV_TS_CALL16(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 16, FT>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
+#define ADV_TS_CALL10(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
+#define ADV_TS_CALL16(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL10);
   else FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL16);
   if (g.IOBCN > 0) {
@@ -387,11 +387,7 @@ void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
     if (g.cv_max <= 16) LAUNCH("adv_ts_obc", (k_adv_ts_obc<16, FT>), (unsigned)((np + 15) / 16), 256, g, a);
     else LAUNCH("adv_ts_obc", (k_adv_ts_obc<32, FT>), (unsigned)((np + 7) / 8), 256, g, a);
   }
-#define VDIF_TS_CALL(KM)                                                                          \
-  do {                                                                                             \
-    if (g.nsi == 0) TLAUNCH("vdif_ts", (k_vdif_ts_r<KM, true>), g.M + 1, g, a, ff, which);         \
-    else TLAUNCH("vdif_ts", (k_vdif_ts_r<KM, false>), g.M + 1, g, a, ff, which);                   \
-  } while (0)
+#define VDIF_TS_CALL(KM) TLAUNCH("vdif_ts", (k_vdif_ts_r<KM, UN>), g.M + 1, g, a, ff, which)
   FV_KMAX_DISPATCH(g.KBM1, VDIF_TS_CALL);
   TLAUNCH("bcond_ts", k_bcond_ts_sums, g.IOBCN + 1, g, a, which, a.obcsum);
   if (g.IOBCN > 0) TLAUNCH("bcond_ts", k_bcond_ts_layers, (long)g.IOBCN * g.KBM1, g, a, which, (const double*)a.obcsum);
@@ -401,54 +397,52 @@ void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
 
 // ADV_Q(Q, QF) with FCT_Q2 (adv_q.F, fct_q2.F) on h->cur with the scratch
 // of `a`.
-template <typename FT>
+template <typename FT, bool UN>
 void enqueue_adv_q(fvgpu_handle* h, IntArgs& a, double* q, double* qf, int fct) {
   const DevGrid& g = h->g;
   const double qmean1 = (double)1.E-8f;
   if (h->two_phase_q) {
-#define CVREC_Q_CALL(RM) TLAUNCH("cvrec_q", (k_cvrec<1, RM, FT>), g.M + 1, g, a, q, nullptr, qmean1, 2, g.KBM1)
+#define CVREC_Q_CALL(RM) TLAUNCH("cvrec_q", (k_cvrec<1, RM, FT, UN>), g.M + 1, g, a, q, nullptr, qmean1, 2, g.KBM1)
     FV_RMAX_DISPATCH(g.ring_max, CVREC_Q_CALL);
-    TLAUNCH("cvflux_q", k_cvflux_q<FT>, g.N + 1, g, a);
+    TLAUNCH("cvflux_q", (k_cvflux_q<FT, UN>), g.N + 1, g, a);
   } else {
-#define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1 - 1, 3)), 256, g, a, q, nullptr, qmean1)
+#define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT, UN>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1 - 1, 3)), 256, g, a, q, nullptr, qmean1)
     FV_RMAX_DISPATCH(g.ring_max, CVRF_Q_CALL);
   }
-#define ADV_Q_CALL10(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 10, FT>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
-#define ADV_Q_CALL16(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 16, FT>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
+#define ADV_Q_CALL10(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
+#define ADV_Q_CALL16(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL10);
   else FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL16);
 }
 
-template <typename FT>
+// UN: identical sigma columns (the kernels' UNI)
+template <typename FT, bool UN>
 void enqueue_internal_step_t(fvgpu_handle* h) {
   const DevGrid& g = h->g;
   IntArgs& a = h->ia;
   const long mk = g.m1 * g.KB, nk = g.n1 * g.KB;
   LAUNCH("int_clock", k_int_clock, 1, 64, g, h->clk, a.qdis, h->ec, 1, g.isplit);
-#define ADJ1_CALL(KM) TLAUNCH("adjust1_brough", k_adjust1_brough<KM>, g.N + 1, g, a)
+#define ADJ1_CALL(KM) TLAUNCH("adjust1_brough", (k_adjust1_brough<KM, UN>), g.N + 1, g, a)
   FV_KMAX_DISPATCH(g.KBM1, ADJ1_CALL);
-  LAUNCH("adv3d_blk", (k_uv_blk<0, FT>), g.ub_tile.nblk, 256, g, a);
-  TLAUNCH("baropg", k_baropg, g.N + 1, g, a, (int)h->md->p.barotropic);
+  LAUNCH("adv3d_blk", (k_uv_blk<0, FT, UN>), g.ub_tile.nblk, 256, g, a);
+  TLAUNCH("baropg", k_baropg<UN>, g.N + 1, g, a, (int)h->md->p.barotropic);
   if (!h->md->p.barotropic) TLAUNCH("rho1_roundtrip", k_rho1_roundtrip, (long)g.KBM1 * g.m1, g, a);
   {
     ExtArgs e = make_ext_args(h, 0, h->ext[0], h->ext[0], nullptr);
     LAUNCH("advave_int", (k_ext_stage<16, FT, true>), g.ub_tile.nblk, 256, h->dg, e);
   }
   for (int iext = 1; iext <= g.isplit; ++iext) enqueue_external_step_t<FT>(h, iext, h->ec + (iext - 1));
-#define ADJ2_CALL(KM) TLAUNCH("adjust2", k_adjust2<KM>, g.N + 1, g, a)
+#define ADJ2_CALL(KM) TLAUNCH("adjust2", (k_adjust2<KM, UN>), g.N + 1, g, a)
   FV_KMAX_DISPATCH(g.KBM1, ADJ2_CALL);
-#define VERTVL_CALL(SM) LAUNCH("vertvl", k_vertvl_tile<SM>, g.nt_nblk, 256, g, a)
+#define VERTVL_CALL(SM) LAUNCH("vertvl", (k_vertvl_tile<SM, UN>), g.nt_nblk, 256, g, a)
   FV_SMAX_DISPATCH(g.cv_max, VERTVL_CALL);
   N2E3D(a.wts, a.w);
 #define VISCOFH_CALL(RM) TLAUNCH_LAYERS("viscofh", k_viscofh_r<RM>, g.M + 1, g.KBM1, 3, g, a)
   FV_RMAX_DISPATCH(g.ve_max, VISCOFH_CALL);
-  LAUNCH("advuv_blk", (k_uv_blk<1, FT>), dim3(g.ub_run.nblk, layer_chunks(h, g.ub_run.nblk, g.KBM1, 6)), 256, g, a);
-#define VDIF_UV_CALL(KM) do {                                                              \
-    if (g.esi == 0) LAUNCH("vdif_uv", (k_vdif_uv_r<KM, true>), (unsigned)((g.N + 127) / 128), 256, g, a);      \
-    else LAUNCH("vdif_uv", (k_vdif_uv_r<KM, false>), (unsigned)((g.N + 127) / 128), 256, g, a);                \
-  } while (0)
+  LAUNCH("advuv_blk", (k_uv_blk<1, FT, UN>), dim3(g.ub_run.nblk, layer_chunks(h, g.ub_run.nblk, g.KBM1, 6)), 256, g, a);
+#define VDIF_UV_CALL(KM) LAUNCH("vdif_uv", (k_vdif_uv_r<KM, UN>), (unsigned)((g.N + 127) / 128), 256, g, a)
   FV_KMAX_DISPATCH(g.KBM1, VDIF_UV_CALL);
-  LAUNCH("wreal", k_wreal, nb(g.N), 256, g, a);
+  LAUNCH("wreal", k_wreal<UN>, nb(g.N), 256, g, a);
   const int fct = h->md->p.scalar_positivity ? 1 : 0;
   if (h->md->p.vertical_closure && h->closure_mode == 1) {
     // learned closure: features, MFMA inference, realizability, then the
@@ -462,18 +456,18 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     LAUNCH("zero", k_zero_int, 1, 64, h->cl_nfall, 1);
     TLAUNCH("closure_apply", k_closure_apply, g.M, g, a, h->cl_yp, a.gx, h->cl_flag, h->cl_nfall);
     TLAUNCH("fallback_q2f", k_fallback_q2f, g.M + 1, g, a, (const int*)h->cl_flag);
-#define VDIF_QM_CALL(RM) TLAUNCH("vdif_q", k_vdif_q<RM>, g.M + 1, g, a, a.vhpair, h->cl_flag)
+#define VDIF_QM_CALL(RM) TLAUNCH("vdif_q", (k_vdif_q<RM, UN>), g.M + 1, g, a, a.vhpair, h->cl_flag)
     // (vdif_q also stores Q2 = Q2F, Q2L = Q2LF for its columns)
     FV_RMAX_DISPATCH(g.ve_max, VDIF_QM_CALL);
   } else if (h->md->p.vertical_closure) {
     // ADV_Q of Q2 on the main stream, of Q2L on stream2 (own scratch)
     fork_streams(h, FV_CONC_3D);
     on_stream2(h, FV_CONC_3D);
-    enqueue_adv_q<FT>(h, h->ib, a.q2l, a.q2lf, fct);
+    enqueue_adv_q<FT, UN>(h, h->ib, a.q2l, a.q2lf, fct);
     on_stream1(h);
-    enqueue_adv_q<FT>(h, a, a.q2, a.q2f, fct);
+    enqueue_adv_q<FT, UN>(h, a, a.q2, a.q2f, fct);
     join_streams(h, FV_CONC_3D);
-#define VDIF_Q_CALL(RM) TLAUNCH("vdif_q", k_vdif_q<RM>, g.M + 1, g, a, a.vhpair, (const int*)nullptr)
+#define VDIF_Q_CALL(RM) TLAUNCH("vdif_q", (k_vdif_q<RM, UN>), g.M + 1, g, a, a.vhpair, (const int*)nullptr)
     // VDIF_Q, then Q2 = Q2F and Q2L = Q2LF (internal_step.F:1029-1035) in
     // the same kernel, the elimination coefficients in `vhpair`.
     FV_RMAX_DISPATCH(g.ve_max, VDIF_Q_CALL);
@@ -489,14 +483,14 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
   if (t_on && s_on) {
     fork_streams(h, FV_CONC_3D);
     on_stream2(h, FV_CONC_3D);
-    enqueue_ts_pass<FT>(h, h->ib, 2, fct);
+    enqueue_ts_pass<FT, UN>(h, h->ib, 2, fct);
     on_stream1(h);
-    enqueue_ts_pass<FT>(h, a, 1, fct);
+    enqueue_ts_pass<FT, UN>(h, a, 1, fct);
     join_streams(h, FV_CONC_3D);
   } else if (t_on) {
-    enqueue_ts_pass<FT>(h, a, 1, fct);
+    enqueue_ts_pass<FT, UN>(h, a, 1, fct);
   } else if (s_on) {
-    enqueue_ts_pass<FT>(h, a, 2, fct);
+    enqueue_ts_pass<FT, UN>(h, a, 2, fct);
   }
   if (!g.river_ts_specified && g.NUMQBC > 0) LAUNCH("adjust_ts", k_adjust_ts, 1, 256, g, a);
   if (!h->md->p.barotropic) {
@@ -519,8 +513,14 @@ void enqueue_external_step(fvgpu_handle* h, int iext) {
 }
 
 void enqueue_internal_step(fvgpu_handle* h) {
-  if (h->precision == FV_MIXED) enqueue_internal_step_t<float>(h);
-  else enqueue_internal_step_t<double>(h);
+  const bool uniform = h->g.nsi == 0;
+  if (h->precision == FV_MIXED) {
+    if (uniform) enqueue_internal_step_t<float, true>(h);
+    else enqueue_internal_step_t<float, false>(h);
+  } else {
+    if (uniform) enqueue_internal_step_t<double, true>(h);
+    else enqueue_internal_step_t<double, false>(h);
+  }
 }
 
 // Wind stress of element wind speeds (PSIMPLE_DRAG, mod_bulk.F:58-90),

@@ -89,7 +89,7 @@ __global__ void k_copy(double* dst, const double* src, long n) {
 
 // ADJUST2D3D(1) (adjust2d3d.F:52-63), BCOND_GCN(5,0) (bcond_gcn.F:537-616)
 // and BOTTOM_ROUGHNESS (brough.F:88-151) for one element column.
-template <int KMAX>
+template <int KMAX, bool UNI>
 __global__ __launch_bounds__(256) void k_adjust1_brough(DevGrid g, IntArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < 1 || i > g.N) return;
@@ -136,6 +136,7 @@ __global__ __launch_bounds__(256) void k_adjust1_brough(DevGrid g, IntArgs a) {
 
 // BAROPG (baropg.F:33-166) with the RMEAN round trip of RHO applied to the
 // element's own column; the node round trip is k_rho1_roundtrip.
+template <bool UNI>
 __global__ void k_baropg(DevGrid g, IntArgs a, int barotropic) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > g.N) return;
@@ -220,7 +221,7 @@ __global__ void k_rho1_roundtrip(DevGrid g, IntArgs a) {
 }
 
 // ADJUST2D3D(2) (adjust2d3d.F:65-110).
-template <int KMAX>
+template <int KMAX, bool UNI>
 __global__ __launch_bounds__(256) void k_adjust2(DevGrid g, IntArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > g.N) return;
@@ -276,6 +277,7 @@ __global__ __launch_bounds__(256) void k_n2e3d(DevGrid g, const double* nvar, do
 // WREAL (wreal.F:32-140): one thread per element column, its layers taken
 // eight at a time with the eight layers' loads issued before their
 // arithmetic.
+template <bool UNI>
 __global__ __launch_bounds__(256) void k_wreal(DevGrid g, IntArgs a) {
   const int i = (int)xcd_thread() + 1;
   if (i > g.N) return;

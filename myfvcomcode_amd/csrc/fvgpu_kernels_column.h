@@ -50,8 +50,8 @@ __global__ __launch_bounds__(256) void k_vdif_uv_r(DevGrid g, IntArgs a) {
   const bool solve = d1 > 0.0;
   const long n1 = g.n1;
   double* X = f ? a.vf : a.uf;
-  auto dz1 = [&](int k) { return sige_u<UNI>(g, g.dz1, i, k); };
-  auto dzz1 = [&](int k) { return sige_u<UNI>(g, g.dzz1, i, k); };
+  auto dz1 = [&](int k) { return DZ1(i, k); };
+  auto dzz1 = [&](int k) { return DZZ1(i, k); };
   // KM1 of level k+1 and X of layer k (past the column: its last)
   double kmp[KMAX + FV_AHEAD + 1], xk[KMAX + FV_AHEAD + 1];
   auto ahead = [&](auto kc) {
@@ -123,8 +123,8 @@ __global__ __launch_bounds__(256) void k_vdif_ts_r(DevGrid g, IntArgs a, double*
   const int KBM1 = g.KBM1, KBM2 = g.KBM2;
   const double dti = g.dti, umolpr = g.umol * 1.E0, d = a.d[i];
   const long m1 = g.m1;
-  auto dz = [&](int k) { return sign_u<UNI>(g, g.dz, i, k); };
-  auto dzz = [&](int k) { return sign_u<UNI>(g, g.dzz, i, k); };
+  auto dz = [&](int k) { return DZ(i, k); };
+  auto dzz = [&](int k) { return DZZ(i, k); };
   double VHF[KMAX + 1], VHPF[KMAX + 1];
   // KH of level k+1 and F of layer k (past the column: its last)
   double khp[KMAX + FV_AHEAD + 1], fk[KMAX + FV_AHEAD + 1];
@@ -240,7 +240,7 @@ struct Q25Loads {
 // instruction cache, and no load could cross a level's branch).  62,500
 // elements x 40 layers: 257 -> 173 us; 1,000,000 x 40: 1277 -> 1082 us (4.9 GB,
 // 4.5 TB/s; 2 waves a SIMD instead of 3).
-template <int RMAX>
+template <int RMAX, bool UNI>
 __global__ __launch_bounds__(256) void k_vdif_q(DevGrid g, IntArgs a, double2* vhs, const int* only) {
   constexpr int UP = 4;
   const int i = (int)xcd_thread();

@@ -84,7 +84,7 @@ __device__ __forceinline__ void cv_load(const DevGrid& g, const IntArgs& a, int 
   if (KIND == 0) L.vh = a.viscofh[ko + i];
 }
 
-template <int KIND, int RMAX, typename FT>
+template <int KIND, int RMAX, typename FT, bool UNI>
 __device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntArgs& a, int i, const RingGeo<RMAX>& rg,
                                                    double art2, double nn, const CvLoads<RMAX>& L,
                                                    const double* mean, double cmean, int k) {
@@ -138,18 +138,18 @@ __device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntAr
   return r;
 }
 
-template <int KIND, int RMAX, typename FT>
+template <int KIND, int RMAX, typename FT, bool UNI>
 __device__ __forceinline__ CvRecT<FT> cv_record(const DevGrid& g, const IntArgs& a, int i, const RingGeo<RMAX>& rg,
                                                 double art2, double nn, const double* f, const double* mean,
                                                 double cmean, int k) {
   CvLoads<RMAX> L;
   cv_load<KIND, RMAX>(g, a, i, rg, f, mean, cmean, k, L);
-  return cv_record_of<KIND, RMAX, FT>(g, a, i, rg, art2, nn, L, mean, cmean, k);
+  return cv_record_of<KIND, RMAX, FT, UNI>(g, a, i, rg, art2, nn, L, mean, cmean, k);
 }
 
 // Ring gradient / bounds of field f at node i for the layers [k0, k1], one
 // thread per node with its ring in registers.
-template <int KIND, int RMAX, typename FT>
+template <int KIND, int RMAX, typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_cvrec(DevGrid g, IntArgs a, const double* f, const double* mean,
                                                double cmean, int k0, int k1) {
   const int i = (int)xcd_thread();
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void k_cvrec(DevGrid g, IntArgs a, const doubl
   ring_geo_load<RMAX>(g, i, rg);
   const double art2 = g.art2[i], nn = g.nn_hvc[i];
   for (int k = k0; k <= k1; ++k)
-    rec[(long)(k - 1) * g.m1 + i] = cv_record<KIND, RMAX, FT>(g, a, i, rg, art2, nn, f, mean, cmean, k);
+    rec[(long)(k - 1) * g.m1 + i] = cv_record<KIND, RMAX, FT, UNI>(g, a, i, rg, art2, nn, f, mean, cmean, k);
 }
 
 // Min and max of field f over the NBSN ring of node i at layer offset ko,
@@ -290,7 +290,7 @@ __device__ __forceinline__ void cv_faces(const ElemFaces<FT>& f, const CvRecT<FT
 // The two nodes of a face enter the diffusive terms through sums, which are
 // the same in either order, and the upwind value through FIJ1 (side IA) and
 // FIJ2 (side IB), exchanged when IA is node B.
-template <typename FT>
+template <typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_cvflux_ts(DevGrid g, IntArgs a) {
   const int e = (int)xcd_thread();
   if (e < 1 || e > g.N) return;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a) {
 // Phase 3 of ADV_T/ADV_S (adv_t.F:507-1052): ordered sub-edge sums (in FP64
 // whatever the flux type), bottom gradients for VDIF_TS, vertical flux,
 // rivers, the update TF1 = (T1 - XFLUX/ART1*DTI/(DT*DZ))*DT/DTFA and FCT.
-template <int SMAX, int RMAX, typename FT>
+template <int SMAX, int RMAX, typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, const double* f1, double* ff,
                                                         const double* fdis, int which, int fct) {
   const int i = (int)xcd_thread();
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
 // on layer interfaces k = 2..KBM1, the element velocity interpolated to the
 // interface with DZ1 weights (once for the three faces); faces as in
 // k_cvflux_ts.
-template <typename FT>
+template <typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_cvflux_q(DevGrid g, IntArgs a) {
   const int e = (int)xcd_thread();
   if (e < 1 || e > g.N) return;
@@ -510,7 +510,7 @@ struct CvRecLds {
 // other kernels read (rec_keep: OBC nodes and their sub-edge neighbours)
 // and, for the tracer, at the bottom layer (the bottom gradients of
 // VDIF_TS).
-template <int KIND, int RMAX, typename FT>
+template <int KIND, int RMAX, typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const double* fld, const double* mean,
                                                    double cmean) {
   __shared__ CvRecLds<FT> srec[2];
@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
       if (s < nk) {
         if (nact) {
           if (!ahead) cv_load<KIND, RMAX>(g, a, i, rg, fld, mean, cmean, k, L);
-          const CvRecT<FT> r = cv_record_of<KIND, RMAX, FT>(g, a, i, rg, art2, nnv, L, mean, cmean, k);
+          const CvRecT<FT> r = cv_record_of<KIND, RMAX, FT, UNI>(g, a, i, rg, art2, nnv, L, mean, cmean, k);
           srec[s & 1].put(t, r);
           if (keep || (KIND == 0 && k == g.KBM1)) rec[(long)(k - 1) * g.m1 + i] = r;
         }
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
 }
 
 // Phase 3 of ADV_Q (adv_q.F:340-390): ordered sums, vertical flux, update.
-template <int SMAX, int RMAX, typename FT>
+template <int SMAX, int RMAX, typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, const double* q, double* qf, int fct) {
   const int i = (int)xcd_thread();
   if (i > g.M) return;
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, cons
 // element-layer velocity is loaded once per tile, and the per-layer sums
 // read LDS instead of gathering the elements' velocities again for each of
 // their nodes.
-template <int SMAX>
+template <int SMAX, bool UNI>
 __global__ __launch_bounds__(256) void k_vertvl_tile(DevGrid g, IntArgs a) {
   __shared__ double sterm[2][3 * FV_NTE];
   const int b = xcd_block(), t = threadIdx.x;

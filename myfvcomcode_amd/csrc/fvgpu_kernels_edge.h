@@ -42,7 +42,7 @@ struct UvFluxLds {
   FT xadv[256], yadv[256], fx[256], fy[256], visc[256];
 };
 
-template <int MODE, typename FT>
+template <int MODE, typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
   __shared__ UvRecsLds<FT> sr;
   __shared__ UvFluxLds<FT> sf;
