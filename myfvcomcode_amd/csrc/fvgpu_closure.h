@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void k_closure_features(DevGrid g, IntArgs a, 
     double fv[RMAX];
     static_for<RMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      fv[j] = f[eo + re[j]];
+      fv[j] = at(f + eo, re[j]);
     });
     double s = 0.0;
     static_for<RMAX>([&](auto jc) {

@@ -270,7 +270,10 @@ __global__ __launch_bounds__(256) void k_n2e3d(DevGrid g, const double* nvar, do
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     const int k = k0 + q;
-    if (k <= kmax) evar[EI(g, i, k)] = one_third * (nvar[NI(g, j1, k)] + nvar[NI(g, j2, k)] + nvar[NI(g, j3, k)]);
+    if (k <= kmax) {
+      const double* nk = nvar + (long)(k - 1) * g.m1;
+      evar[EI(g, i, k)] = one_third * (at(nk, j1) + at(nk, j2) + at(nk, j3));
+    }
   }
 }
 

@@ -298,8 +298,8 @@ __global__ __launch_bounds__(256) void k_vdif_q(DevGrid g, IntArgs a, double2* v
     const long eo = (long)(k - 1) * g.n1;
     static_for<RMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      ur[j] = a.u[eo + re[j]];
-      vr[j] = a.v[eo + re[j]];
+      ur[j] = at(a.u + eo, re[j]);
+      vr[j] = at(a.v + eo, re[j]);
     });
   };
   auto ring_avg = [&](const double (&fv)[RMAX]) {
@@ -312,15 +312,15 @@ __global__ __launch_bounds__(256) void k_vdif_q(DevGrid g, IntArgs a, double2* v
   };
   auto load_level = [&](int k) {
     Q25Loads<RMAX> r;
-    const long q = (long)(k - 1) * m1 + i;
-    r.rho = a.rho1[q];
-    r.kq = KQ[q + m1];
-    r.q2 = a.q2[q];
-    r.q2l = a.q2l[q];
-    r.km = KM[q];
-    r.kh = KH[q];
-    r.q2f = Q2F[q];
-    r.q2lf = Q2LF[q];
+    const long ko = (long)(k - 1) * m1;
+    r.rho = at(a.rho1 + ko, i);
+    r.kq = at(KQ + (ko + m1), i);
+    r.q2 = at(a.q2 + ko, i);
+    r.q2l = at(a.q2l + ko, i);
+    r.km = at(KM + ko, i);
+    r.kh = at(KH + ko, i);
+    r.q2f = at(Q2F + ko, i);
+    r.q2lf = at(Q2LF + ko, i);
     r.dzz = DZZ(i, k - 1);
     r.dz = DZ(i, k);
     r.z = ZN(i, k);

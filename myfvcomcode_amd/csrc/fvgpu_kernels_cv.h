@@ -77,11 +77,11 @@ __device__ __forceinline__ void cv_load(const DevGrid& g, const IntArgs& a, int 
   // read node 0) so that the loads issue together
   static_for<RMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    L.fv[j] = f[ko + rg.rn[j]];
-    if (KIND == 0) L.mv[j] = mean ? mean[ko + rg.rn[j]] : cmean;
+    L.fv[j] = at(f + ko, rg.rn[j]);
+    if (KIND == 0) L.mv[j] = mean ? at(mean + ko, rg.rn[j]) : cmean;
   });
-  L.c = f[ko + i];
-  if (KIND == 0) L.vh = a.viscofh[ko + i];
+  L.c = at(f + ko, i);
+  if (KIND == 0) L.vh = at(a.viscofh + ko, i);
 }
 
 template <int KIND, int RMAX, typename FT, bool UNI>
@@ -95,7 +95,7 @@ __device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntAr
   double mv[RMAX];
   static_for<RMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    mv[j] = KIND == 0 ? L.mv[j] : (mean ? mean[ko + rg.rn[j]] : cmean);
+    mv[j] = KIND == 0 ? L.mv[j] : (mean ? at(mean + ko, rg.rn[j]) : cmean);
   });
   double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
   double f1 = fv[0];
@@ -122,7 +122,7 @@ __device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntAr
   if (KIND == 0) {
     vhn = L.vh * nn;
   } else {
-    const double vfa = (a.viscofh[ko + i] * DZ(i, k - 1) + a.viscofh[ko - g.m1 + i] * DZ(i, k)) /
+    const double vfa = (at(a.viscofh + ko, i) * DZ(i, k - 1) + at(a.viscofh + (ko - g.m1), i) * DZ(i, k)) /
                        (DZ(i, k) + DZ(i, k - 1));
     vhn = vfa * nn;
   }
@@ -166,9 +166,9 @@ __global__ __launch_bounds__(256) void k_cvrec(DevGrid g, IntArgs a, const doubl
 // the ring alone (entry NTSN repeats entry 1), in the order k_cvrec forms
 // them: the FCT bounds (fct_t.F:74-80, fct_q2.F:60-66).
 template <int RMAX>
-__device__ __forceinline__ void ring_bounds(const int (&rn)[RMAX], int nt, const double* f, long ko, double& lo,
+__device__ __forceinline__ void ring_bounds(const int (&rn)[RMAX], const double* f, long ko, double& lo,
                                             double& hi) {
-  lo = f[ko + rn[0]];
+  lo = at(f + ko, rn[0]);
   hi = lo;
   // Slots past the ring repeat its first node (min and max are unchanged),
   // so every load is unconditional and all of them issue before the first
@@ -176,21 +176,21 @@ __device__ __forceinline__ void ring_bounds(const int (&rn)[RMAX], int nt, const
   static_for<RMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
     if (j >= 1) {
-      const double v = f[ko + (j < nt - 1 ? rn[j] : rn[0])];
+      const double v = at(f + ko, rn[j]);
       lo = fmin(lo, v);
       hi = fmax(hi, v);
     }
   });
 }
 
+// The ring alone: entry NTSN repeats entry 1, and so do the slots past it.
 template <int RMAX>
-__device__ __forceinline__ int load_ring(const DevGrid& g, int i, int (&rn)[RMAX]) {
+__device__ __forceinline__ void load_ring(const DevGrid& g, int i, int (&rn)[RMAX]) {
   const int o = g.nbsn_off[i], nt = g.ntsn[i];
   static_for<RMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    rn[j] = j < nt ? g.nbsn[o + j] : 0;
+    rn[j] = g.nbsn[o + (j < nt - 1 ? j : 0)];
   });
-  return nt;
 }
 
 // Face flux of ADV_T/ADV_S through sub-edge c at layer k (adv_t.F:440-500),
@@ -368,27 +368,24 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
   const bool isobc = g.isonb[i] == 2;
   const long cs = (long)g.NCV + 1;
   int rn[RMAX];
-  const int nt = clip ? load_ring<RMAX>(g, i, rn) : 0;
+  if (clip) load_ring<RMAX>(g, i, rn);
   int k0, k1;
   layer_share(1, g.KBM1, k0, k1);
   for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.m1;
     const FT* fl = (const FT*)a.cvflux + (long)(k - 1) * cs;
-    // all SMAX loads issue together (slots past the node's count read the
-    // unused entry 0); the sum takes the node's own terms in sub-edge order
+    // all SMAX loads issue together; the sum takes the node's terms in
+    // sub-edge order, subtracting on side IB, and the slots past its count
+    // add the unused entry 0, which is zero and leaves it as it is
     FT xv[SMAX];
     static_for<SMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      xv[j] = fl[ce[j] >> 1];
+      xv[j] = at(fl, ce[j] >> 1);
     });
     double xflux = 0.0;
     static_for<SMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      if (j < n) {
-        const double x = (double)xv[j];
-        if (ce[j] & 1) xflux = xflux - x;
-        else xflux = xflux + x;
-      }
+      xflux = xflux + flip_sign((double)xv[j], ce[j]);
     });
     if (k == g.KBM1) {  // ADV_T and ADV_S both set the bottom-gradient terms VDIF_TS reads
       const CvRecT<FT> r = ((const CvRecT<FT>*)a.rec)[ko + i];
@@ -396,16 +393,16 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
       a.pfpyb[i] = (double)r.gy;
       a.ah_bottom[i] = (g.fact * a.viscofh[ko + i] + g.fm1) * g.nn_hvc[i];
     }
-    const double fk = f1[ko + i], dzk = DZ(i, k);
+    const double fk = at(f1 + ko, i), dzk = DZ(i, k);
     // DZ-weighted values at the layer's upper (nu/du) and lower (nd/dd)
     // interfaces: the vertical flux (adv_t.F:873-881) and the FCT bounds
     // (fct_t.F:82-101) use the same expressions.  The neighbours are loaded
     // unconditionally (layer 1 reads itself as its upper neighbour, level
     // KB exists below KBM1) so that the loads issue together.
     const long kup = k != 1 ? ko - g.m1 : ko;
-    const double fup = f1[kup + i], dzm = DZ(i, k != 1 ? k - 1 : k);
-    const double fdn = f1[ko + g.m1 + i], dzp = DZ(i, k + 1);
-    const double wk = a.wts[ko + i], wkp = a.wts[ko + g.m1 + i];
+    const double fup = at(f1 + kup, i), dzm = DZ(i, k != 1 ? k - 1 : k);
+    const double fdn = at(f1 + (ko + g.m1), i), dzp = DZ(i, k + 1);
+    const double wk = at(a.wts + ko, i), wkp = at(a.wts + (ko + g.m1), i);
     double temp, nu = 0.0, du = 1.0, nd = 0.0, dd = 1.0;
     const bool has_up = k != 1, has_dn = k == 1 || k != g.KBM1;   // the reference's branch order
     if (has_up) {
@@ -434,7 +431,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
     double x = (fk - xflux / art1 * (g.dti / (a.dt[i] * dzk))) * (a.dt[i] / a.dtfa[i]);
     if (clip) {  // FCT_T / FCT_S (fct_t.F:74-101)
       double tmin, tmax;
-      ring_bounds<RMAX>(rn, nt, f1, ko, tmin, tmax);
+      ring_bounds<RMAX>(rn, f1, ko, tmin, tmax);
       if (has_up) { const double v = nu / du; tmax = fmax(tmax, v); tmin = fmin(tmin, v); }
       if (has_dn) { const double v = nd / dd; tmax = fmax(tmax, v); tmin = fmin(tmin, v); }
       if (tmin - x > 0.0) x = tmin;
@@ -567,7 +564,7 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
       if (s > 0) {
         const int k = k0 + s - 1;
         const long eo = (long)(k - 1) * g.n1;
-        const double uk = a.u[eo + e], vk = a.v[eo + e];
+        const double uk = at(a.u + eo, e), vk = at(a.v + eo, e);
         const double dz1k = DZ1(e, k);
         if (eact) {
           const CvRecLds<FT>& sr = srec[(s - 1) & 1];
@@ -592,8 +589,12 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
 }
 
 // Phase 3 of ADV_Q (adv_q.F:340-390): ordered sums, vertical flux, update.
+// Held to 3 waves a SIMD: with the 4 that its registers would allow, the
+// workgroups' layers spread over more lines than an L2 holds and the faces
+// and ring values shared by neighbours are fetched again (1,000,000 elements
+// x 40 layers: 650 us at 4, 506 at 3; 532 before its 32-bit addresses).
 template <int SMAX, int RMAX, typename FT, bool UNI>
-__global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, const double* q, double* qf, int fct) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_adv_q_gather(DevGrid g, IntArgs a, const double* q, double* qf, int fct) {
   const int i = (int)xcd_thread();
   if (i > g.M) return;
   if (i == 0) {
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, cons
   const long cs = (long)g.NCV + 1;
   const bool clip = fct && !g.fct_skip[i];
   int rn[RMAX];
-  const int nt = clip ? load_ring<RMAX>(g, i, rn) : 0;
+  if (clip) load_ring<RMAX>(g, i, rn);
   if (blockIdx.y == 0) {
     qf[NI(g, i, 1)] = 0.0;
     qf[NI(g, i, g.KB)] = 0.0;
@@ -621,35 +622,32 @@ __global__ __launch_bounds__(256) void k_adv_q_gather(DevGrid g, IntArgs a, cons
   for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.m1;
     const FT* fl = (const FT*)a.cvflux + (long)(k - 1) * cs;
-    // all SMAX loads issue together (slots past the node's count read the
-    // unused entry 0); the sum takes the node's own terms in sub-edge order
+    // all SMAX loads issue together; the sum takes the node's terms in
+    // sub-edge order, subtracting on side IB, and the slots past its count
+    // add the unused entry 0, which is zero and leaves it as it is
     FT xv[SMAX];
     static_for<SMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      xv[j] = fl[ce[j] >> 1];
+      xv[j] = at(fl, ce[j] >> 1);
     });
     double xflux = 0.0;
     static_for<SMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      if (j < n) {
-        const double x = (double)xv[j];
-        if (ce[j] & 1) xflux = xflux - x;
-        else xflux = xflux + x;
-      }
+      xflux = xflux + flip_sign((double)xv[j], ce[j]);
     });
-    const double temp = a.wts[ko - g.m1 + i] * q[ko - g.m1 + i] - a.wts[ko + g.m1 + i] * q[ko + g.m1 + i];
+    const double qup = at(q + (ko - g.m1), i), qdn = at(q + (ko + g.m1), i), qk = at(q + ko, i);
+    const double temp = at(a.wts + (ko - g.m1), i) * qup - at(a.wts + (ko + g.m1), i) * qdn;
     xflux = xflux + temp * art1 * DZZ(i, k - 1) / (DZ(i, k - 1) + DZ(i, k));
-    const double qk = q[ko + i];
     double x = (qk - xflux / art1 * (dti / (dtn * DZZ(i, k - 1)))) * (dtn / dn);
     if (clip) {  // FCT_Q2 / FCT_Q2L (fct_q2.F:60-95)
       double qmin, qmax;
-      ring_bounds<RMAX>(rn, nt, q, ko, qmin, qmax);
+      ring_bounds<RMAX>(rn, q, ko, qmin, qmax);
       if (k != 2) {
-        const double v = (qk * DZZ(i, k - 2) + q[ko - g.m1 + i] * DZZ(i, k - 1)) / (DZZ(i, k - 1) + DZZ(i, k - 2));
+        const double v = (qk * DZZ(i, k - 2) + qup * DZZ(i, k - 1)) / (DZZ(i, k - 1) + DZZ(i, k - 2));
         qmax = fmax(qmax, v); qmin = fmin(qmin, v);
       }
       if (k == 2 || k != g.KBM1) {
-        const double v = (qk * DZZ(i, k) + q[ko + g.m1 + i] * DZZ(i, k - 1)) / (DZZ(i, k) + DZZ(i, k - 1));
+        const double v = (qk * DZZ(i, k) + qdn * DZZ(i, k - 1)) / (DZZ(i, k) + DZZ(i, k - 1));
         qmax = fmax(qmax, v); qmin = fmin(qmin, v);
       }
       if (qmin - x > 0.0) x = qmin;
@@ -707,7 +705,7 @@ __global__ __launch_bounds__(256) void k_vertvl_tile(DevGrid g, IntArgs a) {
         u0 = u1; v0 = v1; z0 = z1;
         if (s + 2 < KBM1) {
           const long kn = (long)(s + 2) * g.n1;
-          u1 = a.u[kn + e]; v1 = a.v[kn + e]; z1 = DZ1(e, s + 3);
+          u1 = at(a.u + kn, e); v1 = at(a.v + kn, e); z1 = DZ1(e, s + 3);
         }
         if (eact) {
           const double dij = dt1 * dz;
@@ -821,8 +819,8 @@ __global__ __launch_bounds__(256) void k_viscofh_r(DevGrid g, IntArgs a) {
     double ur[RMAX], vr[RMAX];
     static_for<RMAX>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      ur[j] = a.u[ko + re[j]];
-      vr[j] = a.v[ko + re[j]];
+      ur[j] = at(a.u + ko, re[j]);
+      vr[j] = at(a.v + ko, re[j]);
     });
     double pupx = 0.0, pupy = 0.0, pvpx = 0.0, pvpy = 0.0;
     {
@@ -843,7 +841,7 @@ __global__ __launch_bounds__(256) void k_viscofh_r(DevGrid g, IntArgs a) {
       }
     });
     {
-      const double uu = a.u[ko + el], vv = a.v[ko + el];
+      const double uu = at(a.u + ko, el), vv = at(a.v + ko, el);
       pupx = pupx + uu * ryl; pupy = pupy + uu * rxl;
       pvpx = pvpx + vv * ryl; pvpy = pvpy + vv * rxl;
       if (bnd) {

@@ -109,9 +109,9 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
   const int xs[4] = {x, x1, x2, x3};
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const long f = (long)(k0 - 1) * g.n1 + xs[q];
-    pu[q] = U[f];
-    pv[q] = V[f];
+    const long f = (long)(k0 - 1) * g.n1;
+    pu[q] = at(U + f, xs[q]);
+    pv[q] = at(V + f, xs[q]);
   }
   for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.n1;
@@ -121,8 +121,8 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
     const long kp = ko + g.n1, km = k != 1 ? ko - g.n1 : ko;
     double ck = 0.0, ok = 0.0, wk = 0.0, wp = 0.0, cp = 0.0, cm = 0.0, rk = 0.0;
     if (MODE == 1) {
-      ck = C[ko + io]; ok = O[ko + io]; wk = a.w[ko + io]; wp = a.w[kp + io];
-      cp = C[kp + io]; cm = C[km + io]; rk = R[ko + io];
+      ck = at(C + ko, io); ok = at(O + ko, io); wk = at(a.w + ko, io); wp = at(a.w + kp, io);
+      cp = at(C + kp, io); cm = at(C + km, io); rk = at(R + ko, io);
     }
     const double dzk = DZ1(io, k), dzp = DZ1(io, k + 1), dzm = DZ1(io, k != 1 ? k - 1 : k);
     if (ract) {
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void k_uv_blk(DevGrid g, IntArgs a) {
     }
     if (k < k1) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) { pu[q] = U[kp + xs[q]]; pv[q] = V[kp + xs[q]]; }
+      for (int q = 0; q < 4; ++q) { pu[q] = at(U + kp, xs[q]); pv[q] = at(V + kp, xs[q]); }
     }
     __syncthreads();
     if (eact) {
