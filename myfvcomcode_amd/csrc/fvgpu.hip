@@ -98,7 +98,6 @@ struct fvgpu_handle {
   int concurrent = 3;     // bit 0: the 3-D chain pairs on stream2
   // CV records then face fluxes in two launches (1) or one fused launch
   // (0), for ADV_T/ADV_S and for ADV_Q
-  int two_phase_ts = 0, two_phase_q = 0;
   // wind speeds at the start (wu0, wv0) and end (wu1, wv1) of the coming
   // internal step; once they differ, every external step forms its own
   // stress (ws2x, ws2y), otherwise it uses the end stress g.wsx/g.wsy
@@ -370,14 +369,8 @@ void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
   double* ff = which == 1 ? a.tf1 : a.sf1;
   const double* fm = which == 1 ? a.tmean1 : a.smean1;
   const double* fdis = which == 1 ? g.tdis : g.sdis;
-  if (h->two_phase_ts) {
-#define CVREC_TS_CALL(RM) TLAUNCH("cvrec_ts", (k_cvrec<0, RM, FT, UN>), g.M + 1, g, a, f1, fm, 0.0, 1, g.KBM1)
-    FV_RMAX_DISPATCH(g.ring_max, CVREC_TS_CALL);
-    TLAUNCH("cvflux_ts", (k_cvflux_ts<FT, UN>), g.N + 1, g, a);
-  } else {
 #define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT, UN>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1, 3)), 256, g, a, f1, fm, 0.0)
-    FV_RMAX_DISPATCH(g.ring_max, CVRF_TS_CALL);
-  }
+  FV_RMAX_DISPATCH(g.ring_max, CVRF_TS_CALL);
 #define ADV_TS_CALL10(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
 #define ADV_TS_CALL16(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL10);
@@ -401,14 +394,8 @@ template <typename FT, bool UN>
 void enqueue_adv_q(fvgpu_handle* h, IntArgs& a, double* q, double* qf, int fct) {
   const DevGrid& g = h->g;
   const double qmean1 = (double)1.E-8f;
-  if (h->two_phase_q) {
-#define CVREC_Q_CALL(RM) TLAUNCH("cvrec_q", (k_cvrec<1, RM, FT, UN>), g.M + 1, g, a, q, nullptr, qmean1, 2, g.KBM1)
-    FV_RMAX_DISPATCH(g.ring_max, CVREC_Q_CALL);
-    TLAUNCH("cvflux_q", (k_cvflux_q<FT, UN>), g.N + 1, g, a);
-  } else {
 #define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT, UN>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1 - 1, 3)), 256, g, a, q, nullptr, qmean1)
-    FV_RMAX_DISPATCH(g.ring_max, CVRF_Q_CALL);
-  }
+  FV_RMAX_DISPATCH(g.ring_max, CVRF_Q_CALL);
 #define ADV_Q_CALL10(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
 #define ADV_Q_CALL16(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL10);
@@ -718,18 +705,8 @@ int build_lists(fvgpu_handle* h) {
     };
     std::vector<int> ids(N);
     for (int e = 1; e <= N; ++e) ids[e - 1] = e;
-    std::vector<int> mark(M + 1, -1);
+    std::vector<int> mark(M + 1, -1), nloc(M + 1, 0);
     int stamp = 0;
-    auto distinct_nodes = [&](int lo, int hi) {
-      ++stamp;
-      int n = 0;
-      for (int q = lo; q < hi; ++q)
-        for (int j = 0; j < 3; ++j) {
-          const int nd = md->nv[(size_t)j * (N + 1) + ids[q]];
-          if (mark[nd] != stamp) { mark[nd] = stamp; ++n; }
-        }
-      return n;
-    };
     // the elements' edges, and they with the other elements of those edges,
     // number at most 256 each (the blocked momentum kernels)
     std::vector<int> emark(N + 1, -1), cmark(NE + 1, -1);
@@ -752,12 +729,68 @@ int build_lists(fvgpu_handle* h) {
       }
       return nr <= 256 && nc <= 256;
     };
-    std::vector<std::pair<int, int>> stack = component_ranges(ids, ecomp), leaves;
+    // a block's tables; false if its nodes, or they with the nodes of their
+    // rings, are too many
+    const int rw = (g.ring_max + 3) / 4;
+    g.cvr_w = rw;
+    std::vector<int> bnn, bne, bnodes, belems, stn, rnn, rnodes, rloc, loc((size_t)N + 1, 0);
+    std::vector<char> seen(M + 1, 0);
+    auto add_block = [&](int lo, int hi) {
+      if (hi - lo > FV_CVB || !tile_fits(lo, hi)) return false;
+      std::sort(ids.begin() + lo, ids.begin() + hi);
+      ++stamp;
+      int rn[FV_CVH], nr = 0;
+      auto position = [&](int nd) {
+        if (mark[nd] != stamp) {
+          if (nr == FV_CVH) return -1;
+          mark[nd] = stamp;
+          nloc[nd] = nr;
+          rn[nr++] = nd;
+        }
+        return nloc[nd];
+      };
+      for (int q = lo; q < hi; ++q) {
+        int packed = 0;
+        for (int j = 0; j < 3; ++j) {
+          const int x = position(md->nv[(size_t)j * (N + 1) + ids[q]]);
+          if (x < 0 || x >= FV_CVB) return false;
+          packed |= x << (8 * j);
+        }
+        loc[ids[q]] = packed;
+      }
+      const int nn = nr;
+      const size_t r0 = rloc.size();
+      rloc.resize(r0 + (size_t)rw * FV_CVB, 0);
+      for (int t = 0; t < nn; ++t) {
+        const int* ring = md->nbsn + md->nbsn_off[rn[t]];
+        for (int j = 0; j < md->ntsn[rn[t]]; ++j) {
+          const int x = position(ring[j]);
+          if (x < 0) { rloc.resize(r0); return false; }
+          rloc[r0 + (j / 4) * FV_CVB + t] |= x << (8 * (j % 4));
+        }
+      }
+      bnn.push_back(nn);
+      bne.push_back(hi - lo);
+      rnn.push_back(nr);
+      bnodes.insert(bnodes.end(), rn, rn + nn);
+      bnodes.resize(bnn.size() * FV_CVB, 1);
+      belems.insert(belems.end(), ids.begin() + lo, ids.begin() + hi);
+      belems.resize(bnn.size() * FV_CVB, 1);
+      rnodes.insert(rnodes.end(), rn, rn + nr);
+      rnodes.resize(bnn.size() * FV_CVH, rn[0]);
+      for (int t = 0; t < nn; ++t) {
+        stn.push_back((rn[t] << 1) | (seen[rn[t]] ? 0 : 1));
+        seen[rn[t]] = 1;
+      }
+      stn.resize(bnn.size() * FV_CVB, 2);
+      return true;
+    };
+    std::vector<std::pair<int, int>> stack = component_ranges(ids, ecomp);
     while (!stack.empty()) {
       const std::pair<int, int> r = stack.back();
       stack.pop_back();
       const int lo = r.first, hi = r.second, n = hi - lo;
-      if (n <= FV_CVB && distinct_nodes(lo, hi) <= FV_CVB && tile_fits(lo, hi)) { leaves.push_back(r); continue; }
+      if (add_block(lo, hi)) continue;
       double x0 = md->xc[ids[lo]], x1 = x0, y0 = md->yc[ids[lo]], y1 = y0;
       for (int q = lo + 1; q < hi; ++q) {
         const double x = md->xc[ids[q]], y = md->yc[ids[q]];
@@ -770,35 +803,7 @@ int build_lists(fvgpu_handle* h) {
       stack.push_back({mid, hi});
       stack.push_back({lo, mid});
     }
-    const int nblk = (int)leaves.size();
-    std::vector<int> bnn(nblk, 0), bne(nblk, 0), bnodes((size_t)nblk * FV_CVB, 1), belems((size_t)nblk * FV_CVB, 1);
-    std::vector<int> loc((size_t)N + 1, 0), nloc(M + 1, 0), stn((size_t)nblk * FV_CVB, 2);
-    std::vector<char> seen(M + 1, 0);
-    for (int b = 0; b < nblk; ++b) {
-      const int lo = leaves[b].first, hi = leaves[b].second;
-      std::sort(ids.begin() + lo, ids.begin() + hi);
-      ++stamp;
-      int nn = 0;
-      for (int q = lo; q < hi; ++q) {
-        const int e = ids[q];
-        belems[(size_t)b * FV_CVB + (q - lo)] = e;
-        int packed = 0;
-        for (int j = 0; j < 3; ++j) {
-          const int nd = md->nv[(size_t)j * (N + 1) + e];
-          if (mark[nd] != stamp) {
-            mark[nd] = stamp;
-            nloc[nd] = nn;
-            stn[(size_t)b * FV_CVB + nn] = (nd << 1) | (seen[nd] ? 0 : 1);
-            seen[nd] = 1;
-            bnodes[(size_t)b * FV_CVB + nn++] = nd;
-          }
-          packed |= nloc[nd] << (8 * j);
-        }
-        loc[e] = packed;
-      }
-      bnn[b] = nn;
-      bne[b] = hi - lo;
-    }
+    const int nblk = (int)bnn.size();
     g.cvb_nblk = nblk;
     tile_own.assign(nblk, {});
     for (int b = 0; b < nblk; ++b)
@@ -898,6 +903,9 @@ int build_lists(fvgpu_handle* h) {
     if (dupload(h, &g.cvb_elems, belems.data(), belems.size())) return 1;
     if (dupload(h, &g.cvb_loc, loc.data(), loc.size())) return 1;
     if (dupload(h, &g.rec_keep, keep.data(), keep.size())) return 1;
+    if (dupload(h, &g.cvr_nn, rnn.data(), rnn.size())) return 1;
+    if (dupload(h, &g.cvr_nodes, rnodes.data(), rnodes.size())) return 1;
+    if (dupload(h, &g.cvr_loc, rloc.data(), rloc.size())) return 1;
     tile_nn.swap(bnn);
   }
   // element blocks of the blocked momentum kernels.  The 2-D stage and
@@ -1266,14 +1274,6 @@ int fvgpu_create(const fv_model* md, int32_t precision, fvgpu_handle** out) {
   HIPCHK(hipGetDevice(&h->device));
   HIPCHK(hipDeviceGetAttribute(&h->cu_count, hipDeviceAttributeMultiprocessorCount, h->device));
   if (!scratch_of(h->device)) { delete h; return 1; }
-  // FP64: CV records + face fluxes in one launch; the FP32 flux form keeps
-  // the two launches (measured faster for it: its records are half the
-  // size, and the two kernels' higher occupancy outweighs their traffic)
-  // the faster form per precision: in FP32 the fused tracer pass (980
-  // against 505 + 620 us) but the two-phase Q2 pass (386 + 491 against
-  // 1013 us), in FP64 both fused
-  h->two_phase_ts = 0;
-  h->two_phase_q = precision == FV_MIXED ? 1 : 0;
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) { delete h; return fail("stream"); }
   h->cur = h->stream;
   h->stage.reserve();
@@ -1876,9 +1876,7 @@ int fvgpu_set_concurrency(fvgpu_handle* h, int32_t mode) {
 }
 
 int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_len) {
-  static const char* fams[] = {"cvrec_ts", "cvrec_q", "cvflux_ts",
-                               "cvflux_q", "adv_ts", "adv_q",
-                               "viscofh", "vdif_q", "vdif_ts", "adjust1_brough", "adjust2", "baropg",
+  static const char* fams[] = {"adv_ts", "adv_q", "viscofh", "vdif_q", "vdif_ts", "adjust1_brough", "adjust2", "baropg",
                                "copy", "closure_features", "closure_apply"};
   static const int cands[] = {64, 128, 256};
   if (steps < 1) return fail("autotune needs at least one step per candidate");

@@ -14,6 +14,7 @@
 #define FV_MAX_CV 32   // control-volume sub-edges per node (twice the node degree)
 #define FV_MAX_RING 16 // NTSN / NTVE bound of the node rings held in registers
 #define FV_CVB 128     // elements and nodes per block of the fused CV kernels
+#define FV_CVH 256     // a block's nodes with the nodes of their rings
 #define FV_NTN 64      // owned nodes per node tile
 #define FV_NTE 192     // elements per node tile
 
@@ -118,6 +119,12 @@ struct DevGrid {
   // at every layer (the OBC nodes and the other ends of their sub-edges).
   int cvb_nblk;
   const int *cvb_nn, *cvb_nodes, *cvb_ne, *cvb_elems, *cvb_loc, *rec_keep;
+  // The block's nodes and the nodes of their rings: cvr_nn[b] (<= FV_CVH)
+  // distinct, cvr_nodes[FV_CVH*b + q], the block's own first and in the order
+  // of cvb_nodes.  Byte j%4 of cvr_loc[(cvr_w*b + j/4)*FV_CVB + t] is the
+  // position q of ring slot j of local node t.
+  int cvr_w;
+  const int *cvr_nn, *cvr_nodes, *cvr_loc;
   StageTab st;
   // Node tiles (VERTVL): tile b owns the nt_nown[b] (<= FV_NTN) nodes
   // nt_nodes[FV_NTN*b + t]; nt_elems[FV_NTE*b + t] are the nt_nel[b]

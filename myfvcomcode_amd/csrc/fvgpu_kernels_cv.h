@@ -4,37 +4,27 @@
 // The reference's scalar advection (ADV_T/ADV_S, ADV_Q) loops over the
 // control-volume sub-edges and scatters each face flux to its two nodes.
 // Here:
-//   1. k_cvrec     one thread per node: ring gradient, ring bounds and the
-//                  viscosity factor of every layer, packed per node-layer
-//                  (CvRec), the node's ring kept in registers across layers;
-//   2. k_cvflux_*  one thread per element: the face fluxes of its three
-//                  sub-edges at every layer, each evaluated once from the
-//                  element's three node records (gathered once per layer
-//                  for the three faces) and its velocity, written to the
-//                  element-major positions 3*(e-1)+j+1 (coalesced);
-//   3. k_*_gather  one thread per node: the node's sub-edge fluxes summed in
+//   1. k_cvrecflux one workgroup per tile of the mesh: the records of its
+//                  nodes (ring gradient, ring bounds and viscosity factor,
+//                  CvRec) formed in LDS layer by layer, and from them the
+//                  face fluxes of the three sub-edges of its elements, each
+//                  evaluated once and written to the element-major positions
+//                  3*(e-1)+j+1 (coalesced);
+//   2. k_*_gather  one thread per node: the node's sub-edge fluxes summed in
 //                  increasing sub-edge order (the reference's scatter order,
 //                  so the sum is bit-identical), then the vertical flux, the
 //                  update and FCT, whose ring bounds come from the field
 //                  itself (the ring's values are in cache beside the node's
-//                  own column) rather than through HBM from phase 1.
+//                  own column) rather than through HBM from the records.
 // Node lists are read slot-major (cvl_ent) so consecutive nodes read
 // consecutive addresses, and workgroups are placed XCD-contiguously.
 #pragma once
 #include "fvgpu_kernels_column.h"
 
-
-// Ring gradient / bounds of field f at node i for the layers [k0, k1]
-// (adv_t.F:219-376 and :469-480; adv_q.F the same on layer interfaces).
-// RMAX >= NTSN bounds the ring held in registers.  The sums are FP64; the
-// record is stored in the flux type FT.
-// kind 0: tracer, VHN = VISCOFH*NN_HVC; kind 1: turbulence, VHN = the
-// DZ-weighted interface viscosity (adv_q.F) times NN_HVC.
-// Ring of node i (RMAX >= NTSN): node indices and the DLTXTRIE/DLTYTRIE
-// factors of its ring segments, in registers across the layers.
+// Ring of node i (RMAX >= NTSN): the DLTXTRIE/DLTYTRIE factors of its ring
+// segments, in registers across the layers.
 template <int RMAX>
 struct RingGeo {
-  int rn[RMAX];
   double rdx[RMAX], rdy[RMAX];
   int nt;
 };
@@ -45,67 +35,40 @@ __device__ __forceinline__ void ring_geo_load(const DevGrid& g, int i, RingGeo<R
   r.nt = nt;
   static_for<RMAX>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    r.rn[j] = j < nt ? g.nbsn[o + j] : 0;
     r.rdx[j] = j < nt - 1 ? g.dltxtrie[o + j] : 0.0;
     r.rdy[j] = j < nt - 1 ? g.dltytrie[o + j] : 0.0;
   });
 }
 
+// The values a record reads: the field C at the node and FV at its ring, for
+// the tracer the mean MV at the ring, and VISCOFH at the layer (VH) and, for
+// ADV_Q, a layer up (VHM).
+template <int RMAX>
+struct CvIn {
+  double fv[RMAX], mv[RMAX];
+  double c, vh, vhm;
+};
+
 // The record of node i at layer k: ring gradient of f and of f - mean
 // (adv_t.F:219-376; adv_q.F:185-230 with the constant mean QMEAN1), the
 // ring bounds with the node (adv_t.F:469-480) and the viscosity factor.
-// kind 0: tracer, VHN = VISCOFH*NN_HVC; kind 1: turbulence, VHN = the
+// KIND 0: tracer, VHN = VISCOFH*NN_HVC; KIND 1: turbulence, VHN = the
 // DZ-weighted interface viscosity (adv_q.F) times NN_HVC.  The sums are
-// FP64; the record is stored in the flux type FT.
-//
-// The values the record reads -- the field at the node and its ring, and
-// for the tracer the mean at the ring and VISCOFH at the layer -- are
-// loaded by cv_load, so that a caller can issue them a layer ahead.
-// (ADV_Q's record keeps its mean and its VISCOFH loads, of two levels, in
-// the record: loaded ahead they measured slower.)
-template <int RMAX>
-struct CvLoads {
-  double fv[RMAX], mv[RMAX];
-  double c, vh;
-};
-
-template <int KIND, int RMAX>
-__device__ __forceinline__ void cv_load(const DevGrid& g, const IntArgs& a, int i, const RingGeo<RMAX>& rg,
-                                        const double* f, const double* mean, double cmean, int k, CvLoads<RMAX>& L) {
-  const long ko = (long)(k - 1) * g.m1;
-  // the ring's values are loaded unconditionally (slots past the ring
-  // read node 0) so that the loads issue together
-  static_for<RMAX>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    L.fv[j] = at(f + ko, rg.rn[j]);
-    if (KIND == 0) L.mv[j] = mean ? at(mean + ko, rg.rn[j]) : cmean;
-  });
-  L.c = at(f + ko, i);
-  if (KIND == 0) L.vh = at(a.viscofh + ko, i);
-}
-
+// FP64 and take the ring's terms in ring order; the record is stored in the
+// flux type FT.
 template <int KIND, int RMAX, typename FT, bool UNI>
-__device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntArgs& a, int i, const RingGeo<RMAX>& rg,
-                                                   double art2, double nn, const CvLoads<RMAX>& L,
-                                                   const double* mean, double cmean, int k) {
-  const long ko = (long)(k - 1) * g.m1;
+__device__ __forceinline__ CvRecT<FT> cv_record(const DevGrid& g, int i, const RingGeo<RMAX>& rg, double art2,
+                                                double nn, const CvIn<RMAX>& L, double cmean, int k) {
   const int nt = rg.nt;
-  const double* fv = L.fv;
-  // the sums take the ring's own terms in ring order
-  double mv[RMAX];
-  static_for<RMAX>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    mv[j] = KIND == 0 ? L.mv[j] : (mean ? at(mean + ko, rg.rn[j]) : cmean);
-  });
   double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
-  double f1 = fv[0];
-  double m1v = mv[0];
+  double f1 = L.fv[0];
+  double m1v = KIND == 0 ? L.mv[0] : cmean;
   double lo = f1, hi = f1;
   static_for<RMAX - 1>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
     if (j < nt - 1) {
-      const double f2 = fv[j + 1];
-      const double m2v = mv[j + 1];
+      const double f2 = L.fv[j + 1];
+      const double m2v = KIND == 0 ? L.mv[j + 1] : cmean;
       const double ffd = 0.5 * (f1 + f2 - m1v - m2v);
       const double ff1 = 0.5 * (f1 + f2);
       s1 = s1 + ff1 * rg.rdy[j];
@@ -122,8 +85,7 @@ __device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntAr
   if (KIND == 0) {
     vhn = L.vh * nn;
   } else {
-    const double vfa = (at(a.viscofh + ko, i) * DZ(i, k - 1) + at(a.viscofh + (ko - g.m1), i) * DZ(i, k)) /
-                       (DZ(i, k) + DZ(i, k - 1));
+    const double vfa = (L.vh * DZ(i, k - 1) + L.vhm * DZ(i, k)) / (DZ(i, k) + DZ(i, k - 1));
     vhn = vfa * nn;
   }
   CvRecT<FT> r;
@@ -138,32 +100,8 @@ __device__ __forceinline__ CvRecT<FT> cv_record_of(const DevGrid& g, const IntAr
   return r;
 }
 
-template <int KIND, int RMAX, typename FT, bool UNI>
-__device__ __forceinline__ CvRecT<FT> cv_record(const DevGrid& g, const IntArgs& a, int i, const RingGeo<RMAX>& rg,
-                                                double art2, double nn, const double* f, const double* mean,
-                                                double cmean, int k) {
-  CvLoads<RMAX> L;
-  cv_load<KIND, RMAX>(g, a, i, rg, f, mean, cmean, k, L);
-  return cv_record_of<KIND, RMAX, FT, UNI>(g, a, i, rg, art2, nn, L, mean, cmean, k);
-}
-
-// Ring gradient / bounds of field f at node i for the layers [k0, k1], one
-// thread per node with its ring in registers.
-template <int KIND, int RMAX, typename FT, bool UNI>
-__global__ __launch_bounds__(256) void k_cvrec(DevGrid g, IntArgs a, const double* f, const double* mean,
-                                               double cmean, int k0, int k1) {
-  const int i = (int)xcd_thread();
-  if (i < 1 || i > g.M) return;
-  CvRecT<FT>* rec = (CvRecT<FT>*)a.rec;
-  RingGeo<RMAX> rg;
-  ring_geo_load<RMAX>(g, i, rg);
-  const double art2 = g.art2[i], nn = g.nn_hvc[i];
-  for (int k = k0; k <= k1; ++k)
-    rec[(long)(k - 1) * g.m1 + i] = cv_record<KIND, RMAX, FT, UNI>(g, a, i, rg, art2, nn, f, mean, cmean, k);
-}
-
 // Min and max of field f over the NBSN ring of node i at layer offset ko,
-// the ring alone (entry NTSN repeats entry 1), in the order k_cvrec forms
+// the ring alone (entry NTSN repeats entry 1), in the order the records form
 // them: the FCT bounds (fct_t.F:74-80, fct_q2.F:60-66).
 template <int RMAX>
 __device__ __forceinline__ void ring_bounds(const int (&rn)[RMAX], const double* f, long ko, double& lo,
@@ -260,7 +198,10 @@ __device__ __forceinline__ FT face_value(const CvRecT<FT>& r, FT x, FT y) {
 }
 
 // The three face fluxes of one element at one layer (adv_t.F:440-500,
-// adv_q.F:200-330) from the records r[3] of its nodes NV(e,1..3), the
+// adv_q.F:200-330).  The two nodes of a face enter the diffusive terms
+// through sums, which are the same in either order, and the upwind value
+// through FIJ1 (side IA) and FIJ2 (side IB), exchanged when IA is node B.
+// From the records r[3] of its nodes NV(e,1..3), the
 // normal velocity (un = V*DLTXE - U*DLTYE) from the element velocity (uk,
 // vk) and the layer thickness dtij; viscosity divided by HPRNU when DIVP.
 template <typename FT, bool DIVP>
@@ -282,33 +223,6 @@ __device__ __forceinline__ void cv_faces(const ElemFaces<FT>& f, const CvRecT<FT
     const FT fyy = dtij * tyy * f.dltx[j];
     const FT sgn = fsign1(un);
     out[j] = -un * dtij * ((one + sgn) * fij2 + (one - sgn) * fij1) * half + fxx + fyy;
-  }
-}
-
-// Phase 2 of ADV_T/ADV_S: the three face fluxes of one element per layer
-// (adv_t.F:440-500), with the geometry held in registers across layers.
-// The two nodes of a face enter the diffusive terms through sums, which are
-// the same in either order, and the upwind value through FIJ1 (side IA) and
-// FIJ2 (side IB), exchanged when IA is node B.
-template <typename FT, bool UNI>
-__global__ __launch_bounds__(256) void k_cvflux_ts(DevGrid g, IntArgs a) {
-  const int e = (int)xcd_thread();
-  if (e < 1 || e > g.N) return;
-  const CvRecT<FT>* rec = (const CvRecT<FT>*)a.rec;
-  FT* cvflux = (FT*)a.cvflux;
-  const ElemFaces<FT> f = elem_faces<FT>(g, e);
-  const int nd[3] = {NV_(e, 1), NV_(e, 2), NV_(e, 3)};
-  const FT fact = (FT)g.fact, half = (FT)0.5, one = (FT)1.0;
-  const double dt1 = a.dt1[e];
-  const long cs = (long)g.NCV + 1, p0 = 3L * (e - 1) + 1;
-  for (int k = 1; k <= g.KBM1; ++k) {
-    const long ko = (long)(k - 1) * g.m1, eo = (long)(k - 1) * g.n1;
-    const FT dtij = (FT)(dt1 * DZ1(e, k));
-    const FT vk = (FT)a.v[eo + e], uk = (FT)a.u[eo + e];
-    CvRecT<FT> r[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) r[q] = rec[ko + nd[q]];
-    cv_faces<FT, false>(f, r, uk, vk, dtij, fact, one, cvflux + (long)(k - 1) * cs + p0);
   }
 }
 
@@ -441,42 +355,6 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
   }
 }
 
-// Phase 2 of ADV_Q (adv_q.F:200-330): the three face fluxes of one element
-// on layer interfaces k = 2..KBM1, the element velocity interpolated to the
-// interface with DZ1 weights (once for the three faces); faces as in
-// k_cvflux_ts.
-template <typename FT, bool UNI>
-__global__ __launch_bounds__(256) void k_cvflux_q(DevGrid g, IntArgs a) {
-  const int e = (int)xcd_thread();
-  if (e < 1 || e > g.N) return;
-  const CvRecT<FT>* rec = (const CvRecT<FT>*)a.rec;
-  FT* cvflux = (FT*)a.cvflux;
-  const ElemFaces<FT> f = elem_faces<FT>(g, e);
-  const int nd[3] = {NV_(e, 1), NV_(e, 2), NV_(e, 3)};
-  const FT fact = (FT)g.fact, rhprnu = (FT)g.hprnu, half = (FT)0.5, one = (FT)1.0;
-  const double dt1 = a.dt1[e];
-  const long cs = (long)g.NCV + 1, p0 = 3L * (e - 1) + 1;
-  double um = a.u[e], vm = a.v[e];   // layer 1
-  for (int k = 2; k <= g.KBM1; ++k) {
-    const long ko = (long)(k - 1) * g.m1, eo = (long)(k - 1) * g.n1;
-    const double uk = a.u[eo + e], vk = a.v[eo + e];
-    const double dz1k = DZ1(e, k), dz1m = DZ1(e, k - 1), dzz1 = DZZ1(e, k - 1);
-    CvRecT<FT> r[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) r[q] = rec[ko + nd[q]];
-    // Every load of the layer is issued before the two divisions: without
-    // the barrier the scheduler trades them for registers and waits on each
-    // record part in turn.
-    __builtin_amdgcn_sched_barrier(0);
-    const FT uq = (FT)((uk * dz1m + um * dz1k) / (dz1k + dz1m));
-    const FT vq = (FT)((vk * dz1m + vm * dz1k) / (dz1k + dz1m));
-    um = uk;
-    vm = vk;
-    const FT dtij = (FT)(dt1 * dzz1);
-    cv_faces<FT, true>(f, r, uq, vq, dtij, fact, rhprnu, cvflux + (long)(k - 1) * cs + p0);
-  }
-}
-
 // The block's records of one layer in LDS, one array per quantity.
 template <typename FT>
 struct CvRecLds {
@@ -494,30 +372,45 @@ struct CvRecLds {
 };
 
 // ADV_T/ADV_S (KIND 0, layers 1..KBM1) or ADV_Q (KIND 1, interfaces
-// 2..KBM1) phases 1 and 2 in one launch.  A workgroup of 256 lanes takes a
-// block of at most FV_CVB = 128 elements and the at most 128 distinct nodes
-// they use (cvb_*: compact tiles of the mesh).  Its first two waves form
-// the nodes' records (one lane per node, ring in registers: cv_record, the
-// same arithmetic as k_cvrec) of layer k into one of two LDS buffers while
-// its last two waves evaluate the elements' three face fluxes (one lane per
-// element: cv_faces, as k_cvflux_*) of layer k-1 from the other buffer; one
-// barrier per layer hands the buffers over.  The two roles hold only their
-// own registers and run side by side.  A node shared by two blocks is
+// 2..KBM1): records and face fluxes in one launch.  A workgroup of 256 lanes
+// takes a block of at most FV_CVB = 128 elements and the at most 128
+// distinct nodes they use (cvb_*: compact tiles of the mesh).  Its first two
+// waves form the nodes' records (one lane per node: cv_record) of layer k
+// while its last two waves evaluate the elements' three face fluxes (one
+// lane per element: cv_faces) of layer k-1 and bring the field of layer k+1
+// at the block's nodes and their rings (cvr_*) into LDS; one barrier per
+// layer hands the two buffers of either kind over.  The two roles hold only
+// their own registers and run side by side.  A node shared by two blocks is
 // formed by both; the records cross HBM only for the nodes whose records
 // other kernels read (rec_keep: OBC nodes and their sub-edge neighbours)
 // and, for the tracer, at the bottom layer (the bottom gradients of
 // VDIF_TS).
+//
+// Bound: the vector memory unit and its latency.  A record read straight
+// from memory takes up to 20 scattered loads a lane, of which two layers
+// could not be kept in flight (160 registers for 2 layers of a ring); a tile
+// and its rings are about 115 nodes, so that a layer is 2 coalesced loads a
+// lane of the face waves, a layer ahead, and a record's values are LDS reads.
+// 1,000,000 elements x 40 layers: FP64 tracer 1164 -> 911 us (1.9 GB, 2.1
+// TB/s), q2 1087 -> 890; FP32 fluxes, tracer 985 -> 706, q2 689 (with records
+// and fluxes in two launches through HBM: 357 + 466).  Exchanging the roles of
+// the waves in every second workgroup (the record waves take twice the
+// instructions of the face waves) changed nothing.
 template <int KIND, int RMAX, typename FT, bool UNI>
 __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const double* fld, const double* mean,
                                                    double cmean) {
   __shared__ CvRecLds<FT> srec[2];
+  // one layer of the field (and for the tracer its mean) at the block's
+  // nodes and their rings
+  constexpr int NF = KIND == 0 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) double sfld[2][FV_CVH * NF];
   const int b = xcd_block(), t = threadIdx.x;
   int k0, k1;
   layer_share(KIND == 0 ? 1 : 2, g.KBM1, k0, k1);
   const int nk = k1 - k0 + 1;       // layers (interfaces) of this workgroup
   if (nk < 1) return;
   // The role is taken from the wave's first lane, so that the branch is
-  // uniform over each wave and both roles pass nk + 1 barriers.
+  // uniform over each wave and both roles pass nk + 2 barriers.
   if (__builtin_amdgcn_readfirstlane(t) < FV_CVB) {
     // records: local node t of the block
     CvRecT<FT>* rec = (CvRecT<FT>*)a.rec;
@@ -525,23 +418,44 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
     const int i = nact ? g.cvb_nodes[(long)FV_CVB * b + t] : 1;
     RingGeo<RMAX> rg;
     ring_geo_load<RMAX>(g, i, rg);
+    constexpr int NW = (RMAX + 3) / 4;   // ring slots four to a word
+    int rw[NW];
+    static_for<NW>([&](auto wc) {
+      constexpr int w = decltype(wc)::value;
+      rw[w] = w < g.cvr_w ? g.cvr_loc[((long)b * g.cvr_w + w) * FV_CVB + t] : 0;
+    });
     const double art2 = g.art2[i], nnv = g.nn_hvc[i];
     const bool keep = nact && g.rec_keep[i] != 0;
-    // the field's values are loaded a layer ahead (rings of up to 10
-    // nodes; the 16-node form has no registers to spare)
-    constexpr bool ahead = RMAX <= 10;
-    CvLoads<RMAX> L;
-    if (ahead) cv_load<KIND, RMAX>(g, a, i, rg, fld, mean, cmean, k0, L);
+    // VISCOFH a layer ahead
+    double vhn = at(a.viscofh + (long)(k0 - 1) * g.m1, i), vhm = 0.0;
+    if (KIND == 1) vhm = at(a.viscofh + (long)(k0 - 2) * g.m1, i);
+    __syncthreads();
     for (int s = 0; s <= nk; ++s) {
       const int k = k0 + s;
       if (s < nk) {
+        CvIn<RMAX> L;
+        L.vh = vhn;
+        L.vhm = vhm;
+        vhm = vhn;
+        vhn = at(a.viscofh + (long)((k < k1 ? k + 1 : k) - 1) * g.m1, i);
+        const double* sf = sfld[s & 1];
+        static_for<RMAX>([&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          const int q = (rw[j / 4] >> (8 * (j % 4))) & 255;
+          if (KIND == 0) {
+            const double2 v = ((const double2*)sf)[q];
+            L.fv[j] = v.x;
+            L.mv[j] = v.y;
+          } else {
+            L.fv[j] = sf[q];
+          }
+        });
+        L.c = sf[NF * t];
         if (nact) {
-          if (!ahead) cv_load<KIND, RMAX>(g, a, i, rg, fld, mean, cmean, k, L);
-          const CvRecT<FT> r = cv_record_of<KIND, RMAX, FT, UNI>(g, a, i, rg, art2, nnv, L, mean, cmean, k);
+          const CvRecT<FT> r = cv_record<KIND, RMAX, FT, UNI>(g, i, rg, art2, nnv, L, cmean, k);
           srec[s & 1].put(t, r);
           if (keep || (KIND == 0 && k == g.KBM1)) rec[(long)(k - 1) * g.m1 + i] = r;
         }
-        if (ahead && s + 1 < nk) cv_load<KIND, RMAX>(g, a, i, rg, fld, mean, cmean, k + 1, L);
       }
       __syncthreads();
     }
@@ -556,15 +470,45 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
     const int l0 = pk & 255, l1 = (pk >> 8) & 255, l2 = (pk >> 16) & 255;
     const FT fact = (FT)g.fact, rhprnu = (FT)g.hprnu, one = (FT)1.0;
     const double dt1 = a.dt1[e];
+    // the velocity a layer ahead
+    double un = a.u[(long)(k0 - 1) * g.n1 + e], vn = a.v[(long)(k0 - 1) * g.n1 + e];
     const long cs = (long)g.NCV + 1, p0 = 3L * (e - 1) + 1;
     // the layer above (ADV_Q's interface interpolation)
     const long em = (long)(KIND == 1 ? k0 - 2 : 0) * g.n1 + e;
     double um = a.u[em], vm = a.v[em];
+    // the field's layers, a layer ahead
+    const int ha = g.cvr_nodes[(long)FV_CVH * b + te], hb = g.cvr_nodes[(long)FV_CVH * b + FV_CVB + te];
+    const bool two = g.cvr_nn[b] > FV_CVB;
+    double fa, fb = 0.0, ma = 0.0, mb = 0.0;
+    auto load = [&](int k) {
+      const long ko = (long)(k - 1) * g.m1;
+      fa = at(fld + ko, ha);
+      if (KIND == 0) ma = at(mean + ko, ha);
+      if (two) {
+        fb = at(fld + ko, hb);
+        if (KIND == 0) mb = at(mean + ko, hb);
+      }
+    };
+    auto stage = [&](double* sf) {
+      if (KIND == 0) {
+        ((double2*)sf)[te] = make_double2(fa, ma);
+        if (two) ((double2*)sf)[FV_CVB + te] = make_double2(fb, mb);
+      } else {
+        sf[te] = fa;
+        if (two) sf[FV_CVB + te] = fb;
+      }
+    };
+    load(k0);
+    stage(sfld[0]);
+    load(k0 < k1 ? k0 + 1 : k0);
+    __syncthreads();
     for (int s = 0; s <= nk; ++s) {
       if (s > 0) {
         const int k = k0 + s - 1;
-        const long eo = (long)(k - 1) * g.n1;
-        const double uk = at(a.u + eo, e), vk = at(a.v + eo, e);
+        const double uk = un, vk = vn;
+        const long eo = (long)((k < k1 ? k + 1 : k) - 1) * g.n1;
+        un = at(a.u + eo, e);
+        vn = at(a.v + eo, e);
         const double dz1k = DZ1(e, k);
         if (eact) {
           const CvRecLds<FT>& sr = srec[(s - 1) & 1];
@@ -582,6 +526,10 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
             cv_faces<FT, true>(f, r, uq, vq, (FT)(dt1 * dzz1), fact, rhprnu, out);
           }
         }
+      }
+      if (s + 1 < nk) {
+        stage(sfld[(s + 1) & 1]);
+        load(k0 + s + 2 < k1 ? k0 + s + 2 : k1);
       }
       __syncthreads();
     }

@@ -41,43 +41,6 @@ def ext_momentum(s, real=R8):
 
 
 # ----------------------------------------------------------------- 3-D mode
-def _cvrec(s, layers, nfields, real):
-    M, RSN = s["M"], s["RSN"]
-    reads = RSN * (I4 + 2 * real) + M * (2 * I4 + 2 * real) + nfields * M * layers * real
-    writes = M * layers * 8 * real
-    return reads + writes
-
-
-def cvrec_ts(s, real=R8):
-    """Ring gradients/bounds + viscosity per node-layer (T or S, KBM1 layers)."""
-    return _cvrec(s, s["KBM1"], 3, real)       # f, mean, VISCOFH
-
-
-def cvrec_q(s, real=R8):
-    """The same for Q2 / Q2L on interfaces 2..KBM1."""
-    return _cvrec(s, s["KBM1"] - 1, 2, real)   # q, VISCOFH
-
-
-def _cvflux(s, rec_layers, uv_layers, real):
-    M, N, NCV = s["M"], s["N"], s["NCV"]
-    reads = (NCV * (3 * I4 + 6 * real)          # NIEC(2), NTRG; DLTXE, DLTYE, DLTXNCVE(2), DLTYNCVE(2)
-             + M * real + N * real              # NN_HVC, DT1
-             + M * rec_layers * 8 * real        # node-layer records
-             + N * uv_layers * 2 * real)        # U, V
-    writes = NCV * rec_layers * real            # face flux
-    return reads + writes
-
-
-def cvflux_ts(s, real=R8):
-    """ADV_T/ADV_S face flux per sub-edge and layer."""
-    return _cvflux(s, s["KBM1"], s["KBM1"], real)
-
-
-def cvflux_q(s, real=R8):
-    """ADV_Q face flux per sub-edge and interface."""
-    return _cvflux(s, s["KBM1"] - 1, s["KBM1"], real)
-
-
 def _cvrecflux(s, layers, nfields, uv_layers, bottom_records, real):
     """Records formed in LDS and face fluxes in one launch: the node fields
     and ring geometry, the element geometry and velocities are read, the
@@ -203,7 +166,7 @@ def n2e3d(s, real=R8):
 
 
 FAMILIES = {f.__name__: f for f in (
-    ext_momentum, cvrec_ts, cvrec_q, cvflux_ts, cvflux_q, cvrecflux_ts, cvrecflux_q,
+    ext_momentum, cvrecflux_ts, cvrecflux_q,
     adv_ts, adv_q,
     adv3d_blk, advuv_blk, vertvl, viscofh, vdif_q, vdif_uv, vdif_ts,
     n2e3d)}
