@@ -7,11 +7,9 @@ constant, MY2.5 closure, DTE = 2 s, ISPLIT = 10 (DTI = 20 s), synthetic
 seeded data.
 
 A step is one INTERNAL_STEP (ISPLIT external steps included).  An untimed
-survey pass (eager launches, every chain on one stream) with HIP events
-around every launch gives each kernel family's own average device time
+survey pass (eager launches) with HIP events around every launch gives each kernel family's own average device time
 ("roofline_by_kernel") and the dominant family; the timed region then runs
-K steps launched eagerly with the independent chains side by side on the
-handle's two streams, the state resident in HBM, and HIP events around
+K steps launched eagerly, the state resident in HBM, and HIP events around
 one in four of the dominant family's launches (events around every launch
 cost about 0.46 ms of a 23.3 ms step), whose average device time is the
 "roofline" figure.  The same step replayed as one hipGraph per step is
@@ -87,16 +85,12 @@ def main():
     dev.synchronize()
     print("bench: warmup done", file=sys.stderr, flush=True)
 
-    # The survey pass (not timed) runs every chain on the handle's main
-    # stream (concurrency 0), eagerly, with HIP events around every launch,
-    # so that no family's event time includes another kernel running beside
-    # it: each family's average device time and the dominant family.  The
-    # timed region then launches eagerly with the chains side by side, with
-    # events around the dominant family's launches only -- events around all
-    # ~300 launches of a step would add about 5 % to it.  The dominant family
-    # (the 2-D momentum stage) runs on the main stream with nothing beside
-    # it, so its event time is its own.
-    dev.set_concurrency(0)
+    # The survey pass (not timed) runs eagerly with HIP events around every
+    # launch: each family's average device time and the dominant family.  The
+    # timed region then launches eagerly with events around the dominant
+    # family's launches only -- events around all the launches of a step would
+    # add to it.  The step is one chain of launches, so that no family's event
+    # time includes another kernel running beside it.
     survey_steps = max(1, min(10, args.steps))
     dev.synchronize()
     dev.set_profiling(True)
@@ -123,12 +117,10 @@ def main():
     # dominant kernel = the modelled family with the largest device time per step
     dom = max(per_kernel, key=lambda k: per_kernel[k]["avg_us"] * per_kernel[k]["launches_per_step"])
 
-    # timed region: K internal steps, launched eagerly with the independent
-    # chains side by side on the handle's two streams, events around one in
+    # timed region: K internal steps, launched eagerly, events around one in
     # PROFILE_EVERY launches of the dominant family (HIP events cannot time
     # launches inside a replayed graph here; the graph replay of the same
     # step is timed as a variant)
-    dev.set_concurrency(3)
     dev.set_profiling(True, kernel=dom, every=PROFILE_EVERY)
     dev.synchronize()
     t0 = time.perf_counter()
@@ -222,7 +214,6 @@ def time_variants(F, model, steps, warmup, fp64_step_s, dti, units, only=None):
             continue
         dev = F.DeviceModel(model, precision=prec)
         graph = True
-        dev.set_concurrency(3)
         if closure:
             dev.set_closure(1, load_params())
         dev.run(warmup, graph=graph)

@@ -387,12 +387,11 @@ void fvgpu_destroy(fvgpu_handle* h);
 
 /* Workgroup size (64, 128 or 256) of one kernel family of the step.      */
 int  fvgpu_set_block(fvgpu_handle* h, const char* family, int32_t block);
-/* Concurrency of the step's independent chains on a second stream of the
- * handle, a bit mask: 1 the S pass beside the T pass and Q2L advection
- * beside Q2; 2 has no effect any more (a 2-D stage is one launch); default
- * 3; 0 runs every chain on the main stream, so that each kernel family's
- * timing is its own.  No counterpart in the reference; results do not
- * depend on it.                                                           */
+/* Concurrency of the step's independent chains: 0..3 are accepted and have
+ * no effect any more.  The T and S passes, and the advection of Q2 and Q2L,
+ * share their launches instead of running on streams of their own, so that
+ * each kernel family's timing is always its own.  No counterpart in the
+ * reference.                                                              */
 int  fvgpu_set_concurrency(fvgpu_handle* h, int32_t mode);
 /* Autotuner: times every kernel family of the step with workgroups of 64,
  * 128 and 256 (`steps` internal steps per candidate), keeps the fastest,

@@ -447,9 +447,8 @@ class DeviceModel:
         _check(L, L.fvgpu_set_forcing(self._h, name.encode(), v.ctypes.data, len(v)), "set_forcing " + name)
 
     def set_concurrency(self, mode):
-        """Independent chains of the step on a second stream, a bit mask:
-        1 the T/S and Q2/Q2L pairs (2 has no effect; default 3), 0 every
-        chain on the main stream (per-kernel timing)."""
+        """Accepts 0..3, without effect: the step's independent chains (T and
+        S, Q2 and Q2L) share their launches."""
         _check(gpu_lib(), gpu_lib().fvgpu_set_concurrency(self._h, int(mode)), "fvgpu_set_concurrency")
 
     def closure_fallbacks(self):

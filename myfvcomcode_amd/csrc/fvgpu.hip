@@ -90,14 +90,6 @@ struct fvgpu_handle {
   int cu_count = 0;       // compute units of the device
   HostStage stage;        // pinned staging of the copies to and from the caller's memory
   hipStream_t stream = nullptr;
-  // Independent chains of the step (the T and S passes, the Q2 and Q2L
-  // advection) fork onto stream2 and join back; both streams have the default priority.  `cur` is the stream the
-  // launch macros enqueue on.
-  hipStream_t stream2 = nullptr, cur = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  int concurrent = 3;     // bit 0: the 3-D chain pairs on stream2
-  // CV records then face fluxes in two launches (1) or one fused launch
-  // (0), for ADV_T/ADV_S and for ADV_Q
   // wind speeds at the start (wu0, wv0) and end (wu1, wv1) of the coming
   // internal step; once they differ, every external step forms its own
   // stress (ws2x, ws2y), otherwise it uses the end stress g.wsx/g.wsy
@@ -111,7 +103,7 @@ struct fvgpu_handle {
   DevClock* clk = nullptr;
   Ext2DState ext[3];      // ext[0] = state / RK base, ext[1], ext[2] stage buffers
   IntArgs ia{};
-  IntArgs ib{};           // ia with its own scratch, for the chain on stream2
+  IntArgs ib{};           // ia with its own scratch, for the second of two passes
   double* phi[2] = {};    // per sub-edge EXTEL terms of a 2-D stage's input and output, element-major
   double* elrk = nullptr; // the RK base elevation of stages 2-4
   double* own2d = nullptr;   // block-order constants of the external steps (ExtArgs::own2d)
@@ -196,12 +188,12 @@ struct Launch {
   Launch(fvgpu_handle* h_, const char* n) : h(h_), name(n) {
     on = h->profiling && (h->profile_only.empty() || h->profile_only == n);
     if (on && h->profile_every > 1) on = h->profile_seen++ % h->profile_every == 0;
-    if (on) { e0 = next_event(h); (void)hipEventRecord(e0, h->cur); }
+    if (on) { e0 = next_event(h); (void)hipEventRecord(e0, h->stream); }
   }
   ~Launch() {
     if (on) {
       e1 = next_event(h);
-      (void)hipEventRecord(e1, h->cur);
+      (void)hipEventRecord(e1, h->stream);
       h->pending.push_back({name, {e0, e1}});
     }
   }
@@ -232,16 +224,16 @@ void drop_graphs(fvgpu_handle* h) {
 #define LAUNCH(NAME, KERNEL, GRID, BLOCK, ...)                                   \
   do {                                                                            \
     Launch l_(h, NAME);                                                           \
-    hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(BLOCK), 0, h->cur, __VA_ARGS__);    \
+    hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(BLOCK), 0, h->stream, __VA_ARGS__);    \
   } while (0)
 
 inline unsigned nb(long n) { return (unsigned)((n + 255) / 256); }
 
-// N2E3D of a node field over layers 1..KB (k_n2e3d's grid: elements by
-// groups of eight layers, x extent a multiple of 8).
-#define N2E3D(NVAR, EVAR)                                                                        \
-  LAUNCH("n2e3d", k_n2e3d, dim3((nb(g.N) + 7) / 8 * 8, (unsigned)((g.KB + 7) / 8)), 256, g, NVAR, EVAR, \
-         g.KB)
+// N2E3D of n node fields over layers 1..KB (k_n2e3d's grid: elements by
+// groups of eight layers by fields, x extent a multiple of 8).
+#define N2E3D(FIELDS, NF)                                                                                   \
+  LAUNCH("n2e3d", k_n2e3d, dim3((nb(g.N) + 7) / 8 * 8, (unsigned)((g.KB + 7) / 8), (unsigned)(NF)), 256, g, \
+         FIELDS, g.KB)
 
 // Launch of a 1-D kernel family over n work items with the family's
 // workgroup size (256 unless the autotuner chose 64 or 128).
@@ -254,7 +246,7 @@ int block_of(const fvgpu_handle* h, const char* name) {
     const int bs_ = block_of(h, NAME);                                                            \
     Launch l_(h, NAME);                                                                           \
     hipLaunchKernelGGL(KERNEL, dim3((unsigned)(((long)(NITEMS) + bs_ - 1) / bs_)), dim3(bs_), 0, \
-                       h->cur, __VA_ARGS__);                                                      \
+                       h->stream, __VA_ARGS__);                                                      \
   } while (0)
 
 // How many shares the n layers of a kernel are split into (its grid's y
@@ -267,7 +259,8 @@ int block_of(const fvgpu_handle* h, const char* name) {
 // 2.14 ms unsplit, 1.94 at 3, 1.96 at 6, 2.02 at 12; 250,000 x 20: 3.28,
 // 3.27, 3.28, 3.35; from 768 workgroups a layer on, nothing is split and
 // nothing changes), but for ADV_UV, whose grid is the most uneven, 6 (62,500
-// elements: 161 us unsplit, 137 at 3, 130 at 6).  adv_ts at 17,000 elements x
+// elements: 161 us unsplit, 137 at 3, 130 at 6), and so for the records and
+// face fluxes of two fields (62,500: 129 us at 3, 121 at 6).  adv_ts at 17,000 elements x
 // 20: 52 -> 17 us, at 62,500 x 40: 101 -> 48 us.
 unsigned layer_chunks(const fvgpu_handle* h, long workgroups, int n, int per_cu) {
   const long want = ((long)per_cu * h->cu_count + workgroups - 1) / std::max(workgroups, 1l);
@@ -280,28 +273,18 @@ unsigned layer_chunks(const fvgpu_handle* h, long workgroups, int n, int per_cu)
     const unsigned nb_ = (unsigned)(((long)(NITEMS) + bs_ - 1) / bs_);                            \
     Launch l_(h, NAME);                                                                           \
     hipLaunchKernelGGL(KERNEL, dim3(nb_, layer_chunks(h, nb_, NLAYERS, PER_CU)), dim3(bs_), 0,     \
-                       h->cur, __VA_ARGS__);                                                      \
+                       h->stream, __VA_ARGS__);                                                      \
   } while (0)
 
-// Fork: work enqueued on stream2 after this waits for everything enqueued
-// on the main stream so far.  Join: the main stream waits for stream2.
-// Under graph capture the events become dependency edges of the graph.
-// `what` is the concurrency bit of the pair; with that bit clear both chains
-// go to the main stream in turn.
-enum { FV_CONC_3D = 1 };
-void fork_streams(fvgpu_handle* h, int what) {
-  if (!(h->concurrent & what)) return;
-  (void)hipEventRecord(h->ev_fork, h->stream);
-  (void)hipStreamWaitEvent(h->stream2, h->ev_fork, 0);
-}
-void join_streams(fvgpu_handle* h, int what) {
-  if (!(h->concurrent & what)) return;
-  (void)hipEventRecord(h->ev_join, h->stream2);
-  (void)hipStreamWaitEvent(h->stream, h->ev_join, 0);
-}
-// enqueue on the second chain's stream / back on the main stream
-void on_stream2(fvgpu_handle* h, int what) { h->cur = (h->concurrent & what) ? h->stream2 : h->stream; }
-void on_stream1(fvgpu_handle* h) { h->cur = h->stream; }
+// The same for n passes (pass_block): their workgroups count together.
+#define TLAUNCH_PASSES(NAME, KERNEL, NITEMS, NLAYERS, PER_CU, NPASS, ...)                           \
+  do {                                                                                            \
+    const int bs_ = block_of(h, NAME);                                                            \
+    const unsigned nb_ = pass_grid(((long)(NITEMS) + bs_ - 1) / bs_, NPASS);                       \
+    Launch l_(h, NAME);                                                                           \
+    hipLaunchKernelGGL(KERNEL, dim3(nb_, layer_chunks(h, nb_, NLAYERS, PER_CU)), dim3(bs_), 0,     \
+                       h->stream, __VA_ARGS__);                                                      \
+  } while (0)
 
 const double ALPHA_RK[5] = {0.0, 0.2500, 1.0 / 3.0, 0.5000, 1.0};
 
@@ -359,45 +342,46 @@ void enqueue_external_step_t(fvgpu_handle* h, int iext, const ExtClock* ec) {
   }
 }
 
-// ADV_T or ADV_S with FCT, VDIF_TS, BCOND_TS, F1 = FF and N2E3D of one
-// tracer (internal_step.F), on h->cur with the scratch of `a`.
+// The pass that advances f to ff with the scratch of `a`.
+Pass make_pass(const IntArgs& a, double* f, double* ff, const double* mean, const double* fdis, int which) {
+  return {f, ff, mean, fdis, which, a.rec, a.cvflux, a.pfpxb, a.pfpyb, a.ah_bottom, a.xflux_obc};
+}
+
+// ADV_T and/or ADV_S with FCT, VDIF_TS and BCOND_TS of the passes P
+// (internal_step.F).
 template <typename FT, bool UN>
-void enqueue_ts_pass(fvgpu_handle* h, IntArgs& a, int which, int fct) {
+void enqueue_ts(fvgpu_handle* h, const Passes& P, int fct) {
   const DevGrid& g = h->g;
-  const long mk = g.m1 * g.KB;
-  double* f1 = which == 1 ? a.t1 : a.s1;
-  double* ff = which == 1 ? a.tf1 : a.sf1;
-  const double* fm = which == 1 ? a.tmean1 : a.smean1;
-  const double* fdis = which == 1 ? g.tdis : g.sdis;
-#define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT, UN>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1, 3)), 256, g, a, f1, fm, 0.0)
+  const IntArgs& a = h->ia;
+  const unsigned nblk = pass_grid(g.cvb_nblk, P.n);
+#define CVRF_TS_CALL(RM) LAUNCH("cvrecflux_ts", (k_cvrecflux<0, RM, FT, UN>), dim3(nblk, layer_chunks(h, nblk, g.KBM1, 6)), 256, g, a, P, 0.0)
   FV_RMAX_DISPATCH(g.ring_max, CVRF_TS_CALL);
-#define ADV_TS_CALL10(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
-#define ADV_TS_CALL16(SM) TLAUNCH_LAYERS("adv_ts", (k_adv_ts_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1, 3, g, a, f1, ff, fdis, which, fct)
+#define ADV_TS_CALL10(SM) TLAUNCH_PASSES("adv_ts", (k_adv_ts_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1, 3, P.n, g, a, P, fct)
+#define ADV_TS_CALL16(SM) TLAUNCH_PASSES("adv_ts", (k_adv_ts_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1, 3, P.n, g, a, P, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL10);
   else FV_SMAX_DISPATCH(g.cv_max, ADV_TS_CALL16);
   if (g.IOBCN > 0) {
     const long np = (long)g.IOBCN * g.KBM1;
-    if (g.cv_max <= 16) LAUNCH("adv_ts_obc", (k_adv_ts_obc<16, FT>), (unsigned)((np + 15) / 16), 256, g, a);
-    else LAUNCH("adv_ts_obc", (k_adv_ts_obc<32, FT>), (unsigned)((np + 7) / 8), 256, g, a);
+    if (g.cv_max <= 16) LAUNCH("adv_ts_obc", (k_adv_ts_obc<16, FT>), dim3((unsigned)((np + 15) / 16), P.n), 256, g, a, P);
+    else LAUNCH("adv_ts_obc", (k_adv_ts_obc<32, FT>), dim3((unsigned)((np + 7) / 8), P.n), 256, g, a, P);
   }
-#define VDIF_TS_CALL(KM) TLAUNCH("vdif_ts", (k_vdif_ts_r<KM, UN>), g.M + 1, g, a, ff, which)
+#define VDIF_TS_CALL(KM) LAUNCH("vdif_ts", (k_vdif_ts_r<KM, UN>), pass_grid((g.M + bs_) / bs_, P.n), bs_, g, a, P)
+  const int bs_ = block_of(h, "vdif_ts");
   FV_KMAX_DISPATCH(g.KBM1, VDIF_TS_CALL);
-  TLAUNCH("bcond_ts", k_bcond_ts_sums, g.IOBCN + 1, g, a, which, a.obcsum);
-  if (g.IOBCN > 0) TLAUNCH("bcond_ts", k_bcond_ts_layers, (long)g.IOBCN * g.KBM1, g, a, which, (const double*)a.obcsum);
-  TLAUNCH("copy", k_copy, mk, f1, ff, mk);
-  N2E3D(f1, which == 1 ? a.t : a.s);
+  if (g.obc_on && g.IOBCN > 0) LAUNCH("bcond_ts", k_bcond_ts, dim3((unsigned)g.IOBCN, P.n), 64, g, a, P);
 }
 
-// ADV_Q(Q, QF) with FCT_Q2 (adv_q.F, fct_q2.F) on h->cur with the scratch
-// of `a`.
+// ADV_Q of Q2 and of Q2L with FCT_Q2 and FCT_Q2L (adv_q.F, fct_q2.F).
 template <typename FT, bool UN>
-void enqueue_adv_q(fvgpu_handle* h, IntArgs& a, double* q, double* qf, int fct) {
+void enqueue_adv_q(fvgpu_handle* h, const Passes& P, int fct) {
   const DevGrid& g = h->g;
+  const IntArgs& a = h->ia;
   const double qmean1 = (double)1.E-8f;
-#define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT, UN>), dim3(g.cvb_nblk, layer_chunks(h, g.cvb_nblk, g.KBM1 - 1, 3)), 256, g, a, q, nullptr, qmean1)
+  const unsigned nblk = pass_grid(g.cvb_nblk, P.n);
+#define CVRF_Q_CALL(RM) LAUNCH("cvrecflux_q", (k_cvrecflux<1, RM, FT, UN>), dim3(nblk, layer_chunks(h, nblk, g.KBM1 - 1, 6)), 256, g, a, P, qmean1)
   FV_RMAX_DISPATCH(g.ring_max, CVRF_Q_CALL);
-#define ADV_Q_CALL10(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
-#define ADV_Q_CALL16(SM) TLAUNCH_LAYERS("adv_q", (k_adv_q_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1 - 1, 3, g, a, q, qf, fct)
+#define ADV_Q_CALL10(SM) TLAUNCH_PASSES("adv_q", (k_adv_q_gather<SM, 10, FT, UN>), g.M + 1, g.KBM1 - 1, 3, P.n, g, a, P, fct)
+#define ADV_Q_CALL16(SM) TLAUNCH_PASSES("adv_q", (k_adv_q_gather<SM, 16, FT, UN>), g.M + 1, g.KBM1 - 1, 3, P.n, g, a, P, fct)
   if (g.ring_max <= 10) FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL10);
   else FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL16);
 }
@@ -406,7 +390,7 @@ void enqueue_adv_q(fvgpu_handle* h, IntArgs& a, double* q, double* qf, int fct) 
 template <typename FT, bool UN>
 void enqueue_internal_step_t(fvgpu_handle* h) {
   const DevGrid& g = h->g;
-  IntArgs& a = h->ia;
+  IntArgs &a = h->ia, &b = h->ib;
   const long mk = g.m1 * g.KB, nk = g.n1 * g.KB;
   LAUNCH("int_clock", k_int_clock, 1, 64, g, h->clk, a.qdis, h->ec, 1, g.isplit);
 #define ADJ1_CALL(KM) TLAUNCH("adjust1_brough", (k_adjust1_brough<KM, UN>), g.N + 1, g, a)
@@ -423,7 +407,7 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
   FV_KMAX_DISPATCH(g.KBM1, ADJ2_CALL);
 #define VERTVL_CALL(SM) LAUNCH("vertvl", (k_vertvl_tile<SM, UN>), g.nt_nblk, 256, g, a)
   FV_SMAX_DISPATCH(g.cv_max, VERTVL_CALL);
-  N2E3D(a.wts, a.w);
+  N2E3D((N2eFields{{a.wts}, {a.w}}), 1);
 #define VISCOFH_CALL(RM) TLAUNCH_LAYERS("viscofh", k_viscofh_r<RM>, g.M + 1, g.KBM1, 3, g, a)
   FV_RMAX_DISPATCH(g.ve_max, VISCOFH_CALL);
   LAUNCH("advuv_blk", (k_uv_blk<1, FT, UN>), dim3(g.ub_run.nblk, layer_chunks(h, g.ub_run.nblk, g.KBM1, 6)), 256, g, a);
@@ -447,13 +431,11 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     // (vdif_q also stores Q2 = Q2F, Q2L = Q2LF for its columns)
     FV_RMAX_DISPATCH(g.ve_max, VDIF_QM_CALL);
   } else if (h->md->p.vertical_closure) {
-    // ADV_Q of Q2 on the main stream, of Q2L on stream2 (own scratch)
-    fork_streams(h, FV_CONC_3D);
-    on_stream2(h, FV_CONC_3D);
-    enqueue_adv_q<FT, UN>(h, h->ib, a.q2l, a.q2lf, fct);
-    on_stream1(h);
-    enqueue_adv_q<FT, UN>(h, a, a.q2, a.q2f, fct);
-    join_streams(h, FV_CONC_3D);
+    Passes P{};
+    P.n = 2;
+    P.p[0] = make_pass(a, a.q2, a.q2f, nullptr, nullptr, 0);
+    P.p[1] = make_pass(b, a.q2l, a.q2lf, nullptr, nullptr, 0);
+    enqueue_adv_q<FT, UN>(h, P, fct);
 #define VDIF_Q_CALL(RM) TLAUNCH("vdif_q", (k_vdif_q<RM, UN>), g.M + 1, g, a, a.vhpair, (const int*)nullptr)
     // VDIF_Q, then Q2 = Q2F and Q2L = Q2LF (internal_step.F:1029-1035) in
     // the same kernel, the elimination coefficients in `vhpair`.
@@ -463,30 +445,29 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     const double umol = h->md->p.umol;
     TLAUNCH("const_mixing", k_const_mixing, mk, a.km, a.kh, umol, umol * h->md->p.vprnu, mk);
   }
-  N2E3D(a.km, a.km1);
-  // ADV_T .. T1 = TF1 on the main stream, the same for S on stream2 (own
-  // scratch); the two passes share no written array
   const bool t_on = h->md->p.temperature_active, s_on = h->md->p.salinity_active;
-  if (t_on && s_on) {
-    fork_streams(h, FV_CONC_3D);
-    on_stream2(h, FV_CONC_3D);
-    enqueue_ts_pass<FT, UN>(h, h->ib, 2, fct);
-    on_stream1(h);
-    enqueue_ts_pass<FT, UN>(h, a, 1, fct);
-    join_streams(h, FV_CONC_3D);
-  } else if (t_on) {
-    enqueue_ts_pass<FT, UN>(h, a, 1, fct);
-  } else if (s_on) {
-    enqueue_ts_pass<FT, UN>(h, a, 2, fct);
+  N2eFields ne{};
+  int nf = 0;
+  auto n2e = [&](const double* nvar, double* evar) { ne.nvar[nf] = nvar; ne.evar[nf++] = evar; };
+  n2e(a.km, a.km1);
+  Passes P{};
+  if (t_on) {
+    P.p[P.n++] = make_pass(a, a.t1, a.tf1, a.tmean1, g.tdis, 1);
+    n2e(a.t1, a.t);
   }
-  if (!g.river_ts_specified && g.NUMQBC > 0) LAUNCH("adjust_ts", k_adjust_ts, 1, 256, g, a);
-  if (!h->md->p.barotropic) {
-    TLAUNCH("dens2", k_dens2, mk, g, a);
-    N2E3D(a.rho1, a.rho);
+  if (s_on) {
+    P.p[P.n++] = make_pass(b, a.s1, a.sf1, a.smean1, g.sdis, 2);
+    n2e(a.s1, a.s);
   }
-  TLAUNCH("copy", k_copy, nk, a.u, a.uf, nk);
-  TLAUNCH("copy", k_copy, nk, a.v, a.vf, nk);
-  TLAUNCH("end_2d", k_end_2d, std::max(g.M, g.N) + 1, g, a);
+  if (P.n > 0) enqueue_ts<FT, UN>(h, P, fct);
+  const bool dens = !h->md->p.barotropic, adjust = !g.river_ts_specified && g.NUMQBC > 0;
+  TLAUNCH("step_end", k_step_end, std::max(mk, nk), g, a, (int)t_on, (int)s_on, (int)(dens && !adjust));
+  if (adjust) {
+    LAUNCH("adjust_ts", k_adjust_ts, 1, 256, g, a);
+    if (dens) TLAUNCH("dens2", k_dens2, mk, g, a);
+  }
+  if (dens) n2e(a.rho1, a.rho);
+  N2E3D(ne, nf);
 }
 
 // One EXTERNAL_STEP by itself: its EXTEL terms and constants are formed
@@ -1183,7 +1164,6 @@ int upload_state(fvgpu_handle* h) {
     a.rec = pr; a.cvflux = pc;
   }
   if (dalloc(h, &a.vhpair, mk)) return 1;
-  if (dalloc(h, &a.obcsum, 5 * (size_t)g.IOBCN)) return 1;
   RW(adx2d, nullptr, n1); RW(ady2d, nullptr, n1); RW(drx2d, nullptr, n1); RW(dry2d, nullptr, n1);
   RW(cbc, nullptr, n1); RW(wubot, nullptr, n1); RW(wvbot, nullptr, n1); RW(tps, nullptr, n1);
   RW(uard, nullptr, n1); RW(vard, nullptr, n1); RW(fluxobn, nullptr, n1);
@@ -1206,7 +1186,7 @@ int upload_state(fvgpu_handle* h) {
   c.isplit = g.isplit; c.iramp = g.iramp; c.depth_fail = 0;
   HIPCHK(h->stage.to_device(h->clk, &c, sizeof(c), h->stream, h->device));
   a.clk = h->clk;
-  // the stream2 chains: the same arrays, their own scratch (node-layer
+  // the second of two passes: the same arrays, their own scratch (node-layer
   // records, face fluxes, bottom gradients, OBC fluxes)
   IntArgs& b = h->ib;
   b = a;
@@ -1219,7 +1199,6 @@ int upload_state(fvgpu_handle* h) {
   }
   if (dalloc(h, &b.pfpxb, m1) || dalloc(h, &b.pfpyb, m1) || dalloc(h, &b.ah_bottom, m1)) return 1;
   if (dalloc(h, &b.xflux_obc, (size_t)g.IOBCN * g.KB)) return 1;
-  if (dalloc(h, &b.obcsum, 5 * (size_t)g.IOBCN)) return 1;
   return 0;
 }
 
@@ -1275,14 +1254,7 @@ int fvgpu_create(const fv_model* md, int32_t precision, fvgpu_handle** out) {
   HIPCHK(hipDeviceGetAttribute(&h->cu_count, hipDeviceAttributeMultiprocessorCount, h->device));
   if (!scratch_of(h->device)) { delete h; return 1; }
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) { delete h; return fail("stream"); }
-  h->cur = h->stream;
   h->stage.reserve();
-  if (hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming) != hipSuccess) {
-    fvgpu_destroy(h);
-    return fail("stream2 / events");
-  }
   if (upload_grid(h) || upload_state(h) || dupload(h, &h->dg, &h->g, 1)) { fvgpu_destroy(h); return 1; }
   HIPCHK(hipStreamSynchronize(h->stream));
   *out = h;
@@ -1530,14 +1502,10 @@ int fvgpu_synchronize(fvgpu_handle* h) {
 void fvgpu_destroy(fvgpu_handle* h) {
   if (!h) return;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->stream2) (void)hipStreamSynchronize(h->stream2);
   drop_graphs(h);
   for (hipEvent_t e : h->event_pool) (void)hipEventDestroy(e);
   for (void* p : h->allocs) (void)hipFree(p);
   h->stage.release();
-  if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
-  if (h->ev_join) (void)hipEventDestroy(h->ev_join);
-  if (h->stream2) (void)hipStreamDestroy(h->stream2);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -1870,9 +1838,7 @@ int fvgpu_set_block(fvgpu_handle* h, const char* family, int32_t block) {
 
 int fvgpu_set_concurrency(fvgpu_handle* h, int32_t mode) {
   if (mode < 0 || mode > 3) return fail("concurrency must be 0..3");
-  h->concurrent = mode;
-  drop_graphs(h);
-  return 0;
+  return 0;   // no effect: the step's independent chains share their launches
 }
 
 int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_len) {
@@ -1894,8 +1860,7 @@ int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_
   HIPCHK(hipMemcpyAsync(arena + off, h->clk, sizeof(DevClock), hipMemcpyDeviceToDevice, h->stream));
   const bool prof = h->profiling;
   const std::string only = h->profile_only;
-  const int conc = h->concurrent, every = h->profile_every;
-  h->concurrent = 0;   // each family timed alone, at every launch
+  const int every = h->profile_every;   // each family timed at every launch
   h->profile_every = 1;
   std::string rep;
   int rc = 0;
@@ -1927,7 +1892,6 @@ int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_
   }
   h->profiling = prof;
   h->profile_only = only;
-  h->concurrent = conc;
   h->profile_every = every;
   h->stats.clear();
   off = 0;

@@ -29,7 +29,6 @@ struct IntArgs {
   // flux buffers, of the flux type FT (double, or float in the mixed form)
   void* rec;             // node-layer records of the field being advected, CvRecT<FT>
   double2* vhpair;       // node-layer pair scratch: VDIF_Q's elimination coefficients
-  double* obcsum;        // BCOND_TS column sums, 5 per OBC node
   void* cvflux;          // per sub-edge, per layer face flux (NCV+1) x KB FT
   // 2-D
   double *adx2d, *ady2d, *drx2d, *dry2d, *cbc, *wubot, *wvbot, *tps, *uard, *vard, *fluxobn;
@@ -39,6 +38,34 @@ struct IntArgs {
   double *qdis, *xflux_obc, *uard_obcn;
   DevClock* clk;
 };
+
+// A field that a launch of the advection, tracer and q2 kernels advances, with
+// its scratch: T and S, and Q2 and Q2L, are advanced by the same launches, one
+// pass each.
+struct Pass {
+  double *f, *ff;             // F1 and FF
+  const double *mean, *fdis;  // tracers: the mean and the rivers' values
+  int which;                  // 1: T, 2: S
+  void *rec, *cvflux;
+  double *pfpxb, *pfpyb, *ah_bottom, *xflux_obc;
+};
+struct Passes {
+  Pass p[2];
+  int n;                      // 1 or 2
+};
+
+// This workgroup's pass, and its block of `nblk` (the grid's x extent is
+// pass_grid(nblk, n)): as xcd_block, with the two passes of a block next to
+// one another on one XCD, so that what they share -- velocities, geometry,
+// lists -- is read from its L2 the second time.  False: no block.
+__device__ __forceinline__ bool pass_block(const Passes& P, int nblk, Pass& p, int& b) {
+  const int two = P.n - 1, j = (int)blockIdx.x >> 3;
+  const bool second = (j & two) != 0;
+  p = second ? P.p[1] : P.p[0];
+  b = ((int)blockIdx.x & 7) * ((nblk + 7) >> 3) + (j >> two);
+  return b < nblk;
+}
+inline unsigned pass_grid(long nblk, int n) { return (unsigned)((nblk + 7) / 8 * 8 * n); }
 
 #define GRID1(n) (((n) + 255) / 256), 256
 
@@ -257,13 +284,21 @@ __global__ __launch_bounds__(256) void k_adjust2(DevGrid g, IntArgs a) {
   });
 }
 
-// N2E3D (mod_main.F:1633-1645) over layers 1..kmax: one thread per element
-// and group of eight layers (blockIdx.y), the group's node loads issued
-// together.  The grid's x extent is a multiple of 8, so every layer group
-// of an element range runs on the same XCD and shares its L2.
-__global__ __launch_bounds__(256) void k_n2e3d(DevGrid g, const double* nvar, double* evar, int kmax) {
+// N2E3D (mod_main.F:1633-1645) of up to four fields (blockIdx.z) over layers
+// 1..kmax: one thread per element and group of eight layers (blockIdx.y), the
+// group's node loads issued together.  The grid's x extent is a multiple of
+// 8, so every layer group of an element range runs on the same XCD and shares
+// its L2.
+struct N2eFields {
+  const double* nvar[4];
+  double* evar[4];
+};
+__global__ __launch_bounds__(256) void k_n2e3d(DevGrid g, N2eFields f, int kmax) {
   const int i = (int)xcd_thread() + 1;
   if (i > g.N) return;
+  const int z = (int)blockIdx.z;
+  const double* nvar = z == 0 ? f.nvar[0] : z == 1 ? f.nvar[1] : z == 2 ? f.nvar[2] : f.nvar[3];
+  double* evar = z == 0 ? f.evar[0] : z == 1 ? f.evar[1] : z == 2 ? f.evar[2] : f.evar[3];
   const int j1 = NV_(i, 1), j2 = NV_(i, 2), j3 = NV_(i, 3);
   const double one_third = 1.0 / 3.0;
   const int k0 = (int)blockIdx.y * 8 + 1;

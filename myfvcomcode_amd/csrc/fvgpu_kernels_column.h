@@ -117,10 +117,32 @@ __global__ __launch_bounds__(256) void k_vdif_uv_r(DevGrid g, IntArgs a) {
 // sigma values as in VDIF_UV (1,000,000 elements x 40 layers: 157 -> 114 us; the
 // loads ahead alone changed nothing).
 template <int KMAX, bool UNI>
-__global__ __launch_bounds__(256) void k_vdif_ts_r(DevGrid g, IntArgs a, double* f, int ncon) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 1 || i > g.M || g.isonb[i] == 2) return;   // OBC columns keep F (vdif_ts.F:259,313)
+__global__ __launch_bounds__(256) void k_vdif_ts_r(DevGrid g, IntArgs a, Passes P) {
+  Pass ps;
+  int b;
+  if (!pass_block(P, (int)(g.M / blockDim.x) + 1, ps, b)) return;
+  const int i = b * (int)blockDim.x + (int)threadIdx.x;
+  if (i < 1 || i > g.M) return;
+  double* f = ps.ff;
+  const int ncon = ps.which;
   const int KBM1 = g.KBM1, KBM2 = g.KBM2;
+  if (g.river_ts_specified) {
+    // BCOND_TS at the river nodes: the last river at the node sets it (the
+    // reference sets TF1 and SF1 in both calls; each pass here sets its own,
+    // which leaves T1 and S1 unchanged, F1 = FF following in both)
+    const int rv = g.node_riv[i];
+    if (rv >= 0) {
+      double w;
+      int last = -1;
+      for (int j = rv; j < g.NUMQBC; ++j)
+        if (river_share(g, j, i, w)) last = j;
+      if (last >= 0) {
+        for (int k = 1; k <= KBM1; ++k) f[NI(g, i, k)] = ps.fdis[last];
+        return;
+      }
+    }
+  }
+  if (g.isonb[i] == 2) return;   // OBC columns keep F (vdif_ts.F:259,313)
   const double dti = g.dti, umolpr = g.umol * 1.E0, d = a.d[i];
   const long m1 = g.m1;
   auto dz = [&](int k) { return DZ(i, k); };
@@ -154,9 +176,9 @@ __global__ __launch_bounds__(256) void k_vdif_ts_r(DevGrid g, IntArgs a, double*
     }
   });
   const double cfb = -dti * (khbottom + umolpr) / (dz(KBM1) * dzz(KBM1 - 1) * d * d);
-  const double tmp1 = a.pfpxb[i] * g.cos_sita[i] + a.pfpyb[i] * g.sin_sita[i];
-  const double tmp2 = a.ah_bottom[i] * g.phpn[i];
-  const double tmp3 = khbottom + umolpr + a.ah_bottom[i] * g.phpn[i] * g.phpn[i];
+  const double tmp1 = ps.pfpxb[i] * g.cos_sita[i] + ps.pfpyb[i] * g.sin_sita[i];
+  const double tmp2 = ps.ah_bottom[i] * g.phpn[i];
+  const double tmp3 = khbottom + umolpr + ps.ah_bottom[i] * g.phpn[i] * g.phpn[i];
   double tmp = tmp1 * tmp2 / tmp3 * (khbottom + umolpr);
   if (g.noflux_bot) {
     if (ncon == 1) { if (tmp1 > 0.0) tmp = 0.0; }

@@ -233,12 +233,13 @@ __device__ __forceinline__ void cv_faces(const ElemFaces<FT>& f, const CvRecT<FT
 // operation), then the first lane sums them in sub-edge order.  Every
 // face's loads issue at once instead of one face after another.
 template <int LP, typename FT>
-__global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a) {
+__global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a, Passes P) {
+  const Pass ps = blockIdx.y == 0 ? P.p[0] : P.p[1];
   __shared__ double sadv[256];
   const int lane = threadIdx.x % LP;
   const long t = (long)blockIdx.x * (256 / LP) + threadIdx.x / LP;
   const bool act = t < (long)g.IOBCN * g.KBM1;
-  const CvRecT<FT>* rec = (const CvRecT<FT>*)a.rec;
+  const CvRecT<FT>* rec = (const CvRecT<FT>*)ps.rec;
   const int obc = act ? (int)(t % g.IOBCN) : 0, k = act ? (int)(t / g.IOBCN) + 1 : 1;
   const int i = g.i_obc_n[obc];
   const int n = act ? g.cv_cnt[i] : 0;
@@ -260,17 +261,21 @@ __global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a) {
   if (!act || lane != 0) return;
   double xadv = 0.0;
   for (int j = 0; j < n; ++j) xadv = xadv + sadv[threadIdx.x + j];
-  a.xflux_obc[(long)(k - 1) * g.IOBCN + obc] = xadv;
+  ps.xflux_obc[(long)(k - 1) * g.IOBCN + obc] = xadv;
 }
 
-// Phase 3 of ADV_T/ADV_S (adv_t.F:507-1052): ordered sub-edge sums (in FP64
+// Phase 2 of ADV_T/ADV_S (adv_t.F:507-1052): ordered sub-edge sums (in FP64
 // whatever the flux type), bottom gradients for VDIF_TS, vertical flux,
 // rivers, the update TF1 = (T1 - XFLUX/ART1*DTI/(DT*DZ))*DT/DTFA and FCT.
 template <int SMAX, int RMAX, typename FT, bool UNI>
-__global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, const double* f1, double* ff,
-                                                        const double* fdis, int which, int fct) {
-  const int i = (int)xcd_thread();
+__global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, Passes P, int fct) {
+  Pass ps;
+  int b;
+  if (!pass_block(P, (int)(g.M / blockDim.x) + 1, ps, b)) return;
+  const int i = b * (int)blockDim.x + (int)threadIdx.x;
   if (i < 1 || i > g.M) return;
+  const double *f1 = ps.f, *fdis = ps.fdis;
+  double* ff = ps.ff;
   const bool clip = fct && !g.fct_skip[i];
   const int n = g.cv_cnt[i];
   int ce[SMAX];
@@ -287,7 +292,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
   layer_share(1, g.KBM1, k0, k1);
   for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.m1;
-    const FT* fl = (const FT*)a.cvflux + (long)(k - 1) * cs;
+    const FT* fl = (const FT*)ps.cvflux + (long)(k - 1) * cs;
     // all SMAX loads issue together; the sum takes the node's terms in
     // sub-edge order, subtracting on side IB, and the slots past its count
     // add the unused entry 0, which is zero and leaves it as it is
@@ -302,10 +307,10 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
       xflux = xflux + flip_sign((double)xv[j], ce[j]);
     });
     if (k == g.KBM1) {  // ADV_T and ADV_S both set the bottom-gradient terms VDIF_TS reads
-      const CvRecT<FT> r = ((const CvRecT<FT>*)a.rec)[ko + i];
-      a.pfpxb[i] = (double)r.gx;
-      a.pfpyb[i] = (double)r.gy;
-      a.ah_bottom[i] = (g.fact * a.viscofh[ko + i] + g.fm1) * g.nn_hvc[i];
+      const CvRecT<FT> r = ((const CvRecT<FT>*)ps.rec)[ko + i];
+      ps.pfpxb[i] = (double)r.gx;
+      ps.pfpyb[i] = (double)r.gy;
+      ps.ah_bottom[i] = (g.fact * a.viscofh[ko + i] + g.fm1) * g.nn_hvc[i];
     }
     const double fk = at(f1 + ko, i), dzk = DZ(i, k);
     // DZ-weighted values at the layer's upper (nu/du) and lower (nd/dd)
@@ -341,7 +346,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, con
             xflux = xflux - a.qdis[j] * w * g.vqdist[(long)(k - 1) * g.NUMQBC + j] * fdis[j];
         }
     }
-    if (which == 1) xflux = xflux - 0.0 * art1;
+    if (ps.which == 1) xflux = xflux - 0.0 * art1;
     double x = (fk - xflux / art1 * (g.dti / (a.dt[i] * dzk))) * (a.dt[i] / a.dtfa[i]);
     if (clip) {  // FCT_T / FCT_S (fct_t.F:74-101)
       double tmin, tmax;
@@ -397,15 +402,17 @@ struct CvRecLds {
 // the waves in every second workgroup (the record waves take twice the
 // instructions of the face waves) changed nothing.
 template <int KIND, int RMAX, typename FT, bool UNI>
-__global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const double* fld, const double* mean,
-                                                   double cmean) {
+__global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, Passes P, double cmean) {
   __shared__ CvRecLds<FT> srec[2];
   // one layer of the field (and for the tracer its mean) at the block's
   // nodes and their rings
   constexpr int NF = KIND == 0 ? 2 : 1;
   __shared__ __attribute__((aligned(16))) double sfld[2][FV_CVH * NF];
-  const int b = xcd_block(), t = threadIdx.x;
-  int k0, k1;
+  const int t = threadIdx.x;
+  Pass ps;
+  int b, k0, k1;
+  if (!pass_block(P, g.cvb_nblk, ps, b)) return;
+  const double *fld = ps.f, *mean = ps.mean;
   layer_share(KIND == 0 ? 1 : 2, g.KBM1, k0, k1);
   const int nk = k1 - k0 + 1;       // layers (interfaces) of this workgroup
   if (nk < 1) return;
@@ -413,7 +420,7 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
   // uniform over each wave and both roles pass nk + 2 barriers.
   if (__builtin_amdgcn_readfirstlane(t) < FV_CVB) {
     // records: local node t of the block
-    CvRecT<FT>* rec = (CvRecT<FT>*)a.rec;
+    CvRecT<FT>* rec = (CvRecT<FT>*)ps.rec;
     const bool nact = t < g.cvb_nn[b];
     const int i = nact ? g.cvb_nodes[(long)FV_CVB * b + t] : 1;
     RingGeo<RMAX> rg;
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
     }
   } else {
     // faces: local element t - FV_CVB of the block
-    FT* cvflux = (FT*)a.cvflux;
+    FT* cvflux = (FT*)ps.cvflux;
     const int te = t - FV_CVB;
     const bool eact = te < g.cvb_ne[b];
     const int e = eact ? g.cvb_elems[(long)FV_CVB * b + te] : 1;
@@ -542,9 +549,14 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, const d
 // and ring values shared by neighbours are fetched again (1,000,000 elements
 // x 40 layers: 650 us at 4, 506 at 3; 532 before its 32-bit addresses).
 template <int SMAX, int RMAX, typename FT, bool UNI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_adv_q_gather(DevGrid g, IntArgs a, const double* q, double* qf, int fct) {
-  const int i = (int)xcd_thread();
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_adv_q_gather(DevGrid g, IntArgs a, Passes P, int fct) {
+  Pass ps;
+  int b;
+  if (!pass_block(P, (int)(g.M / blockDim.x) + 1, ps, b)) return;
+  const int i = b * (int)blockDim.x + (int)threadIdx.x;
   if (i > g.M) return;
+  const double* q = ps.f;
+  double* qf = ps.ff;
   if (i == 0) {
     if (blockIdx.y == 0)
       for (int k = 1; k <= g.KB; ++k) qf[NI(g, 0, k)] = 0.0;
@@ -569,7 +581,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   layer_share(2, g.KBM1, k0, k1);
   for (int k = k0; k <= k1; ++k) {
     const long ko = (long)(k - 1) * g.m1;
-    const FT* fl = (const FT*)a.cvflux + (long)(k - 1) * cs;
+    const FT* fl = (const FT*)ps.cvflux + (long)(k - 1) * cs;
     // all SMAX loads issue together; the sum takes the node's terms in
     // sub-edge order, subtracting on side IB, and the slots past its count
     // add the unused entry 0, which is zero and leaves it as it is

@@ -19,8 +19,9 @@ I4 = 4
 
 def sizes(model):
     h = model.hdr
+    ts = int(bool(h.p.temperature_active)) + int(bool(h.p.salinity_active))   # tracers a launch advances
     return dict(M=h.m, N=h.n, NE=h.ne, NCV=h.ncv, KB=h.kb, KBM1=h.kbm1,
-                RSN=h.nring_sn, RVE=h.nring_ve)
+                RSN=h.nring_sn, RVE=h.nring_ve, TS=ts, N2E=2 + ts + int(not h.p.barotropic))
 
 
 # ----------------------------------------------------------------- 2-D mode
@@ -41,49 +42,52 @@ def ext_momentum(s, real=R8):
 
 
 # ----------------------------------------------------------------- 3-D mode
-def _cvrecflux(s, layers, nfields, uv_layers, bottom_records, real):
-    """Records formed in LDS and face fluxes in one launch: the node fields
-    and ring geometry, the element geometry and velocities are read, the
-    face fluxes (and the bottom layer's records for the tracer) written;
-    no node-layer record crosses HBM."""
+def _cvrecflux(s, layers, own, fields, uv_layers, bottom_records, real):
+    """Records formed in LDS and face fluxes of `fields` fields in one launch:
+    the ring and element geometry, VISCOFH and the velocities are read once,
+    `own` node fields of each field (itself, its mean) read and its face
+    fluxes (and the bottom layer's records for the tracer) written; no other
+    node-layer record crosses HBM."""
     M, N, NCV, RSN = s["M"], s["N"], s["NCV"], s["RSN"]
-    reads = (RSN * (I4 + 2 * real) + M * (2 * I4 + 2 * real)   # ring lists and factors, NTSN, ART2, NN_HVC
-             + nfields * M * layers * real                     # field, mean, VISCOFH
-             + 2 * N * I4 + M * 13 // 10 * I4                  # block element lists and local indices; node lists (about 1.3 per node)
+    reads = (RSN * (1 + 2 * real) + M * (2 * I4 + 2 * real)    # ring slots and factors, NTSN, ART2, NN_HVC
+             + M * layers * real                               # VISCOFH
+             + fields * own * M * layers * real                # field, mean
+             + 2 * N * I4 + M * 32 // 10 * I4                  # block element lists and local indices; the blocks' nodes (about 1.3 per node) and with their rings (1.9)
              + NCV * (3 * I4 + 6 * real) + N * real            # sub-edge geometry, DT1
              + N * uv_layers * 2 * real)                       # U, V
-    writes = NCV * layers * real + (M * 8 * real if bottom_records else 0)
+    writes = fields * (NCV * layers * real + (M * 8 * real if bottom_records else 0))
     return reads + writes
 
 
 def cvrecflux_ts(s, real=R8):
-    """ADV_T/ADV_S records and face fluxes in one launch."""
-    return _cvrecflux(s, s["KBM1"], 3, s["KBM1"], True, real)
+    """ADV_T and ADV_S records and face fluxes in one launch."""
+    return _cvrecflux(s, s["KBM1"], 2, s["TS"], s["KBM1"], True, real)
 
 
 def cvrecflux_q(s, real=R8):
-    """ADV_Q records and face fluxes in one launch."""
-    return _cvrecflux(s, s["KBM1"] - 1, 2, s["KBM1"], False, real)
+    """ADV_Q records and face fluxes of Q2 and Q2L in one launch."""
+    return _cvrecflux(s, s["KBM1"] - 1, 1, 2, s["KBM1"], False, real)
 
 
 def adv_ts(s, real=R8):
-    """Ordered sub-edge sums + vertical flux + update (T or S)."""
+    """Ordered sub-edge sums + vertical flux + update of T and S."""
     M, NCV, KB, KBM1 = s["M"], s["NCV"], s["KB"], s["KBM1"]
-    reads = (M * (3 * I4 + 4 * real) + 2 * NCV * I4   # counts, flags; ART1, DT, DTFA, NN_HVC; slot lists
-             + NCV * KBM1 * real                       # face fluxes
-             + M * KBM1 * real + M * KB * real         # T1, WTS
-             + M * KBM1 * 2 * real                     # FCT ring bounds (RLOHI)
-             + M * (real + 8 * real))                  # bottom VISCOFH and record
-    writes = M * KBM1 * real + 3 * M * real            # TF1; PFPXB, PFPYB, AH_BOTTOM
+    reads = (M * (3 * I4 + 4 * real) + 2 * NCV * I4 + M * (I4 + real)   # counts, flags; ART1, DT, DTFA, NN_HVC; slot lists; bottom VISCOFH
+             + M * KB * real                                   # WTS
+             + s["RSN"] * I4                                   # FCT rings
+             + s["TS"] * (NCV * KBM1 * real                    # face fluxes
+                          + M * KBM1 * real                    # F1
+                          + M * 8 * real))                     # bottom record
+    writes = s["TS"] * (M * KBM1 * real + 3 * M * real)        # FF; PFPXB, PFPYB, AH_BOTTOM
     return reads + writes
 
 
 def adv_q(s, real=R8):
-    """Ordered sub-edge sums + vertical flux + update (Q2 or Q2L)."""
+    """Ordered sub-edge sums + vertical flux + update of Q2 and Q2L."""
     M, NCV, KB, KBM1 = s["M"], s["NCV"], s["KB"], s["KBM1"]
-    reads = (M * (I4 + 3 * real) + 2 * NCV * I4 + NCV * (KBM1 - 1) * real + 2 * M * KB * real
-             + M * (KBM1 - 1) * 2 * real)              # FCT ring bounds (RLOHI)
-    writes = M * KB * real
+    reads = (M * (I4 + 3 * real) + 2 * NCV * I4 + M * KB * real + s["RSN"] * I4
+             + 2 * (NCV * (KBM1 - 1) * real + M * KB * real))
+    writes = 2 * M * KB * real
     return reads + writes
 
 
@@ -154,22 +158,29 @@ def vdif_uv(s, real=R8):
 
 
 def vdif_ts(s, real=R8):
-    """VDIF_TS: implicit vertical diffusion of one tracer."""
+    """VDIF_TS: implicit vertical diffusion of T and S."""
     M, KB, KBM1 = s["M"], s["KB"], s["KBM1"]
-    return M * KB * 2 * real + M * 8 * real + M * KBM1 * real
+    return M * KB * real + M * 5 * real + s["TS"] * (M * 2 * KBM1 * real + M * 3 * real)
+
+
+def step_end(s, real=R8):
+    """T1 = TF1, S1 = SF1 with DENS2 of them, U = UF, V = VF and the 2-D state."""
+    M, N, KB = s["M"], s["N"], s["KB"]
+    return M * KB * (2 * s["TS"] + (s["N2E"] > 2 + s["TS"])) * real + 4 * N * KB * real + (M + N) * 4 * real
 
 
 def n2e3d(s, real=R8):
-    """N2E3D of one node-layer field (KB layers): element mean of its nodes."""
+    """N2E3D of node-layer fields (KB layers): element means of their nodes;
+    the mean of its two launches, of W and of KM1, T, S and RHO."""
     M, N, KB = s["M"], s["N"], s["KB"]
-    return M * KB * real + N * 3 * I4 + N * KB * real
+    return N * 3 * I4 + (s["N2E"] * (M * KB * real + N * KB * real)) // 2
 
 
 FAMILIES = {f.__name__: f for f in (
     ext_momentum, cvrecflux_ts, cvrecflux_q,
     adv_ts, adv_q,
     adv3d_blk, advuv_blk, vertvl, viscofh, vdif_q, vdif_uv, vdif_ts,
-    n2e3d)}
+    step_end, n2e3d)}
 
 
 def bytes_per_launch(name, model, real=R8):

@@ -1,6 +1,7 @@
 """The internal step where the tiles of the fused tracer and q2 kernels carry
-the most: tiles whose nodes and rings exceed two waves, the widest rings, and
-sigma columns that differ from node to node, against the oracle bit for bit."""
+the most: tiles whose nodes and rings exceed two waves, the widest rings,
+sigma columns that differ from node to node, and the deepest columns,
+against the oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -54,7 +55,13 @@ def _sigma_by_node():
     return m
 
 
-CASES = {"stretched": _stretched, "wheel": wheel_mesh, "sigma": _sigma_by_node}
+def _deep():
+    """The most layers the device takes, under an open boundary."""
+    import myfvcomcode_amd as F
+    return F.Model.build(1, nx=13, ny=9, kb=64, n_seamounts=1)
+
+
+CASES = {"stretched": _stretched, "wheel": wheel_mesh, "sigma": _sigma_by_node, "deep": _deep}
 
 
 @pytest.mark.parametrize("name", list(CASES))
