@@ -227,6 +227,13 @@ void drop_graphs(fvgpu_handle* h) {
     hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(BLOCK), 0, h->stream, __VA_ARGS__);    \
   } while (0)
 
+// LAUNCH with LDS bytes of dynamic shared memory.
+#define LAUNCH_LDS(NAME, KERNEL, GRID, BLOCK, LDS, ...)                          \
+  do {                                                                            \
+    Launch l_(h, NAME);                                                           \
+    hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(BLOCK), LDS, h->stream, __VA_ARGS__); \
+  } while (0)
+
 inline unsigned nb(long n) { return (unsigned)((n + 255) / 256); }
 
 // N2E3D of n node fields over layers 1..KB (k_n2e3d's grid: elements by
@@ -386,6 +393,28 @@ void enqueue_adv_q(fvgpu_handle* h, const Passes& P, int fct) {
   else FV_SMAX_DISPATCH(g.cv_max, ADV_Q_CALL16);
 }
 
+// Whether VDIF_Q runs by block of columns (k_vdif_q_blk): where the columns
+// are fewer than three waves a CU, one lane a column (k_vdif_q) leaves the
+// chip waiting on a column's 20 dependent divisions a level; with more, its
+// lanes are the better packed (32,000 columns x 40 layers: 174 us one lane a
+// column, 113 by block; 63,000 x 40: 195, 227; 63,000 x 20: 104, 104; 126,000 x
+// 20: 147, 240).  Twice as many where a subset of the columns is solved, which
+// is seldom all of them (63,000 x 40, the learned closure's fallback: 134, 37).
+// The block's levels have to fit 64 KiB of LDS (KB <= 45).
+bool vdif_q_blocks(const fvgpu_handle* h, bool subset) {
+  const DevGrid& g = h->g;
+  return (long)g.M + 1 <= (subset ? 384l : 192l) * h->cu_count &&
+         (size_t)FV_VQARR * g.KB * FV_VQN * sizeof(double) <= 65536 - 1024;
+}
+#define VDIF_Q_LAUNCH(RM, ONLY)                                                                        \
+  do {                                                                                                 \
+    if (vdif_q_blocks(h, (ONLY) != nullptr))                                                           \
+      LAUNCH_LDS("vdif_q", (k_vdif_q_blk<RM>), (unsigned)((g.M + FV_VQN) / FV_VQN), 256,               \
+                 (size_t)FV_VQARR * g.KB * FV_VQN * sizeof(double), g, a, ONLY);                       \
+    else                                                                                               \
+      TLAUNCH("vdif_q", (k_vdif_q<RM, UN>), g.M + 1, g, a, a.vhpair, ONLY);                            \
+  } while (0)
+
 // UN: identical sigma columns (the kernels' UNI)
 template <typename FT, bool UN>
 void enqueue_internal_step_t(fvgpu_handle* h) {
@@ -427,7 +456,7 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     LAUNCH("zero", k_zero_int, 1, 64, h->cl_nfall, 1);
     TLAUNCH("closure_apply", k_closure_apply, g.M, g, a, h->cl_yp, a.gx, h->cl_flag, h->cl_nfall);
     TLAUNCH("fallback_q2f", k_fallback_q2f, g.M + 1, g, a, (const int*)h->cl_flag);
-#define VDIF_QM_CALL(RM) TLAUNCH("vdif_q", (k_vdif_q<RM, UN>), g.M + 1, g, a, a.vhpair, h->cl_flag)
+#define VDIF_QM_CALL(RM) VDIF_Q_LAUNCH(RM, h->cl_flag)
     // (vdif_q also stores Q2 = Q2F, Q2L = Q2LF for its columns)
     FV_RMAX_DISPATCH(g.ve_max, VDIF_QM_CALL);
   } else if (h->md->p.vertical_closure) {
@@ -436,7 +465,7 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
     P.p[0] = make_pass(a, a.q2, a.q2f, nullptr, nullptr, 0);
     P.p[1] = make_pass(b, a.q2l, a.q2lf, nullptr, nullptr, 0);
     enqueue_adv_q<FT, UN>(h, P, fct);
-#define VDIF_Q_CALL(RM) TLAUNCH("vdif_q", (k_vdif_q<RM, UN>), g.M + 1, g, a, a.vhpair, (const int*)nullptr)
+#define VDIF_Q_CALL(RM) VDIF_Q_LAUNCH(RM, (const int*)nullptr)
     // VDIF_Q, then Q2 = Q2F and Q2L = Q2LF (internal_step.F:1029-1035) in
     // the same kernel, the elimination coefficients in `vhpair`.
     FV_RMAX_DISPATCH(g.ve_max, VDIF_Q_CALL);

@@ -239,6 +239,10 @@ struct Q25Loads {
   double rho, kq, q2, q2l, km, kh, q2f, q2lf, dzz, dz, z, ur[RMAX], vr[RMAX];
 };
 
+// Columns a block of k_vdif_q_blk takes, and its arrays in LDS per level.
+#define FV_VQN 16
+#define FV_VQARR 11
+
 // VDIF_Q, MY2.5 (vdif_q.F:34-551), one thread per node column in two
 // sweeps.  The downward sweep k = 1..KB reads every node-layer value once
 // (sliding windows over RHO1 and KQ, the ring averages of U/V): it forms the
@@ -475,4 +479,193 @@ __global__ __launch_bounds__(256) void k_vdif_q(DevGrid g, IntArgs a, double2* v
       a.q2l[q] = y2;
     }
   }
+}
+
+// VDIF_Q by block of FV_VQN = 16 node columns, for meshes with too few
+// columns to fill the chip (vdif_q_blocks of the host side).  Only the two
+// eliminations are serial in the level: first all 256 lanes form the ring
+// averages of U/V, then the level quantities, PROD and the new KQ/KM/KH and
+// L, a lane for a node and every 16th level, into LDS; then one lane for each
+// node and solve runs the elimination and back-substitution on LDS; then all
+// lanes store the result.  The same operations as k_vdif_q in the same order;
+// `vhs` is not needed and VHP is not parked in Q2F/Q2LF.
+//
+// Bound: latency -- of two rounds of loads, the dependent divisions of the
+// elimination (KBM1 of them instead of about 20 KBM1) -- and with many columns
+// the instructions, which one lane per column packs better.  Channel of 3,200
+// elements x 10 layers: 44 -> 12 us; 17,000 x 20: 80 -> 23; 62,500 x 40: 174 ->
+// 113.  512 lanes a block: 109 at 62,500 x 40, but 29 at 17,000 x 20.
+template <int RMAX>
+__global__ __launch_bounds__(256) void k_vdif_q_blk(DevGrid g, IntArgs a, const int* only) {
+  constexpr int NB = FV_VQN, KL = 256 / NB;
+  enum { sKQ, sU, sV, sAK, sCK, sC1, sC2, sR1, sR2, sF1, sF2 };
+  extern __shared__ double lds[];   // FV_VQARR x KB x NB
+  __shared__ double snode[3][NB];   // L0, Q2F(KB), VHP(1) of Q2
+  const int t = (int)threadIdx.x, n = t % NB, kl = t / NB;
+  const int i0 = xcd_block() * NB + n;
+  const bool col = i0 <= g.M && (!only || only[i0]);   // column subset (the learned closure's fallback)
+  if (!__syncthreads_or(col)) return;
+  const int KB = g.KB, KBM1 = g.KBM1;
+  const double A1 = 0.92, B1 = 16.6, A2 = 0.74, B2 = 10.1, C1 = 0.08, E1 = 1.80, E2 = 1.33, SEF = 1.00;
+  const double KAPPA = 0.40, SMALL = 1.E-8, SURFL = 2.E+5;
+  double* Q2F = a.q2f; double* Q2LF = a.q2lf; double* L = a.l; double* KM = a.km; double* KH = a.kh; double* KQ = a.kq;
+  const long m1 = g.m1;
+  if (i0 == 0 && col) {
+    for (int k = kl + 1; k <= KB; k += KL) {
+      const long q = NI(g, 0, k);
+      if (k == 1 || k == KB) L[q] = 0.0;
+      const double kn0 = (k == 1 || k == KB ? 0.0 : L[q]) * sqrt(fabs(a.q2[q] + SMALL));
+      KQ[q] = 0.5 * (kn0 * KAPPA * 0.0 + KQ[q]);
+      KM[q] = 0.5 * (kn0 * 0.0 + KM[q]);
+      KH[q] = 0.5 * (kn0 * 0.0 * g.vprnu + KH[q]);
+      a.q2[q] = Q2F[q];
+      a.q2l[q] = Q2LF[q];
+    }
+  }
+  const bool act = col && i0 >= 1;
+  const int i = act ? i0 : 1;
+  auto S = [&](int v, int k) -> double& { return lds[(v * KB + (k - 1)) * NB + n]; };
+  const double dti = g.dti, umol = g.umol, d = a.d[i];
+  const int o = g.nbve_off[i], nt = g.ntve[i];
+  int re[RMAX];
+  static_for<RMAX>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    re[j] = j < nt ? g.nbve[o + j] : 0;
+  });
+  const double ntd = (double)nt;
+  auto ring_sum = [&](const double* p) {   // the ring in order, slots past it read element 0
+    double v[RMAX], x = 0.0;
+    static_for<RMAX>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      v[j] = at(p, re[j]);
+    });
+    static_for<RMAX>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if (j < nt) x = x + v[j];
+    });
+    return x;
+  };
+  if (act)
+    for (int k = kl + 1; k <= KB; k += KL) {
+      S(sKQ, k) = at(KQ + (long)(k - 1) * m1, i);
+      if (k <= KBM1) {
+        S(sU, k) = ring_sum(a.u + (long)(k - 1) * g.n1) / ntd;
+        S(sV, k) = ring_sum(a.v + (long)(k - 1) * g.n1) / ntd;
+      }
+    }
+  if (kl == KL - 1) {   // the node's own values
+    const double ramp = a.clk->ramp_int;
+    double wus = 0.0, wvs = 0.0;
+    static_for<RMAX>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const double wx = at(g.wsx, re[j]), wy = at(g.wsy, re[j]);
+      if (j < nt) {
+        wus = wus + (g.wind_on ? -wx * ramp * 0.001 : 0.0);
+        wvs = wvs + (g.wind_on ? -wy * ramp * 0.001 : 0.0);
+      }
+    });
+    wus = wus / ntd; wvs = wvs / ntd;
+    const double utau2 = sqrt(sq(wus) + sq(wvs));
+    snode[0][n] = SURFL * utau2 / g.grav_n[i];
+    const double wub = ring_sum(a.wubot) / ntd, wvb = ring_sum(a.wvbot) / ntd;
+    snode[1][n] = sqrt(sq(wub) + sq(wvb)) * g.const1;
+    snode[2][n] = g.cvhp1 * utau2;
+  }
+  const double coef4 = 18.0 * A1 * A1 + 9.0 * A1 * A2, coef5 = 9.0 * A1 * A2;
+  const double z1 = ZN(i, 1), zkb = ZN(i, KB);
+  __syncthreads();
+  const double l0 = snode[0][n], q2f_kb = snode[1][n], vhp1_1 = snode[2][n];
+  if (act)
+    for (int k = kl + 1; k <= KB; k += KL) {
+      const bool inner = k >= 2 && k <= KBM1;
+      const long ko = (long)(k - 1) * m1, kup = inner ? ko - m1 : ko;
+      const double rho_km1 = at(a.rho1 + kup, i), rho = at(a.rho1 + ko, i);
+      const double q2 = at(a.q2 + ko, i), q2l = at(a.q2l + ko, i), km = at(KM + ko, i), kh = at(KH + ko, i);
+      double q2f = at(Q2F + ko, i), q2lf = at(Q2LF + ko, i);
+      const double dzz = DZZ(i, inner ? k - 1 : 1), dz = DZ(i, inner ? k : 1), dz_km1 = DZ(i, inner ? k - 1 : 1);
+      const double zk = ZN(i, k);
+      const double kq_k = S(sKQ, k);
+      const Q25Level lv = q25_eval(g, i, k, d, l0, q2, q2l, rho_km1, rho, dzz, zk);
+      {
+        // stability functions and the under-relaxed mixing coefficients
+        const double coef1 = A2 * (1.0 - 6.0 * A1 / B1 * lv.stf);
+        const double coef2 = 3.0 * A2 * B2 / lv.stf + 18.0 * A1 * A2;
+        const double coef3 = A1 * (1.0 - 3.0 * C1 - 6.0 * A1 / B1 * lv.stf);
+        const double sh = coef1 / (1.0 - coef2 * lv.gh);
+        const double sm = (coef3 + sh * coef4 * lv.gh) / (1. - coef5 * lv.gh);
+        const double kn = lv.ll * sqrt(lv.q2);
+        const long q = ko + i;
+        KQ[q] = 0.5 * (kn * KAPPA * sm + kq_k);
+        KM[q] = 0.5 * (kn * sm + km);
+        KH[q] = 0.5 * (kn * sh * g.vprnu + kh);
+        L[q] = lv.ll;
+      }
+      if (!inner) continue;
+      // PROD (vdif_q.F:259-302)
+      const double boy = lv.boy;
+      // the reference's KM*0*x**1.5, x >= 0: zero (or NaN) whatever the power
+      double pr = km * 0.0 * (.5 * (-boy + fabs(boy)));
+      if (d > 0.0) {
+        pr = pr + km * SEF * (sq(S(sU, k) - S(sU, k - 1)) + sq(S(sV, k) - S(sV, k - 1))) / sq(dzz * d);
+        pr = pr + kh * boy;
+      }
+      // the threshold before the solves (vdif_q.F:136-145): both to SMALL
+      // if either is at or below it
+      if (q2f <= SMALL || q2lf <= SMALL) { q2f = SMALL; q2lf = SMALL; }
+      S(sAK, k) = -0.5 * dti * (S(sKQ, k + 1) + kq_k + 2.0 * umol) / (dzz * dz * d * d);
+      S(sCK, k) = -0.5 * dti * (S(sKQ, k - 1) + kq_k + 2.0 * umol) / (dzz * dz_km1 * d * d);
+      const double c1 = 2. * dti * lv.dtef + 1., r1 = -2. * dti * pr;
+      S(sC1, k) = c1;
+      S(sR1, k) = r1;
+      S(sF1, k) = q2f;
+      if (d > 0.0) {
+        const double dtef = lv.dtef * (1. + E2 * sq((1. / fabs(zk - z1) + 1. / fabs(zk - zkb)) * lv.ll / (d * KAPPA)));
+        S(sC2, k) = dti * dtef + 1.;
+        S(sR2, k) = dti * (-pr * lv.ll * E1);
+        S(sF2, k) = q2lf;
+      } else {              // D <= 0: VH/VHP keep the first solve's values
+        S(sC2, k) = c1;
+        S(sR2, k) = r1;
+        S(sF2, k) = q2f;
+      }
+    }
+  __syncthreads();
+  if (act && t < 2 * NB) {
+    const int s = t / NB;   // 0: Q2, 1: Q2L
+    double vh = 0.0, vhp = s == 0 || !(d > 0.0) ? vhp1_1 : 0.0;
+#pragma unroll 4
+    for (int k = 2; k <= KBM1; ++k) {
+      const double ak = S(sAK, k), ck = S(sCK, k);
+      const double t1 = 1. / (ak + ck * (1. - vh) - S(sC1 + s, k));
+      vhp = (S(sR1 + s, k) + ck * vhp - S(sF1 + s, k)) * t1;
+      vh = ak * t1;
+      S(sC1 + s, k) = vh;
+      S(sR1 + s, k) = vhp;
+    }
+    double x = s == 0 ? q2f_kb : Q2LF[NI(g, i, KB)];
+#pragma unroll 4
+    for (int k = KBM1; k >= 2; --k) {
+      x = S(sC1 + s, k) * x + S(sR1 + s, k);
+      S(sF1 + s, k) = x;
+    }
+    S(sF1 + s, 1) = 0.0 * x + (s == 0 ? vhp1_1 : 0.0);   // VH(1) = 0, VHP(1) of the two solves
+  }
+  __syncthreads();
+  if (act)
+    for (int k = kl + 1; k <= KB; k += KL) {
+      const long q = (long)(k - 1) * m1 + i;
+      double y1, y2;
+      if (k == KB) {
+        y1 = q2f_kb;
+        y2 = Q2LF[q];
+      } else {
+        y1 = S(sF1, k);
+        y2 = S(sF2, k);
+        if (k >= 2 && (y1 <= SMALL || y2 <= SMALL)) { y1 = SMALL; y2 = SMALL; }
+      }
+      Q2F[q] = y1;
+      Q2LF[q] = y2;
+      a.q2[q] = y1;
+      a.q2l[q] = y2;
+    }
 }

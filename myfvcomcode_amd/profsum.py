@@ -43,7 +43,7 @@ FAMILY_OF = [
     (r"k_ext_stage<\d+, \w+, false", "ext_momentum"),
     (r"k_adv_ts_gather<", "adv_ts"),
     (r"k_adv_q_gather<", "adv_q"), (r"k_vertvl_tile<", "vertvl"),
-    (r"k_viscofh_r<", "viscofh"), (r"k_vdif_q<", "vdif_q"), (r"k_vdif_uv_r<", "vdif_uv"),
+    (r"k_viscofh_r<", "viscofh"), (r"k_vdif_q(_blk)?<", "vdif_q"), (r"k_vdif_uv_r<", "vdif_uv"),
     (r"k_vdif_ts_r<", "vdif_ts"), (r"k_n2e3d\b", "n2e3d"),
     (r"k_cvrecflux<0,", "cvrecflux_ts"), (r"k_cvrecflux<1,", "cvrecflux_q"),
     (r"k_uv_blk<0,", "adv3d_blk"), (r"k_uv_blk<1,", "advuv_blk"),

@@ -29,11 +29,10 @@ def _stretched(nx=33, ny=97, kb=6):
     return m
 
 
-def _sigma_by_node():
+def _sigma_by_node(kb=8):
     """The estuary channel with a power law whose exponent varies by node."""
     import myfvcomcode_amd as F
-    m = F.Model.build(0, nx=41, ny=21, kb=8)
-    kb = m.kb
+    m = F.Model.build(0, nx=41, ny=21, kb=kb)
     p = 1.0 + 0.3 * np.sin(np.arange(m.field3("z").shape[1]) * 0.37)
     z = -((np.arange(kb) / (kb - 1.0))[:, None] ** p[None, :])
 
@@ -61,7 +60,10 @@ def _deep():
     return F.Model.build(1, nx=13, ny=9, kb=64, n_seamounts=1)
 
 
-CASES = {"stretched": _stretched, "wheel": wheel_mesh, "sigma": _sigma_by_node, "deep": _deep}
+CASES = {"stretched": _stretched, "wheel": wheel_mesh, "sigma": _sigma_by_node, "deep": _deep,
+         # up to 45 levels VDIF_Q takes blocks of columns here, past them a lane a column
+         "wheel_45": lambda: wheel_mesh(kb=45), "sigma_46": lambda: _sigma_by_node(kb=46),
+         "wheel_47": lambda: wheel_mesh(kb=47)}
 
 
 @pytest.mark.parametrize("name", list(CASES))
