@@ -713,6 +713,32 @@ int build_lists(fvgpu_handle* h) {
       std::reverse(r.begin(), r.end());   // popped from the back: first component first
       return r;
     };
+    // a range halved at the median of its longer extent: the points with
+    // their coordinates beside them, so that the selection reads memory in
+    // order; short ranges' members are copied to `idv`
+    struct Pt { double x, y; int id; };
+    auto points = [](const std::vector<int>& idv, const double* x, const double* y) {
+      std::vector<Pt> p(idv.size());
+      for (size_t q = 0; q < p.size(); ++q) p[q] = {x[idv[q]], y[idv[q]], idv[q]};
+      return p;
+    };
+    auto halve = [](std::vector<Pt>& p, std::vector<int>& idv, int lo, int hi) {
+      double x0 = p[lo].x, x1 = x0, y0 = p[lo].y, y1 = y0;
+      for (int q = lo + 1; q < hi; ++q) {
+        x0 = std::min(x0, p[q].x); x1 = std::max(x1, p[q].x);
+        y0 = std::min(y0, p[q].y); y1 = std::max(y1, p[q].y);
+      }
+      const int mid = lo + (hi - lo + 1) / 2;
+      if ((x1 - x0) >= (y1 - y0))
+        std::nth_element(p.begin() + lo, p.begin() + mid, p.begin() + hi,
+                         [](const Pt& a, const Pt& b) { return a.x < b.x || (a.x == b.x && a.id < b.id); });
+      else
+        std::nth_element(p.begin() + lo, p.begin() + mid, p.begin() + hi,
+                         [](const Pt& a, const Pt& b) { return a.y < b.y || (a.y == b.y && a.id < b.id); });
+      if (hi - lo <= 4 * FV_CVB)
+        for (int q = lo; q < hi; ++q) idv[q] = p[q].id;
+      return mid;
+    };
     std::vector<int> ids(N);
     for (int e = 1; e <= N; ++e) ids[e - 1] = e;
     std::vector<int> mark(M + 1, -1), nloc(M + 1, 0);
@@ -744,6 +770,12 @@ int build_lists(fvgpu_handle* h) {
     const int rw = (g.ring_max + 3) / 4;
     g.cvr_w = rw;
     std::vector<int> bnn, bne, bnodes, belems, stn, rnn, rnodes, rloc, loc((size_t)N + 1, 0);
+    const size_t nest = (size_t)N / 112 + 16;   // about as many blocks
+    bnodes.reserve(nest * FV_CVB);
+    belems.reserve(nest * FV_CVB);
+    stn.reserve(nest * FV_CVB);
+    rnodes.reserve(nest * FV_CVH);
+    rloc.reserve(nest * rw * FV_CVB);
     std::vector<char> seen(M + 1, 0);
     auto add_block = [&](int lo, int hi) {
       if (hi - lo > FV_CVB || !tile_fits(lo, hi)) return false;
@@ -796,20 +828,13 @@ int build_lists(fvgpu_handle* h) {
       return true;
     };
     std::vector<std::pair<int, int>> stack = component_ranges(ids, ecomp);
+    std::vector<Pt> pts = points(ids, md->xc, md->yc);
     while (!stack.empty()) {
       const std::pair<int, int> r = stack.back();
       stack.pop_back();
-      const int lo = r.first, hi = r.second, n = hi - lo;
+      const int lo = r.first, hi = r.second;
       if (add_block(lo, hi)) continue;
-      double x0 = md->xc[ids[lo]], x1 = x0, y0 = md->yc[ids[lo]], y1 = y0;
-      for (int q = lo + 1; q < hi; ++q) {
-        const double x = md->xc[ids[q]], y = md->yc[ids[q]];
-        x0 = std::min(x0, x); x1 = std::max(x1, x); y0 = std::min(y0, y); y1 = std::max(y1, y);
-      }
-      const double* key = (x1 - x0) >= (y1 - y0) ? md->xc : md->yc;
-      const int mid = lo + (n + 1) / 2;
-      std::nth_element(ids.begin() + lo, ids.begin() + mid, ids.begin() + hi,
-                       [&](int a, int b) { return key[a] < key[b] || (key[a] == key[b] && a < b); });
+      const int mid = halve(pts, ids, lo, hi);
       stack.push_back({mid, hi});
       stack.push_back({lo, mid});
     }
@@ -839,21 +864,14 @@ int build_lists(fvgpu_handle* h) {
         return n;
       };
       std::vector<std::pair<int, int>> st = component_ranges(nids, ncompv), tl;
+      pts = points(nids, md->vx, md->vy);
       while (!st.empty()) {
         const std::pair<int, int> r = st.back();
         st.pop_back();
         const int lo = r.first, hi = r.second, n = hi - lo;
         if (n <= FV_NTN && elems_around(lo, hi) <= FV_NTE) { tl.push_back(r); continue; }
         if (n == 1) return fail("a node has more elements around it than a node tile holds");
-        double x0 = md->vx[nids[lo]], x1 = x0, y0 = md->vy[nids[lo]], y1 = y0;
-        for (int q = lo + 1; q < hi; ++q) {
-          const double x = md->vx[nids[q]], y = md->vy[nids[q]];
-          x0 = std::min(x0, x); x1 = std::max(x1, x); y0 = std::min(y0, y); y1 = std::max(y1, y);
-        }
-        const double* key = (x1 - x0) >= (y1 - y0) ? md->vx : md->vy;
-        const int mid = lo + (n + 1) / 2;
-        std::nth_element(nids.begin() + lo, nids.begin() + mid, nids.begin() + hi,
-                         [&](int a, int b) { return key[a] < key[b] || (key[a] == key[b] && a < b); });
+        const int mid = halve(pts, nids, lo, hi);
         st.push_back({mid, hi});
         st.push_back({lo, mid});
       }

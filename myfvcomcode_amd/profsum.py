@@ -46,7 +46,7 @@ FAMILY_OF = [
     (r"k_viscofh_r<", "viscofh"), (r"k_vdif_q(_blk)?<", "vdif_q"), (r"k_vdif_uv_r<", "vdif_uv"),
     (r"k_vdif_ts_r<", "vdif_ts"), (r"k_n2e3d\b", "n2e3d"),
     (r"k_cvrecflux<0,", "cvrecflux_ts"), (r"k_cvrecflux<1,", "cvrecflux_q"),
-    (r"k_uv_blk<0,", "adv3d_blk"), (r"k_uv_blk<1,", "advuv_blk"),
+    (r"k_uv_blk<0,", "adv3d_blk"), (r"k_uv_blk<1,", "advuv_blk"), (r"k_step_end\b", "step_end"),
 ]
 
 
