@@ -182,7 +182,7 @@ def main():
         "config": {"workload": "FVCOM INTERNAL_STEP, %dx%d-node jittered mesh, %d elements x %d layers, "
                                "DTE=2 s ISPLIT=10, MY2.5, plain FP64" % (args.nx, args.ny, n, kbm1),
                    "elements": n, "layers": kbm1, "dti_s": dti,
-                   "mode": "eager launches, independent chains on two streams"},
+                   "mode": "eager launches"},
         "elem_layer_steps_per_s": rate,
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": pk["achieved_GBps"], "peak": PEAK_HBM / 1e9,
                      "unit": "GB/s", "frac": pk["frac"], "traffic": traffic,

@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) void k_stage_tables(DevGrid g, StageTab st, co
 }
 
 // One 2-D stage by element tile.  A workgroup of 256 lanes takes a compact
-// tile of at most 128 elements (DevGrid::ub_tile; its nodes in st_nodes) and
+// tile of at most 128 elements (DevGrid::ub_tile, cvb_*) and
 // does the whole stage for it, so that neither the edge terms nor the new
 // elevation cross HBM between launches:
 //   1. lanes 0, 1, ..: the least-squares velocity gradients of the tile's
@@ -321,9 +321,9 @@ __global__ __launch_bounds__(256) void k_stage_tables(DevGrid g, StageTab st, co
 // base elevation from a copy (stage 4 writes over the base).
 //
 // Bound: on a large mesh HBM (1,000,000 elements in FP64: 622 MB a stage,
-// 151 us, 4.1 TB/s; as separate elevation, edge and momentum kernels 196 us,
+// 147 us, 4.2 TB/s; as separate elevation, edge and momentum kernels 196 us,
 // 180 with the first two side by side), on a small one the launches and the
-// dependent loads of one tile (3,200 elements: 21 -> 8 us a stage).  The
+// dependent loads of one tile (3,200 elements: 21 -> 9 us a stage).  The
 // constants come in block order because gathering them by index had every
 // tile wait for one more load and fetch rows of partly used lines (206 ->
 // 164 us); the own elements' data is loaded after the node part, so that
