@@ -1325,11 +1325,13 @@ int fvgpu_internal_step(fvgpu_handle* h) {
 int fvgpu_external_step(fvgpu_handle* h, int32_t iext) {
   // the clock as INTERNAL_STEP would set it for IINT+1, then one EXTERNAL_STEP
   enqueue_external_step(h, iext);
+  const hipError_t launched = hipGetLastError();
   // restore IINT (this call does not complete an internal step)
   DevClock c;
   HIPCHK(h->stage.to_host(&c, h->clk, sizeof(c), h->stream, h->device));
   c.iint -= 1;
   HIPCHK(h->stage.to_device(h->clk, &c, sizeof(c), h->stream, h->device));
+  HIPCHK(launched);
   return 0;
 }
 
@@ -1621,6 +1623,7 @@ extern "C" int fvgpu_diagnostics(fvgpu_handle* h, fv_diag* out) {
   const int nblk = 256;
   DiagAcc* part = (DiagAcc*)h->diag_part;
   hipLaunchKernelGGL(k_diag_partial, dim3(nblk), dim3(256), 0, h->stream, h->g, h->ia, part);
+  HIPCHK(hipGetLastError());
   std::vector<DiagAcc> hp(nblk);
   HIPCHK(h->stage.to_host(hp.data(), part, sizeof(DiagAcc) * nblk, h->stream, h->device));
   DevClock c;

@@ -49,9 +49,18 @@ class HostStage {
   char *small_ = nullptr, *large_ = nullptr;
   std::mutex mu_;   // the staging serves one copy at a time
 
+  // Clears the error of a call whose failure is an answer here -- unless an
+  // error was pending before it, as that of a launch, which the caller has yet
+  // to report.
+  static void answered(hipError_t pending) {
+    if (pending == hipSuccess) (void)hipGetLastError();
+  }
+
   static bool pinned(char*& p, size_t n) {
-    if (!p && hipHostMalloc((void**)&p, n, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();   // no staging: the caller copies directly
+    if (p) return true;
+    const hipError_t pending = hipPeekAtLastError();
+    if (hipHostMalloc((void**)&p, n, hipHostMallocDefault) != hipSuccess) {
+      answered(pending);   // no staging: the caller copies directly
       p = nullptr;
     }
     return p != nullptr;
@@ -63,8 +72,10 @@ class HostStage {
     if (n == 0) return hipStreamSynchronize(stream);
     // memory the runtime knows (pinned, or the device's) needs no staging
     hipPointerAttribute_t at_{};
-    const bool known = hipPointerGetAttributes(&at_, host) == hipSuccess && at_.type != hipMemoryTypeUnregistered;
-    if (!known) (void)hipGetLastError();
+    const hipError_t pending = hipPeekAtLastError();
+    const hipError_t asked = hipPointerGetAttributes(&at_, host);
+    if (asked != hipSuccess) answered(pending);
+    const bool known = asked == hipSuccess && at_.type != hipMemoryTypeUnregistered;
     std::unique_lock<std::mutex> lock(mu_, std::defer_lock);
     if (!known) lock.lock();
     if (!known && n <= SMALL && pinned(small_, SMALL)) {
