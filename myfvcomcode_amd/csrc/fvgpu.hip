@@ -1398,6 +1398,7 @@ int ens_update(fvgpu_handle* h, const char* name, int32_t nrens, const int64_t* 
   const int64_t* off = node ? node_off : elem_off;
   const size_t ls = node ? m1 : n1;
   if (len < 1) return fail("ensemble update: empty member slice");
+  if (!x5 || !off) return fail("ensemble update: null argument");
   for (int i = 0; i < nrens; ++i)
     if (off[i] < 0 || (size_t)(off[i] + len + 1) > ls) return fail("ensemble update: member slice outside the array");
   if (!stage) {
@@ -1457,6 +1458,7 @@ int fvgpu_set_forcing(fvgpu_handle* h, const char* name, const double* host, int
   if (n == "wind") {
     if (!h->md->p.wind_on) return fail("the model was created without wind");
     if ((size_t)len != 2 * n1) return fail("wind: expected UUWIND then VVWIND, 2*(N+1) values");
+    if (!host) return fail("wind: null argument");
     const bool varies =
         !h->wind_varies && std::memcmp(h->wind_end.data(), host, 2 * n1 * sizeof(double)) != 0;
     // the new speeds (by way of the external steps' stress buffers, which
@@ -1816,6 +1818,7 @@ int32_t fvmlp_nparams(void) { return MLP_NPARAM; }
 
 int fvmlp_grad(fvmlp* t, const int32_t* idx, int32_t B, float* grad, float* loss) {
   if (B < 1 || B > t->bmax) return fail("fvmlp_grad: batch size outside [1, bmax]");
+  if (!grad) return fail("fvmlp_grad: null argument");
   const int* didx = nullptr;
   if (idx) {
     for (int b = 0; b < B; ++b)

@@ -70,6 +70,7 @@ class HostStage {
   // the device or down to the host
   hipError_t copy(char* host, char* dev, size_t n, bool up, hipStream_t stream, int device) {
     if (n == 0) return hipStreamSynchronize(stream);
+    if (!host || !dev) return hipErrorInvalidValue;
     // memory the runtime knows (pinned, or the device's) needs no staging
     hipPointerAttribute_t at_{};
     const hipError_t pending = hipPeekAtLastError();

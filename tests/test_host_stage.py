@@ -119,6 +119,51 @@ def test_copies_and_pending_errors(tmp_path):
 """)
 
 
+def test_null_host_memory_is_refused(tmp_path):
+    _run(tmp_path, r"""
+  for (size_t n : sizes) {
+    HostStage st;
+    std::vector<char> dev(n);
+    CHECK(st.to_device(dev.data(), nullptr, n, nullptr, 0) == hipErrorInvalidValue);
+    CHECK(st.to_host(nullptr, dev.data(), n, nullptr, 0) == hipErrorInvalidValue);
+    CHECK(st.to_host(nullptr, dev.data(), 0, nullptr, 0) == hipSuccess);
+    st.release();
+  }
+""")
+
+
+@pytest.mark.gpu
+def test_null_arguments_are_errors(built):
+    """Null host memory at the entry points that copy: an error, whatever the
+    size, and the handle goes on."""
+    import numpy as np
+    import myfvcomcode_amd as F
+    L = F.gpu_lib()
+    m = F.Model.build(1, nx=181, ny=121, kb=12, n_seamounts=1)   # T1 above the size that is copied by chunks
+    m.set_river(5, 1.0)
+    dev = F.DeviceModel(m)
+    dev.run(1)
+    print("case: null host memory", flush=True)
+    for n in ("el", "t1"):
+        k = len(dev.get(n))
+        assert L.fvgpu_get_state(dev._h, n.encode(), None, k) != 0
+        assert L.fvgpu_put_state(dev._h, n.encode(), None, k) != 0
+    assert L.fvgpu_set_forcing(dev._h, b"wind", None, 2 * (m.n + 1)) != 0
+    assert L.fvgpu_set_forcing(dev._h, b"tdis", None, 1) != 0
+    off = np.zeros(2, np.int64)
+    assert L.fvgpu_ensemble_update(dev._h, b"el", 2, off.ctypes.data, off.ctypes.data, 2, 2, None) != 0
+    assert L.fvgpu_ensemble_update(dev._h, b"el", 2, None, None, 2, 2, off.ctypes.data) != 0
+    t = F.Trainer(np.ones((64, 8), np.float32), np.ones((64, 2), np.float32), bmax=64)
+    assert L.fvmlp_set_params(t._h, None) != 0
+    t.set_params(np.zeros(L.fvmlp_nparams(), np.float32))
+    assert L.fvmlp_get_params(t._h, None) != 0
+    assert L.fvmlp_grad(t._h, None, 64, None, None) != 0
+    assert L.fvmlp_infer(t._h, 0, 64, 1, None) != 0
+    assert np.isfinite(t.grad(batch=64)[1]).all()
+    dev.run(1)
+    assert dev.diagnostics().iint == 2
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("call", ["external_step", "diagnostics"])
 def test_launch_error_is_reported(built, call):
