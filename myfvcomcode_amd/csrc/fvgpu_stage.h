@@ -16,10 +16,9 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 class HostStage {
  public:
@@ -90,23 +89,23 @@ class HostStage {
     if (!known && n > SMALL && pinned(large_, 2 * CHUNK * THREADS)) {
       // chunks small enough that every thread has some
       const size_t chunk = std::min(CHUNK, std::max<size_t>(CHUNK / 4, n / (2 * THREADS) / 4096 * 4096));
-      std::vector<hipError_t> err(THREADS, hipSuccess);
-      std::vector<std::thread> helpers;
+      hipError_t err[THREADS] = {};
+      std::thread helpers[THREADS];
       int started = 1;
       // lane j of `lanes` takes the chunks j, j + lanes, ...: fixed before
       // the first helper starts, so a helper that cannot be started leaves
       // its chunks to the caller
       auto lane = [&](int j) { err[j] = run_lane(host, dev, n, chunk, j, THREADS, up, stream, device); };
       try {
-        for (; started < THREADS; ++started) helpers.emplace_back(lane, started);
-      } catch (const std::system_error&) {
+        for (; started < THREADS; ++started) helpers[started] = std::thread(lane, started);
+      } catch (const std::exception&) {   // no thread, or no memory for one
       }
       int here = device;
       (void)hipGetDevice(&here);
       lane(0);
       for (int j = started; j < THREADS; ++j) lane(j);
       if (here != device) (void)hipSetDevice(here);
-      for (std::thread& t : helpers) t.join();
+      for (int j = 1; j < started; ++j) helpers[j].join();
       for (hipError_t e : err)
         if (e != hipSuccess) return e;
       return hipStreamSynchronize(stream);

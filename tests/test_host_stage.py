@@ -68,6 +68,16 @@ inline hipError_t hipEventDestroy(hipEvent_t e) { std::free(e); __atomic_sub_fet
 MAIN = r"""
 #include "fvgpu_stage.h"
 #include <cstdio>
+#include <new>
+#include <vector>
+thread_local int news = -1;   // allocations of this thread that succeed before one fails; -1: all
+void* operator new(size_t n) {
+  if (news >= 0 && news-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
 static const size_t sizes[] = {8, HostStage::SMALL, HostStage::SMALL + 1, 40u << 20};
 static std::vector<char> bytes(size_t n) {
@@ -129,6 +139,27 @@ def test_null_host_memory_is_refused(tmp_path):
     CHECK(st.to_host(nullptr, dev.data(), 0, nullptr, 0) == hipSuccess);
     st.release();
   }
+""")
+
+
+def test_no_memory_for_the_helpers(tmp_path):
+    """A copy whose helper threads cannot be had is done by the caller; no
+    exception leaves it, whichever allocation fails."""
+    _run(tmp_path, r"""
+  for (size_t n : sizes)
+    for (int k = 0; k < 6; ++k) {
+      HostStage st;
+      std::vector<char> a = bytes(n), dev(n), b(n);
+      news = k;
+      const hipError_t up = st.to_device(dev.data(), a.data(), n, nullptr, 0);
+      news = k;
+      const hipError_t down = st.to_host(b.data(), dev.data(), n, nullptr, 0);
+      news = -1;
+      CHECK(up == hipSuccess && down == hipSuccess);
+      CHECK(a == dev && a == b);
+      st.release();
+      CHECK(live == 0);
+    }
 """)
 
 
