@@ -184,23 +184,26 @@ __device__ __forceinline__ double ext_node_update(const DevGrid& g, const ExtArg
   return elrk - dtk * xflux / art1;
 }
 
-// The open-boundary condition of OBC node i (index obc): its elevation from
-// the unconstrained one.  1/2: BCOND_ASL (mod_obcs.F:552-582), then the RK
-// blend (external_step.F:262-266); 3/4: BCOND_ASL_CLP (mod_obcs.F:599-617);
-// 5/6: BCOND_GWI (mod_obcs.F:624-658) and 7/8: BCOND_BKI (mod_obcs.F:665-699)
-// from the new elevation el2 of the interior neighbour NEXT_OBC; 9/10:
-// BCOND_ORE (mod_obcs.F:706-737) from the stage input EL and the elevations
-// ELM1/ELM2 one and two stages back.
-__device__ __forceinline__ double ext_obc_value(const DevGrid& g, const ExtArgs& a, int i, int obc, int ty,
-                                                double elrk, double elf, double el2) {
-  if (ty <= 2) {
-    if (g.obc_elev) {
-      const double rk_time = a.ec->time + g.dte * (a.alpha - 1.0);
-      elf = tide_force(g, obc, rk_time, a.ec->ramp);
-    }
-    return elrk + a.alpha * (elf - elrk);
+// The elevation of OBC node `obc` of TYPE_OBC 1..4 from the unconstrained
+// one.  1/2: BCOND_ASL (mod_obcs.F:552-582), then the RK blend
+// (external_step.F:262-266); 3/4: BCOND_ASL_CLP (mod_obcs.F:599-617).
+__device__ __forceinline__ double ext_obc_given(const DevGrid& g, const ExtArgs& a, int obc, int ty, double elrk,
+                                                double elf) {
+  if (ty > 2) return 0.0;
+  if (g.obc_elev) {
+    const double rk_time = a.ec->time + g.dte * (a.alpha - 1.0);
+    elf = tide_force(g, obc, rk_time, a.ec->ramp);
   }
-  if (ty <= 4) return 0.0;
+  return elrk + a.alpha * (elf - elrk);
+}
+
+// The open-boundary condition of OBC node i (index obc) of TYPE_OBC 5..10.
+// 5/6: BCOND_GWI (mod_obcs.F:624-658) and 7/8: BCOND_BKI (mod_obcs.F:665-699)
+// from the new elevation el2 of the neighbour NEXT_OBC; 9/10: BCOND_ORE
+// (mod_obcs.F:706-737) from the stage input EL and the elevations ELM1/ELM2
+// one and two stages back.
+__device__ __forceinline__ double ext_obc_radiated(const DevGrid& g, const ExtArgs& a, int i, int obc, int ty,
+                                                   double elrk, double el2) {
   if (ty >= 9) {
     const int i2 = g.next_obc[obc], i3 = g.next_obc2[obc];
     const double cl = (a.elm2[i2] - a.cur.el[i2]) / (a.cur.el[i2] + a.elm2[i2] - 2.0 * a.elm1[i3]);
@@ -426,21 +429,24 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
       const double elrk = at(a.elrk, j);
       if (keep && a.elrk_copy) a.elrk_copy[j] = elrk;
       const int ty = obc >= 0 ? g.type_obc[obc] : 0;
-      // GWI / BKI need their interior neighbour's new elevation: a second
-      // pass forms it, as the tile that has that node does
+      // GWI / BKI need their neighbour's new elevation: a second pass forms
+      // it, as the tile that has that node does.  The grid's NEXT_OBC are
+      // interior nodes; one that a host has set to an OBC node of TYPE_OBC
+      // 1..4 enters with its given elevation.
       double elf = 0.0, el2 = 0.0, xobc = 0.0;
-      int id = j, rv = nd.w;
+      int id = j, rv = nd.w, ob = obc;
       double ar = art1, er = elrk;
       if (n0)
         static_for<SMAX>([&](auto jc) { ce[decltype(jc)::value] = 0; });
       for (bool next = false;;) {
         double xo;
-        const double e = ext_node_update<SMAX>(g, a, id, ce, rv, !next && obc >= 0, ar, er, xo);
+        const double e = ext_node_update<SMAX>(g, a, id, ce, rv, ob >= 0, ar, er, xo);
         if (next) { el2 = e; break; }
         elf = e;
         xobc = xo;
         if (ty < 5 || ty > 8) break;
         id = g.next_obc[obc];
+        ob = g.node_obc[id];
         static_for<SMAX>([&](auto jc) {
           constexpr int q = decltype(jc)::value;
           ce[q] = q < st.nslot ? g.cvl_ent[(long)q * g.m1 + id] : 0;
@@ -450,7 +456,16 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
         next = true;
       }
       if (obc >= 0) {
-        elf = ext_obc_value(g, a, j, obc, ty, elrk, elf, el2);
+        // the given elevation: the node's own, or that of the neighbour which
+        // it radiates from
+        const bool own = ty < 5;
+        const int ty2 = own ? ty : ob >= 0 ? g.type_obc[ob] : 5;
+        if (ty2 < 5) {
+          const double e = ext_obc_given(g, a, ob, ty2, er, own ? elf : el2);
+          if (own) elf = e;
+          else el2 = e;
+        }
+        if (!own) elf = ext_obc_radiated(g, a, j, obc, ty, elrk, el2);
         // FLUX_OBN's flux defect (mod_obcs.F:1196) and, in the last stage,
         // the node's UARD_OBCN share (external_step.F:423-430)
         if (nact) s_fobn[tn] = -(elf - elrk) * art1 / (a.alpha * g.dte) - xobc;
