@@ -1017,8 +1017,6 @@ int build_lists(fvgpu_handle* h) {
     }
     if (upload_blocks(g.ub_run)) return 1;
     if (build_blocks(tile_own) > 256) return fail("an element tile exceeds the blocked momentum kernels' records");
-    for (int c = 1; c <= NE; ++c)
-      if (md->isbc[c] < 0 || md->isbc[c] > 2) return fail("ISBC outside 0..2");
     if (upload_blocks(g.ub_tile)) return 1;
     // the 2-D stage's tables, filled on the device
     const size_t nt = tile_own.size();

@@ -40,14 +40,15 @@ struct UvBlocks {
 //                    another element, INT_MIN for a pad
 //   edge[256*b + t]  the record slots of IA and IB in bits 0-7 and 8-15, the
 //                    node slots of IENODE in bits 16-22 and 23-29, ISBC in
-//                    bits 30-31; all ones for a pad
+//                    bits 30-31 (3: not 0..2, read it); all ones for a pad
 //   egeo[(6*b + q)*256 + t]  XIJC-XC and YIJC-YC of IA, the same of IB,
 //                    DLTXC, DLTYC
 //   node[FV_CVB*b + t]  {2*node + 1 in the first block that has it, 0, OBC
 //                    index or -1, river index or -1}, x = -1 for a pad
 //   list[(nslot*b + j)*FV_CVB + t]  the node's cvl_ent list
 //   nd[(2*b + q)*FV_CVB + t]  ART1, H
-//   elem[FV_CVB*b + t]  {epos, cvb_loc, ISBCE + 4 if it has rivers, IUCP}
+//   elem[FV_CVB*b + t]  {epos, cvb_loc, ISBCE (0 where it is not 0..3) + 4
+//                    if it has rivers, IUCP}
 //   ed[(12*b + q)*FV_CVB + t]  EPOR, GRAV_E, ART, COR, H1, CC_SPONGE, DLTXE
 //                    and DLTYE of the three sub-edges
 // a12, art and cc_hvc are DevGrid's.

@@ -264,7 +264,8 @@ __global__ __launch_bounds__(256) void k_stage_tables(DevGrid g, StageTab st, co
   double v[6] = {};
   if (t < B.ne[b]) {
     const int c = B.edges[256 * b + t], ia = IEC_(c, 1), ib = IEC_(c, 2);
-    pl = (unsigned)B.eloc[256 * b + t] | (unsigned)g.isbc[c] << 30;
+    const int isbc = g.isbc[c];
+    pl = (unsigned)B.eloc[256 * b + t] | (unsigned)(isbc >= 0 && isbc <= 2 ? isbc : 3) << 30;
     // the edge's nodes are nodes of whichever of its elements the tile owns
     const int sa = pl & 255, sb = (pl >> 8) & 255;
     const int e = B.elems[256 * b + (sa < nown ? sa : sb)], loc = g.cvb_loc[e];
@@ -290,8 +291,9 @@ __global__ __launch_bounds__(256) void k_stage_tables(DevGrid g, StageTab st, co
   st.nd[(2 * b + 1) * FV_CVB + t] = nact ? g.h[i] : 0.0;
   const bool oact = t < nown;
   const int e = oact ? B.elems[256 * b + t] : 0;
+  const int isbce = g.isbce[e] >= 0 && g.isbce[e] <= 3 ? g.isbce[e] : 0;
   st.elem[FV_CVB * b + t] = oact ? make_int4(B.epos[e], g.cvb_loc[e],
-                                             (g.isbce[e] & 3) | (g.re_off[e] < g.re_off[e + 1] ? 4 : 0), g.iucp[e])
+                                             isbce | (g.re_off[e] < g.re_off[e + 1] ? 4 : 0), g.iucp[e])
                                  : make_int4(0, 0, 0, 0);
   double w[12] = {};
   if (oact) {
@@ -532,7 +534,8 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     sf.elij[t] = 0.5 * (s_el[n1] + s_el[n2]);
     sf.dlx[t] = eg[4];
     sf.dly[t] = eg[5];
-    sf.isbc[t] = (int)(pl >> 30);
+    const int isbc = (int)(pl >> 30);
+    sf.isbc[t] = isbc < 3 ? isbc : g.isbc[g.ub_tile.edges[256L * b + t]];
   }
   __syncthreads();
   if (!oact) return;

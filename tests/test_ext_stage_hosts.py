@@ -38,3 +38,18 @@ def test_next_obc_is_an_obc_node(built, radiating):
     m = _model([3, radiating, 4])
     m.field("next_obc")[1::3] = m.field("i_obc_n")[0::3][:len(m.field("next_obc")[1::3])]
     _parity(m, "TYPE_OBC %d beside 3" % radiating)
+
+
+def test_boundary_marks_of_any_value(built):
+    """ISBC enters the edge terms as a number; an ISBCE other than 1, 2 and 3
+    marks nothing."""
+    m = _model([1])
+    rng = np.random.default_rng(4)
+    c = rng.permutation(np.arange(1, m.hdr.ne + 1))
+    for k, v in enumerate((3, -1, 7, 4, 2)):
+        m.field("isbc")[c[40 * k:40 * (k + 1)]] = v
+    e = rng.permutation(np.flatnonzero(m.field("isbce")[1:] == 0) + 1)
+    for k, v in enumerate((4, 5, 6, 7, -2, -1)):
+        m.field("isbce")[e[20 * k:20 * (k + 1)]] = v
+    dev = _parity(m, "ISBC and ISBCE of any value")
+    assert np.isfinite(dev.get("ua")).all()
