@@ -350,6 +350,7 @@ void enqueue_external_step_t(fvgpu_handle* h, int iext, const ExtClock* ec) {
   const Ext2DState* nxt[5] = {nullptr, &h->ext[1], &h->ext[2], &h->ext[1], &h->ext[0]};
   for (int K = 1; K <= 4; ++K) {
     ExtArgs a = make_ext_args(h, K, *cur[K], *nxt[K], ec);
+    if (g.fobn) LAUNCH("ext_fobn", k_ext_fobn, nb(g.IOBCN), 256, h->dg, a);
 #define EXT_STAGE_CALL(SM) LAUNCH("ext_momentum", (k_ext_stage<SM, FT, false>), g.ub_tile.nblk, 256, h->dg, a)
     FV_SMAX_DISPATCH(g.cv_max, EXT_STAGE_CALL);
     if (g.obc_ore) LAUNCH("elm_shift", k_elm_shift, nb(g.M + 1), 256, g, a);
@@ -629,11 +630,12 @@ int build_lists(fvgpu_handle* h) {
     if (md->nadjc_obc[i] > 0) fo.push_back({md->adjc_obc[i], (i << 1) | 0});
     if (md->nadjc_obc[i] > 1) fo.push_back({md->adjc_obc[(size_t)IOBCN + i], (i << 1) | 1});
   }
+  bool far = false;   // a contribution goes to an element that does not have the node
   for (const auto& [e, x] : fo) {
     const int j = md->i_obc_n[x >> 1];
-    if (md->nv[e] != j && md->nv[(size_t)N + 1 + e] != j && md->nv[2 * ((size_t)N + 1) + e] != j)
-      return fail("an OBC node's adjacent cell does not have the node");
+    far = far || (md->nv[e] != j && md->nv[(size_t)N + 1 + e] != j && md->nv[2 * ((size_t)N + 1) + e] != j);
   }
+  if (far && dalloc(h, &g.fobn, (size_t)IOBCN)) return 1;
   // CSR over elements 0..N of (element, entry) pairs, each element's entries in their order
   auto element_csr = [&](std::vector<std::pair<int, int>>& v, std::vector<int>& off, std::vector<int>& ent_) {
     std::stable_sort(v.begin(), v.end(), [](const auto& p, const auto& q) { return p.first < q.first; });

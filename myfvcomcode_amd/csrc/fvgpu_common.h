@@ -143,6 +143,7 @@ struct DevGrid {
   const int *next_obc2;
   int obc_radiate;                 // some OBC node has TYPE_OBC 5..10
   int obc_ore;                     // some OBC node has TYPE_OBC 9/10 (Orlanski)
+  double* fobn;                    // the OBC nodes' flux defects where k_ext_fobn forms them, else null
   const double *fluxf_obc, *dltn_obc, *emean, *apt, *phai, *period;
   const int *inodeq;               // node river: its node, else 0
   const int *icellq, *n_icellq;    // edge river: its cell and the two nodes of its solid edge, else 0

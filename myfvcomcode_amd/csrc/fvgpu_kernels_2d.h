@@ -218,6 +218,34 @@ __device__ __forceinline__ double ext_obc_radiated(const DevGrid& g, const ExtAr
   return ty <= 6 ? (cc * el2 + elrk) / cp : (cc * el2 + elrk * (1.0 - g.dte / 10800.0)) / cp;
 }
 
+// FLUX_OBN's flux defect (mod_obcs.F:1196) of every OBC node, as k_ext_stage
+// forms it, for a mesh on which an element that it goes to does not have the
+// node, so that the node's tile cannot hand it over (the grid's ADJC_OBC are
+// cells around the node; a host may set others).  One thread per OBC node,
+// before the stage.
+__global__ void k_ext_fobn(const DevGrid* __restrict__ gp, ExtArgs a) {
+  const DevGrid& g = *gp;
+  const int obc = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (obc >= g.IOBCN) return;
+  auto update = [&](int i, int ob, double& xobc) {
+    int ce[FV_MAX_CV];
+    static_for<FV_MAX_CV>([&](auto jc) {
+      constexpr int q = decltype(jc)::value;
+      ce[q] = q < g.cv_max ? g.cvl_ent[(long)q * g.m1 + i] : 0;
+    });
+    const double e = ext_node_update<FV_MAX_CV>(g, a, i, ce, g.node_riv[i], ob >= 0, g.art1[i], a.elrk[i], xobc);
+    const int ty = ob >= 0 ? g.type_obc[ob] : 5;
+    return ty < 5 ? ext_obc_given(g, a, ob, ty, a.elrk[i], e) : e;
+  };
+  const int j = g.i_obc_n[obc], ty = g.type_obc[obc];
+  const double elrk = a.elrk[j];
+  double xobc, x2, el2 = 0.0;
+  double elf = update(j, obc, xobc);
+  if (ty >= 5 && ty <= 8) el2 = update(g.next_obc[obc], g.node_obc[g.next_obc[obc]], x2);
+  if (ty >= 5) elf = ext_obc_radiated(g, a, j, obc, ty, elrk, el2);
+  g.fobn[obc] = -(elf - elrk) * g.art1[j] / (a.alpha * g.dte) - xobc;
+}
+
 // ASSIGN_ELM1_TO_ELM2 (mod_obcs.F:178-199) at the end of a stage
 // (external_step.F:333): ELM2 = ELM1, ELM1 = the stage input EL.  Run
 // after k_ext_stage, the only reader; launched only when Orlanski nodes exist.
@@ -549,9 +577,9 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     } else {
       for (int p = g.fo_off[i]; p < g.fo_off[i + 1]; ++p) {
         const int ent = g.fo_obc[p], ob = ent >> 1, slot = ent & 1;
-        const int j = g.i_obc_n[ob];   // one of the element's nodes
+        const int j = g.i_obc_n[ob];   // one of the element's nodes, or g.fobn has it
         const int ln = j == NV_(i, 1) ? nl & 255 : j == NV_(i, 2) ? (nl >> 8) & 255 : (nl >> 16) & 255;
-        fl = fl + g.fluxf_obc[(long)slot * g.IOBCN + ob] * s_fobn[ln];
+        fl = fl + g.fluxf_obc[(long)slot * g.IOBCN + ob] * (g.fobn ? g.fobn[ob] : s_fobn[ln]);
       }
       a.fluxobn[i] = fl;
     }

@@ -53,3 +53,14 @@ def test_boundary_marks_of_any_value(built):
         m.field("isbce")[e[20 * k:20 * (k + 1)]] = v
     dev = _parity(m, "ISBC and ISBCE of any value")
     assert np.isfinite(dev.get("ua")).all()
+
+
+@pytest.mark.parametrize("types", [[1], [5, 2, 8, 3, 9]])
+def test_flux_to_a_cell_without_the_node(built, types):
+    """OBC nodes whose flux defects go to boundary cells elsewhere (each
+    node's cells exchanged with those of the node across the boundary)."""
+    m = _model(types)
+    adjc = m.field("adjc_obc").reshape(2, -1)
+    adjc[:, 1:-1] = adjc[:, 1:-1][:, ::-1].copy()
+    assert (m.field("isbce")[adjc[adjc > 0]] == 2).any()
+    _parity(m, "TYPE_OBC %s, cells exchanged" % types)
