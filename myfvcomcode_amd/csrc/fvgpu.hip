@@ -94,6 +94,7 @@ struct fvgpu_handle {
   // internal step; once they differ, every external step forms its own
   // stress (ws2x, ws2y), otherwise it uses the end stress g.wsx/g.wsy
   double *wu0 = nullptr, *wv0 = nullptr, *wu1 = nullptr, *wv1 = nullptr, *ws2x = nullptr, *ws2y = nullptr;
+  double* wnew = nullptr;   // new speeds on their way into wu1 and wv1
   int wind_varies = 0;
   std::vector<double> wind_end;   // wu1 then wv1, kept on the host until the wind first varies
   DevGrid g{};
@@ -1136,7 +1137,7 @@ int upload_grid(fvgpu_handle* h) {
       if (dupload(h, &src, w0s[q], n1)) return 1;
       *dst[q] = (double*)src;
     }
-    if (dalloc(h, &h->ws2x, n1) || dalloc(h, &h->ws2y, n1)) return 1;
+    if (dalloc(h, &h->ws2x, n1) || dalloc(h, &h->ws2y, n1) || dalloc(h, &h->wnew, 2 * n1)) return 1;
     h->wind_varies = std::memcmp(md->uuwind0, md->uuwind, n1 * sizeof(double)) != 0 ||
                      std::memcmp(md->vvwind0, md->vvwind, n1 * sizeof(double)) != 0;
     if (!h->wind_varies) {
@@ -1461,13 +1462,12 @@ int fvgpu_set_forcing(fvgpu_handle* h, const char* name, const double* host, int
     if (!host) return fail("wind: null argument");
     const bool varies =
         !h->wind_varies && std::memcmp(h->wind_end.data(), host, 2 * n1 * sizeof(double)) != 0;
-    // the new speeds (by way of the external steps' stress buffers, which
-    // every external step fills again) become the end of the coming step,
-    // the previous end its start
-    HIPCHK(h->stage.to_device(h->ws2x, host, n1 * sizeof(double), h->stream, h->device));
-    HIPCHK(h->stage.to_device(h->ws2y, host + n1, n1 * sizeof(double), h->stream, h->device));
+    // the new speeds become the end of the coming step, the previous end its
+    // start; on their way they wait in memory of their own, so that a thread
+    // which enqueues steps meanwhile does not write over them
+    HIPCHK(h->stage.to_device(h->wnew, host, 2 * n1 * sizeof(double), h->stream, h->device));
     hipLaunchKernelGGL(k_wind_shift, dim3(nb((long)n1)), dim3(256), 0, h->stream, (long)n1, h->wu0, h->wv0, h->wu1,
-                       h->wv1, (const double*)h->ws2x, (const double*)h->ws2y, (double*)g.wsx, (double*)g.wsy);
+                       h->wv1, (const double*)h->wnew, (const double*)(h->wnew + n1), (double*)g.wsx, (double*)g.wsy);
     HIPCHK(hipGetLastError());
     if (varies) {
       // the captured step gains the per-external-step stress kernel
