@@ -1791,8 +1791,11 @@ int fvmlp_create(int64_t n, const float* x, const float* y, int32_t bmax, fvmlp*
     fvmlp_destroy(t);
     return 1;
   }
-  if (t->stage.to_device(t->X, x, (size_t)n * MLP_IN * sizeof(float), t->stream, t->device) != hipSuccess ||
-      t->stage.to_device(t->Y, y, (size_t)n * MLP_OUT * sizeof(float), t->stream, t->device) != hipSuccess) {
+  // directly: the staging's large buffer would be pinned for two copies
+  // (400,000 samples, trainer made: 0.90 ms through it, 0.62 directly)
+  if (hipMemcpyAsync(t->X, x, (size_t)n * MLP_IN * sizeof(float), hipMemcpyHostToDevice, t->stream) != hipSuccess ||
+      hipMemcpyAsync(t->Y, y, (size_t)n * MLP_OUT * sizeof(float), hipMemcpyHostToDevice, t->stream) != hipSuccess ||
+      hipStreamSynchronize(t->stream) != hipSuccess) {
     fvmlp_destroy(t);
     return fail("fvmlp_create: copying the samples");
   }
