@@ -1411,23 +1411,24 @@ int ens_update(fvgpu_handle* h, const char* name, int32_t nrens, const int64_t* 
     }
     stage = h->ens_buf;
   }
-  double* dx5 = stage;
-  long* doff = (long*)(stage + FV_ENS_MAX * FV_ENS_MAX);
+  // X5, then the offsets: nrens*(nrens + 1) words of the staging
   static_assert(sizeof(long) == sizeof(double), "offsets are staged beside X5");
   double up[FV_ENS_MAX * FV_ENS_MAX + FV_ENS_MAX];
-  std::memcpy(up, x5, (size_t)nrens * nrens * sizeof(double));
+  const size_t nx = (size_t)nrens * nrens;
+  std::memcpy(up, x5, nx * sizeof(double));
   for (int i = 0; i < nrens; ++i) {
     const long o = (long)off[i];
-    std::memcpy(&up[FV_ENS_MAX * FV_ENS_MAX + i], &o, sizeof(o));
+    std::memcpy(&up[nx + i], &o, sizeof(o));
   }
-  HIPCHK(h->stage.to_device(stage, up, (size_t)(FV_ENS_MAX * FV_ENS_MAX + nrens) * sizeof(double), h->stream,
-                            h->device));
+  HIPCHK(h->stage.to_device(stage, up, (nx + nrens) * sizeof(double), h->stream, h->device));
+  const double* dx5 = stage;
+  const long* doff = (const long*)(stage + nx);
   const long total = (long)len * nl;
   // persistent blocks: two per CU (the 65 KB of LDS each allows two)
   const long ntiles = (total + FV_ENS_TILE - 1) / FV_ENS_TILE;
   const unsigned blocks = (unsigned)std::max(1L, std::min(ntiles, 2L * std::max(h->cu_count, 1)));
-  hipLaunchKernelGGL(k_ens_update, dim3(blocks), dim3(256), 0, h->stream, arr, (const long*)doff, (long)len,
-                     (long)ls, nl, (int)nrens, (const double*)dx5);
+  hipLaunchKernelGGL(k_ens_update, dim3(blocks), dim3(256), 0, h->stream, arr, doff, (long)len,
+                     (long)ls, nl, (int)nrens, dx5);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
   return 0;
