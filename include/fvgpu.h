@@ -385,7 +385,9 @@ int  fvgpu_synchronize(fvgpu_handle* h);
 int  fvgpu_stream_copy(fvgpu_handle* h, int64_t n, int32_t reps, double* avg_us);
 void fvgpu_destroy(fvgpu_handle* h);
 
-/* Workgroup size (64, 128 or 256) of one kernel family of the step.      */
+/* Workgroup size (64, 128 or 256) of one kernel family of the step, as
+ * fvgpu_autotune reports them; a family whose workgroups have a fixed size
+ * keeps it.                                                              */
 int  fvgpu_set_block(fvgpu_handle* h, const char* family, int32_t block);
 /* Concurrency of the step's independent chains: 0..3 are accepted and have
  * no effect any more.  The T and S passes, and the advection of Q2 and Q2L,
@@ -393,9 +395,9 @@ int  fvgpu_set_block(fvgpu_handle* h, const char* family, int32_t block);
  * each kernel family's timing is always its own.  No counterpart in the
  * reference.                                                              */
 int  fvgpu_set_concurrency(fvgpu_handle* h, int32_t mode);
-/* Autotuner: times every kernel family of the step with workgroups of 64,
- * 128 and 256 (`steps` internal steps per candidate), keeps the fastest,
- * and restores the model state afterwards.  `report` receives
+/* Autotuner: times every kernel family of the step that has a choice with
+ * workgroups of 64, 128 and 256 (`steps` internal steps per candidate),
+ * keeps the fastest, and restores the model state afterwards.  `report` receives
  * "family=size:time;..." (may be NULL).                                  */
 int  fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_len);
 

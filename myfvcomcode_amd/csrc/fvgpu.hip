@@ -1907,7 +1907,7 @@ int fvgpu_set_concurrency(fvgpu_handle* h, int32_t mode) {
 
 int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_len) {
   static const char* fams[] = {"adv_ts", "adv_q", "viscofh", "vdif_q", "vdif_ts", "adjust1_brough", "adjust2", "baropg",
-                               "copy", "closure_features", "closure_apply"};
+                               "step_end", "closure_features", "closure_apply"};
   static const int cands[] = {64, 128, 256};
   if (steps < 1) return fail("autotune needs at least one step per candidate");
   // save the state; every candidate runs real steps
@@ -1929,6 +1929,8 @@ int fvgpu_autotune(fvgpu_handle* h, int32_t steps, char* report, int64_t report_
   std::string rep;
   int rc = 0;
   for (const char* f : fams) {
+    // VDIF_Q by block of columns has one workgroup size
+    if (!std::strcmp(f, "vdif_q") && vdif_q_blocks(h, h->closure_mode == 1)) continue;
     double best = 1e30;
     int bestc = 256;
     bool seen = false;
