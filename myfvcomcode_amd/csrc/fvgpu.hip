@@ -1078,7 +1078,7 @@ int upload_grid(fvgpu_handle* h) {
   UP(dltxnec, md->nring_ve); UP(dltynec, md->nring_ve);
   UP(xc, n1); UP(yc, n1); UP(art, n1); UP(h1, n1); UP(cor, n1); UP(cc_hvc, n1); UP(cc_sponge, n1);
   UP(cc_z0b, n1); UP(grav_e, n1); UP(epor, n1); UP(isbce, n1); UP(iucp, n1);
-  UP(nv, 3 * n1); UP(nbe, 3 * n1); UP(a1u, 4 * n1); UP(a2u, 4 * n1); UP(awx, 3 * n1); UP(awy, 3 * n1);
+  UP(nv, 3 * n1); UP(nbe, 3 * n1); UP(awx, 3 * n1); UP(awy, 3 * n1);
   {
     std::vector<double> a12(8 * n1);
     for (size_t e = 0; e < n1; ++e)
@@ -1097,13 +1097,11 @@ int upload_grid(fvgpu_handle* h) {
   if (p.type_tsobc == 4)
     for (size_t k = 0; k < ob; ++k)
       if (md->next_obc2[k] <= 0) return fail("TYPE_TSOBC 4 needs NEXT_OBC2 for every OBC node");
-  g.obc_radiate = 0;
   g.obc_ore = 0;
   for (size_t k = 0; k < ob; ++k) {
-    if (md->type_obc[k] >= 5) g.obc_radiate = 1;
     if (md->type_obc[k] >= 9) g.obc_ore = 1;
   }
-  UP(i_obc_n, ob); UP(next_obc, ob); UP(nadjc_obc, ob); UP(adjc_obc, 2 * ob); UP(fluxf_obc, 2 * ob);
+  UP(i_obc_n, ob); UP(next_obc, ob); UP(fluxf_obc, 2 * ob);
   UP(type_obc, ob); UP(next_obc2, ob);
   UP(dltn_obc, ob); UP(emean, ob); UP(apt, ob * nt); UP(phai, ob * nt); UP(period, nt);
   for (size_t k = 0; k < nr; ++k)

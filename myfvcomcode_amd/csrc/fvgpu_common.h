@@ -83,7 +83,7 @@ struct DevGrid {
   const double *xc, *yc, *art, *h1, *cor, *cc_hvc, *cc_sponge, *cc_z0b, *grav_e, *epor;
   const double *sin_alpha, *cos_alpha, *wsx, *wsy;
   const int *isbce, *iucp, *nv, *nbe;
-  const double *a1u, *a2u, *awx, *awy;
+  const double *awx, *awy;
   const double* a12;               // A1U(e,1..4), A2U(e,1..4) of element e at 8e..8e+7 (64-byte aligned)
   // edges and CV sub-edges
   const int *iec, *ienode, *isbc, *niec, *ntrg;
@@ -139,9 +139,7 @@ struct DevGrid {
   // consecutive elements for ADV_UV.
   UvBlocks ub_tile, ub_run;
   // OBC / tide / rivers
-  const int *i_obc_n, *next_obc, *nadjc_obc, *adjc_obc, *type_obc;
-  const int *next_obc2;
-  int obc_radiate;                 // some OBC node has TYPE_OBC 5..10
+  const int *i_obc_n, *next_obc, *type_obc, *next_obc2;
   int obc_ore;                     // some OBC node has TYPE_OBC 9/10 (Orlanski)
   double* fobn;                    // the OBC nodes' flux defects where k_ext_fobn forms them, else null
   const double *fluxf_obc, *dltn_obc, *emean, *apt, *phai, *period;
@@ -215,8 +213,6 @@ __device__ __forceinline__ double sige_u(const DevGrid& g, const double* a, int 
 #define ZZ1(i, k) sige_u<UNI>(g, g.zz1, i, k)
 #define NV_(i, j) g.nv[(long)((j)-1) * g.n1 + (i)]
 #define NBE_(i, j) g.nbe[(long)((j)-1) * g.n1 + (i)]
-#define A1U_(i, j) g.a1u[(long)((j)-1) * g.n1 + (i)]
-#define A2U_(i, j) g.a2u[(long)((j)-1) * g.n1 + (i)]
 #define AWX_(i, j) g.awx[(long)((j)-1) * g.n1 + (i)]
 #define AWY_(i, j) g.awy[(long)((j)-1) * g.n1 + (i)]
 #define IEC_(e, j) g.iec[(long)((j)-1) * (g.NE + 1) + (e)]
