@@ -922,16 +922,18 @@ int build_lists(fvgpu_handle* h) {
       if (dupload(h, &g.nt_elems, telems.data(), telems.size())) return 1;
       if (dupload(h, &g.nt_lpos, tlpos.data(), tlpos.size())) return 1;
     }
-    std::vector<int> keep(M + 1, 0);
+    std::vector<int> keep(M + 1, -1);
     for (int i = 0; i < md->iobcn; ++i) {
       const int j = md->i_obc_n[i];
-      keep[j] = 1;
+      keep[j] = 0;
       for (int q = off[j]; q < off[j + 1]; ++q) {
         const int c = ent[q] >> 1;
-        keep[md->niec[c]] = 1;
-        keep[md->niec[(size_t)(NCV + 1) + c]] = 1;
+        keep[md->niec[c]] = 0;
+        keep[md->niec[(size_t)(NCV + 1) + c]] = 0;
       }
     }
+    for (int& k : keep)
+      if (k == 0) k = g.nkeep++;
     if (dupload(h, &g.cvb_nn, bnn.data(), bnn.size())) return 1;
     if (dupload(h, &g.cvb_nodes, bnodes.data(), bnodes.size())) return 1;
     for (int i = 1; i <= M; ++i)
@@ -1209,10 +1211,11 @@ int upload_state(fvgpu_handle* h) {
   RW(viscofh, nullptr, mk);
   RW(gx, nullptr, mk);
   // flux buffers sized for FP64 (the mixed form uses the first half)
+  const size_t nrec = m1 + (size_t)g.nkeep * g.KBM1;
   {
     CvRecT<double>* pr = nullptr;
     double* pc = nullptr;
-    if (dalloc(h, &pr, mk)) return 1;
+    if (dalloc(h, &pr, nrec)) return 1;
     if (dalloc(h, &pc, ((size_t)g.NCV + 1) * g.KB)) return 1;
     a.rec = pr; a.cvflux = pc;
   }
@@ -1246,7 +1249,7 @@ int upload_state(fvgpu_handle* h) {
   {
     CvRecT<double>* pr = nullptr;
     double* pc = nullptr;
-    if (dalloc(h, &pr, mk)) return 1;
+    if (dalloc(h, &pr, nrec)) return 1;
     if (dalloc(h, &pc, ((size_t)g.NCV + 1) * g.KB)) return 1;
     b.rec = pr; b.cvflux = pc;
   }

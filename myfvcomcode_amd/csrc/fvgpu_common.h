@@ -116,9 +116,12 @@ struct DevGrid {
   // the cvb_ne[b] (<= FV_CVB) elements cvb_elems[FV_CVB*b + t] and the
   // cvb_nn[b] (<= FV_CVB) distinct nodes they use, cvb_nodes[FV_CVB*b + t];
   // cvb_loc[e] packs the local indices of NV(e,1..3) in bits 0-7, 8-15,
-  // 16-23.  rec_keep[i] = 1 for the nodes whose records other kernels read
-  // at every layer (the OBC nodes and the other ends of their sub-edges).
-  int cvb_nblk;
+  // 16-23.  The nodes whose records other kernels read at every layer (the
+  // OBC nodes and the other ends of their sub-edges) are numbered 0 .. nkeep-1
+  // in rec_keep[i], -1 at the others.  A pass's records (Pass::rec): node i's
+  // of the bottom layer at i, that of number q at layer k at
+  // m1 + (k-1)*nkeep + q.
+  int cvb_nblk, nkeep;
   const int *cvb_nn, *cvb_nodes, *cvb_ne, *cvb_elems, *cvb_loc, *rec_keep;
   // The block's nodes and the nodes of their rings: cvr_nn[b] (<= FV_CVH)
   // distinct, cvr_nodes[FV_CVH*b + q], the block's own first and in the order

@@ -27,7 +27,7 @@ struct IntArgs {
   double* gx;            // node-layer scratch (PROD of VDIF_Q)
   double *elm1, *elm2;   // the elevation one and two RK stages back (Orlanski OBC)
   // flux buffers, of the flux type FT (double, or float in the mixed form)
-  void* rec;             // node-layer records of the field being advected, CvRecT<FT>
+  void* rec;             // records of the field being advected that other kernels read, CvRecT<FT>
   double2* vhpair;       // node-layer pair scratch: VDIF_Q's elimination coefficients
   void* cvflux;          // per sub-edge, per layer face flux (NCV+1) x KB FT
   // 2-D

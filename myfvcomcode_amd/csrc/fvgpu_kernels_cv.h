@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a, Passes
   const int obc = act ? (int)(t % g.IOBCN) : 0, k = act ? (int)(t / g.IOBCN) + 1 : 1;
   const int i = g.i_obc_n[obc];
   const int n = act ? g.cv_cnt[i] : 0;
-  const long ko = (long)(k - 1) * g.m1, eo = (long)(k - 1) * g.n1;
+  const long eo = (long)(k - 1) * g.n1, ro = g.m1 + (long)(k - 1) * g.nkeep;
   if (lane < n) {
     const int e = g.cv_ent[g.cv_off[i] + lane], c = e >> 1;
     const int ia = NIEC_(c, 1), ib = NIEC_(c, 2), i1 = g.ntrg[c];
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a, Passes
     const FT visc0 = (FT)(g.fm1 * 0.5 * (g.nn_hvc[ia] + g.nn_hvc[ib]));
     const CvFace<FT> r = cv_face<FT>(un, dtij, dltx, dlty, (FT)DLTXNCVE_(c, 1), (FT)DLTYNCVE_(c, 1),
                                      (FT)DLTXNCVE_(c, 2), (FT)DLTYNCVE_(c, 2), (FT)g.fact, visc0,
-                                     rec[ko + ia], rec[ko + ib]);
+                                     rec[ro + g.rec_keep[ia]], rec[ro + g.rec_keep[ib]]);
     const double adv = (double)(r.exflux - r.fxx - r.fyy);
     sadv[threadIdx.x] = (e & 1) ? -adv : adv;
   }
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256) void k_adv_ts_gather(DevGrid g, IntArgs a, Pas
       xflux = xflux + flip_sign((double)xv[j], ce[j]);
     });
     if (k == g.KBM1) {  // ADV_T and ADV_S both set the bottom-gradient terms VDIF_TS reads
-      const CvRecT<FT> r = ((const CvRecT<FT>*)ps.rec)[ko + i];
+      const CvRecT<FT> r = ((const CvRecT<FT>*)ps.rec)[i];
       ps.pfpxb[i] = (double)r.gx;
       ps.pfpyb[i] = (double)r.gy;
       ps.ah_bottom[i] = (g.fact * a.viscofh[ko + i] + g.fm1) * g.nn_hvc[i];
@@ -386,10 +386,9 @@ struct CvRecLds {
 // at the block's nodes and their rings (cvr_*) into LDS; one barrier per
 // layer hands the two buffers of either kind over.  The two roles hold only
 // their own registers and run side by side.  A node shared by two blocks is
-// formed by both; the records cross HBM only for the nodes whose records
-// other kernels read (rec_keep: OBC nodes and their sub-edge neighbours)
-// and, for the tracer, at the bottom layer (the bottom gradients of
-// VDIF_TS).
+// formed by both; the records cross HBM only for the tracer, at the nodes
+// whose records other kernels read (rec_keep: OBC nodes and their sub-edge
+// neighbours) and at the bottom layer (the bottom gradients of VDIF_TS).
 //
 // Bound: the vector memory unit and its latency.  A record read straight
 // from memory takes up to 20 scattered loads a lane, of which two layers
@@ -433,7 +432,7 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, Passes 
       rw[w] = w < g.cvr_w ? g.cvr_loc[((long)b * g.cvr_w + w) * FV_CVB + t] : 0;
     });
     const double art2 = g.art2[i], nnv = g.nn_hvc[i];
-    const bool keep = nact && g.rec_keep[i] != 0;
+    const int keep = nact ? g.rec_keep[i] : -1;
     // VISCOFH a layer ahead
     double vhn = at(a.viscofh + (long)(k0 - 1) * g.m1, i), vhm = 0.0;
     if (KIND == 1) vhm = at(a.viscofh + (long)(k0 - 2) * g.m1, i);
@@ -462,7 +461,8 @@ __global__ __launch_bounds__(256) void k_cvrecflux(DevGrid g, IntArgs a, Passes 
         if (nact) {
           const CvRecT<FT> r = cv_record<KIND, RMAX, FT, UNI>(g, i, rg, art2, nnv, L, cmean, k);
           srec[s & 1].put(t, r);
-          if (keep || (KIND == 0 && k == g.KBM1)) rec[(long)(k - 1) * g.m1 + i] = r;
+          if (KIND == 0 && keep >= 0) rec[g.m1 + (long)(k - 1) * g.nkeep + keep] = r;
+          if (KIND == 0 && k == g.KBM1) rec[i] = r;
         }
       }
       __syncthreads();
