@@ -107,6 +107,7 @@ struct fvgpu_handle {
   IntArgs ib{};           // ia with its own scratch, for the second of two passes
   double* phi[2] = {};    // per sub-edge EXTEL terms of a 2-D stage's input and output, element-major
   double* elrk = nullptr; // the RK base elevation of stages 2-4
+  int stage_odd = 0;      // the 2-D stage's tables are not as the grid builder makes them (k_ext_stage's ODD)
   double* own2d = nullptr;   // block-order constants of the external steps (ExtArgs::own2d)
   ExtClock* ec = nullptr; // clocks of the external steps (ISPLIT of them, at least one)
   double* ens_buf = nullptr;  // X5 and member offsets of fvgpu_ensemble_update
@@ -352,8 +353,11 @@ void enqueue_external_step_t(fvgpu_handle* h, int iext, const ExtClock* ec) {
   for (int K = 1; K <= 4; ++K) {
     ExtArgs a = make_ext_args(h, K, *cur[K], *nxt[K], ec);
     if (g.fobn) LAUNCH("ext_fobn", k_ext_fobn, nb(g.IOBCN), 256, h->dg, a);
-#define EXT_STAGE_CALL(SM) LAUNCH("ext_momentum", (k_ext_stage<SM, FT, false>), g.ub_tile.nblk, 256, h->dg, a)
-    FV_SMAX_DISPATCH(g.cv_max, EXT_STAGE_CALL);
+#define EXT_STAGE_CALL(SM) LAUNCH("ext_momentum", (k_ext_stage<SM, FT, false, false>), g.ub_tile.nblk, 256, h->dg, a)
+    if (h->stage_odd)
+      LAUNCH("ext_momentum", (k_ext_stage<FV_MAX_CV, FT, false, true>), g.ub_tile.nblk, 256, h->dg, a);
+    else
+      FV_SMAX_DISPATCH(g.cv_max, EXT_STAGE_CALL);
     if (g.obc_ore) LAUNCH("elm_shift", k_elm_shift, nb(g.M + 1), 256, g, a);
   }
 }
@@ -438,7 +442,8 @@ void enqueue_internal_step_t(fvgpu_handle* h) {
   if (!h->md->p.barotropic) TLAUNCH("rho1_roundtrip", k_rho1_roundtrip, (long)g.KBM1 * g.m1, g, a);
   {
     ExtArgs e = make_ext_args(h, 0, h->ext[0], h->ext[0], nullptr);
-    LAUNCH("advave_int", (k_ext_stage<16, FT, true>), g.ub_tile.nblk, 256, h->dg, e);
+    if (h->stage_odd) LAUNCH("advave_int", (k_ext_stage<16, FT, true, true>), g.ub_tile.nblk, 256, h->dg, e);
+    else LAUNCH("advave_int", (k_ext_stage<16, FT, true, false>), g.ub_tile.nblk, 256, h->dg, e);
   }
   for (int iext = 1; iext <= g.isplit; ++iext) enqueue_external_step_t<FT>(h, iext, h->ec + (iext - 1));
 #define ADJ2_CALL(KM) TLAUNCH("adjust2", (k_adjust2<KM, UN>), g.N + 1, g, a)
@@ -637,6 +642,9 @@ int build_lists(fvgpu_handle* h) {
     far = far || (md->nv[e] != j && md->nv[(size_t)N + 1 + e] != j && md->nv[2 * ((size_t)N + 1) + e] != j);
   }
   if (far && dalloc(h, &g.fobn, (size_t)IOBCN)) return 1;
+  h->stage_odd = far;
+  for (int c = 1; c <= NE; ++c)
+    if (md->isbc[c] < 0 || md->isbc[c] > 2) h->stage_odd = 1;
   // CSR over elements 0..N of (element, entry) pairs, each element's entries in their order
   auto element_csr = [&](std::vector<std::pair<int, int>>& v, std::vector<int>& off, std::vector<int>& ent_) {
     std::stable_sort(v.begin(), v.end(), [](const auto& p, const auto& q) { return p.first < q.first; });
@@ -663,6 +671,8 @@ int build_lists(fvgpu_handle* h) {
     for (int q = 0; q < 2; ++q)
       if (nd[q] > 0) { nriv[nd[q]] = j; skip[nd[q]] = 1; }
   }
+  for (int i = 0; i < IOBCN; ++i)
+    if (md->type_obc[i] >= 5 && md->type_obc[i] <= 8 && nobc[md->next_obc[i]] >= 0) h->stage_odd = 1;
   if (dupload(h, &g.node_obc, nobc.data(), nobc.size())) return 1;
   if (dupload(h, &g.node_riv, nriv.data(), nriv.size())) return 1;
   if (dupload(h, &g.fct_skip, skip.data(), skip.size())) return 1;

@@ -40,7 +40,7 @@ struct UvBlocks {
 //                    another element, INT_MIN for a pad
 //   edge[256*b + t]  the record slots of IA and IB in bits 0-7 and 8-15, the
 //                    node slots of IENODE in bits 16-22 and 23-29, ISBC in
-//                    bits 30-31 (3: not 0..2, read it); all ones for a pad
+//                    bits 30-31 (3: not 0..2); all ones for a pad
 //   egeo[(6*b + q)*256 + t]  XIJC-XC and YIJC-YC of IA, the same of IB,
 //                    DLTXC, DLTYC
 //   node[FV_CVB*b + t]  {2*node + 1 in the first block that has it, 0, OBC

@@ -366,6 +366,12 @@ __global__ __launch_bounds__(256) void k_stage_tables(DevGrid g, StageTab st, co
 // (internal_step.F:387-392) instead of a stage: ADX2D/ADY2D -= the sums, the
 // accumulators of the coming external steps set to zero
 // (internal_step.F:395-397) and the first stage's sub-edge terms formed.
+//
+// ODD: for tables that a host has set otherwise than the grid builder does
+// (fvgpu_handle::stage_odd) -- ISBC outside 0..2, a radiating node whose
+// NEXT_OBC is an OBC node, an ADJC_OBC without its node.  A kernel of its own:
+// in the others' code the three cost 1 % of a 3,200-element step (515.4 us,
+// 510.6 without).
 template <typename FT>
 struct ExtRecsLds {   // one array per quantity: a wave's reads of one spread over the banks
   FT u[256], v[256], c1[256], c2[256], c5[256], c6[256], p[256], cc[256];
@@ -377,7 +383,7 @@ struct ExtFluxLds {
   int isbc[256];
 };
 
-template <int SMAX, typename FT, bool INT>
+template <int SMAX, typename FT, bool INT, bool ODD>
 __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ gp, ExtArgs a) {
   const DevGrid& g = *gp;   // in device memory, for the boundary parts: by value its pointers
                             // overflow the scalar registers
@@ -460,23 +466,25 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
       if (keep && a.elrk_copy) a.elrk_copy[j] = elrk;
       const int ty = obc >= 0 ? g.type_obc[obc] : 0;
       // GWI / BKI need their neighbour's new elevation: a second pass forms
-      // it, as the tile that has that node does.  The grid's NEXT_OBC are
-      // interior nodes; one that a host has set to an OBC node of TYPE_OBC
-      // 1..4 enters with its given elevation.
+      // it, as the tile that has that node does (ODD: an OBC node of TYPE_OBC
+      // 1..4 with its given elevation)
       double elf = 0.0, el2 = 0.0, xobc = 0.0;
-      int id = j, rv = nd.w, ob = obc;
+      int id = j, rv = nd.w;
       double ar = art1, er = elrk;
       if (n0)
         static_for<SMAX>([&](auto jc) { ce[decltype(jc)::value] = 0; });
       for (bool next = false;;) {
         double xo;
+        const int ob = ODD && next ? g.node_obc[id] : next ? -1 : obc;
         const double e = ext_node_update<SMAX>(g, a, id, ce, rv, ob >= 0, ar, er, xo);
-        if (next) { el2 = e; break; }
+        if (next) {
+          el2 = ODD && ob >= 0 && g.type_obc[ob] < 5 ? ext_obc_given(g, a, ob, g.type_obc[ob], er, e) : e;
+          break;
+        }
         elf = e;
         xobc = xo;
         if (ty < 5 || ty > 8) break;
         id = g.next_obc[obc];
-        ob = g.node_obc[id];
         static_for<SMAX>([&](auto jc) {
           constexpr int q = decltype(jc)::value;
           ce[q] = q < st.nslot ? g.cvl_ent[(long)q * g.m1 + id] : 0;
@@ -486,16 +494,7 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
         next = true;
       }
       if (obc >= 0) {
-        // the given elevation: the node's own, or that of the neighbour which
-        // it radiates from
-        const bool own = ty < 5;
-        const int ty2 = own ? ty : ob >= 0 ? g.type_obc[ob] : 5;
-        if (ty2 < 5) {
-          const double e = ext_obc_given(g, a, ob, ty2, er, own ? elf : el2);
-          if (own) elf = e;
-          else el2 = e;
-        }
-        if (!own) elf = ext_obc_radiated(g, a, j, obc, ty, elrk, el2);
+        elf = ty < 5 ? ext_obc_given(g, a, obc, ty, elrk, elf) : ext_obc_radiated(g, a, j, obc, ty, elrk, el2);
         // FLUX_OBN's flux defect (mod_obcs.F:1196) and, in the last stage,
         // the node's UARD_OBCN share (external_step.F:423-430)
         if (nact) s_fobn[tn] = -(elf - elrk) * art1 / (a.alpha * g.dte) - xobc;
@@ -562,8 +561,7 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     sf.elij[t] = 0.5 * (s_el[n1] + s_el[n2]);
     sf.dlx[t] = eg[4];
     sf.dly[t] = eg[5];
-    const int isbc = (int)(pl >> 30);
-    sf.isbc[t] = isbc < 3 ? isbc : g.isbc[g.ub_tile.edges[256L * b + t]];
+    sf.isbc[t] = ODD ? g.isbc[g.ub_tile.edges[256L * b + t]] : (int)(pl >> 30);
   }
   __syncthreads();
   if (!oact) return;
@@ -577,9 +575,9 @@ __global__ __launch_bounds__(256) void k_ext_stage(const DevGrid* __restrict__ g
     } else {
       for (int p = g.fo_off[i]; p < g.fo_off[i + 1]; ++p) {
         const int ent = g.fo_obc[p], ob = ent >> 1, slot = ent & 1;
-        const int j = g.i_obc_n[ob];   // one of the element's nodes, or g.fobn has it
+        const int j = g.i_obc_n[ob];   // one of the element's nodes (ODD: or g.fobn has it)
         const int ln = j == NV_(i, 1) ? nl & 255 : j == NV_(i, 2) ? (nl >> 8) & 255 : (nl >> 16) & 255;
-        fl = fl + g.fluxf_obc[(long)slot * g.IOBCN + ob] * (g.fobn ? g.fobn[ob] : s_fobn[ln]);
+        fl = fl + g.fluxf_obc[(long)slot * g.IOBCN + ob] * (ODD && g.fobn ? g.fobn[ob] : s_fobn[ln]);
       }
       a.fluxobn[i] = fl;
     }
