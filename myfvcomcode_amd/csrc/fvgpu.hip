@@ -603,8 +603,6 @@ int build_lists(fvgpu_handle* h) {
     g.ring_max = std::max(g.ring_max, md->ntsn[i]);
     g.ve_max = std::max(g.ve_max, md->ntve[i]);
   }
-  if (dupload(h, &g.cv_off, off.data(), off.size())) return 1;
-  if (dupload(h, &g.cv_ent, ent.data(), ent.size())) return 1;
   {
     int smax = 0;
     for (int i = 0; i <= M; ++i) smax = std::max(smax, cnt[i]);
@@ -944,6 +942,16 @@ int build_lists(fvgpu_handle* h) {
     }
     for (int& k : keep)
       if (k == 0) k = g.nkeep++;
+    std::vector<int4> osub((size_t)md->iobcn * g.cv_max, int4{-1, 0, 0, 0});
+    for (int i = 0; i < md->iobcn; ++i) {
+      const int j = md->i_obc_n[i];
+      for (int q = off[j]; q < off[j + 1]; ++q) {
+        const int c = ent[q] >> 1;
+        osub[(size_t)i * g.cv_max + (q - off[j])] =
+            int4{ent[q], md->ntrg[c], keep[md->niec[c]], keep[md->niec[(size_t)(NCV + 1) + c]]};
+      }
+    }
+    if (dupload(h, &g.obc_sub, osub.data(), osub.size())) return 1;
     if (dupload(h, &g.cvb_nn, bnn.data(), bnn.size())) return 1;
     if (dupload(h, &g.cvb_nodes, bnodes.data(), bnodes.size())) return 1;
     for (int i = 1; i <= M; ++i)
@@ -1102,7 +1110,7 @@ int upload_grid(fvgpu_handle* h) {
   }
   const size_t ne1 = md->ne + 1, cv1 = md->ncv + 1;
   UP(iec, 2 * ne1); UP(ienode, 2 * ne1); UP(isbc, ne1); UP(xijc, ne1); UP(yijc, ne1); UP(dltxc, ne1); UP(dltyc, ne1);
-  UP(niec, 2 * cv1); UP(ntrg, cv1); UP(dltxe, cv1); UP(dltye, cv1); UP(dltxncve, 2 * cv1); UP(dltyncve, 2 * cv1);
+  UP(niec, 2 * cv1); UP(dltxe, cv1); UP(dltye, cv1); UP(dltxncve, 2 * cv1); UP(dltyncve, 2 * cv1);
   const size_t ob = md->iobcn, nt = md->ntide, nr = md->numqbc;
   for (size_t k = 0; k < ob; ++k)
     if (md->type_obc[k] < 1 || md->type_obc[k] > 10) return fail("TYPE_OBC must be 1..10");

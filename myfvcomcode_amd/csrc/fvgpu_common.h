@@ -86,16 +86,16 @@ struct DevGrid {
   const double *awx, *awy;
   const double* a12;               // A1U(e,1..4), A2U(e,1..4) of element e at 8e..8e+7 (64-byte aligned)
   // edges and CV sub-edges
-  const int *iec, *ienode, *isbc, *niec, *ntrg;
+  const int *iec, *ienode, *isbc, *niec;
   const double *xijc, *yijc, *dltxc, *dltyc, *dltxe, *dltye, *dltxncve, *dltyncve;
   // sigma (per column, or one column for all: nsk ..)
   const double *z, *zz, *dz, *dzz, *z1, *zz1, *dz1, *dzz1;
   // gather lists
-  const int *cv_off, *cv_ent;      // node -> (cv<<1 | side), sorted by cv
-  // the same lists slot-major (entry j of node i at j*m1+i, j < cv_cnt[i]):
-  // consecutive nodes read consecutive addresses for each slot.  cvl_ent
-  // holds (p<<1 | side), p the element-major position of the sub-edge's
-  // flux in the per-layer flux buffers (below).
+  // node -> control-volume sub-edges in increasing order, slot-major (entry j
+  // of node i at j*m1+i, j < cv_cnt[i]): consecutive nodes read consecutive
+  // addresses for each slot.  cvl_ent holds (p<<1 | side), p the
+  // element-major position of the sub-edge's flux in the per-layer flux
+  // buffers (below).
   int cv_max;
   int ring_max, ve_max;            // max NTSN, max NTVE
   const int *cv_cnt, *cvl_ent;
@@ -120,9 +120,11 @@ struct DevGrid {
   // OBC nodes and the other ends of their sub-edges) are numbered 0 .. nkeep-1
   // in rec_keep[i], -1 at the others.  A pass's records (Pass::rec): node i's
   // of the bottom layer at i, that of number q at layer k at
-  // m1 + (k-1)*nkeep + q.
+  // m1 + (k-1)*nkeep + q.  obc_sub[cv_max*n + j]: sub-edge j of OBC node n
+  // (2*sub-edge + side, its NTRG, the numbers of its nodes IA and IB), or -1.
   int cvb_nblk, nkeep;
   const int *cvb_nn, *cvb_nodes, *cvb_ne, *cvb_elems, *cvb_loc, *rec_keep;
+  const int4* obc_sub;
   // The block's nodes and the nodes of their rings: cvr_nn[b] (<= FV_CVH)
   // distinct, cvr_nodes[FV_CVH*b + q], the block's own first and in the order
   // of cvb_nodes.  Byte j%4 of cvr_loc[(cvr_w*b + j/4)*FV_CVB + t] is the

@@ -241,21 +241,20 @@ __global__ __launch_bounds__(256) void k_adv_ts_obc(DevGrid g, IntArgs a, Passes
   const bool act = t < (long)g.IOBCN * g.KBM1;
   const CvRecT<FT>* rec = (const CvRecT<FT>*)ps.rec;
   const int obc = act ? (int)(t % g.IOBCN) : 0, k = act ? (int)(t / g.IOBCN) + 1 : 1;
-  const int i = g.i_obc_n[obc];
-  const int n = act ? g.cv_cnt[i] : 0;
+  const int4 sub = act && lane < g.cv_max ? g.obc_sub[(long)obc * g.cv_max + lane] : make_int4(-1, 0, 0, 0);
+  const int n = act ? g.cv_cnt[g.i_obc_n[obc]] : 0;
   const long eo = (long)(k - 1) * g.n1, ro = g.m1 + (long)(k - 1) * g.nkeep;
-  if (lane < n) {
-    const int e = g.cv_ent[g.cv_off[i] + lane], c = e >> 1;
-    const int ia = NIEC_(c, 1), ib = NIEC_(c, 2), i1 = g.ntrg[c];
+  if (sub.x >= 0) {
+    const int c = sub.x >> 1, i1 = sub.y, ia = NIEC_(c, 1), ib = NIEC_(c, 2);
     const FT dltx = (FT)g.dltxe[c], dlty = (FT)g.dltye[c];
     const FT dtij = (FT)(a.dt1[i1] * DZ1(i1, k));
     const FT un = (FT)a.v[eo + i1] * dltx - (FT)a.u[eo + i1] * dlty;
     const FT visc0 = (FT)(g.fm1 * 0.5 * (g.nn_hvc[ia] + g.nn_hvc[ib]));
     const CvFace<FT> r = cv_face<FT>(un, dtij, dltx, dlty, (FT)DLTXNCVE_(c, 1), (FT)DLTYNCVE_(c, 1),
                                      (FT)DLTXNCVE_(c, 2), (FT)DLTYNCVE_(c, 2), (FT)g.fact, visc0,
-                                     rec[ro + g.rec_keep[ia]], rec[ro + g.rec_keep[ib]]);
+                                     rec[ro + sub.z], rec[ro + sub.w]);
     const double adv = (double)(r.exflux - r.fxx - r.fyy);
-    sadv[threadIdx.x] = (e & 1) ? -adv : adv;
+    sadv[threadIdx.x] = (sub.x & 1) ? -adv : adv;
   }
   __syncthreads();
   if (!act || lane != 0) return;
