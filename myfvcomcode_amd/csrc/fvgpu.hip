@@ -1770,7 +1770,7 @@ int malloc_mlp(fvmlp* t, T** p, size_t n) {
 // the first B: its gradient and loss into G, and with step >= 1 the AdamW
 // step.
 int mlp_batch(fvmlp* t, const int* didx, MlpDraw draw, int B, int step, float lr, float wd) {
-  const int blocks = std::min((B + MLP_GRP - 1) / MLP_GRP, MLP_BLOCKS);
+  const int blocks = std::min(B / MLP_GRP + (B % MLP_GRP != 0), MLP_BLOCKS);
   hipLaunchKernelGGL(k_mlp_batch, dim3(blocks), dim3(256), 0, t->stream, t->P, t->X, t->Y, didx, draw, B, t->part);
   hipLaunchKernelGGL(k_mlp_update, dim3((MLP_PART + 31) / 32), dim3(256), 0, t->stream, t->part, blocks, t->G, t->P,
                      t->Mo, t->Ve, step, lr, wd, 0.9f, 0.999f, 1e-8f);

@@ -171,9 +171,9 @@ __global__ __launch_bounds__(256) void k_mlp_batch(const float* __restrict__ P, 
   const float b3 = P[MLP_OFF_B3 + (t & 1)];
   mlp_f32x4 gW2[4] = {}, gW1 = {}, gB2 = {}, gW3 = {};
   float lacc = 0.0f, dacc = 0.0f;
-  for (int g0 = blockIdx.x * MLP_GRP; g0 < B; g0 += gridDim.x * MLP_GRP) {
+  for (long g0 = (long)blockIdx.x * MLP_GRP; g0 < B; g0 += (long)gridDim.x * MLP_GRP) {
     if (t < MLP_GRP) {
-      const int b = g0 + t;
+      const long b = g0 + t;
       float4 xa = make_float4(0.f, 0.f, 0.f, 0.f);
       float x4 = 0.0f;
       float2 y = make_float2(1.f, 1.f);
