@@ -11,7 +11,7 @@ survey pass (eager launches) with HIP events around every launch gives each kern
 ("roofline_by_kernel") and the dominant family; the timed region then runs
 K steps launched eagerly, the state resident in HBM, and HIP events around
 one in four of the dominant family's launches (events around every launch
-cost about 0.46 ms of a 23.3 ms step), whose average device time is the
+cost about 0.3 ms of an 18.8 ms step), whose average device time is the
 "roofline" figure.  The same step replayed as one hipGraph per step is
 timed among the variants.  The CPU baseline is the serial FP64 oracle on a
 bounded sample of the same workload (the same generator at 251x126 nodes,

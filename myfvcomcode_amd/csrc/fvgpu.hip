@@ -15,8 +15,8 @@
 //    the fourth stage written in place over the RK base (pointwise reads
 //    only), so the state returns to fixed buffers after every external step
 //    and one internal step can be captured as a replayable hipGraph;
-//  * time-dependent scalars (RAMP, ExtTime) live in a device clock updated
-//    by single-thread kernels, never by host writes between launches.
+//  * time-dependent scalars (RAMP, ExtTime) live in a device clock that a
+//    kernel of one workgroup updates, never host writes between launches.
 #include "fvgpu_closure.h"
 #include "fvgpu_stage.h"
 #include "../../include/fvgpu.h"
@@ -269,15 +269,17 @@ int block_of(const fvgpu_handle* h, const char* name) {
 // extent) whose layers are independent of one another, given its workgroups
 // per layer: so many that about `per_cu` workgroups a CU are in the grid -- a
 // mesh with fewer leaves CUs idle while each of its lanes walks the column
-// alone -- but at least 2 layers a share, over which a lane's constants and
-// lists are read once.  3 is what the registers of these kernels let a CU
-// hold: more measured slower (62,500 elements x 40 layers, one graph a step:
-// 2.14 ms unsplit, 1.94 at 3, 1.96 at 6, 2.02 at 12; 250,000 x 20: 3.28,
-// 3.27, 3.28, 3.35; from 768 workgroups a layer on, nothing is split and
-// nothing changes), but for ADV_UV, whose grid is the most uneven, 6 (62,500
-// elements: 161 us unsplit, 137 at 3, 130 at 6), and so for the records and
-// face fluxes of two fields (62,500: 129 us at 3, 121 at 6).  adv_ts at 17,000 elements x
-// 20: 52 -> 17 us, at 62,500 x 40: 101 -> 48 us.
+// alone -- but at most n/2, since a lane's constants and lists are read once
+// over its share (layer_share: two layers or more, the last share excepted).
+// From per_cu workgroups a CU on (on 256 CUs 768 at 3, 1,536 at 6) nothing is
+// split and nothing changes.
+// 3 is what the registers of these kernels let a CU hold: more measured slower
+// (62,500 elements x 40 layers, one graph a step: 2.14 ms unsplit, 1.94 at 3,
+// 1.96 at 6, 2.02 at 12; 250,000 x 20: 3.28, 3.27, 3.28, 3.35), but for ADV_UV,
+// whose grid is the most uneven, 6 (62,500 elements: 161 us unsplit, 137 at 3,
+// 130 at 6), and so for the records and face fluxes of two fields (62,500: 129
+// us at 3, 121 at 6).  adv_ts at 17,000 elements x 20: 52 -> 17 us, at 62,500 x
+// 40: 101 -> 48 us.
 unsigned layer_chunks(const fvgpu_handle* h, long workgroups, int n, int per_cu) {
   const long want = ((long)per_cu * h->cu_count + workgroups - 1) / std::max(workgroups, 1l);
   return (unsigned)std::max(1l, std::min(want, (long)n / 2));
@@ -545,7 +547,9 @@ int build_lists(fvgpu_handle* h) {
   const fv_model* md = h->md;
   const int M = md->m, N = md->n, NE = md->ne, NCV = md->ncv;
   DevGrid& g = h->g;
-  // per-layer byte offsets of entities and flux positions are 32-bit (at())
+  // per-layer byte offsets of entities and flux positions are 32-bit (at()).
+  // The limit is 179 million elements, whose smallest state (3 layers, 2.9 KB an
+  // element) is 520 GB: no mesh that the card holds meets it.
   if (8ll * std::max<long long>({(long long)M + 1, (long long)N + 1, (long long)NCV + 1}) >= (1ll << 32))
     return fail("the mesh exceeds 32-bit byte offsets per layer");
   // node -> CV sub-edges sorted by sub-edge index

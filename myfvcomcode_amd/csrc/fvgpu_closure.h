@@ -142,7 +142,8 @@ typedef float mlp_f32x4 __attribute__((ext_vector_type(4)));
 #define MLP_LCG_C 1442695040888963407ull
 struct MlpDraw { unsigned long long state; long n; };
 
-// The LCG's state `steps` steps on (composition by doubling).
+// The LCG's state `steps` steps on, by composing its step with itself and
+// doubling (Brown, Random number generation with arbitrary strides, 1994).
 __host__ __device__ inline unsigned long long mlp_lcg_skip(unsigned long long st, unsigned long long steps) {
   unsigned long long a = MLP_LCG_A, c = MLP_LCG_C;
   for (; steps; steps >>= 1) {

@@ -395,8 +395,8 @@ struct CvRecLds {
 // and its rings are about 115 nodes, so that a layer is 2 coalesced loads a
 // lane of the face waves, a layer ahead, and a record's values are LDS reads.
 // 1,000,000 elements x 40 layers: FP64 tracer 1164 -> 911 us a field
-// (two in one launch 1730: 4.6 GB, 2.7 TB/s), q2 1087 -> 890; FP32 fluxes, tracer
-// 985 -> 706, q2 689 (with records
+// (two in one launch 1730: 4.6 GB, 2.7 TB/s), q2 1087 -> 890 (two 1570); FP32
+// fluxes, tracer 985 -> 706, q2 689 (with records
 // and fluxes in two launches through HBM: 357 + 466).  Exchanging the roles of
 // the waves in every second workgroup (the record waves take twice the
 // instructions of the face waves) changed nothing.
