@@ -767,25 +767,21 @@ int build_lists(fvgpu_handle* h) {
     int stamp = 0;
     // the elements' edges, and they with the other elements of those edges,
     // number at most 256 each (the blocked momentum kernels)
-    std::vector<int> emark(N + 1, -1), cmark(NE + 1, -1);
+    // (an edge between two of them is met from both, any other once)
+    std::vector<int> emark(N + 1, -1);
     auto tile_fits = [&](int lo, int hi) {
-      ++stamp;
-      int nr = 0, nc = 0;
-      for (int q = lo; q < hi; ++q) {
-        const int e = ids[q];
-        if (emark[e] != stamp) { emark[e] = stamp; ++nr; }
+      const int own = stamp += 2, other = own - 1;
+      int nr = hi - lo, inner = 0, outer = 0;
+      for (int q = lo; q < hi; ++q) emark[ids[q]] = own;
+      for (int q = lo; q < hi; ++q)
         for (int j = 0; j < 3; ++j) {
-          const int c = ed[3 * (size_t)e + j] >> 1;
-          if (cmark[c] == stamp) continue;
-          cmark[c] = stamp;
-          ++nc;
-          for (int side = 0; side < 2; ++side) {
-            const int x = md->iec[(size_t)side * (NE + 1) + c];
-            if (emark[x] != stamp) { emark[x] = stamp; ++nr; }
-          }
+          const int en = ed[3 * (size_t)ids[q] + j];
+          const int x = md->iec[(en & 1 ? 0 : (size_t)(NE + 1)) + (en >> 1)];
+          if (emark[x] == own) { ++inner; continue; }
+          ++outer;
+          if (emark[x] != other) { emark[x] = other; ++nr; }
         }
-      }
-      return nr <= 256 && nc <= 256;
+      return nr <= 256 && inner / 2 + outer <= 256;
     };
     // a block's tables; false if its nodes, or they with the nodes of their
     // rings, are too many
